@@ -459,6 +459,7 @@ __global__ __launch_bounds__(256) void varlen_k_stream_kernel(const VarlenKParam
   const i32x4 g_rsrc = make_buffer_resource(p.gidx, (uint32_t)(p.total_rows * 4));
   const uint32_t lds_p = smem_base, lds_q = smem_base + 2 * 32768;
   ki32x8 state = {}, next = {}, geo = {};
+  ki32x16 tok = {};  // the gather indices of the gathered stream's next stage, from one statement to the next
   {
     int32_t ps, qs;
     first_offsets(cur, ps, qs);
@@ -474,11 +475,12 @@ __global__ __launch_bounds__(256) void varlen_k_stream_kernel(const VarlenKParam
   geo[SMOE_MM_LDSQ] = (int32_t)lds_q;
   geo[SMOE_MM_WLDS] = wave * (NINSTR * 1024);
   if constexpr (SG) {
-    SMOE_TILE_PROLOGUE_MM_QG(pra, qra, pv, qv, p_rsrc, q_rsrc, state, pvn, qvn, half, g_rsrc, next, geo);
+    SMOE_TILE_PROLOGUE_MM_QG(pra, qra, pv, qv, p_rsrc, q_rsrc, state, tok, pvn, qvn, half, g_rsrc, next, geo);
   } else {
-    SMOE_TILE_PROLOGUE_MM_PG(pra, qra, pv, qv, p_rsrc, q_rsrc, state, pvn, qvn, half, g_rsrc, next, geo);
+    SMOE_TILE_PROLOGUE_MM_PG(pra, qra, pv, qv, p_rsrc, q_rsrc, state, tok, pvn, qvn, half, g_rsrc, next, geo);
   }
   uniform(state);
+  uniform(tok);
   uniform(p_rsrc);
   uniform(q_rsrc);
   // the prologue has requested one token-side stage and two weight-side stages of the first tile
@@ -500,12 +502,13 @@ __global__ __launch_bounds__(256) void varlen_k_stream_kernel(const VarlenKParam
     next[SMOE_MM_RLEFTN] = nxt.row_end - (nxt.row_begin + wave * 16);
     next[SMOE_MM_SNEXT] = stages_of(nxt);
     if constexpr (SG) {
-      SMOE_TILE_LOOP_MM_QG(pra, qra, pv, qv, p_rsrc, q_rsrc, state, pvn, qvn, half, g_rsrc, next, geo);
+      SMOE_TILE_LOOP_MM_QG(pra, qra, pv, qv, p_rsrc, q_rsrc, state, tok, pvn, qvn, half, g_rsrc, next, geo);
     } else {
-      SMOE_TILE_LOOP_MM_PG(pra, qra, pv, qv, p_rsrc, q_rsrc, state, pvn, qvn, half, g_rsrc, next, geo);
+      SMOE_TILE_LOOP_MM_PG(pra, qra, pv, qv, p_rsrc, q_rsrc, state, tok, pvn, qvn, half, g_rsrc, next, geo);
     }
     // (the compiler takes the scalar results of an assembly statement for per-lane values; say that they are uniform)
     uniform(state);
+    uniform(tok);
     uniform(p_rsrc);
     uniform(q_rsrc);
     // both streams are on nxt now; their next tile is the one after it

@@ -620,7 +620,7 @@ def mm_emit_tile(gp: bool, gq: bool) -> list[str]:
     em(f"s_sub_u32 s{MS_DQ}, 0, s{MS_QCUR}")
     for line in mm_move_read_addresses():
         em(line)
-    # the index run requested behind the last loads must not land in registers the compiler owns again
+    # the index run requested behind the last loads has landed before the statement hands it out (operand "tok")
     em("s_waitcnt lgkmcnt(0)")
     em("s_nop 15")
     em("s_nop 7")
@@ -631,7 +631,7 @@ def mm_operands():
     outs = [
         (vrange(MV_PRA, 2 * FM), "pra"), (vrange(MV_QRA, 2 * FN), "qra"), (vrange(MV_PV, P_INSTR), "pv"),
         (vrange(MV_QV, Q_INSTR), "qv"), (srange(MS_PRSRC, 4), "prsrc"), (srange(MS_QRSRC, 4), "qrsrc"),
-        (srange(MS_ST, 8), "state"),
+        (srange(MS_ST, 8), "state"), (srange(MS_TOK, RPW), "tok"),
     ]
     ins = [
         (vrange(MV_PVN, P_INSTR), "pvn"), (vrange(MV_QVN, Q_INSTR), "qvn"), (vrange(MV_HALF, 1), "half"),
@@ -651,7 +651,7 @@ def mm_statement(name: str, lines: list[str], with_matrix: bool) -> str:
     clob = [f"v{i}" for i in range(MV_T, MV_T + 2)]
     if with_matrix:
         clob += [f"v{i}" for i in range(0, 128)] + [f"a{i}" for i in range(256)]
-    clob += [f"s{i}" for i in range(MS_PCUR, MS_A1 + 1)] + [f"s{i}" for i in range(MS_TOK, MS_TOK + 16)]
+    clob += [f"s{i}" for i in range(MS_PCUR, MS_A1 + 1)]
     clob += ["scc", "memory"]
     params = ", ".join(n for _, n in outs + ins)
     body = [f"#define {name}({params}) \\", "  asm volatile( \\"]
@@ -675,8 +675,7 @@ def mm_layout_defines() -> list[str]:
     return [f"#define SMOE_MM_{k} {v}" for k, v in names.items()]
 
 
-def statement(name: str, qmn: bool) -> str:
-    lines = emit_tile(qmn)
+def tile_operands(qmn: bool):
     nq = n_qoff(qmn)
     outs = [
         (vrange(V_PV, P_INSTR), "pv"), (vrange(V_QV, Q_INSTR), "qv"), (srange(S_QRSRC, 4), "qrsrc"),
@@ -690,6 +689,13 @@ def statement(name: str, qmn: bool) -> str:
         (srange(S_NMID, 1), "nmid"), (srange(S_LDSP, 1), "ldsp"), (srange(S_LDSQ, 1), "ldsq"),
         (srange(S_WLDS, 1), "wlds"),
     ]
+    return outs, ins
+
+
+def statement(name: str, qmn: bool) -> str:
+    lines = emit_tile(qmn)
+    nq = n_qoff(qmn)
+    outs, ins = tile_operands(qmn)
     clob = [f"v{i}" for i in range(0, 128)]
     clob += [f"v{i}" for i in range(V_PRA, V_PRA + 2)]
     clob += [f"v{i}" for i in range(V_QRA, V_QRA + nq)]

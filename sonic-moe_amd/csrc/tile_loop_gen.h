@@ -1673,7 +1673,7 @@
 #define SMOE_MM_LDSP 3
 #define SMOE_MM_LDSQ 4
 #define SMOE_MM_WLDS 5
-#define SMOE_TILE_PROLOGUE_MM_QG(pra, qra, pv, qv, prsrc, qrsrc, state, pvn, qvn, half, grsrc, next, geo) \
+#define SMOE_TILE_PROLOGUE_MM_QG(pra, qra, pv, qv, prsrc, qrsrc, state, tok, pvn, qvn, half, grsrc, next, geo) \
   asm volatile( \
     "s_add_u32 s62, s55, s57\n\t" \
     "s_add_u32 s62, s62, 32768\n\t" \
@@ -1914,12 +1914,11 @@
     "s_buffer_load_dwordx16 s[72:87], s[32:35], s37\n\t" \
     "s_add_u32 s37, s37, 256\n\t" \
     "s_waitcnt vmcnt(0) lgkmcnt(0)\n\t" \
-    : "+{v[160:175]}"(pra), "+{v[176:191]}"(qra), "+{v[128:135]}"(pv), "+{v[136:143]}"(qv), "+{s[24:27]}"(prsrc), "+{s[28:31]}"(qrsrc), "+{s[36:43]}"(state) \
+    : "+{v[160:175]}"(pra), "+{v[176:191]}"(qra), "+{v[128:135]}"(pv), "+{v[136:143]}"(qv), "+{s[24:27]}"(prsrc), "+{s[28:31]}"(qrsrc), "+{s[36:43]}"(state), "+{s[72:87]}"(tok) \
     : "{v[144:151]}"(pvn), "{v[152:159]}"(qvn), "{v194}"(half), "{s[32:35]}"(grsrc), "{s[44:51]}"(next), "{s[52:59]}"(geo) \
-    : "v192", "v193", "s60", "s61", "s62", "s63", "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", "s72", "s73", \
-      "s74", "s75", "s76", "s77", "s78", "s79", "s80", "s81", "s82", "s83", "s84", "s85", "s86", "s87", "scc", "memory")
+    : "v192", "v193", "s60", "s61", "s62", "s63", "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", "scc", "memory")
 
-#define SMOE_TILE_LOOP_MM_QG(pra, qra, pv, qv, prsrc, qrsrc, state, pvn, qvn, half, grsrc, next, geo) \
+#define SMOE_TILE_LOOP_MM_QG(pra, qra, pv, qv, prsrc, qrsrc, state, tok, pvn, qvn, half, grsrc, next, geo) \
   asm volatile( \
     "s_barrier\n\t" \
     "s_add_u32 s62, s41, s57\n\t" \
@@ -3140,7 +3139,7 @@
     "s_waitcnt lgkmcnt(0)\n\t" \
     "s_nop 15\n\t" \
     "s_nop 7\n\t" \
-    : "+{v[160:175]}"(pra), "+{v[176:191]}"(qra), "+{v[128:135]}"(pv), "+{v[136:143]}"(qv), "+{s[24:27]}"(prsrc), "+{s[28:31]}"(qrsrc), "+{s[36:43]}"(state) \
+    : "+{v[160:175]}"(pra), "+{v[176:191]}"(qra), "+{v[128:135]}"(pv), "+{v[136:143]}"(qv), "+{s[24:27]}"(prsrc), "+{s[28:31]}"(qrsrc), "+{s[36:43]}"(state), "+{s[72:87]}"(tok) \
     : "{v[144:151]}"(pvn), "{v[152:159]}"(qvn), "{v194}"(half), "{s[32:35]}"(grsrc), "{s[44:51]}"(next), "{s[52:59]}"(geo) \
     : "v192", "v193", "v0", "v1", "v2", "v3", "v4", "v5", "v6", "v7", "v8", "v9", "v10", "v11", "v12", "v13", \
       "v14", "v15", "v16", "v17", "v18", "v19", "v20", "v21", "v22", "v23", "v24", "v25", "v26", "v27", "v28", "v29", \
@@ -3166,10 +3165,9 @@
       "a206", "a207", "a208", "a209", "a210", "a211", "a212", "a213", "a214", "a215", "a216", "a217", "a218", "a219", "a220", "a221", \
       "a222", "a223", "a224", "a225", "a226", "a227", "a228", "a229", "a230", "a231", "a232", "a233", "a234", "a235", "a236", "a237", \
       "a238", "a239", "a240", "a241", "a242", "a243", "a244", "a245", "a246", "a247", "a248", "a249", "a250", "a251", "a252", "a253", \
-      "a254", "a255", "s60", "s61", "s62", "s63", "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", "s72", "s73", \
-      "s74", "s75", "s76", "s77", "s78", "s79", "s80", "s81", "s82", "s83", "s84", "s85", "s86", "s87", "scc", "memory")
+      "a254", "a255", "s60", "s61", "s62", "s63", "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", "scc", "memory")
 
-#define SMOE_TILE_PROLOGUE_MM_PG(pra, qra, pv, qv, prsrc, qrsrc, state, pvn, qvn, half, grsrc, next, geo) \
+#define SMOE_TILE_PROLOGUE_MM_PG(pra, qra, pv, qv, prsrc, qrsrc, state, tok, pvn, qvn, half, grsrc, next, geo) \
   asm volatile( \
     "s_buffer_load_dwordx16 s[72:87], s[32:35], s36\n\t" \
     "s_add_u32 s36, s36, 256\n\t" \
@@ -3332,12 +3330,11 @@
     "buffer_load_dwordx4 v143, s[28:31], s37 offen lds\n\t" \
     "s_add_u32 s37, s37, s53\n\t" \
     "s_waitcnt vmcnt(0) lgkmcnt(0)\n\t" \
-    : "+{v[160:175]}"(pra), "+{v[176:191]}"(qra), "+{v[128:135]}"(pv), "+{v[136:143]}"(qv), "+{s[24:27]}"(prsrc), "+{s[28:31]}"(qrsrc), "+{s[36:43]}"(state) \
+    : "+{v[160:175]}"(pra), "+{v[176:191]}"(qra), "+{v[128:135]}"(pv), "+{v[136:143]}"(qv), "+{s[24:27]}"(prsrc), "+{s[28:31]}"(qrsrc), "+{s[36:43]}"(state), "+{s[72:87]}"(tok) \
     : "{v[144:151]}"(pvn), "{v[152:159]}"(qvn), "{v194}"(half), "{s[32:35]}"(grsrc), "{s[44:51]}"(next), "{s[52:59]}"(geo) \
-    : "v192", "v193", "s60", "s61", "s62", "s63", "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", "s72", "s73", \
-      "s74", "s75", "s76", "s77", "s78", "s79", "s80", "s81", "s82", "s83", "s84", "s85", "s86", "s87", "scc", "memory")
+    : "v192", "v193", "s60", "s61", "s62", "s63", "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", "scc", "memory")
 
-#define SMOE_TILE_LOOP_MM_PG(pra, qra, pv, qv, prsrc, qrsrc, state, pvn, qvn, half, grsrc, next, geo) \
+#define SMOE_TILE_LOOP_MM_PG(pra, qra, pv, qv, prsrc, qrsrc, state, tok, pvn, qvn, half, grsrc, next, geo) \
   asm volatile( \
     "s_barrier\n\t" \
     "s_add_u32 s62, s41, s57\n\t" \
@@ -4558,7 +4555,7 @@
     "s_waitcnt lgkmcnt(0)\n\t" \
     "s_nop 15\n\t" \
     "s_nop 7\n\t" \
-    : "+{v[160:175]}"(pra), "+{v[176:191]}"(qra), "+{v[128:135]}"(pv), "+{v[136:143]}"(qv), "+{s[24:27]}"(prsrc), "+{s[28:31]}"(qrsrc), "+{s[36:43]}"(state) \
+    : "+{v[160:175]}"(pra), "+{v[176:191]}"(qra), "+{v[128:135]}"(pv), "+{v[136:143]}"(qv), "+{s[24:27]}"(prsrc), "+{s[28:31]}"(qrsrc), "+{s[36:43]}"(state), "+{s[72:87]}"(tok) \
     : "{v[144:151]}"(pvn), "{v[152:159]}"(qvn), "{v194}"(half), "{s[32:35]}"(grsrc), "{s[44:51]}"(next), "{s[52:59]}"(geo) \
     : "v192", "v193", "v0", "v1", "v2", "v3", "v4", "v5", "v6", "v7", "v8", "v9", "v10", "v11", "v12", "v13", \
       "v14", "v15", "v16", "v17", "v18", "v19", "v20", "v21", "v22", "v23", "v24", "v25", "v26", "v27", "v28", "v29", \
@@ -4584,5 +4581,4 @@
       "a206", "a207", "a208", "a209", "a210", "a211", "a212", "a213", "a214", "a215", "a216", "a217", "a218", "a219", "a220", "a221", \
       "a222", "a223", "a224", "a225", "a226", "a227", "a228", "a229", "a230", "a231", "a232", "a233", "a234", "a235", "a236", "a237", \
       "a238", "a239", "a240", "a241", "a242", "a243", "a244", "a245", "a246", "a247", "a248", "a249", "a250", "a251", "a252", "a253", \
-      "a254", "a255", "s60", "s61", "s62", "s63", "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", "s72", "s73", \
-      "s74", "s75", "s76", "s77", "s78", "s79", "s80", "s81", "s82", "s83", "s84", "s85", "s86", "s87", "scc", "memory")
+      "a254", "a255", "s60", "s61", "s62", "s63", "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", "scc", "memory")

@@ -270,6 +270,23 @@ def _sval(w: Wave, tok: str) -> int:
     return int(tok, 0)
 
 
+def scramble_compiler_registers(w, operands) -> None:
+    """Between two statements the compiler owns every register that is not an operand: whatever a statement left in one
+    (it may have declared it clobbered) is gone when the next one starts."""
+    kept = set()
+    for reg, _ in operands[0] + operands[1]:
+        m = re.fullmatch(r"([sv])(?:(\d+)|\[(\d+):(\d+)\])", reg)
+        lo, hi = (m[2], m[2]) if m[2] else (m[3], m[4])
+        kept |= {(m[1], r) for r in range(int(lo), int(hi) + 1)}
+    for r in range(102):
+        if ("s", r) not in kept:
+            w.s[r] = 0x5bad0000 + r
+    for r in range(256):
+        if ("v", r) not in kept:
+            w.v[r] = 0x7bad0000 + r
+            w.vt[r] = -1
+
+
 def run_wave(w: Wave, lines: list[str]):
     """generator: executes the statement for one wave, yields at every barrier"""
     labels = {ln[:-1]: i for i, ln in enumerate(lines) if ln.endswith(":")}
@@ -519,6 +536,7 @@ def simulate(prob: Problem, lds_base: int = 0) -> dict:
         for w in waves:
             w.tile = tile
             w.acc_seen = {}
+            scramble_compiler_registers(w, G.tile_operands(prob.qmn))
         gens = [run_wave(w, lines) for w in waves]
         alive = [True] * G.NW
         while any(alive):
@@ -684,6 +702,7 @@ def simulate_mm(prob: ProblemMM) -> dict:
             w.acc_seen = {}
             w.s[G.MS_NMID] = stages(tile) - 2
             set_next(w, nxt)
+            scramble_compiler_registers(w, G.mm_operands())
         gens = [run_wave(w, lines) for w in waves]
         alive = [True] * G.NW
         while any(alive):
