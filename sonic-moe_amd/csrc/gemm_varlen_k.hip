@@ -298,51 +298,40 @@ __global__ __launch_bounds__(C::NT) void varlen_k_kernel(const VarlenKParams p) 
 
 
 // ---- the same GEMM on the hand-scheduled loop, as a stream of tiles ---------------------------------------------------
-// Schedule.  The 32 tiles an XCD's 32 workgroups run side by side are one block (BA_T x BB_T tiles) of ONE expert's
-// output, as in the blocked order above - so all of them have the same length (the expert's token count) and a
-// persistent workgroup that takes tile i of every block of its XCD is balanced against its 31 neighbours by
-// construction.  Across the XCDs the blocks are dealt by cost: experts sorted by token count, largest first (or in the
-// caller's expert_schedule_order), their blocks laid out in that order and dealt to the XCDs in snake order
-// 0..7, 7..0, so every XCD gets one of the larger and one of the smaller blocks of each run of 16.  No queue, no
-// atomics: the table is built by one small kernel per launch and every workgroup knows its next tiles in advance,
-// which is what lets the load streams of the loop run across tile boundaries.
-//   table: int32 count[8] (rounds per XCD), then block[8][max_rounds] (block id = expert * blocks_per_expert + block)
+// Schedule.  The tiles an XCD's 32 workgroups run side by side form one UNIT.  Experts are sorted by token count, largest
+// first (or taken in the caller's expert_schedule_order), their tiles laid out in that order, and the units of that
+// sequence dealt to the XCDs in snake order 0..7, 7..0, so every XCD gets one of the larger and one of the smaller units
+// of each run of 16.  Two kinds of unit:
+//   blocks  (nb > 0) 32 tiles = ba x bb tiles of ONE expert's output, where the output splits into such blocks: all 32
+//           workgroups run the same number of stages and share ba + bb operand panels in the XCD's L2;
+//   chunks  (nb == 0) `chunk` consecutive tiles of the sequence, across expert borders: for outputs of a few tiles per
+//           expert or of ragged tile counts.  Neighbours in the sorted order have nearly the same length, and a workgroup
+//           walks its chunks alternately from the front and from the back, so the longer experts at the front do not pile
+//           up on the same workgroups.  Launches of less than 256 tiles use shorter chunks and so all eight XCDs.
+//           Against the eight-wavefront kernel, one tile per workgroup, that such outputs ran on before: H = 768,
+//           I = 256, E = 128, 2560 rows per expert (12 and 6 tiles per expert) dW1 297 -> 212 us = 1216 TFLOP/s, dW2
+//           179 -> 130; H = 1536, I = 256, 375 rows per expert dW1 123 -> 96, dW2 64 -> 56.
+// No queue, no atomics: one small kernel per launch sorts the experts, everything else is arithmetic on the round number,
+// and every workgroup knows its next tiles in advance, which is what lets the load streams of the loop run across tile
+// boundaries.
 constexpr int SCHED_MAX_E = 4096;
 
-static inline size_t block_schedule_bytes(int64_t blocks_total) {
-  return (size_t)(8 + 8 * ((blocks_total + 7) / 8 + 1)) * sizeof(int32_t);
-}
-
-__global__ __launch_bounds__(1024) void build_block_schedule_kernel(const int32_t* __restrict__ off,
-                                                                    const int32_t* __restrict__ order, int E, int nb,
-                                                                    int max_rounds, int32_t* __restrict__ table) {
+__global__ __launch_bounds__(1024) void sort_experts_kernel(const int32_t* __restrict__ off,
+                                                            const int32_t* __restrict__ order, int E,
+                                                            int32_t* __restrict__ sorted) {
   __shared__ int32_t cost[SCHED_MAX_E];
   const int tid = threadIdx.x;
   for (int e = tid; e < E; e += 1024) cost[e] = off[e + 1] - off[e];
   __syncthreads();
-  const int64_t total = (int64_t)E * nb;
   for (int e = tid; e < E; e += 1024) {
-    int pos = 0;  // position of expert e in the schedule order
     if (order != nullptr) {
-      for (int i = 0; i < E; i++) pos = order[i] == e ? i : pos;
+      sorted[e] = order[e];
     } else {
+      int pos = 0;
       const int c = cost[e];
       for (int o = 0; o < E; o++) pos += (cost[o] > c || (cost[o] == c && o < e)) ? 1 : 0;
+      sorted[pos] = e;
     }
-    for (int j = 0; j < nb; j++) {
-      const int64_t seq = (int64_t)pos * nb + j;
-      const int r = (int)(seq & 15);
-      const int x = r < 8 ? r : 15 - r;
-      const int64_t round = 2 * (seq >> 4) + (r >= 8 ? 1 : 0);
-      table[8 + (int64_t)x * max_rounds + round] = e * nb + j;
-    }
-  }
-  if (tid < 8) {
-    const int rem = (int)(total & 15);
-    int n = (int)(2 * (total >> 4));
-    if (tid < (rem < 8 ? rem : 8)) n += 1;
-    if (rem > 8 && tid > 15 - rem) n += 1;
-    table[tid] = n;
   }
 }
 
@@ -355,13 +344,15 @@ __global__ __launch_bounds__(1024) void build_block_schedule_kernel(const int32_
 typedef int32_t ki32x8 __attribute__((ext_vector_type(8)));
 typedef int32_t ki32x16 __attribute__((ext_vector_type(16)));
 
-struct BlockShape {
-  int nb, nbj, ba, bb;  // blocks per expert, blocks along b, tiles per block along a / b
+struct UnitShape {
+  int nb, nbj, ba, bb;  // blocks per expert (0: the units are chunks), blocks along b, tiles per block along a / b
+  int chunk;            // tiles of a chunk, at most 32
+  int units;            // units of the launch
 };
 
 template <bool RG, bool SG>
-__global__ __launch_bounds__(256) void varlen_k_stream_kernel(const VarlenKParams p, const BlockShape bs,
-                                                              const int32_t* table, int max_rounds) {
+__global__ __launch_bounds__(256) void varlen_k_stream_kernel(const VarlenKParams p, const UnitShape us,
+                                                              const int32_t* sorted_experts) {
   static_assert(RG != SG, "exactly one operand is gathered");
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   typedef ElemMma Mma;
@@ -374,22 +365,36 @@ __global__ __launch_bounds__(256) void varlen_k_stream_kernel(const VarlenKParam
 
   typedef const __attribute__((address_space(4))) int32_t* const_i32_ptr;
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;  // workgroup b runs on XCD b % 8
-  const const_i32_ptr tab = (const_i32_ptr)table, off = (const_i32_ptr)p.off;
-  const int rounds = tab[xcd];
-  if (rounds == 0) return;
-  const const_i32_ptr blocks = tab + 8 + (int64_t)xcd * max_rounds;
+  const const_i32_ptr sorted = (const_i32_ptr)sorted_experts, off = (const_i32_ptr)p.off;
   struct Tile {
     int e, row_begin, row_end, a0, b0;
   };
-  // past the XCD's last round: an empty expert - every load out of range
+  auto unit_of = [&](int r) { return 16 * (r >> 1) + ((r & 1) ? 15 - xcd : xcd); };
+  auto chunk_tile = [&](int r) { return unit_of(r) * us.chunk + ((r & 1) ? us.chunk - 1 - slot : slot); };
+  const int rest = us.units & 15;
+  int rounds = 2 * (us.units >> 4) + (xcd < rest ? 1 : 0) + (rest > 8 && xcd > 15 - rest ? 1 : 0);
+  const int tiles_e = p.tiles_a * p.tiles_b;
+  if (us.nb == 0) {
+    if (slot >= us.chunk) return;
+    // the sequence's last chunk may be short; it is the last one its XCD works on
+    if (rounds > 0 && chunk_tile(rounds - 1) >= tiles_e * p.E) rounds--;
+  }
+  if (rounds == 0) return;
+  // past the workgroup's last round: an empty expert - every load out of range
   auto tile_at = [&](int r) {
     Tile t = {0, 0, 0, 0, 0};
     if (r < rounds) {
-      const int B = blocks[r];
-      t.e = B / bs.nb;
-      const int blk = B - t.e * bs.nb;
-      t.a0 = ((blk / bs.nbj) * bs.ba + slot / bs.bb) * BA;
-      t.b0 = ((blk % bs.nbj) * bs.bb + slot % bs.bb) * BB;
+      if (us.nb > 0) {
+        const int B = unit_of(r), pos = B / us.nb, blk = B - pos * us.nb;
+        t.e = sorted[pos];
+        t.a0 = ((blk / us.nbj) * us.ba + slot / us.bb) * BA;
+        t.b0 = ((blk % us.nbj) * us.bb + slot % us.bb) * BB;
+      } else {
+        const int v = chunk_tile(r), pos = v / tiles_e, within = v - pos * tiles_e;
+        t.e = sorted[pos];
+        t.a0 = (within / p.tiles_b) * BA;
+        t.b0 = (within % p.tiles_b) * BB;
+      }
       t.row_begin = off[t.e];
       t.row_end = off[t.e + 1];
     }
@@ -563,42 +568,48 @@ static int launch_varlen_k(const VarlenKParams& pin, hipStream_t st, void* works
   SMOE_REQUIRE(p.r_stride > 0 && p.r_stride < (1ll << 31) && p.s_stride > 0 && p.s_stride < (1ll << 31),
                SMOE_ERR_UNSUPPORTED, "weight-grad gemm: operand row stride out of range");
   if constexpr (C::R_GATHER != C::S_GATHER && C::BA == 256 && C::BB == 256) {
-    // The tile streams on the hand-scheduled loop: whole blocks of 32 tiles per expert, a schedule table in the
-    // workspace, and 32-bit byte offsets for both operands (the streams run a few stages past an expert's end before
-    // they stop; rows past the end are told by a wrapped offset).
+    // The tile streams on the hand-scheduled loop: the experts' order in the workspace, and 32-bit byte offsets for both
+    // operands (the streams run a few stages past an expert's end before they stop; rows past the end are told by a
+    // wrapped offset).
     const int64_t lim = (1ll << 32) - (1ll << 16);
     const int64_t r_rows = C::R_GATHER ? p.gather_rows : p.total_rows + 8 * C::BK;
     const int64_t s_rows = C::S_GATHER ? p.gather_rows : p.total_rows + 8 * C::BK;
     const bool fits = p.off != nullptr && p.gidx != nullptr && p.gather_rows > 0 && (r_rows + 1) * p.r_stride * 2 < lim &&
                       (s_rows + 1) * p.s_stride * 2 < lim && (p.total_rows + 8 * C::BK) * 4 < lim;
-    // a block is ba x bb tiles with ba * bb = 32, as square as the tile counts allow (fewest operand panels per block)
-    BlockShape bs = {0, 0, 0, 0};
-    bool whole_blocks = false;
-    for (int bb : {8, 4, 16, 2, 32, 1}) {
-      if (p.tiles_b % bb == 0 && p.tiles_a % (32 / bb) == 0) {
-        bs.bb = bb;
-        bs.ba = 32 / bb;
-        whole_blocks = true;
-        break;
+    // What a stream saves is the turnaround between the tiles of a workgroup and, per stage, the hand-scheduled loop; it
+    // costs a launch that sorts the experts.  With at most one tile per workgroup and short experts nothing of that is
+    // left (H = 512, I = 256, E = 8, 32 tiles: 256 rows per expert 12.7 us one-tile, 14.1 + 3.2 stream; 1024 rows 27.3 /
+    // 29.2; 4096 rows 85 / 77.  H = 768, E = 32, 192 tiles: 1024 rows 36 / 31, 4096 rows 144 / 103).
+    const bool long_enough = total > 256 || p.total_rows >= 1024ll * p.E;
+    if (tuning().gemm_asm && fits && long_enough && p.E <= SCHED_MAX_E && total < (1ll << 30) && workspace != nullptr &&
+        (size_t)p.E * sizeof(int32_t) <= workspace_bytes) {
+      // a block is ba x bb tiles with ba * bb = 32, as square as the tile counts allow (fewest operand panels per block)
+      UnitShape us = {0, 0, 0, 0, 0, 0};
+      if (total >= 256) {
+        for (int bb : {8, 4, 16, 2, 32, 1}) {
+          if (p.tiles_b % bb == 0 && p.tiles_a % (32 / bb) == 0) {
+            us.bb = bb;
+            us.ba = 32 / bb;
+            us.nbj = p.tiles_b / us.bb;
+            us.nb = (p.tiles_a / us.ba) * us.nbj;
+            us.units = us.nb * p.E;
+            break;
+          }
+        }
       }
-    }
-    if (tuning().gemm_asm && fits && whole_blocks && p.E <= SCHED_MAX_E && workspace != nullptr) {
-      bs.nbj = p.tiles_b / bs.bb;
-      bs.nb = (p.tiles_a / bs.ba) * bs.nbj;
-      const int64_t blocks_total = (int64_t)bs.nb * p.E;
-      if (block_schedule_bytes(blocks_total) <= workspace_bytes && blocks_total < (1ll << 30)) {
-        const int max_rounds = (int)((blocks_total + 7) / 8 + 1);
-        static LdsLimitOnce lds_limit_asm;
-        auto akern = varlen_k_stream_kernel<C::R_GATHER, C::S_GATHER>;
-        const int rc_a = lds_limit_asm.ensure((const void*)akern, 160 * 1024);
-        if (rc_a) return rc_a;
-        hipLaunchKernelGGL(build_block_schedule_kernel, dim3(1), dim3(1024), 0, st, p.off, p.order, p.E, bs.nb, max_rounds,
-                           (int32_t*)workspace);
-        SMOE_LAUNCH_CHECK();
-        hipLaunchKernelGGL(akern, dim3(256), dim3(256), 160 * 1024, st, p, bs, (const int32_t*)workspace, max_rounds);
-        SMOE_LAUNCH_CHECK();
-        return SMOE_OK;
+      if (us.nb == 0) {
+        us.chunk = total < 256 ? (int)ceil_div(total, 8) : 32;
+        us.units = (int)ceil_div(total, us.chunk);
       }
+      static LdsLimitOnce lds_limit_asm;
+      auto akern = varlen_k_stream_kernel<C::R_GATHER, C::S_GATHER>;
+      const int rc_a = lds_limit_asm.ensure((const void*)akern, 160 * 1024);
+      if (rc_a) return rc_a;
+      hipLaunchKernelGGL(sort_experts_kernel, dim3(1), dim3(1024), 0, st, p.off, p.order, p.E, (int32_t*)workspace);
+      SMOE_LAUNCH_CHECK();
+      hipLaunchKernelGGL(akern, dim3(256), dim3(256), 160 * 1024, st, p, us, (const int32_t*)workspace);
+      SMOE_LAUNCH_CHECK();
+      return SMOE_OK;
     }
   }
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(C::NT), C::SMEM, st, p);

@@ -322,6 +322,50 @@ def test_kernel_selection_knobs(dev, tuning, knob, value):
             assert torch.equal(a, b), name
 
 
+@pytest.mark.parametrize("T,H,I,E,K,skew,empty", [
+    (3100, 64, 64, 3, 1, 0.0, ()),           # one tile per expert, three tiles in all: chunks of one tile
+    (6000, 768, 256, 11, 2, 1.0, (4, 10)),   # 66 and 33 tiles: chunks shorter than 32
+    (2000, 768, 320, 43, 3, 1.2, (0, 42)),   # 387 and 258 tiles of ragged width: whole chunks and a short last one
+    (3000, 1472, 704, 16, 4, 0.5, (7,)),     # 36 and 18 tiles per expert
+])
+def test_weight_gradients_in_chunks(dev, tuning, T, H, I, E, K, skew, empty):
+    """Outputs that do not split into blocks of 32 tiles run as tile streams over chunks of tiles of several experts:
+    against the oracle (bf16 rounding of the stored result, as everywhere) and, bit for bit, against the one-tile kernel,
+    which adds the same products in the same order."""
+    _, bwd = _ops()
+    _, w1, w2 = make_weights(E, H, I, dev, seed=T)
+    idx, scores, meta, md = make_tc_routing(T, E, K, dev, seed=T + 1, skew=skew, empty=empty)
+    g = torch.Generator().manual_seed(T + 2)
+    TK = T * K
+    x, dout = (torch.randn(T, H, generator=g).to(torch.bfloat16).to(dev) for _ in range(2))
+    dz = torch.randn(TK, 2 * I, generator=g).to(torch.bfloat16).to(dev)
+    y1s = torch.randn(TK, I, generator=g).to(torch.bfloat16).to(dev)
+    s_flat = torch.from_numpy(scores).to(dev).view(-1)
+    off, gidx, sidx = (md[k] for k in ("expert_frequency_offset", "x_gather_idx", "s_scatter_idx"))
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def run():
+        dw1 = torch.full((E, 2 * I, H), 3.0, dtype=torch.bfloat16, device=dev)
+        dw2 = torch.full((E, H, I), 3.0, dtype=torch.bfloat16, device=dev)
+        bwd._up_projection_backward(x, w1.permute(1, 2, 0), None, dw1.permute(1, 2, 0), dz, None, off, None, gidx, sidx,
+                                    True, stream)
+        bwd._down_projection_weight_grad(dout, y1s, dw2.permute(1, 2, 0), None, s_flat, off, None, gidx, sidx, stream)
+        return dw1, dw2
+
+    dw1, dw2 = run()
+    for e in range(E):
+        lo, hi = int(off[e]), int(off[e + 1])
+        tok = gidx[lo:hi].long()
+        ref1, ref2 = dz[lo:hi].float().t() @ x[tok].float(), dout[tok].float().t() @ y1s[lo:hi].float()
+        if lo == hi:
+            assert not dw1[e].any() and not dw2[e].any()
+        else:
+            assert rel_l2(dw1[e], ref1) < TOL and rel_l2(dw2[e], ref2) < TOL, e
+    tuning("gemm_asm", 0)
+    for a, b in zip((dw1, dw2), run()):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("stream_kernels", [1, 0])
 @pytest.mark.parametrize("order_kind", ["reversed", "largest_first", "random"])
 def test_expert_schedule_order(dev, tuning, order_kind, stream_kernels):
