@@ -1279,6 +1279,7 @@ struct Tuning {
   int gemm_asm;             // 1: the tile streams run on the hand-scheduled four-wavefront loop (tile_loop_gen.h)
   int gemm_group_tiles;     // most token tiles of one expert that sweep the feature tiles together (tile streams)
   int gemm_group_snake;     // 1: consecutive groups of an expert sweep the feature tiles in opposite directions
+  int gemm_skinny_rows;     // most token rows per expert, on average, that take the skinny forward GEMM (0: none do)
 };
 const Tuning& tuning();
 
@@ -1389,6 +1390,25 @@ struct StreamTiles {
     return t;
   }
 };
+
+// ---- forward grouped GEMM for few token rows per expert (gemm_skinny.hip) ------------------------------------------
+struct SkinnyGemm {
+  const uint16_t* P;  // token operand, K-major; rows gathered by gidx, or the grouped rows themselves (gidx null)
+  int64_t p_stride, p_rows;
+  const int32_t* gidx;
+  const uint16_t* Q;  // weights, K-major
+  int64_t q_stride_e, q_stride_row;
+  const int32_t* off;
+  const uint16_t* bias;  // nullable
+  uint16_t* out0;        // z (nullable with an activation) resp. y2
+  int64_t out0_stride;
+  uint16_t* out1;  // y1, with an activation
+  int64_t out1_stride;
+  int N, Kdim, E;
+  bool first_blocks;  // set by the launcher: how the workgroups are dealt to the experts
+};
+bool skinny_gemm_takes(const SkinnyGemm& g, int64_t TK);
+int launch_skinny_gemm(const SkinnyGemm& g, int act, int64_t TK, hipStream_t st);  // act -1: no activation
 
 int launch_ds_finalize(const float* ds_partial, int ncols, const int32_t* sidx, float* ds, int64_t TK, hipStream_t st);
 

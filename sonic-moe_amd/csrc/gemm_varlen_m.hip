@@ -724,6 +724,26 @@ static bool offsets_fit32(const VarlenMParams& p, bool qmn, bool all_rows) {
 
 template <class C, int ROLE, int ACT>
 static int launch_varlen_m(VarlenMParams& p, const int32_t* off, void* workspace, int64_t TK, int E, hipStream_t st) {
+  if constexpr (!C::QMN && (ROLE == ROLE_UP_FWD || ROLE == ROLE_PLAIN)) {
+    SkinnyGemm g = {};
+    g.P = p.P;
+    g.p_stride = p.p_stride;
+    g.p_rows = p.gidx ? p.p_rows : TK;
+    g.gidx = p.gidx;
+    g.Q = p.Q;
+    g.q_stride_e = p.q_stride_e;
+    g.q_stride_row = p.q_stride_row;
+    g.off = off;
+    g.bias = p.bias;
+    g.out0 = p.out0;
+    g.out0_stride = p.out0_stride;
+    g.out1 = p.out1;
+    g.out1_stride = p.out1_stride;
+    g.N = p.N;
+    g.Kdim = p.Kdim;
+    g.E = E;
+    if (skinny_gemm_takes(g, TK)) return launch_skinny_gemm(g, ROLE == ROLE_UP_FWD ? ACT : -1, TK, st);
+  }
   static LdsLimitOnce lds_limit;
   auto kern = varlen_m_kernel<C, ROLE, ACT>;
   {
