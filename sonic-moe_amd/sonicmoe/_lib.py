@@ -149,4 +149,6 @@ def require_device(*tensors: torch.Tensor | None) -> None:
 
 
 def current_stream_handle() -> int:
+    if torch.cuda.is_initialized():  # the Stream object behind current_stream() costs several us
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
     return torch.cuda.current_stream().cuda_stream

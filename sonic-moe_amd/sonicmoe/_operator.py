@@ -1,0 +1,46 @@
+"""Operators of the `sonicmoe::` namespace and how the layer calls them.
+
+Every operator is a torch custom op: what traces, transforms or intercepts PyTorch calls sees it.  The dispatcher's way
+to such an op costs about 20 us of host time per call, more than most of its kernels take on a few tokens; where nothing
+looks on, `run` calls the operator's Python body (its argument checks and the C entry point) directly.
+"""
+
+from __future__ import annotations
+
+import torch
+
+from .enums import LIBRARY_NAME
+
+# argument types for which the dispatcher would do nothing but call the body: not tensor subclasses
+_PLAIN = frozenset((torch.Tensor, torch.nn.Parameter, type(None), int, float, bool, str))
+
+
+def operator(name: str, mutates_args: set[str]):
+    """torch.library.custom_op in this package's namespace; the undecorated function is kept as `.body`."""
+
+    def register(body):
+        op = torch.library.custom_op(f"{LIBRARY_NAME}::{name}", mutates_args=mutates_args)(body)
+        op.body = body
+        return op
+
+    return register
+
+
+def run(op, *args) -> None:
+    """op(*args) for outputs that were allocated for this call and that nothing has saved yet (the dispatcher would also
+    count the mutation in their version counters)."""
+    if torch.compiler.is_compiling():
+        op(*args)
+        return
+    if (
+        torch._C._len_torch_dispatch_stack() == 0  # dispatch modes: fake tensors, make_fx, profiling counters
+        and torch._C._functorch.peek_interpreter_stack() is None  # vmap, grad, functionalization
+        and not torch._C._is_torch_function_mode_enabled()
+        and torch._C._get_tracing_state() is None  # torch.jit.trace
+    ):
+        for a in args:
+            if type(a) not in _PLAIN:
+                break
+        else:
+            op = getattr(op, "body", op)  # (a plain function put in an operator's place is called as it is)
+    op(*args)

@@ -18,7 +18,8 @@ import torch.nn.functional as F
 
 from .. import _lib
 from ..count_cumsum import count_cumsum
-from ..enums import LIBRARY_NAME, ActivationType, is_glu
+from .._operator import operator, run
+from ..enums import ActivationType, is_glu
 from .backward import (
     _down_projection_backward,
     _down_projection_weight_grad,
@@ -63,8 +64,8 @@ from .utils import enable_quack_gemm, is_using_quack_gemm
 # ---------------------------------------------------------------------------------------------------------------
 
 
-@torch.library.custom_op(
-    f"{LIBRARY_NAME}::_routing_metadata",
+@operator(
+    "_routing_metadata",
     mutates_args={"freq", "off", "x_gather_idx", "s_scatter_idx", "s_reverse_scatter_idx", "tok_off"},
 )
 def _routing_metadata(
@@ -120,7 +121,7 @@ def _build_metadata(expert_idx: torch.Tensor, token_idx: torch.Tensor | None, T:
     expert_idx = expert_idx.contiguous().to(torch.int32)
     if token_idx is not None:
         token_idx = token_idx.contiguous().to(torch.int32)
-    _routing_metadata(expert_idx, token_idx, T, K, freq, off, gidx, sidx, ridx, tok_off)
+    run(_routing_metadata, expert_idx, token_idx, T, K, freq, off, gidx, sidx, ridx, tok_off)
     return freq, off, gidx, sidx, ridx, tok_off
 
 
@@ -175,7 +176,7 @@ class TC_Softmax_Topk_Router_Function(torch.autograd.Function):
         T = router_logits.size(0)
         scores = torch.empty(T, K, dtype=torch.float32, device=router_logits.device)
         indices = torch.empty(T, K, dtype=torch.int32, device=router_logits.device)
-        _softmax_topk_fwd(router_logits, scores, indices, E, K)
+        run(_softmax_topk_fwd, router_logits, scores, indices, E, K)
         ctx.save_for_backward(scores, indices)
         ctx.E, ctx.K, ctx.logits_dtype = E, K, router_logits.dtype
         ctx.mark_non_differentiable(indices)
@@ -185,7 +186,7 @@ class TC_Softmax_Topk_Router_Function(torch.autograd.Function):
     def backward(ctx, dscores: torch.Tensor, _unused):
         scores, indices = ctx.saved_tensors
         dlogits = torch.zeros(scores.size(0), ctx.E, dtype=ctx.logits_dtype, device=scores.device)
-        _softmax_topk_bwd(dlogits, None, dscores, scores, indices, ctx.K)
+        run(_softmax_topk_bwd, dlogits, None, dscores, scores, indices, ctx.K)
         return dlogits, None, None
 
 
@@ -285,9 +286,9 @@ def _experts_forward(x, w1, b1, w2, b2, scores_flat, off, gidx, ridx, tok_off, K
     y1 = None if is_using_fp8_forward() else torch.empty(TK, I, dtype=x.dtype, device=x.device)
     if _FUSED_COMBINE and sidx is not None and not is_using_fp8_forward():
         # down projection + combine in one kernel (atomic adds onto a zeroed output); y2 does not exist
-        _up_projection_forward(x, w1, z, y1, b1, off, order, gidx, stream_id, activation_type.value, glu, inference)
+        run(_up_projection_forward, x, w1, z, y1, b1, off, order, gidx, stream_id, activation_type.value, glu, inference)
         o = torch.zeros(T, H, dtype=x.dtype, device=x.device)
-        _down_projection_forward_combine(w2, y1, o, b2, scores_flat, off, order, gidx, sidx, stream_id)
+        run(_down_projection_forward_combine, w2, y1, o, b2, scores_flat, off, order, gidx, sidx, stream_id)
         return o, z
     y2 = torch.empty(TK, H, dtype=x.dtype, device=x.device)
     if is_using_fp8_forward():
@@ -299,19 +300,20 @@ def _experts_forward(x, w1, b1, w2, b2, scores_flat, off, gidx, ridx, tok_off, K
         # y1 leaves the up-projection already quantised (from the fp32 accumulator); its bf16 form is not stored
         y1q = torch.empty(TK, I, dtype=torch.uint8, device=x.device)
         y1s = torch.empty(I // 128, TK, dtype=torch.int32, device=x.device)
-        _up_projection_forward_fp8(
+        run(
+            _up_projection_forward_fp8,
             xq, xs, w1q, w1s, z, None, b1, off, gidx, E, stream_id, activation_type.value, glu, y1q, y1s
         )
         del xq, xs, w1q, w1s
         w2q, w2s = quantize_weight(w2)
-        _down_projection_forward_fp8(y1q, y1s, w2q, w2s, y2, b2, off, E, stream_id)
+        run(_down_projection_forward_fp8, y1q, y1s, w2q, w2s, y2, b2, off, E, stream_id)
         del y1q, y1s, w2q, w2s
     else:
-        _up_projection_forward(x, w1, z, y1, b1, off, order, gidx, stream_id, activation_type.value, glu, inference)
-        _down_projection_forward(w2, y1, y2, b2, off, order, gidx, stream_id)
+        run(_up_projection_forward, x, w1, z, y1, b1, off, order, gidx, stream_id, activation_type.value, glu, inference)
+        run(_down_projection_forward, w2, y1, y2, b2, off, order, gidx, stream_id)
     del y1
     o = torch.empty(T, H, dtype=x.dtype, device=x.device)
-    _router_forward(y2, o, scores_flat, ridx, tok_off, K_or_maxK, H, is_varlen_K)
+    run(_router_forward, y2, o, scores_flat, ridx, tok_off, K_or_maxK, H, is_varlen_K)
     return o, z
 
 
@@ -332,16 +334,17 @@ def _experts_backward(dout, x, w1, w2, b2, z, scores_flat, off, gidx, sidx, ridx
     db2 = None if b2 is None else torch.empty_like(b2)
     dz = torch.empty_like(z)
     ds = torch.empty(TK, dtype=torch.float32, device=x.device)
-    _down_projection_backward(
+    run(
+        _down_projection_backward,
         dout, z, w2, dw2, dz, ds, b2, db2, scores_flat, off, order, gidx, sidx, stream_id, glu, activation_type.value
     )
     dw1 = torch.empty_like(w1)
     db1 = torch.empty(w1.size(2), w1.size(0), dtype=x.dtype, device=x.device) if has_b1 else None
     dx_expanded = torch.empty(TK, H, dtype=x.dtype, device=x.device)
-    _up_projection_backward(x, w1, dx_expanded, dw1, dz, db1, off, order, gidx, sidx, glu, stream_id)
+    run(_up_projection_backward, x, w1, dx_expanded, dw1, dz, db1, off, order, gidx, sidx, glu, stream_id)
     del dz
     dx = torch.empty(T, H, dtype=x.dtype, device=x.device)
-    _token_broadcast_backward(dx, dx_expanded, ridx, tok_off, K_or_maxK, H, is_varlen_K)
+    run(_token_broadcast_backward, dx, dx_expanded, ridx, tok_off, K_or_maxK, H, is_varlen_K)
     return dx, dw1, db1, dw2, db2, ds
 
 
@@ -362,25 +365,25 @@ def _experts_backward_fp8(dout, x, w1, w2, b2, z, scores_flat, off, gidx, sidx, 
     dzq_scales = torch.empty(N1 // 128, TK, dtype=torch.int32, device=x.device)
     y1s = torch.empty(TK, I, dtype=x.dtype, device=x.device)
     ds = torch.empty(TK, dtype=torch.float32, device=x.device)
-    _down_projection_backward_fp8(doutq, dout_scales, w2tq, w2t_scales, z, dz, dzq, dzq_scales, y1s, ds, scores_flat,
+    run(_down_projection_backward_fp8, doutq, dout_scales, w2tq, w2t_scales, z, dz, dzq, dzq_scales, y1s, ds, scores_flat,
                                   off, gidx, sidx, E, stream_id, activation_type.value, glu)
     del doutq, dout_scales, w2tq, w2t_scales
     if b2 is not None:  # y2 = y1 W2^T + b2 puts <dout, b2> into the score gradient
-        _score_grad_bias_term(dout, b2, ds, off, gidx, sidx, stream_id)
+        run(_score_grad_bias_term, dout, b2, ds, off, gidx, sidx, stream_id)
     dw2 = torch.empty_like(w2)
     db2 = None if b2 is None else torch.empty_like(b2)
-    _down_projection_weight_grad(dout, y1s, dw2, db2, scores_flat, off, order, gidx, sidx, stream_id)
+    run(_down_projection_weight_grad, dout, y1s, dw2, db2, scores_flat, off, order, gidx, sidx, stream_id)
     del y1s
     w1tq, w1t_scales = quantize_expert_weight_transposed(w1)
     dx_expanded = torch.empty(TK, H, dtype=x.dtype, device=x.device)
-    _down_projection_forward_fp8(dzq, dzq_scales, w1tq, w1t_scales, dx_expanded, None, off, E, stream_id)
+    run(_down_projection_forward_fp8, dzq, dzq_scales, w1tq, w1t_scales, dx_expanded, None, off, E, stream_id)
     del dzq, dzq_scales, w1tq, w1t_scales
     dw1 = torch.empty_like(w1)
     db1 = torch.empty(w1.size(2), w1.size(0), dtype=x.dtype, device=x.device) if has_b1 else None
-    _up_projection_backward(x, w1, None, dw1, dz, db1, off, order, gidx, sidx, glu, stream_id)
+    run(_up_projection_backward, x, w1, None, dw1, dz, db1, off, order, gidx, sidx, glu, stream_id)
     del dz
     dx = torch.empty(T, H, dtype=x.dtype, device=x.device)
-    _token_broadcast_backward(dx, dx_expanded, ridx, tok_off, K_or_maxK, H, is_varlen_K)
+    run(_token_broadcast_backward, dx, dx_expanded, ridx, tok_off, K_or_maxK, H, is_varlen_K)
     return dx, dw1, db1, dw2, db2, ds
 
 
@@ -445,7 +448,7 @@ def _router_wgrad(dlogits: torch.Tensor, x: torch.Tensor, like: torch.Tensor) ->
             and H % 8 == 0)
     if fast and T >= 256 and os.environ.get("SMOE_ROUTER_WGRAD", "1") != "0":
         partial = torch.empty(router_weight_grad_chunks(T, E, H), E, H, dtype=x.dtype, device=x.device)
-        _router_weight_grad(dlogits.contiguous(), x.contiguous(), partial)
+        run(_router_weight_grad, dlogits.contiguous(), x.contiguous(), partial)
         return partial.sum(0, dtype=torch.float32).to(like.dtype) if partial.size(0) > 1 else partial[0]
     return dlogits.t() @ x
 
@@ -467,14 +470,14 @@ class _TCLayerFunction(torch.autograd.Function):
         if _FUSED_ROUTER and router_fused_supported(x, router_w):
             router_logits = torch.empty(T, E, dtype=x.dtype, device=x.device)
             colsum = torch.empty(router_fused_partials(T, E), E, dtype=torch.float32, device=x.device)
-            _router_forward_fused(x, router_w.contiguous(), router_logits, scores, indices, colsum)
+            run(_router_forward_fused, x, router_w.contiguous(), router_logits, scores, indices, colsum)
             # picked up by switch_loss() when it is handed this very tensor (MoE.forward does that).  Under torch.compile
             # a tensor attribute does not survive tracing: the loss then takes its own pass over the logits.
             if not torch.compiler.is_compiling():
                 router_logits._smoe_softmax_colsum_partials = (colsum, router_logits._version)
         else:
             router_logits = F.linear(x, router_w)
-            _softmax_topk_fwd(router_logits, scores, indices, E, K)
+            run(_softmax_topk_fwd, router_logits, scores, indices, E, K)
         freq, off, gidx, sidx, ridx, tok_off = _build_metadata(indices.view(-1), None, T, E, K)
         scores_flat = scores.view(-1)
         order = _schedule_order(off)
@@ -500,7 +503,7 @@ class _TCLayerFunction(torch.autograd.Function):
             has_b1, ctx.order, ctx.fp8_backward,
         )
         dlogits = torch.zeros(T, E, dtype=logits_dtype, device=x.device)
-        _softmax_topk_bwd(dlogits, None, ds.view(T, K), scores, indices, K)
+        run(_softmax_topk_bwd, dlogits, None, ds.view(T, K), scores, indices, K)
         if dlogits_outside is not None:
             dlogits = dlogits + dlogits_outside
         dwr = _router_wgrad(dlogits, x, router_w) if ctx.needs_input_grad[1] else None
@@ -525,9 +528,9 @@ class _SwitchLossFunction(torch.autograd.Function):
         aux = torch.empty(1, dtype=torch.float32, device=logits.device)
         partials, version = getattr(router_logits, "_smoe_softmax_colsum_partials", (None, None))
         if partials is not None and version == router_logits._version and router_logits.dim() == 2:
-            _switch_loss_from_partials(partials, freq, acc, aux)  # the fused router already summed the softmax columns
+            run(_switch_loss_from_partials, partials, freq, acc, aux)  # the fused router already summed the softmax columns
         else:
-            _switch_loss_fwd(logits, freq, acc, aux)
+            run(_switch_loss_fwd, logits, freq, acc, aux)
         ctx.save_for_backward(logits, freq, acc)
         ctx.logits_shape = router_logits.shape
         return aux.view(())
@@ -536,7 +539,7 @@ class _SwitchLossFunction(torch.autograd.Function):
     def backward(ctx, grad_aux: torch.Tensor):
         logits, freq, acc = ctx.saved_tensors
         dlogits = torch.empty_like(logits, memory_format=torch.contiguous_format)
-        _switch_loss_bwd(logits, freq, acc, grad_aux.reshape(1).float().contiguous(), dlogits)
+        run(_switch_loss_bwd, logits, freq, acc, grad_aux.reshape(1).float().contiguous(), dlogits)
         return dlogits.view(ctx.logits_shape), None
 
 

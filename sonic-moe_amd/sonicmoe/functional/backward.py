@@ -7,12 +7,13 @@ from typing import Optional
 import torch
 
 from .. import _lib
-from ..enums import ACTIVATION_CODE, LIBRARY_NAME, ActivationType
+from .._operator import operator
+from ..enums import ACTIVATION_CODE, ActivationType
 from ..utils import expert_major_strides
 from .forward import _check_schedule_order, _elem_dtype, _gather_sum, _gemm_workspace
 
 
-@torch.library.custom_op(f"{LIBRARY_NAME}::_up_projection_backward", mutates_args={"dw1", "dx_expanded", "db1"})
+@operator("_up_projection_backward", mutates_args={"dw1", "dx_expanded", "db1"})
 def _up_projection_backward(
     x: torch.Tensor,
     w1: torch.Tensor,
@@ -68,7 +69,7 @@ def _up_projection_backward(
     _lib.check(rc, "_up_projection_backward")
 
 
-@torch.library.custom_op(f"{LIBRARY_NAME}::_down_projection_backward", mutates_args={"dw2", "dz", "ds", "db2"})
+@operator("_down_projection_backward", mutates_args={"dw2", "dz", "ds", "db2"})
 def _down_projection_backward(
     dout: torch.Tensor,
     z: torch.Tensor,
@@ -140,7 +141,7 @@ def _down_projection_backward(
     _lib.check(rc, "_down_projection_backward")
 
 
-@torch.library.custom_op(f"{LIBRARY_NAME}::_down_projection_weight_grad", mutates_args={"dw2", "db2"})
+@operator("_down_projection_weight_grad", mutates_args={"dw2", "db2"})
 def _down_projection_weight_grad(
     dout: torch.Tensor,
     y1s: torch.Tensor,
@@ -176,7 +177,7 @@ def _down_projection_weight_grad(
     _lib.check(rc, "_down_projection_weight_grad")
 
 
-@torch.library.custom_op(f"{LIBRARY_NAME}::_token_broadcast_backward", mutates_args={"dx_reduced"})
+@operator("_token_broadcast_backward", mutates_args={"dx_reduced"})
 def _token_broadcast_backward(
     dx_reduced: torch.Tensor,
     dx_expanded: torch.Tensor,
@@ -200,7 +201,7 @@ def _token_broadcast_backward(
     )
 
 
-@torch.library.custom_op(f"{LIBRARY_NAME}::_softmax_topk_bwd", mutates_args={"dlogits_full"})
+@operator("_softmax_topk_bwd", mutates_args={"dlogits_full"})
 def _softmax_topk_bwd(
     dlogits_full: torch.Tensor,
     dlogits: Optional[torch.Tensor],
@@ -234,7 +235,7 @@ def _softmax_topk_bwd(
     _lib.check(rc, "_softmax_topk_bwd")
 
 
-@torch.library.custom_op(f"{LIBRARY_NAME}::_topk_bwd", mutates_args={"dlogits_full"})
+@operator("_topk_bwd", mutates_args={"dlogits_full"})
 def _topk_bwd(dlogits_full: torch.Tensor, dtopk_values: torch.Tensor, topk_indices: torch.Tensor, K: int) -> None:
     """dlogits_full[t, idx[t,k]] = dtopk_values[t,k]: backward of `_topk_fwd` without the softmax fusion; the caller
     zero-fills dlogits_full (sonicmoe/functional/backward.py:589-610 of the reference, which has no caller for it)."""
@@ -251,7 +252,7 @@ def _topk_bwd(dlogits_full: torch.Tensor, dtopk_values: torch.Tensor, topk_indic
     _lib.check(rc, "_topk_bwd")
 
 
-@torch.library.custom_op(f"{LIBRARY_NAME}::_router_weight_grad", mutates_args={"partial"})
+@operator("_router_weight_grad", mutates_args={"partial"})
 def _router_weight_grad(dlogits: torch.Tensor, x: torch.Tensor, partial: torch.Tensor) -> None:
     """partial[c] (E, H) = dlogits[rows of chunk c]^T x[rows of chunk c]; the chunks are partial.size(0) equal token
     ranges.  Their sum is the weight gradient of router_logits = F.linear(x, router_w)."""
@@ -274,7 +275,7 @@ def router_weight_grad_chunks(T: int, E: int, H: int) -> int:
     return max(1, min(64, -(-256 // tiles), T // 256))
 
 
-@torch.library.custom_op(f"{LIBRARY_NAME}::_switch_loss_bwd", mutates_args={"dlogits"})
+@operator("_switch_loss_bwd", mutates_args={"dlogits"})
 def _switch_loss_bwd(router_logits: torch.Tensor, expert_frequency: torch.Tensor, acc: torch.Tensor,
                      grad_aux: torch.Tensor, dlogits: torch.Tensor) -> None:
     """dlogits (T, E) = grad_aux * d aux / d router_logits for the switch loss; acc as left by _switch_loss_fwd.  The

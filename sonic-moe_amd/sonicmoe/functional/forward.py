@@ -9,7 +9,8 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
-from ..enums import ACTIVATION_CODE, LIBRARY_NAME, ActivationType
+from .._operator import operator
+from ..enums import ACTIVATION_CODE, ActivationType
 from ..utils import expert_major_strides
 
 
@@ -63,7 +64,7 @@ def _check_schedule_order(order: torch.Tensor | None, E: int) -> None:
                          f"{order.dtype} {tuple(order.shape)}")
 
 
-@torch.library.custom_op(f"{LIBRARY_NAME}::_topk_fwd", mutates_args={"values", "indices"})
+@operator("_topk_fwd", mutates_args={"values", "indices"})
 def _topk_fwd(
     x: torch.Tensor, k: int, values: torch.Tensor, indices: torch.Tensor, require_softmax_fusion: bool = True
 ) -> None:
@@ -89,16 +90,14 @@ def _topk_fwd(
     _lib.check(rc, "_topk_fwd")
 
 
-@torch.library.custom_op(
-    f"{LIBRARY_NAME}::_softmax_topk_fwd", mutates_args={"topk_router_score", "topk_router_indices"}
-)
+@operator("_softmax_topk_fwd", mutates_args={"topk_router_score", "topk_router_indices"})
 def _softmax_topk_fwd(
     router_logits: torch.Tensor, topk_router_score: torch.Tensor, topk_router_indices: torch.Tensor, E: int, K: int
 ) -> None:
-    _topk_fwd(router_logits, K, topk_router_score, topk_router_indices, True)
+    _topk_fwd.body(router_logits, K, topk_router_score, topk_router_indices, True)
 
 
-@torch.library.custom_op(f"{LIBRARY_NAME}::_up_projection_forward", mutates_args={"z", "y1"})
+@operator("_up_projection_forward", mutates_args={"z", "y1"})
 def _up_projection_forward(
     x: torch.Tensor,
     w1: torch.Tensor,
@@ -149,7 +148,7 @@ def _up_projection_forward(
     _lib.check(rc, "_up_projection_forward")
 
 
-@torch.library.custom_op(f"{LIBRARY_NAME}::_down_projection_forward", mutates_args={"y2"})
+@operator("_down_projection_forward", mutates_args={"y2"})
 def _down_projection_forward(
     w2: torch.Tensor,
     y1: torch.Tensor,
@@ -190,7 +189,7 @@ def _down_projection_forward(
     _lib.check(rc, "_down_projection_forward")
 
 
-@torch.library.custom_op(f"{LIBRARY_NAME}::_down_projection_forward_combine", mutates_args={"o"})
+@operator("_down_projection_forward_combine", mutates_args={"o"})
 def _down_projection_forward_combine(
     w2: torch.Tensor,
     y1: torch.Tensor,
@@ -268,7 +267,7 @@ def _gather_sum(src, out, weights, ridx, tok_off, K, H, is_varlen_K, what):
     _lib.check(rc, what)
 
 
-@torch.library.custom_op(f"{LIBRARY_NAME}::_router_forward", mutates_args={"o"})
+@operator("_router_forward", mutates_args={"o"})
 def _router_forward(
     y2: torch.Tensor,
     o: torch.Tensor,
@@ -293,7 +292,7 @@ def _router_forward(
     )
 
 
-@torch.library.custom_op(f"{LIBRARY_NAME}::_switch_loss_fwd", mutates_args={"acc", "aux"})
+@operator("_switch_loss_fwd", mutates_args={"acc", "aux"})
 def _switch_loss_fwd(router_logits: torch.Tensor, expert_frequency: torch.Tensor, acc: torch.Tensor,
                      aux: torch.Tensor) -> None:
     """acc (E) fp32 = column sums of softmax(router_logits) in fp32; aux (1) fp32 = E * <acc / |acc|_1, freq / |freq|_1>:
@@ -323,8 +322,8 @@ def router_fused_supported(x: torch.Tensor, router_w: torch.Tensor) -> bool:
             and 16 <= E <= 256 and H % 256 == 0 and x.size(0) > 0)
 
 
-@torch.library.custom_op(
-    f"{LIBRARY_NAME}::_router_forward_fused", mutates_args={"router_logits", "topk_scores", "topk_indices", "colsum_partial"}
+@operator(
+    "_router_forward_fused", mutates_args={"router_logits", "topk_scores", "topk_indices", "colsum_partial"}
 )
 def _router_forward_fused(x: torch.Tensor, router_w: torch.Tensor, router_logits: torch.Tensor,
                           topk_scores: torch.Tensor, topk_indices: torch.Tensor,
@@ -356,7 +355,7 @@ def router_fused_partials(T: int, E: int) -> int:
     return int(_lib.lib().smoe_router_fused_partials(T, E))
 
 
-@torch.library.custom_op(f"{LIBRARY_NAME}::_switch_loss_from_partials", mutates_args={"acc", "aux"})
+@operator("_switch_loss_from_partials", mutates_args={"acc", "aux"})
 def _switch_loss_from_partials(colsum_partial: torch.Tensor, expert_frequency: torch.Tensor, acc: torch.Tensor,
                                aux: torch.Tensor) -> None:
     """acc, aux of `_switch_loss_fwd` from the column-sum partials `_router_forward_fused` wrote."""

@@ -16,7 +16,8 @@ from contextlib import contextmanager
 import torch
 
 from .. import _lib
-from ..enums import ACTIVATION_CODE, LIBRARY_NAME, ActivationType
+from .._operator import operator, run
+from ..enums import ACTIVATION_CODE, ActivationType
 from .forward import _elem_dtype, _gemm_workspace
 
 _FP8_FORWARD = False
@@ -54,7 +55,7 @@ def is_using_fp8_backward() -> bool:
     return _FP8_BACKWARD
 
 
-@torch.library.custom_op(f"{LIBRARY_NAME}::_mx_quantize", mutates_args={"q", "scales"})
+@operator("_mx_quantize", mutates_args={"q", "scales"})
 def _mx_quantize(src: torch.Tensor, q: torch.Tensor, scales: torch.Tensor) -> None:
     """src (R, C) bf16 -> q (R, C) uint8 e4m3 codes, scales (C/128, R) int32 (four exponent bytes per word)."""
     _lib.require_device(src, q, scales)
@@ -75,7 +76,7 @@ def mx_quantize(t: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         raise NotImplementedError(f"mx_quantize: {C} columns are not a multiple of 128")
     q = torch.empty(R, C, dtype=torch.uint8, device=t.device)
     scales = torch.empty(C // 128, R, dtype=torch.int32, device=t.device)
-    _mx_quantize(t, q, scales)
+    run(_mx_quantize, t, q, scales)
     return q, scales
 
 
@@ -121,9 +122,7 @@ def quantize_expert_weight(w_view: torch.Tensor) -> tuple[torch.Tensor, torch.Te
     return q, scales
 
 
-@torch.library.custom_op(
-    f"{LIBRARY_NAME}::_up_projection_forward_fp8", mutates_args={"z", "y1", "y1q", "y1q_scales"}
-)
+@operator("_up_projection_forward_fp8", mutates_args={"z", "y1", "y1q", "y1q_scales"})
 def _up_projection_forward_fp8(
     xq: torch.Tensor,
     x_scales: torch.Tensor,
@@ -177,7 +176,7 @@ def _up_projection_forward_fp8(
     _lib.check(rc, "_up_projection_forward_fp8")
 
 
-@torch.library.custom_op(f"{LIBRARY_NAME}::_down_projection_forward_fp8", mutates_args={"y2"})
+@operator("_down_projection_forward_fp8", mutates_args={"y2"})
 def _down_projection_forward_fp8(
     y1q: torch.Tensor,
     y1_scales: torch.Tensor,
@@ -215,7 +214,7 @@ def _down_projection_forward_fp8(
     _lib.check(rc, "_down_projection_forward_fp8")
 
 
-@torch.library.custom_op(f"{LIBRARY_NAME}::_mx_quantize_transposed", mutates_args={"q", "scales"})
+@operator("_mx_quantize_transposed", mutates_args={"q", "scales"})
 def _mx_quantize_transposed(src: torch.Tensor, q: torch.Tensor, scales: torch.Tensor) -> None:
     """src (E, R, C) bf16 (last dimension contiguous) -> q (E, C, R) uint8, the transposed matrices quantised along R,
     scales (R/128, E*C) int32."""
@@ -232,9 +231,7 @@ def _mx_quantize_transposed(src: torch.Tensor, q: torch.Tensor, scales: torch.Te
     _lib.check(rc, "_mx_quantize_transposed")
 
 
-@torch.library.custom_op(
-    f"{LIBRARY_NAME}::_mx_quantize_both", mutates_args={"q_rows", "scales_rows", "q_t", "scales_t"}
-)
+@operator("_mx_quantize_both", mutates_args={"q_rows", "scales_rows", "q_t", "scales_t"})
 def _mx_quantize_both(src: torch.Tensor, q_rows: torch.Tensor, scales_rows: torch.Tensor, q_t: torch.Tensor,
                       scales_t: torch.Tensor) -> None:
     """src (E, R, C) bf16 -> both quantised copies from one pass over src: q_rows (E*R, C) / scales_rows (C/128, E*R) as
@@ -281,7 +278,7 @@ def quantize_expert_weight_both(w_view: torch.Tensor) -> tuple[torch.Tensor, tor
     scales = torch.empty(K // 128, E * N, dtype=torch.int32, device=w.device)
     qt = torch.empty(E, K, N, dtype=torch.uint8, device=w.device)
     scales_t = torch.empty(N // 128, E * K, dtype=torch.int32, device=w.device)
-    _mx_quantize_both(w.detach(), q, scales, qt, scales_t)
+    run(_mx_quantize_both, w.detach(), q, scales, qt, scales_t)
     if _CACHE_WEIGHTS:
         if len(_WEIGHT_CACHE) >= _WEIGHT_CACHE_MAX:
             _WEIGHT_CACHE.pop(next(iter(_WEIGHT_CACHE)))
@@ -313,12 +310,12 @@ def quantize_expert_weight_transposed(w_view: torch.Tensor) -> tuple[torch.Tenso
                                   f"in % 64 == 0")
     q = torch.empty(E, K, N, dtype=torch.uint8, device=w.device)
     scales = torch.empty(N // 128, E * K, dtype=torch.int32, device=w.device)
-    _mx_quantize_transposed(w.detach(), q, scales)
+    run(_mx_quantize_transposed, w.detach(), q, scales)
     return q.view(E * K, N), scales
 
 
-@torch.library.custom_op(
-    f"{LIBRARY_NAME}::_down_projection_backward_fp8", mutates_args={"dz", "dzq", "dzq_scales", "y1s", "ds"}
+@operator(
+    "_down_projection_backward_fp8", mutates_args={"dz", "dzq", "dzq_scales", "y1s", "ds"}
 )
 def _down_projection_backward_fp8(
     doutq: torch.Tensor,
@@ -386,7 +383,7 @@ def _down_projection_backward_fp8(
     _lib.check(rc, "_down_projection_backward_fp8")
 
 
-@torch.library.custom_op(f"{LIBRARY_NAME}::_score_grad_bias_term", mutates_args={"ds"})
+@operator("_score_grad_bias_term", mutates_args={"ds"})
 def _score_grad_bias_term(
     dout: torch.Tensor,
     b2: torch.Tensor,

@@ -1,0 +1,91 @@
+"""`run` calls an operator's body directly only where nothing observes the dispatcher."""
+
+import pytest
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.overrides import TorchFunctionMode
+from torch.utils._python_dispatch import TorchDispatchMode
+
+from sonicmoe._operator import operator, run
+
+BODY_CALLS = []
+
+
+@operator("_test_copy", mutates_args={"out"})
+def _test_copy(x: torch.Tensor, out: torch.Tensor, scale: float) -> None:
+    BODY_CALLS.append(type(x))
+    out.copy_(x * scale)
+
+
+@_test_copy.register_fake
+def _(x, out, scale):
+    return None
+
+
+class Tagged(torch.Tensor):
+    pass
+
+
+class Seen(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.ops = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.ops.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.fixture(autouse=True)
+def _clear():
+    BODY_CALLS.clear()
+
+
+def test_plain_tensors_skip_the_dispatcher(monkeypatch):
+    x, out = torch.randn(3), torch.zeros(3)
+    with monkeypatch.context() as m:
+        m.setattr(type(_test_copy), "__call__", lambda self, *args: pytest.fail("went through the dispatcher"))
+        run(_test_copy, x, out, 2.0)
+        assert torch.equal(out, x * 2) and BODY_CALLS == [torch.Tensor]
+        with torch.no_grad():
+            run(_test_copy, torch.nn.Parameter(x), out, 3.0)
+        assert torch.equal(out, x * 3)
+
+
+def test_dispatch_modes_see_the_operator():
+    x, out = torch.randn(3), torch.zeros(3)
+    with Seen() as seen:
+        run(_test_copy, x, out, 2.0)
+    assert any("_test_copy" in op for op in seen.ops)
+    with FakeTensorMode():
+        run(_test_copy, torch.empty(3), torch.empty(3), 2.0)
+    assert len(BODY_CALLS) == 1  # the fake call stopped at the fake implementation
+
+
+def test_function_modes_subclasses_and_tracing_take_the_operator(monkeypatch):
+    taken = []
+    monkeypatch.setattr(type(_test_copy), "__call__", lambda self, *args: taken.append(args))
+
+    class Mode(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    x, out = torch.randn(3), torch.zeros(3)
+    with Mode():
+        run(_test_copy, x, out, 2.0)
+    run(_test_copy, x.as_subclass(Tagged), out, 2.0)
+    torch.jit.trace(lambda t: (run(_test_copy, t, out, 2.0), t + 1)[1], x, check_trace=False)
+    torch.vmap(lambda t: (run(_test_copy, t, out, 2.0), t)[1])(torch.randn(2, 3))
+    assert len(taken) == 4 and not BODY_CALLS
+
+
+def test_compiled_code_keeps_the_operator():
+    seen = []
+
+    def backend(gm, _inputs):
+        seen.extend(str(n.target) for n in gm.graph.nodes)
+        return gm.forward
+
+    out = torch.zeros(3)
+    torch.compile(lambda t, o: (run(_test_copy, t, o, 2.0), o + 1)[1], backend=backend, fullgraph=True)(torch.ones(3), out)
+    assert any("_test_copy" in t for t in seen) and torch.equal(out, torch.full((3,), 2.0))
