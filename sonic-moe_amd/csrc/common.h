@@ -96,6 +96,14 @@ SMOE_DEV float elem_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 #endif
 SMOE_DEV float elem_bits_to_f32(uint32_t h) { return elem_lo(h); }
 
+// The value as the compiler cannot see through it.  Between a group of loads and the selects that drop some of them: the
+// compiler turns `c < n ? p[c] : v` over a clamped index back into a load under a condition, and such loads are waited for
+// one by one.
+SMOE_DEV uint32_t opaque(uint32_t v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
 // 1 / (1 + e^-x) with the hardware reciprocal (1 ulp): a correctly rounded division is a dozen instructions per value
 SMOE_DEV float fast_sigmoid(float x) { return __builtin_amdgcn_rcpf(1.0f + __expf(-x)); }
 

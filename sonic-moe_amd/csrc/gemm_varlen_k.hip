@@ -329,6 +329,7 @@ __global__ __launch_bounds__(1024) void sort_experts_kernel(const int32_t* __res
     } else {
       int pos = 0;
       const int c = cost[e];
+#pragma unroll 8
       for (int o = 0; o < E; o++) pos += (cost[o] > c || (cost[o] == c && o < e)) ? 1 : 0;
       sorted[pos] = e;
     }

@@ -12,10 +12,12 @@ namespace smoe {
 // top-K + softmax
 // ============================================================================================================
 // One row is owned by a group of G consecutive lanes (G a power of two <= 64); lane g of the group holds the
-// VPL consecutive columns [g*VPL, (g+1)*VPL) as 64-bit keys
-//     key = (order-preserving image of the fp32 value) << 32 | (0xffffffff - column)
-// so that the maximum key is the largest value and, among equal values, the lowest column.  K rounds of
-// "group arg-max, then retire the winner" give the winners in descending order.
+// VPL consecutive columns [g*VPL, (g+1)*VPL) as keys
+//     key = (order-preserving image of the value's bits) << W | (2^W - 1 - column)
+// with W = 32 for fp32 and W = 16 for the 16-bit types, so that the maximum key is the largest value and, among equal
+// values, the lowest column.  K rounds of "group arg-max, then retire the winner" give the winners in descending order.
+// A round is a chain of maxima, one instruction each on 32-bit keys and three on 64-bit ones (one row, E = 128, K = 8:
+// 8.3 -> 5.8 us; T = 40960, E = 256: 32 -> 26 us).
 
 SMOE_DEV uint32_t orderable(uint32_t bits) { return bits ^ ((bits >> 31) ? 0xffffffffu : 0x80000000u); }
 SMOE_DEV uint32_t unorderable(uint32_t o) { return o ^ ((o >> 31) ? 0x80000000u : 0xffffffffu); }
@@ -42,11 +44,48 @@ __device__ __forceinline__ uint32_t load_as_f32_bits<float>(const float* p) {
   return __float_as_uint(*p);
 }
 
+template <typename T>
+struct TopkKey;
+template <>
+struct TopkKey<float> {
+  typedef uint64_t Key;
+  static __device__ __forceinline__ uint32_t load(const float* p, uint32_t clear_mask) {
+    return __float_as_uint(*p) & clear_mask;
+  }
+  static __device__ __forceinline__ Key make(uint32_t bits, int col) {
+    return ((uint64_t)orderable(bits) << 32) | (uint64_t)(0xffffffffu - (uint32_t)col);
+  }
+  static __device__ __forceinline__ float value(Key k) { return __uint_as_float(unorderable((uint32_t)(k >> 32))); }
+  static __device__ __forceinline__ int column(Key k) { return (int)(0xffffffffu - (uint32_t)k); }
+  static __device__ __forceinline__ Key shfl_xor(Key k, int m) { return shfl_xor_u64(k, m); }
+};
+// (clearing the low bits of the fp32 image, log2(E) <= 12 of them, does not touch a 16-bit value)
+template <typename T>
+struct TopkKey16 {
+  typedef uint32_t Key;
+  static __device__ __forceinline__ uint32_t load(const T* p, uint32_t) { return *(const uint16_t*)p; }
+  static __device__ __forceinline__ Key make(uint32_t bits, int col) {
+    return (bits ^ ((bits >> 15) ? 0xffffu : 0x8000u)) << 16 | (0xffffu - (uint32_t)col);
+  }
+  static __device__ __forceinline__ float value(Key k) {
+    const uint16_t o = (uint16_t)(k >> 16), bits = o ^ ((o >> 15) ? 0x8000u : 0xffffu);
+    return __uint_as_float(load_as_f32_bits<T>((const T*)&bits));
+  }
+  static __device__ __forceinline__ int column(Key k) { return (int)(0xffffu - (k & 0xffffu)); }
+  static __device__ __forceinline__ Key shfl_xor(Key k, int m) { return __shfl_xor(k, m, 64); }
+};
+template <>
+struct TopkKey<uint16_t> : TopkKey16<uint16_t> {};
+template <>
+struct TopkKey<__half> : TopkKey16<__half> {};
+
 template <typename T, int VPL>
 __global__ __launch_bounds__(256) void topk_softmax_kernel(const T* __restrict__ logits, int64_t row_stride,
                                                            int64_t Trows, int E, int K, int G, uint32_t clear_mask,
                                                            float* __restrict__ scores, int32_t* __restrict__ indices,
                                                            int do_softmax) {
+  // the winners' scores, K per row of the workgroup, until their sum is known
+  extern __shared__ float won[];
   const int lane_in_block = threadIdx.x;
   const int rows_per_block = 256 / G;
   const int g = lane_in_block % G;
@@ -54,45 +93,59 @@ __global__ __launch_bounds__(256) void topk_softmax_kernel(const T* __restrict__
   const bool row_ok = row < Trows;
   const int64_t rrow = row_ok ? row : 0;
 
-  uint64_t key[VPL];
+  typedef TopkKey<T> TK;
+  typedef typename TK::Key Key;
+  Key key[VPL];
   const T* src = logits + rrow * row_stride;
+  // all loads of a lane at once, those past the end from the last column (taken under a condition each, they were VPL
+  // round trips to memory: one row, E = 128, K = 8 10.7 -> 8.3 us)
+  uint32_t bits[VPL];
 #pragma unroll
   for (int i = 0; i < VPL; i++) {
     const int col = g * VPL + i;
-    uint64_t k = 0;  // 0 = retired / out of range: below every real key (real keys have a non-zero column part)
-    if (col < E) {
-      uint32_t bits = load_as_f32_bits<T>(src + col) & clear_mask;
-      k = ((uint64_t)orderable(bits) << 32) | (uint64_t)(0xffffffffu - (uint32_t)col);
-    }
-    key[i] = k;
+    bits[i] = TK::load(src + (col < E ? col : E - 1), clear_mask);
+  }
+#pragma unroll
+  for (int i = 0; i < VPL; i++) {
+    const int col = g * VPL + i;
+    // 0 = retired / out of range: below every real key (real keys have a non-zero column part)
+    const uint32_t v = opaque(bits[i]);
+    key[i] = col < E ? TK::make(v, col) : 0;
   }
 
   float vmax = 0.f, esum = 0.f;
   for (int r = 0; r < K; r++) {
-    uint64_t best = key[0];
+    Key best = key[0];
 #pragma unroll
     for (int i = 1; i < VPL; i++) best = key[i] > best ? key[i] : best;
     for (int m = 1; m < G; m <<= 1) {
-      uint64_t o = shfl_xor_u64(best, m);
+      const Key o = TK::shfl_xor(best, m);
       best = o > best ? o : best;
     }
 #pragma unroll
     for (int i = 0; i < VPL; i++) key[i] = (key[i] == best) ? 0 : key[i];
     if (g == 0 && row_ok) {
-      const float v = __uint_as_float(unorderable((uint32_t)(best >> 32)));
-      const int col = (int)(0xffffffffu - (uint32_t)best);
+      const float v = TK::value(best);
+      const int col = TK::column(best);
       float outv = v;
       if (do_softmax) {
         if (r == 0) vmax = v;
         outv = expf(v - vmax);
         esum += outv;
       }
-      scores[row * K + r] = outv;
+      if (do_softmax) {
+        won[lane_in_block / G * K + r] = outv;
+      } else {
+        scores[row * K + r] = outv;
+      }
       indices[row * K + r] = col;
     }
   }
-  if (do_softmax && g == 0 && row_ok) {
-    for (int r = 0; r < K; r++) scores[row * K + r] = scores[row * K + r] / esum;
+  if (do_softmax) {  // the row's lanes are lanes of one wavefront
+    const float sum = __shfl(esum, lane_in_block & 63 & -G, 64);
+    __builtin_amdgcn_wave_barrier();
+    if (row_ok)
+      for (int r = g; r < K; r += G) scores[row * K + r] = won[lane_in_block / G * K + r] / sum;
   }
 }
 
@@ -105,10 +158,12 @@ static int launch_topk(const void* logits, int64_t T_, int E, int K, int64_t row
   while (vpl * G < E) vpl <<= 1;
   const int rows_per_block = 256 / G;
   const dim3 grid((unsigned)ceil_div(T_, rows_per_block)), block(256);
+  // at most 16 KiB: G < 64 lanes own at most 16 G columns, so K <= 16 G; G = 64 makes 4 rows of K <= 64
+  const size_t won_bytes = softmax ? (size_t)rows_per_block * K * sizeof(float) : 0;
   const T* p = (const T*)logits;
 #define SMOE_TOPK_CASE(V)                                                                                          \
   case V:                                                                                                          \
-    hipLaunchKernelGGL((topk_softmax_kernel<T, V>), grid, block, 0, st, p, row_stride, T_, E, K, G, clear_mask,    \
+    hipLaunchKernelGGL((topk_softmax_kernel<T, V>), grid, block, won_bytes, st, p, row_stride, T_, E, K, G, clear_mask,    \
                        scores, indices, softmax);                                                                  \
     break;
   switch (vpl) {
@@ -253,6 +308,20 @@ __global__ __launch_bounds__(1024) void inclusive_scan_kernel(const int32_t* __r
 // segment rebuilds off[] from freq, seeds a cursor per expert and assigns positions with ballot-based ranking.
 constexpr int SEG = 1024;
 constexpr int META_WAVES = 4;
+constexpr int SEG_STEPS = SEG / 64;
+
+// The expert ids of a wavefront's segment, -1 past the end: all loads before the first use (taken one step at a time, and
+// under a condition each, every step of the histogram and of the ranking began with a round trip to memory; the three
+// passes at TK = 48008, E = 128: 25.2 -> 22.8 us).
+SMOE_DEV void load_segment(const int32_t* __restrict__ expert_idx, int64_t lo, int64_t TK, int lane, int (&ids)[SEG_STEPS]) {
+#pragma unroll
+  for (int i = 0; i < SEG_STEPS; i++) {
+    const int64_t j = lo + i * 64 + lane;
+    ids[i] = TK > 0 ? expert_idx[j < TK ? j : TK - 1] : -1;
+  }
+#pragma unroll
+  for (int i = 0; i < SEG_STEPS; i++) ids[i] = lo + i * 64 + lane < TK ? (int)opaque(ids[i]) : -1;
+}
 
 __global__ __launch_bounds__(64 * META_WAVES) void meta_hist_kernel(const int32_t* __restrict__ expert_idx,
                                                                     int64_t TK, int E, int NS,
@@ -262,14 +331,13 @@ __global__ __launch_bounds__(64 * META_WAVES) void meta_hist_kernel(const int32_
   int32_t* hist = lds + (size_t)wave * E;
   const int s = blockIdx.x * META_WAVES + wave;
   if (s >= NS) return;
+  int ids[SEG_STEPS];
+  load_segment(expert_idx, (int64_t)s * SEG, TK, lane, ids);
   for (int e = lane; e < E; e += 64) hist[e] = 0;
   __builtin_amdgcn_wave_barrier();
-  const int64_t lo = (int64_t)s * SEG;
-  const int64_t hi = lo + SEG < TK ? lo + SEG : TK;
-  for (int64_t j = lo + lane; j < hi; j += 64) {
-    const int e = expert_idx[j];
-    if (e >= 0 && e < E) atomicAdd(&hist[e], 1);
-  }
+#pragma unroll
+  for (int i = 0; i < SEG_STEPS; i++)
+    if (ids[i] >= 0 && ids[i] < E) atomicAdd(&hist[ids[i]], 1);
   __builtin_amdgcn_wave_barrier();
   for (int e = lane; e < E; e += 64) hist_t[(size_t)e * NS + s] = hist[e];
 }
@@ -294,6 +362,45 @@ __global__ __launch_bounds__(256) void meta_scan_kernel(const int32_t* __restric
   if (lane == 0) freq[e] = carry;
 }
 
+// One step of the counting sort for a wavefront: lane l holds slot j (consecutive over the lanes, `valid` a prefix of them)
+// of expert e.  Slots of the same expert take consecutive positions from that expert's cursor, in lane order.
+SMOE_DEV void place_slots(int e, int64_t j, bool valid, int lane, const int32_t* __restrict__ token_idx, int64_t TK,
+                          int64_t T, int E, int K, int ebits, int32_t* cursor, int32_t* __restrict__ gidx,
+                          int32_t* __restrict__ sidx, int32_t* __restrict__ ridx, int32_t* __restrict__ tok_off) {
+  const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+  const bool in_range = valid && e >= 0 && e < E;
+  if (!in_range) e = 0;
+  uint64_t peers = __ballot(in_range);
+  for (int b = 0; b < ebits; b++) {
+    const uint64_t bal = __ballot((e >> b) & 1);
+    peers &= ((e >> b) & 1) ? bal : ~bal;
+  }
+  int32_t pos = 0;
+  if (in_range) {
+    pos = cursor[e] + __popcll(peers & lt_mask);
+  }
+  __builtin_amdgcn_wave_barrier();
+  if (in_range && (peers >> lane) >> 1 == 0) cursor[e] = pos + 1;  // highest peer lane advances the cursor
+  __builtin_amdgcn_wave_barrier();
+  if (in_range) {
+    sidx[pos] = (int32_t)j;
+    ridx[j] = pos;
+    gidx[pos] = token_idx ? token_idx[j] : (int32_t)(j / K);
+  }
+  if (tok_off && valid) {
+    if (token_idx) {
+      const int32_t t = token_idx[j];
+      const int32_t tprev = j == 0 ? -1 : token_idx[j - 1];
+      for (int32_t u = tprev + 1; u <= t; u++) tok_off[u] = (int32_t)j;
+      if (j == TK - 1)
+        for (int64_t u = (int64_t)t + 1; u <= T; u++) tok_off[u] = (int32_t)TK;
+    } else {
+      if (j % K == 0) tok_off[j / K] = (int32_t)j;
+      if (j == TK - 1) tok_off[T] = (int32_t)TK;
+    }
+  }
+}
+
 __global__ __launch_bounds__(64 * META_WAVES) void meta_scatter_kernel(
     const int32_t* __restrict__ expert_idx, const int32_t* __restrict__ token_idx, int64_t TK, int64_t T, int E,
     int K, int NS, int ebits, const int32_t* __restrict__ freq, const int32_t* __restrict__ base_t,
@@ -304,6 +411,9 @@ __global__ __launch_bounds__(64 * META_WAVES) void meta_scatter_kernel(
   int32_t* cursor = lds + (size_t)wave * E;
   const int s = blockIdx.x * META_WAVES + wave;
   if (s >= NS) return;
+  const int64_t lo = (int64_t)s * SEG;
+  int ids[SEG_STEPS];
+  load_segment(expert_idx, lo, TK, lane, ids);
 
   // exclusive scan of freq -> off (every segment needs it; segment 0 also publishes it)
   int32_t carry = 0;
@@ -325,47 +435,81 @@ __global__ __launch_bounds__(64 * META_WAVES) void meta_scatter_kernel(
   if (s == 0 && lane == 0) off[E] = carry;
   __builtin_amdgcn_wave_barrier();
 
-  const int64_t lo = (int64_t)s * SEG;
-  const int64_t hi = lo + SEG < TK ? lo + SEG : TK;
-  const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-  for (int64_t j0 = lo; j0 < hi; j0 += 64) {
-    const int64_t j = j0 + lane;
-    const bool valid = j < hi;
-    int e = valid ? expert_idx[j] : 0;
-    const bool in_range = valid && e >= 0 && e < E;
-    if (!in_range) e = 0;
-    uint64_t peers = __ballot(in_range);
-    for (int b = 0; b < ebits; b++) {
-      const uint64_t bal = __ballot((e >> b) & 1);
-      peers &= ((e >> b) & 1) ? bal : ~bal;
-    }
-    int32_t pos = 0;
-    if (in_range) {
-      pos = cursor[e] + __popcll(peers & lt_mask);
-    }
-    __builtin_amdgcn_wave_barrier();
-    if (in_range && (peers >> lane) >> 1 == 0) cursor[e] = pos + 1;  // highest peer lane advances the cursor
-    __builtin_amdgcn_wave_barrier();
-    if (in_range) {
-      sidx[pos] = (int32_t)j;
-      ridx[j] = pos;
-      gidx[pos] = token_idx ? token_idx[j] : (int32_t)(j / K);
-    }
-    if (tok_off && valid) {
-      if (token_idx) {
-        const int32_t t = token_idx[j];
-        const int32_t tprev = j == 0 ? -1 : token_idx[j - 1];
-        for (int32_t u = tprev + 1; u <= t; u++) tok_off[u] = (int32_t)j;
-        if (j == TK - 1)
-          for (int64_t u = (int64_t)t + 1; u <= T; u++) tok_off[u] = (int32_t)TK;
-      } else {
-        if (j % K == 0) tok_off[j / K] = (int32_t)j;
-        if (j == TK - 1) tok_off[T] = (int32_t)TK;
-      }
-    }
+#pragma unroll
+  for (int i = 0; i < SEG_STEPS; i++) {
+    const int64_t j = lo + i * 64 + lane;
+    if (lo + i * 64 < TK)
+      place_slots(ids[i], j, j < TK, lane, token_idx, TK, T, E, K, ebits, cursor, gidx, sidx, ridx, tok_off);
   }
   if (tok_off && TK == 0 && s == 0)
     for (int64_t u = lane; u <= T; u += 64) tok_off[u] = 0;
+}
+
+// The three passes as one workgroup, for few slots: what they cost there is launches and one round trip to memory after
+// the other.  Wavefront w owns M1_STEPS * 64 consecutive slots at most, whose expert ids it reads once, all at the start;
+// histograms, scan and cursors stay in LDS.  The line at M1_SLOTS: one compute unit ranks 64 slots of each of its 16
+// wavefronts in about a microsecond, the three launches and their dependent reads take 20.  Three passes -> one, us:
+// 8 slots, E = 128 7.5 -> 4.5; 512 slots 14.7 -> 4.7; 3108 slots, E = 48 21.8 -> 7.3; 8192 slots, E = 128 24.6 -> 12.8.
+constexpr int M1_WAVES = 16, M1_STEPS = 8, M1_SLOTS = M1_WAVES * M1_STEPS * 64, M1_MAX_E = 512;
+
+__global__ __launch_bounds__(64 * M1_WAVES) void meta_one_kernel(
+    const int32_t* __restrict__ expert_idx, const int32_t* __restrict__ token_idx, int TK, int64_t T, int E, int K,
+    int ebits, int steps, int32_t* __restrict__ freq, int32_t* __restrict__ off, int32_t* __restrict__ gidx,
+    int32_t* __restrict__ sidx, int32_t* __restrict__ ridx, int32_t* __restrict__ tok_off) {
+  extern __shared__ int32_t lds[];  // M1_WAVES x E
+  __shared__ int32_t wave_total[M1_WAVES];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int32_t* cursor = lds + wave * E;
+  const int first = wave * steps * 64 + lane;
+  int ids[M1_STEPS];
+#pragma unroll
+  for (int i = 0; i < M1_STEPS; i++) {
+    const int j = first + i * 64;
+    ids[i] = i < steps && TK > 0 ? expert_idx[j < TK ? j : TK - 1] : -1;  // (no condition per lane: no wait per load)
+  }
+#pragma unroll
+  for (int i = 0; i < M1_STEPS; i++) ids[i] = first + i * 64 < TK ? (int)opaque(ids[i]) : -1;
+  for (int e = lane; e < E; e += 64) cursor[e] = 0;
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int i = 0; i < M1_STEPS; i++)
+    if (ids[i] >= 0 && ids[i] < E) atomicAdd(&cursor[ids[i]], 1);
+  __syncthreads();
+  // thread e: the wavefronts' counts of expert e become their starts inside the expert, the total the expert's count
+  int32_t total = 0;
+  if (tid < E) {
+#pragma unroll
+    for (int w = 0; w < M1_WAVES; w++) {
+      const int32_t n = lds[w * E + tid];
+      lds[w * E + tid] = total;
+      total += n;
+    }
+  }
+  int32_t upto = total;
+  for (int d = 1; d < 64; d <<= 1) {
+    const int32_t o = __shfl_up(upto, d, 64);
+    if (lane >= d) upto += o;
+  }
+  if (lane == 63) wave_total[wave] = upto;
+  __syncthreads();
+  int32_t begin = upto - total;
+  for (int w = 0; w < wave; w++) begin += wave_total[w];
+  if (tid < E) {
+    freq[tid] = total;
+    off[tid] = begin;
+    if (tid == E - 1) off[E] = begin + total;
+#pragma unroll
+    for (int w = 0; w < M1_WAVES; w++) lds[w * E + tid] += begin;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < M1_STEPS; i++) {
+    const int j = first + i * 64;
+    if (i < steps && j - lane < TK)
+      place_slots(ids[i], j, j < TK, lane, token_idx, TK, T, E, K, ebits, cursor, gidx, sidx, ridx, tok_off);
+  }
+  if (tok_off && TK == 0)
+    for (int64_t u = tid; u <= T; u += 64 * M1_WAVES) tok_off[u] = 0;
 }
 
 }  // namespace smoe
@@ -522,6 +666,14 @@ static int launch_routing_metadata(const int32_t* expert_idx, const int32_t* tok
   int32_t* base_t = hist_t + (size_t)E * NS;
   int ebits = 0;
   while ((1 << ebits) < E) ebits++;
+  if (TK <= M1_SLOTS && E <= M1_MAX_E) {
+    const int steps = (int)ceil_div(TK, 64 * M1_WAVES);
+    hipLaunchKernelGGL(meta_one_kernel, dim3(1), dim3(64 * M1_WAVES), (size_t)M1_WAVES * E * sizeof(int32_t), st, expert_idx,
+                       token_idx, (int)TK, T, E, K, ebits, steps, freq, off, x_gather_idx, s_scatter_idx,
+                       s_reverse_scatter_idx, tok_off);
+    SMOE_LAUNCH_CHECK();
+    return SMOE_OK;
+  }
   const dim3 grid_seg((unsigned)ceil_div(NS, META_WAVES)), block_seg(64 * META_WAVES);
   const size_t smem = (size_t)META_WAVES * E * sizeof(int32_t);
   hipLaunchKernelGGL(meta_hist_kernel, grid_seg, block_seg, smem, st, expert_idx, TK, E, NS, hist_t);
