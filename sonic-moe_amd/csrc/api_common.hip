@@ -21,7 +21,7 @@ void set_error(const char* fmt, ...) {
 
 namespace {
 std::once_flag g_tuning_once;
-Tuning g_tuning = {1, 0, 2, 1, 1, 8, 1, 16};
+Tuning g_tuning = {1, 0, 2, 1, 1, 8, 1, 1, 16};
 
 struct Knob {
   const char* name;
@@ -37,6 +37,7 @@ const Knob g_knobs[] = {
     {"gemm_asm", "SMOE_GEMM_ASM", &Tuning::gemm_asm, 0, 1, 1},
     {"gemm_group_tiles", "SMOE_GEMM_GROUP_TILES", &Tuning::gemm_group_tiles, 1, TILE_GROUP_MAX, 8},
     {"gemm_group_snake", "SMOE_GEMM_GROUP_SNAKE", &Tuning::gemm_group_snake, 0, 1, 1},
+    {"gemm_small_tiles", "SMOE_GEMM_SMALL_TILES", &Tuning::gemm_small_tiles, 0, 2, 1},
     {"gemm_skinny_rows", "SMOE_GEMM_SKINNY_ROWS", &Tuning::gemm_skinny_rows, 0, 1 << 20, 16},
 };
 

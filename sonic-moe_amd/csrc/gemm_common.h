@@ -1279,6 +1279,7 @@ struct Tuning {
   int gemm_asm;             // 1: the tile streams run on the hand-scheduled four-wavefront loop (tile_loop_gen.h)
   int gemm_group_tiles;     // most token tiles of one expert that sweep the feature tiles together (tile streams)
   int gemm_group_snake;     // 1: consecutive groups of an expert sweep the feature tiles in opposite directions
+  int gemm_small_tiles;     // 1: grouped GEMMs whose 256 x 256 tiles are too few or mostly padding take 128 x 128; 2: all do
   int gemm_skinny_rows;     // most token rows per expert, on average, that take the skinny forward GEMM (0: none do)
 };
 const Tuning& tuning();

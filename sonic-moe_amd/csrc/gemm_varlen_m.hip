@@ -8,6 +8,8 @@
 #include "gemm_common.h"
 #include "tile_loop_gen.h"
 
+#include <math.h>
+
 namespace smoe {
 
 // ROLE_COMBINE: the down-projection forward that adds its score-weighted rows onto the tokens' output rows instead of
@@ -271,6 +273,8 @@ __global__ __launch_bounds__(C::NT) void varlen_m_kernel(const VarlenMParams p) 
     da.ds_partial = p.ds_partial;
     da.ds_cols = p.ds_cols;
     da.ds_col = nt * C::WN + wn;
+    // the table has DS_COLS_PER_TILE columns per 256 of the output: a last tile of 128 fills the missing ones too
+    if (C::BN == 128 && nt == p.n_tiles - 1 && (nt & 1) == 0) da.ds_pad_col1 = da.ds_col + C::WN + 1;
     da.m_base = m_base;
     da.row_end = row_end;
     da.n_base = n_base;
@@ -722,6 +726,59 @@ static bool offsets_fit32(const VarlenMParams& p, bool qmn, bool all_rows) {
   return p.q_stride_row > 0 && q_rows * p.q_stride_row * 2 <= lim;
 }
 
+// 128 x 128 tiles, four wavefronts as 2 x 2, two workgroups to a compute unit: for problems whose 256 x 256 tiles do not
+// fill the chip, fill it unevenly (288 tiles on 256 compute units) or are mostly padding.  Per product of full tiles
+// this kernel is half as slow again (0.0025 us per tile and stage of 64 over the whole chip, against 1.6 us per stage and
+// round of 256 tiles), per tile of a few rows it wastes less.
+template <bool QMN>
+using SmallCfg = Cfg<128, 128, 2, 2, QMN, 64, 2>;
+
+// Where the line lies: the time of either kernel in us as measured, bf16, SwiGLU, even load, weights out of the caches,
+// E x rows per expert of (H, I); "a/b" is 256 / 128 for up, down, dz, dx:
+//   8 x 256 of (512, 256)      23/13 16/9 42/19 20/12         8 x 2048    26/26 18/17 48/29 23/23
+//   48 x 85 of (1472, 704)     76/58 43/34 56/47 68/60        48 x 341    110/111 59/60 111/79 99/108
+//   128 x 32 of (768, 256)     36/28 27/20 42/25 39/30        128 x 512   80/91 48/58 95/76 74/88
+//   128 x 64 of (1536, 256)    56/49 38/34 59/36 59/53        128 x 128   59/73 39/42 64/53 65/69
+//   128 x 32 of (4096, 1024)   383/550 210/222 223/227 399/522
+// The terms: 256-row tiles come in rounds of one per compute unit, a round that is not full costs most of a full one, and
+// the epilogue of dz costs as much as 15 stages; of the 128-row tiles an unfilled chip runs any number in the time of its
+// latencies; 4.3 TB/s is what that kernel draws from memory.  A small margin goes to the 256-row tiles.
+static bool small_tiles_pay(const VarlenMParams& p, int role, int64_t TK, int E, int cus) {
+  const Tuning& tune = tuning();
+  if (tune.gemm_small_tiles != 1) return tune.gemm_small_tiles == 2;
+  const double experts = (double)(TK < E ? TK : E), rows = (double)TK / E, stages = p.Kdim / 64.0;
+  // token tiles: one per expert while the rows stay clear of the tile's height, else half a tile of padding each
+  const double m256 = rows <= 192 ? experts : E * (rows / 256 + 0.5);
+  const double m128 = rows <= 96 ? experts : E * (rows / 128 + 0.5);
+  const double full = m256 * (double)ceil_div(p.N, 256) / cus, up = ceil(full);
+  const double rounds = role == ROLE_DZ ? up : full < 1 ? 1 : 0.6 * up + 0.4 * full;
+  const double t256 = rounds * (1.6 * stages + (role == ROLE_DZ ? 24 : role == ROLE_UP_FWD ? 6 : 5)) + 0.15 * stages + 4;
+  double waves = m128 * (double)ceil_div(p.N, 128) / (2.0 * cus);  // of two workgroups per compute unit
+  if (waves > 1) waves = 0.6 * waves + 0.4 * ceil(waves);
+  double t128 = 9 + 512 * waves * (0.0025 * stages + (role == ROLE_DZ ? 0.023 : 0.003));
+  const double bytes = 2.0 * (experts * p.N * p.Kdim + (double)TK * ((double)p.N + p.Kdim));
+  if (t128 < bytes / 4.3e6) t128 = bytes / 4.3e6;
+  return t128 < 0.95 * t256;
+}
+
+template <class C, int ROLE, int ACT>
+static int launch_small_tiles(VarlenMParams& p, const int32_t* off, void* workspace, int64_t TK, int E, hipStream_t st) {
+  static LdsLimitOnce lds_limit;
+  auto kern = varlen_m_kernel<C, ROLE, ACT>;
+  const int rc_attr = lds_limit.ensure((const void*)kern, C::SMEM);
+  if (rc_attr) return rc_attr;
+  p.tm = carve_tile_map(workspace, TK, E, C::BM);
+  const int rc = launch_build_tile_map(off, p.order, E, C::BM, p.tm, st);
+  if (rc) return rc;
+  p.n_tiles = (int)ceil_div(p.N, C::BN);
+  if (ROLE == ROLE_DZ) p.ds_cols = (int)ceil_div(p.N, 256) * DS_COLS_PER_TILE;
+  const int64_t grid = ceil_div(max_token_tiles(TK, E, C::BM) * p.n_tiles, 8) * 8;
+  SMOE_REQUIRE(grid < (1ll << 31) && tile_map_fits(TK, E, C::BM), SMOE_ERR_UNSUPPORTED, "grouped gemm: too many tiles");
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(C::NT), C::SMEM, st, p);
+  SMOE_LAUNCH_CHECK();
+  return SMOE_OK;
+}
+
 template <class C, int ROLE, int ACT>
 static int launch_varlen_m(VarlenMParams& p, const int32_t* off, void* workspace, int64_t TK, int E, hipStream_t st) {
   if constexpr (!C::QMN && (ROLE == ROLE_UP_FWD || ROLE == ROLE_PLAIN)) {
@@ -743,6 +800,12 @@ static int launch_varlen_m(VarlenMParams& p, const int32_t* off, void* workspace
     g.Kdim = p.Kdim;
     g.E = E;
     if (skinny_gemm_takes(g, TK)) return launch_skinny_gemm(g, ROLE == ROLE_UP_FWD ? ACT : -1, TK, st);
+  }
+  if constexpr (ROLE != ROLE_COMBINE) {
+    int cus = 0;
+    const int rc_cu = device_compute_units(&cus);
+    if (rc_cu) return rc_cu;
+    if (small_tiles_pay(p, ROLE, TK, E, cus)) return launch_small_tiles<SmallCfg<C::QMN>, ROLE, ACT>(p, off, workspace, TK, E, st);
   }
   static LdsLimitOnce lds_limit;
   auto kern = varlen_m_kernel<C, ROLE, ACT>;
