@@ -112,6 +112,14 @@ int smoe_topk_softmax_fwd(const void* logits, int dtype, int64_t T, int E, int K
 int smoe_softmax_topk_bwd(void* dlogits, int dtype, int64_t row_stride, const void* dlogits_add, const float* dscores,
                           const float* scores, const int32_t* indices, int64_t T, int K, void* stream);
 
+/* The whole gradient of the router logits, every element written: dlogits[t, e] = outside[t, e] (0 when outside is NULL)
+ * + s_k (ds_k - sum_j ds_j s_j) where e = idx[t, k], added in fp32 and rounded once.  smoe_softmax_topk_bwd onto a zero
+ * fill and an addition, in one pass.  outside has dlogits' dtype, its rows outside_stride elements apart; it is not
+ * dlogits itself. */
+int smoe_router_logit_grad(void* dlogits, int dtype, int64_t row_stride, const void* outside, int64_t outside_stride,
+                           const float* dscores, const float* scores, const int32_t* indices, int64_t T, int E, int K,
+                           void* stream);
+
 /* Backward of the top-K WITHOUT softmax (smoe_topk_softmax_fwd with softmax == 0): dlogits[t, indices[t, k]] =
  * dvalues[t, k]; the caller zero-fills dlogits.  Replaces sonicmoe::_topk_bwd (sonicmoe/functional/backward.py:559-610;
  * no caller inside the reference's layer entry points).  dvalues (T, K) fp32 contiguous, dlogits has `dtype`. */
@@ -241,6 +249,9 @@ int smoe_up_projection_backward(const void* x, const void* w1, int64_t w1_stride
  * dlogits (T, E) and x (T, H) contiguous bf16; E and H multiples of 8. */
 int smoe_router_weight_grad(const void* dlogits, const void* x, void* partial, int64_t T, int E, int H, int chunks,
                             void* stream);
+
+/* That sum: out[i] = sum of partial[c][i] over the chunks, in fp32 and chunk order, i < n; n a multiple of 8, bf16. */
+int smoe_sum_chunks(const void* partial, int chunks, int64_t n, void* out, void* stream);
 
 /* The router in one pass over x (bf16): logits = x Wr^T, the top-K winners of every row with their softmax scores, and
  * optionally the column sums of the full row softmax, all from the GEMM's accumulators.  Replaces the chain

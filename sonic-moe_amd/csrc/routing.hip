@@ -224,6 +224,65 @@ __global__ __launch_bounds__(256) void softmax_topk_bwd_kernel(T* __restrict__ d
   }
 }
 
+// The whole gradient of the router logits: the scatter above onto whatever gradient reached the logits from outside (the
+// load-balancing loss), or onto zeros, in one pass that writes every row.  As a zero fill, the scatter and an add it was
+// three launches and five passes over (T, E); T = 6001, E = 128, K = 8: 11.2 -> 4.0 us, T = 40960: 17.5 -> 10.0.
+// A thread owns VEC columns of a row and looks for the row's K winners among them.
+template <typename T, int VEC>
+__global__ __launch_bounds__(256) void router_logit_grad_kernel(T* __restrict__ dlogits, int64_t row_stride,
+                                                                const T* __restrict__ outside, int64_t outside_stride,
+                                                                const float* __restrict__ dscores,
+                                                                const float* __restrict__ scores,
+                                                                const int32_t* __restrict__ indices, int64_t Trows, int E,
+                                                                int K, int pieces, int rows_per_block) {
+  struct alignas(sizeof(T) * VEC) Pack {
+    T e[VEC];
+  };
+  const int64_t row = (int64_t)blockIdx.x * rows_per_block + threadIdx.x / pieces;
+  if ((int)threadIdx.x / pieces >= rows_per_block || row >= Trows) return;
+  const float* g = dscores + row * K;
+  const float* s = scores + row * K;
+  const int32_t* ix = indices + row * K;
+  float dot = 0.f;
+  for (int k = 0; k < K; k++) dot += g[k] * s[k];
+  for (int piece = threadIdx.x % pieces; piece * VEC < E; piece += pieces) {
+    const int c0 = piece * VEC;
+    float v[VEC];
+    Pack p;
+    if (outside != nullptr) p = *(const Pack*)(outside + row * outside_stride + c0);
+#pragma unroll
+    for (int j = 0; j < VEC; j++) v[j] = outside != nullptr ? __uint_as_float(load_as_f32_bits<T>(&p.e[j])) : 0.f;
+    for (int k = 0; k < K; k++) {
+      const int c = ix[k] - c0;
+      const float add = s[k] * (g[k] - dot);
+#pragma unroll
+      for (int j = 0; j < VEC; j++) v[j] = c == j ? v[j] + add : v[j];
+    }
+#pragma unroll
+    for (int j = 0; j < VEC; j++) store_from_f32<T>(&p.e[j], v[j]);
+    *(Pack*)(dlogits + row * row_stride + c0) = p;
+  }
+}
+
+template <typename T>
+static void launch_router_logit_grad(void* dlogits, int64_t row_stride, const void* outside, int64_t outside_stride,
+                                     const float* dscores, const float* scores, const int32_t* indices, int64_t T_, int E,
+                                     int K, hipStream_t st) {
+  constexpr int VEC = 16 / sizeof(T);
+  const bool wide = E % VEC == 0 && row_stride % VEC == 0 && aligned16(dlogits) &&
+                    (outside == nullptr || (outside_stride % VEC == 0 && aligned16(outside)));
+  const int pieces = (int)ceil_div(E, wide ? VEC : 1);
+  const int columns = pieces < 256 ? pieces : 256;  // threads of a row
+  const int rows_per_block = 256 / columns;
+  const dim3 grid((unsigned)ceil_div(T_, rows_per_block)), block(256);
+  if (wide)
+    hipLaunchKernelGGL((router_logit_grad_kernel<T, VEC>), grid, block, 0, st, (T*)dlogits, row_stride, (const T*)outside,
+                       outside_stride, dscores, scores, indices, T_, E, K, columns, rows_per_block);
+  else
+    hipLaunchKernelGGL((router_logit_grad_kernel<T, 1>), grid, block, 0, st, (T*)dlogits, row_stride, (const T*)outside,
+                       outside_stride, dscores, scores, indices, T_, E, K, columns, rows_per_block);
+}
+
 // Backward of the un-fused top-K (values without softmax): the gradient of a selected logit is the gradient of its
 // value.  One thread per token; the caller has zero-filled dlogits.
 template <typename T>
@@ -599,6 +658,33 @@ extern "C" int smoe_softmax_topk_bwd(void* dlogits, int dtype, int64_t row_strid
       break;
     default:
       set_error("softmax_topk_bwd: unknown dtype %d", dtype);
+      return SMOE_ERR_INVALID;
+  }
+  SMOE_LAUNCH_CHECK();
+  return SMOE_OK;
+}
+
+extern "C" int smoe_router_logit_grad(void* dlogits, int dtype, int64_t row_stride, const void* outside,
+                                      int64_t outside_stride, const float* dscores, const float* scores,
+                                      const int32_t* indices, int64_t T, int E, int K, void* stream) {
+  SMOE_REQUIRE(T >= 0 && T < (1ll << 31) && E >= 1 && K >= 1, SMOE_ERR_INVALID, "router_logit_grad: bad sizes");
+  if (T == 0) return SMOE_OK;
+  SMOE_REQUIRE(dlogits && dscores && scores && indices, SMOE_ERR_INVALID, "router_logit_grad: null pointer");
+  SMOE_REQUIRE(row_stride >= E && (outside == nullptr || outside_stride >= E || T == 1), SMOE_ERR_INVALID,
+               "router_logit_grad: row stride below E");
+  hipStream_t st = (hipStream_t)stream;
+  switch (dtype) {
+    case SMOE_DT_BF16:
+      launch_router_logit_grad<uint16_t>(dlogits, row_stride, outside, outside_stride, dscores, scores, indices, T, E, K, st);
+      break;
+    case SMOE_DT_F16:
+      launch_router_logit_grad<__half>(dlogits, row_stride, outside, outside_stride, dscores, scores, indices, T, E, K, st);
+      break;
+    case SMOE_DT_F32:
+      launch_router_logit_grad<float>(dlogits, row_stride, outside, outside_stride, dscores, scores, indices, T, E, K, st);
+      break;
+    default:
+      set_error("router_logit_grad: unknown dtype %d", dtype);
       return SMOE_ERR_INVALID;
   }
   SMOE_LAUNCH_CHECK();

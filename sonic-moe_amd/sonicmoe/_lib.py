@@ -31,6 +31,7 @@ _SIGNATURES = {
     "smoe_count_cumsum": (c_int, [_P, _I, _L, _I, _P, _P, _P]),
     "smoe_topk_softmax_fwd": (c_int, [_P, _I, _L, _I, _I, _L, _P, _P, _I, _P]),
     "smoe_softmax_topk_bwd": (c_int, [_P, _I, _L, _P, _P, _P, _P, _L, _I, _P]),
+    "smoe_router_logit_grad": (c_int, [_P, _I, _L, _P, _L, _P, _P, _P, _L, _I, _I, _P]),
     "smoe_topk_bwd": (c_int, [_P, _I, _L, _P, _P, _L, _I, _P]),
     "smoe_routing_metadata_workspace_bytes": (c_size_t, [_L, _I]),
     "smoe_routing_metadata": (c_int, [_P, _P, _L, _L, _I, _I, _P, _P, _P, _P, _P, _P, _P, _Z, _P]),
@@ -56,6 +57,7 @@ _SIGNATURES = {
         [_P, _P, _L, _L, _P, _P, _L, _L, _P, _P, _P, _P, _P, _L, _L, _I, _I, _I, _I, _P, _Z, _P],
     ),
     "smoe_router_weight_grad": (c_int, [_P, _P, _P, _L, _I, _I, _I, _P]),
+    "smoe_sum_chunks": (c_int, [_P, _I, _L, _P, _P]),
     "smoe_router_fused_partials": (ctypes.c_int64, [_L, _I]),
     "smoe_router_forward_fused": (c_int, [_P, _P, _L, _I, _I, _I, _P, _P, _P, _P, _P]),
     "smoe_switch_loss_from_partials": (c_int, [_P, _L, _I, _P, _P, _P, _P]),

@@ -23,8 +23,10 @@ from ..enums import ActivationType, is_glu
 from .backward import (
     _down_projection_backward,
     _down_projection_weight_grad,
+    _router_logit_grad,
     _router_weight_grad,
     _softmax_topk_bwd,
+    _sum_chunks,
     _switch_loss_bwd,
     _token_broadcast_backward,
     _up_projection_backward,
@@ -449,7 +451,11 @@ def _router_wgrad(dlogits: torch.Tensor, x: torch.Tensor, like: torch.Tensor) ->
     if fast and T >= 256 and os.environ.get("SMOE_ROUTER_WGRAD", "1") != "0":
         partial = torch.empty(router_weight_grad_chunks(T, E, H), E, H, dtype=x.dtype, device=x.device)
         run(_router_weight_grad, dlogits.contiguous(), x.contiguous(), partial)
-        return partial.sum(0, dtype=torch.float32).to(like.dtype) if partial.size(0) > 1 else partial[0]
+        if partial.size(0) == 1:
+            return partial[0]
+        dw = torch.empty(E, H, dtype=x.dtype, device=x.device)
+        run(_sum_chunks, partial, dw)
+        return dw.to(like.dtype)
     return dlogits.t() @ x
 
 
@@ -502,10 +508,10 @@ class _TCLayerFunction(torch.autograd.Function):
             dout, x, w1, w2, b2, z, scores.view(-1), off, gidx, sidx, ridx, tok_off, K, False, activation_type, stream_id,
             has_b1, ctx.order, ctx.fp8_backward,
         )
-        dlogits = torch.zeros(T, E, dtype=logits_dtype, device=x.device)
-        run(_softmax_topk_bwd, dlogits, None, ds.view(T, K), scores, indices, K)
-        if dlogits_outside is not None:
-            dlogits = dlogits + dlogits_outside
+        dlogits = torch.empty(T, E, dtype=logits_dtype, device=x.device)
+        if dlogits_outside is not None and (dlogits_outside.stride(1) != 1 or dlogits_outside.stride(0) < E):
+            dlogits_outside = dlogits_outside.clone(memory_format=torch.contiguous_format)
+        run(_router_logit_grad, dlogits, dlogits_outside, ds.view(T, K), scores, indices)
         dwr = _router_wgrad(dlogits, x, router_w) if ctx.needs_input_grad[1] else None
         if ctx.needs_input_grad[0]:
             dx.addmm_(dlogits, router_w)  # dx_experts + dlogits Wr in the GEMM's epilogue

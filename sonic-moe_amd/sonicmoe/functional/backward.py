@@ -235,6 +235,32 @@ def _softmax_topk_bwd(
     _lib.check(rc, "_softmax_topk_bwd")
 
 
+@operator("_router_logit_grad", mutates_args={"dlogits"})
+def _router_logit_grad(
+    dlogits: torch.Tensor,
+    outside: Optional[torch.Tensor],
+    dtopk_score: torch.Tensor,
+    topk_router_score: torch.Tensor,
+    topk_router_indices: torch.Tensor,
+) -> None:
+    """dlogits (T, E) = outside (or zeros), plus the gradient of `_softmax_topk_bwd` at the selected logits; every element
+    is written."""
+    _lib.require_device(dlogits, outside, dtopk_score, topk_router_score, topk_router_indices)
+    if dlogits.dtype not in _lib.DT_CODE:
+        raise NotImplementedError(f"_router_logit_grad: unsupported dtype {dlogits.dtype}")
+    assert outside is None or (outside.dtype == dlogits.dtype and outside.shape == dlogits.shape and outside.stride(1) == 1)
+    T, E = dlogits.shape
+    dtopk_score = dtopk_score.contiguous().float()
+    assert topk_router_score.is_contiguous() and topk_router_indices.is_contiguous() and dlogits.stride(1) == 1
+    assert dtopk_score.shape == topk_router_score.shape == topk_router_indices.shape
+    rc = _lib.lib().smoe_router_logit_grad(
+        _lib.ptr(dlogits), _lib.DT_CODE[dlogits.dtype], dlogits.stride(0), _lib.ptr(outside),
+        0 if outside is None else outside.stride(0), _lib.ptr(dtopk_score), _lib.ptr(topk_router_score),
+        _lib.ptr(topk_router_indices), T, E, dtopk_score.size(1), _lib.current_stream_handle(),
+    )
+    _lib.check(rc, "_router_logit_grad")
+
+
 @operator("_topk_bwd", mutates_args={"dlogits_full"})
 def _topk_bwd(dlogits_full: torch.Tensor, dtopk_values: torch.Tensor, topk_indices: torch.Tensor, K: int) -> None:
     """dlogits_full[t, idx[t,k]] = dtopk_values[t,k]: backward of `_topk_fwd` without the softmax fusion; the caller
@@ -266,6 +292,17 @@ def _router_weight_grad(dlogits: torch.Tensor, x: torch.Tensor, partial: torch.T
         _lib.ptr(dlogits), _lib.ptr(x), _lib.ptr(partial), T, E, H, partial.size(0), _lib.current_stream_handle()
     )
     _lib.check(rc, "_router_weight_grad")
+
+
+@operator("_sum_chunks", mutates_args={"out"})
+def _sum_chunks(partial: torch.Tensor, out: torch.Tensor) -> None:
+    """out = partial.sum(0), added in fp32."""
+    _lib.require_device(partial, out)
+    dt = _elem_dtype(("partial", partial), ("out", out))
+    assert partial.is_contiguous() and out.is_contiguous() and partial.shape[1:] == out.shape
+    rc = _lib.lib(dt).smoe_sum_chunks(_lib.ptr(partial), partial.size(0), out.numel(), _lib.ptr(out),
+                                      _lib.current_stream_handle())
+    _lib.check(rc, "_sum_chunks")
 
 
 def router_weight_grad_chunks(T: int, E: int, H: int) -> int:

@@ -1,0 +1,73 @@
+"""Gradient of the router logits in one pass, and the sum of the token chunks of the router's weight gradient."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+EPS = {torch.bfloat16: 2.0**-7, torch.float16: 2.0**-10, torch.float32: 2.0**-23}  # spacing of the values at 1 (8, 11, 24 bits)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("outside", ["none", "dense", "padded rows", "odd offset"])
+@pytest.mark.parametrize("T,E,K", [(1, 8, 2), (257, 128, 8), (33, 100, 5), (19, 2056, 4), (5, 4096, 16), (700, 3, 3)])
+def test_router_logit_grad(dev, T, E, K, outside, dtype):
+    from sonicmoe.functional import backward as bwd
+
+    g = torch.Generator().manual_seed(T * E + K)
+    idx = torch.stack([torch.randperm(E, generator=g)[:K] for _ in range(T)]).to(torch.int32).to(dev)
+    scores = torch.rand(T, K, generator=g).softmax(1).to(dev)
+    ds = torch.randn(T, K, generator=g).to(dev)
+    out_grad = None
+    if outside != "none":
+        pad, lead = {"dense": (0, 0), "padded rows": (16, 0), "odd offset": (3, 1)}[outside]
+        out_grad = torch.randn(T, E + pad, generator=g).to(dtype).to(dev)[:, lead : lead + E]
+    dlogits = torch.full((T, E), 7.0, dtype=dtype, device=dev)
+    bwd._router_logit_grad(dlogits, out_grad, ds, scores, idx)
+    ref = torch.zeros(T, E, dtype=torch.float64, device=dev) if out_grad is None else out_grad.double()
+    s, d = scores.double(), ds.double()
+    add = s * (d - (s * d).sum(1, keepdim=True))
+    ref = ref.scatter_add(1, idx.long(), add)
+    # one rounding to the stored type, and fp32 sums of K products: (K + 3) roundings of at most |s| |ds| each
+    bound = EPS[dtype] * ref.abs() / 2 + (K + 3) * 2.0**-24 * (d.abs().sum(1, keepdim=True) + ref.abs()) + 1e-7
+    assert ((dlogits.double() - ref).abs() <= bound).all()
+    if out_grad is not None:  # what no expert was picked for passes through
+        picked = torch.zeros(T, E, dtype=torch.bool, device=dev).scatter(1, idx.long(), True)
+        assert torch.equal(dlogits[~picked], out_grad[~picked])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("chunks,E,H", [(1, 8, 8), (3, 8, 264), (4, 16, 128), (64, 128, 768)])
+def test_sum_chunks(dev, chunks, E, H, dtype):
+    from sonicmoe.functional import backward as bwd
+
+    partial = torch.randn(chunks, E, H, generator=torch.Generator().manual_seed(chunks)).to(dtype).to(dev)
+    out = torch.full((E, H), 7.0, dtype=dtype, device=dev)
+    bwd._sum_chunks(partial, out)
+    ref = partial.double().sum(0)
+    bound = EPS[dtype] * ref.abs() / 2 + chunks * 2.0**-24 * partial.double().abs().sum(0) + 1e-7
+    assert ((out.double() - ref).abs() <= bound).all()
+
+
+def test_gradient_from_outside_in_any_layout(dev):
+    """The gradient that reaches router_logits may be expanded, transposed or narrowed."""
+    from sonicmoe import MoE
+    from sonicmoe.enums import ActivationType
+    from sonicmoe.functional import moe_TC_softmax_topk_layer
+
+    torch.manual_seed(3)
+    moe = MoE(16, 2, 128, 64, ActivationType.SWIGLU, False, 0.02).to(device=dev, dtype=torch.bfloat16)
+    x = torch.randn(64, 128, device=dev).to(torch.bfloat16)
+    base = torch.randn(16, 64, device=dev).to(torch.bfloat16)
+    row = torch.randn(16, device=dev).to(torch.bfloat16)
+
+    def dx(grad):
+        xi = x.clone().requires_grad_()
+        out, logits, _ = moe_TC_softmax_topk_layer(xi, moe.router.weight, moe.c_fc.weight.permute(1, 2, 0), None,
+                                                   moe.c_proj.weight.permute(1, 2, 0), None, 2,
+                                                   torch.cuda.current_stream().cuda_stream)
+        return torch.autograd.grad([out, logits], [xi, moe.router.weight], [torch.ones_like(out), grad])
+
+    for grad in (base.t(), row.expand(64, 16)):
+        for a, b in zip(dx(grad), dx(grad.contiguous().clone())):
+            assert torch.equal(a, b)
