@@ -860,14 +860,22 @@ extern "C" int smoe_mx_quantize(const void* src, int64_t src_stride, int64_t R, 
 // ---- scale words of a gathered token operand in grouped row order ---------------------------------------------------
 // The GEMM kernels fetch one scale word per tile row and stage.  Through the gather index that is one cache line per
 // row (64 scattered 4-byte reads per load instruction); from a table in grouped order it is two lines per 64 rows.
-// dst[g][m] = src[g][gidx[m]] for the KB 128-element blocks of the contraction.
+// dst[g][m] = src[g][gidx[m]] for the KB 128-element blocks of the contraction, GS_BLOCKS of them to a thread: all its loads
+// before its stores (as one loop over 32 blocks per thread, 64 workgroups for 16384 rows: 11.0 -> 5.1 us).
+constexpr int GS_BLOCKS = 4;
 __global__ __launch_bounds__(256) void gather_scale_rows_kernel(const uint32_t* __restrict__ src, int64_t src_rows,
                                                                 const int32_t* __restrict__ gidx,
                                                                 uint32_t* __restrict__ dst, int64_t TK, int KB) {
   const int64_t m = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (m >= TK) return;
   const int64_t r = gidx[m];
-  for (int g = 0; g < KB; g++) dst[(int64_t)g * TK + m] = src[(int64_t)g * src_rows + r];
+  const int g0 = blockIdx.y * GS_BLOCKS;
+  uint32_t v[GS_BLOCKS];
+#pragma unroll
+  for (int i = 0; i < GS_BLOCKS; i++) v[i] = src[(int64_t)(g0 + i < KB ? g0 + i : KB - 1) * src_rows + r];
+#pragma unroll
+  for (int i = 0; i < GS_BLOCKS; i++)
+    if (g0 + i < KB) dst[(int64_t)(g0 + i) * TK + m] = v[i];
 }
 
 static size_t grouped_scales_offset(int64_t TK, int E) { return (tile_map_bytes(TK, E) + 255) / 256 * 256; }
@@ -880,7 +888,8 @@ static int group_token_scales(Fp8Params& p, void* workspace, size_t workspace_by
   const size_t at = grouped_scales_offset(TK, E);
   if (p.gidx == nullptr || workspace_bytes < at + (size_t)KB * TK * sizeof(uint32_t)) return SMOE_OK;
   uint32_t* dst = (uint32_t*)((char*)workspace + at);
-  hipLaunchKernelGGL(gather_scale_rows_kernel, dim3((unsigned)ceil_div(TK, 256)), dim3(256), 0, st, p.p_scales,
+  hipLaunchKernelGGL(gather_scale_rows_kernel, dim3((unsigned)ceil_div(TK, 256), (unsigned)ceil_div(KB, GS_BLOCKS)), dim3(256),
+                     0, st, p.p_scales,
                      p.p_rows, p.gidx, dst, TK, KB);
   SMOE_LAUNCH_CHECK();
   p.p_scales = dst;
