@@ -11,8 +11,10 @@ import torch
 
 from .enums import LIBRARY_NAME
 
-# argument types for which the dispatcher would do nothing but call the body: not tensor subclasses
-_PLAIN = frozenset((torch.Tensor, torch.nn.Parameter, type(None), int, float, bool, str))
+# The dispatcher would do nothing but call the body for these values and for tensors that are no subclass, have memory (a
+# meta tensor stops at the fake implementation) and hold their values as they are (a lazily negated view is resolved).
+_TENSORS = (torch.Tensor, torch.nn.Parameter)
+_VALUES = frozenset((type(None), int, float, bool, str))
 
 
 def operator(name: str, mutates_args: set[str]):
@@ -37,9 +39,11 @@ def run(op, *args) -> None:
         and torch._C._functorch.peek_interpreter_stack() is None  # vmap, grad, functionalization
         and not torch._C._is_torch_function_mode_enabled()
         and torch._C._get_tracing_state() is None  # torch.jit.trace
+        and not args[0].is_meta  # (every operator's first argument is a tensor, and all of one call are on one device)
     ):
         for a in args:
-            if type(a) not in _PLAIN:
+            kind = type(a)
+            if kind not in _VALUES and (kind not in _TENSORS or a.is_neg()):
                 break
         else:
             op = getattr(op, "body", op)  # (a plain function put in an operator's place is called as it is)

@@ -89,3 +89,32 @@ def test_compiled_code_keeps_the_operator():
     out = torch.zeros(3)
     torch.compile(lambda t, o: (run(_test_copy, t, o, 2.0), o + 1)[1], backend=backend, fullgraph=True)(torch.ones(3), out)
     assert any("_test_copy" in t for t in seen) and torch.equal(out, torch.full((3,), 2.0))
+
+
+def test_meta_tensors_stop_at_the_fake_implementation():
+    run(_test_copy, torch.empty(3, device="meta"), torch.empty(3, device="meta"), 2.0)
+    assert not BODY_CALLS
+
+
+def test_lazily_negated_views_are_resolved():
+    x, out = torch.randn(3), torch.zeros(3)
+    seen = []
+    body = _test_copy.body
+    _test_copy.body = lambda *args: seen.append(args)
+    try:
+        run(_test_copy, torch._neg_view(x), out, 2.0)
+    finally:
+        _test_copy.body = body
+    assert not seen and torch.equal(out, -x * 2)
+
+
+def test_layer_shapes_on_the_meta_device():
+    from sonicmoe import MoE
+    from sonicmoe.enums import ActivationType
+
+    with torch.device("meta"):
+        moe = MoE(8, 2, 128, 64, ActivationType.SWIGLU, False, 0.02).to(torch.bfloat16)
+        x = torch.empty(32, 128, dtype=torch.bfloat16, requires_grad=True)
+    out, aux = moe(x)
+    (dx,) = torch.autograd.grad(out, [x], torch.empty_like(out))
+    assert out.shape == dx.shape == (32, 128) and aux.shape == () and out.is_meta
