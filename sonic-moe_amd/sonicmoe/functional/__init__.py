@@ -453,9 +453,11 @@ def _router_wgrad(dlogits: torch.Tensor, x: torch.Tensor, like: torch.Tensor) ->
         run(_router_weight_grad, dlogits.contiguous(), x.contiguous(), partial)
         if partial.size(0) == 1:
             return partial[0]
+        if like.dtype != x.dtype:  # (fp32 router weights under autocast: the sum keeps its 32 bits)
+            return partial.sum(0, dtype=torch.float32).to(like.dtype)
         dw = torch.empty(E, H, dtype=x.dtype, device=x.device)
         run(_sum_chunks, partial, dw)
-        return dw.to(like.dtype)
+        return dw
     return dlogits.t() @ x
 
 

@@ -49,6 +49,24 @@ def test_sum_chunks(dev, chunks, E, H, dtype):
     assert ((out.double() - ref).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gradient_of_fp32_router_weights(dev, dtype):
+    """fp32 router weights beside 16-bit logits (autocast): the chunks' sum is not rounded to 16 bits on its way."""
+    from sonicmoe.functional import _router_wgrad
+    from sonicmoe.functional.backward import _router_weight_grad, router_weight_grad_chunks
+
+    T, E, H = 1500, 16, 264
+    g = torch.Generator().manual_seed(9)
+    dlogits, x = torch.randn(T, E, generator=g).to(dtype).to(dev), torch.randn(T, H, generator=g).to(dtype).to(dev)
+    dw = _router_wgrad(dlogits, x, torch.empty(E, H, device=dev))
+    partial = torch.empty(router_weight_grad_chunks(T, E, H), E, H, dtype=dtype, device=dev)
+    assert partial.size(0) > 1
+    _router_weight_grad(dlogits, x, partial)
+    assert dw.dtype == torch.float32
+    assert ((dw.double() - partial.double().sum(0)).abs() <= partial.size(0) * 2.0**-24 * partial.double().abs().sum(0)).all()
+    assert not torch.equal(dw, dw.to(dtype).float())  # more than 16 bits are there
+
+
 def test_gradient_from_outside_in_any_layout(dev):
     """The gradient that reaches router_logits may be expanded, transposed or narrowed."""
     from sonicmoe import MoE
