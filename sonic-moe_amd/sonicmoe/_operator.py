@@ -12,7 +12,8 @@ import torch
 from .enums import LIBRARY_NAME
 
 # The dispatcher would do nothing but call the body for these values and for tensors that are no subclass, have memory (a
-# meta tensor stops at the fake implementation) and hold their values as they are (a lazily negated view is resolved).
+# meta tensor stops at the fake implementation, a zero tensor without memory is filled) and hold their values as they are
+# (a lazily negated view is resolved).
 _TENSORS = (torch.Tensor, torch.nn.Parameter)
 _VALUES = frozenset((type(None), int, float, bool, str))
 
@@ -43,7 +44,7 @@ def run(op, *args) -> None:
     ):
         for a in args:
             kind = type(a)
-            if kind not in _VALUES and (kind not in _TENSORS or a.is_neg()):
+            if kind not in _VALUES and (kind not in _TENSORS or a.is_neg() or a._is_zerotensor()):
                 break
         else:
             op = getattr(op, "body", op)  # (a plain function put in an operator's place is called as it is)

@@ -108,6 +108,17 @@ def test_lazily_negated_views_are_resolved():
     assert not seen and torch.equal(out, -x * 2)
 
 
+def test_zero_tensors_without_memory_are_filled():
+    out, seen = torch.ones(3), []
+    body = _test_copy.body
+    _test_copy.body = lambda *args: seen.append(args)
+    try:
+        run(_test_copy, torch._efficientzerotensor((3,)), out, 2.0)
+    finally:
+        _test_copy.body = body
+    assert not seen and not out.any()
+
+
 def test_layer_shapes_on_the_meta_device():
     from sonicmoe import MoE
     from sonicmoe.enums import ActivationType
