@@ -1,8 +1,9 @@
 """Operators of the `sonicmoe::` namespace and how the layer calls them.
 
 Every operator is a torch custom op: what traces, transforms or intercepts PyTorch calls sees it.  The dispatcher's way
-to such an op costs about 20 us of host time per call, more than most of its kernels take on a few tokens; where nothing
-looks on, `run` calls the operator's Python body (its argument checks and the C entry point) directly.
+to such an op costs about 20 us of host time per call, more than most of its kernels take on a few tokens; where none of
+the observers below looks on, `run` calls the operator's Python body (its argument checks and the C entry point) directly.
+An ExecutionTraceObserver without a profiler around it gives no sign of itself: its trace lacks the operators.
 """
 
 from __future__ import annotations
@@ -40,6 +41,7 @@ def run(op, *args) -> None:
         and torch._C._functorch.peek_interpreter_stack() is None  # vmap, grad, functionalization
         and not torch._C._is_torch_function_mode_enabled()
         and torch._C._get_tracing_state() is None  # torch.jit.trace
+        and not torch.autograd._profiler_enabled()  # its rows come from the dispatcher
         and not args[0].is_meta  # (every operator's first argument is a tensor, and all of one call are on one device)
     ):
         for a in args:

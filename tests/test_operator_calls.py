@@ -79,6 +79,14 @@ def test_function_modes_subclasses_and_tracing_take_the_operator(monkeypatch):
     assert len(taken) == 4 and not BODY_CALLS
 
 
+def test_profilers_see_the_operator():
+    x, out = torch.randn(3), torch.zeros(3)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU], record_shapes=True) as profile:
+        run(_test_copy, x, out, 2.0)
+    (row,) = [r for r in profile.key_averages(group_by_input_shape=True) if r.key == "sonicmoe::_test_copy"]
+    assert row.count == 1 and row.input_shapes[:2] == [[3], [3]]
+
+
 def test_compiled_code_keeps_the_operator():
     seen = []
 
