@@ -244,12 +244,14 @@ def _router_logit_grad(
     topk_router_indices: torch.Tensor,
 ) -> None:
     """dlogits (T, E) = outside (or zeros), plus the gradient of `_softmax_topk_bwd` at the selected logits; every element
-    is written."""
+    is written.  `outside` may have any strides."""
     _lib.require_device(dlogits, outside, dtopk_score, topk_router_score, topk_router_indices)
     if dlogits.dtype not in _lib.DT_CODE:
         raise NotImplementedError(f"_router_logit_grad: unsupported dtype {dlogits.dtype}")
-    assert outside is None or (outside.dtype == dlogits.dtype and outside.shape == dlogits.shape and outside.stride(1) == 1)
+    assert outside is None or (outside.dtype == dlogits.dtype and outside.shape == dlogits.shape)
     T, E = dlogits.shape
+    if outside is not None and (outside.stride(1) != 1 or outside.stride(0) < E):
+        outside = outside.clone(memory_format=torch.contiguous_format)
     dtopk_score = dtopk_score.contiguous().float()
     assert topk_router_score.is_contiguous() and topk_router_indices.is_contiguous() and dlogits.stride(1) == 1
     assert dtopk_score.shape == topk_router_score.shape == topk_router_indices.shape

@@ -67,8 +67,9 @@ def test_gradient_of_fp32_router_weights(dev, dtype):
     assert not torch.equal(dw, dw.to(dtype).float())  # more than 16 bits are there
 
 
-def test_gradient_from_outside_in_any_layout(dev):
-    """The gradient that reaches router_logits may be expanded, transposed or narrowed."""
+@pytest.fixture
+def layer_grads(dev):
+    """Gradients of a small layer for a gradient of its output and one of its router logits."""
     from sonicmoe import MoE
     from sonicmoe.enums import ActivationType
     from sonicmoe.functional import moe_TC_softmax_topk_layer
@@ -76,16 +77,29 @@ def test_gradient_from_outside_in_any_layout(dev):
     torch.manual_seed(3)
     moe = MoE(16, 2, 128, 64, ActivationType.SWIGLU, False, 0.02).to(device=dev, dtype=torch.bfloat16)
     x = torch.randn(64, 128, device=dev).to(torch.bfloat16)
-    base = torch.randn(16, 64, device=dev).to(torch.bfloat16)
-    row = torch.randn(16, device=dev).to(torch.bfloat16)
 
-    def dx(grad):
+    def grads(grad, dout=torch.ones_like):
         xi = x.clone().requires_grad_()
         out, logits, _ = moe_TC_softmax_topk_layer(xi, moe.router.weight, moe.c_fc.weight.permute(1, 2, 0), None,
                                                    moe.c_proj.weight.permute(1, 2, 0), None, 2,
                                                    torch.cuda.current_stream().cuda_stream)
-        return torch.autograd.grad([out, logits], [xi, moe.router.weight], [torch.ones_like(out), grad])
+        return torch.autograd.grad([out, logits], [xi, moe.router.weight], [dout(out), grad])
 
+    return grads
+
+
+def test_gradient_from_outside_in_any_layout(dev, layer_grads):
+    """The gradient that reaches router_logits may be expanded, transposed or narrowed."""
+    base = torch.randn(16, 64, device=dev).to(torch.bfloat16)
+    row = torch.randn(16, device=dev).to(torch.bfloat16)
     for grad in (base.t(), row.expand(64, 16)):
-        for a, b in zip(dx(grad), dx(grad.contiguous().clone())):
+        for a, b in zip(layer_grads(grad), layer_grads(grad.contiguous().clone())):
             assert torch.equal(a, b)
+
+
+def test_zero_gradients_without_memory(dev, layer_grads):
+    zero = torch._efficientzerotensor((64, 16), dtype=torch.bfloat16, device=dev)
+    for a, b in zip(layer_grads(zero), layer_grads(torch.zeros(64, 16, dtype=torch.bfloat16, device=dev))):
+        assert torch.equal(a, b)
+    for a in layer_grads(zero, lambda out: torch._efficientzerotensor(out.shape, dtype=out.dtype, device=dev)):
+        assert not a.any()
