@@ -103,3 +103,11 @@ def test_zero_gradients_without_memory(dev, layer_grads):
         assert torch.equal(a, b)
     for a in layer_grads(zero, lambda out: torch._efficientzerotensor(out.shape, dtype=out.dtype, device=dev)):
         assert not a.any()
+
+
+def test_sparse_gradient_from_outside(dev, layer_grads):
+    """A sparse gradient (an embedding lookup on the logits, say) counts as the dense one."""
+    rows = torch.tensor([5, 9, 5], device=dev)
+    grad = torch.sparse_coo_tensor(rows[None], torch.randn(3, 16, device=dev).to(torch.bfloat16), (64, 16))
+    for a, b in zip(layer_grads(grad), layer_grads(grad.to_dense())):
+        assert torch.equal(a, b)
