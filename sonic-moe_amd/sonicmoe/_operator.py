@@ -18,6 +18,13 @@ from .enums import LIBRARY_NAME
 _TENSORS = (torch.Tensor, torch.nn.Parameter)
 _VALUES = frozenset((type(None), int, float, bool, str))
 
+# Dispatch keys of a plain tensor under which somebody else may register an implementation of an operator (the operator's
+# own registrations are under alias keys), and the names, "namespace/operator/key", of all that Python code has registered
+# (a torch without that record: every call takes the dispatcher).
+_KEYS = ("CUDA", "AutogradCUDA", "AutocastCUDA", "CPU", "AutogradCPU", "AutocastCPU", "BackendSelect",
+         "CompositeImplicitAutograd")
+_REGISTERED = getattr(torch.library, "_impls", None)
+
 
 def operator(name: str, mutates_args: set[str]):
     """torch.library.custom_op in this package's namespace; the undecorated function is kept as `.body`."""
@@ -25,6 +32,7 @@ def operator(name: str, mutates_args: set[str]):
     def register(body):
         op = torch.library.custom_op(f"{LIBRARY_NAME}::{name}", mutates_args=mutates_args)(body)
         op.body = body
+        op.elsewhere = frozenset(f"{LIBRARY_NAME}/{name}/{key}" for key in _KEYS)
         return op
 
     return register
@@ -49,5 +57,7 @@ def run(op, *args) -> None:
             if kind not in _VALUES and (kind not in _TENSORS or a.is_neg() or a._is_zerotensor()):
                 break
         else:
-            op = getattr(op, "body", op)  # (a plain function put in an operator's place is called as it is)
+            # (a plain function put in an operator's place is called as it is)
+            if hasattr(op, "body") and _REGISTERED is not None and _REGISTERED.isdisjoint(op.elsewhere):
+                op = op.body
     op(*args)

@@ -87,6 +87,31 @@ def test_profilers_see_the_operator():
     assert row.count == 1 and row.input_shapes[:2] == [[3], [3]]
 
 
+@pytest.mark.parametrize("how", ["Library.impl", "register_kernel"])
+def test_implementations_registered_elsewhere_are_called(how):
+    @operator(f"_test_{how.split('.')[0].lower()}", mutates_args={"out"})
+    def op(x: torch.Tensor, out: torch.Tensor) -> None:
+        out.copy_(x)
+
+    def sevens(x, out):
+        out.fill_(7.0)
+
+    x, out = torch.ones(3), torch.zeros(3)
+    run(op, x, out)
+    assert torch.equal(out, x)
+    if how == "Library.impl":
+        with torch.library._scoped_library("sonicmoe", "IMPL") as lib:
+            lib.impl(op._name, sevens, "CPU")
+            run(op, x, out)
+        assert out.eq(7).all()
+        run(op, x, out)
+        assert torch.equal(out, x)
+    else:
+        torch.library.register_kernel(f"sonicmoe::{op._name}", "cpu", sevens)
+        run(op, x, out)
+        assert out.eq(7).all()
+
+
 def test_compiled_code_keeps_the_operator():
     seen = []
 
