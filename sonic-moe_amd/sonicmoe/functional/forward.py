@@ -9,7 +9,7 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
-from .._operator import operator
+from .._operator import operator, run
 from ..enums import ACTIVATION_CODE, ActivationType
 from ..utils import expert_major_strides
 
@@ -94,7 +94,7 @@ def _topk_fwd(
 def _softmax_topk_fwd(
     router_logits: torch.Tensor, topk_router_score: torch.Tensor, topk_router_indices: torch.Tensor, E: int, K: int
 ) -> None:
-    _topk_fwd.body(router_logits, K, topk_router_score, topk_router_indices, True)
+    run(_topk_fwd, router_logits, K, topk_router_score, topk_router_indices, True)
 
 
 @operator("_up_projection_forward", mutates_args={"z", "y1"})

@@ -112,6 +112,19 @@ def test_implementations_registered_elsewhere_are_called(how):
         assert out.eq(7).all()
 
 
+def test_operator_inside_an_operator():
+    """The softmax router is built on the plain top-K operator; who looks on sees both."""
+    from sonicmoe.functional.forward import _softmax_topk_fwd
+
+    calls = []
+    logits, scores, indices = torch.randn(4, 8), torch.empty(4, 2), torch.empty(4, 2, dtype=torch.int32)
+    with torch.library._scoped_library("sonicmoe", "IMPL") as lib:
+        lib.impl("_topk_fwd", lambda *args: calls.append(args[1]), "CPU")
+        _softmax_topk_fwd(logits, scores, indices, 8, 2)
+        run(_softmax_topk_fwd, logits, scores, indices, 8, 2)
+    assert calls == [2, 2]
+
+
 def test_compiled_code_keeps_the_operator():
     seen = []
 
