@@ -21,7 +21,7 @@ void set_error(const char* fmt, ...) {
 
 namespace {
 std::once_flag g_tuning_once;
-Tuning g_tuning = {1, 0, 2, 1, 1, 8, 1, 1, 16};
+Tuning g_tuning = {1, 0, 2, 1, 1, 8, 1, 1, -1, 16};
 
 struct Knob {
   const char* name;
@@ -38,6 +38,7 @@ const Knob g_knobs[] = {
     {"gemm_group_tiles", "SMOE_GEMM_GROUP_TILES", &Tuning::gemm_group_tiles, 1, TILE_GROUP_MAX, 8},
     {"gemm_group_snake", "SMOE_GEMM_GROUP_SNAKE", &Tuning::gemm_group_snake, 0, 1, 1},
     {"gemm_small_tiles", "SMOE_GEMM_SMALL_TILES", &Tuning::gemm_small_tiles, 0, 2, 1},
+    {"varlen_k_stream_rows", "SMOE_VARLEN_K_STREAM_ROWS", &Tuning::varlen_k_stream_rows, 0, 1 << 30, -1},
     {"gemm_skinny_rows", "SMOE_GEMM_SKINNY_ROWS", &Tuning::gemm_skinny_rows, 0, 1 << 20, 16},
 };
 
@@ -147,8 +148,8 @@ extern "C" int smoe_set_tuning(const char* name, int value) {
   for (const smoe::Knob& k : smoe::g_knobs) {
     if (strcmp(name, k.name) != 0) continue;
     if (value < 0) value = k.def;
-    SMOE_REQUIRE(value >= k.lo && value <= k.hi, SMOE_ERR_INVALID, "set_tuning: %s = %d outside [%d, %d]", name, value,
-                 k.lo, k.hi);
+    SMOE_REQUIRE(value == k.def || (value >= k.lo && value <= k.hi), SMOE_ERR_INVALID, "set_tuning: %s = %d outside [%d, %d]",
+                 name, value, k.lo, k.hi);
     smoe::g_tuning.*(k.field) = value;
     return SMOE_OK;
   }

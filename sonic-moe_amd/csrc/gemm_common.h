@@ -1280,6 +1280,7 @@ struct Tuning {
   int gemm_group_tiles;     // most token tiles of one expert that sweep the feature tiles together (tile streams)
   int gemm_group_snake;     // 1: consecutive groups of an expert sweep the feature tiles in opposite directions
   int gemm_small_tiles;     // 1: grouped GEMMs whose 256 x 256 tiles are too few or mostly padding take 128 x 128; 2: all do
+  int varlen_k_stream_rows; // least rows per expert, on average, of a weight-gradient stream; -1 (default): by output shape
   int gemm_skinny_rows;     // most token rows per expert, on average, that take the skinny forward GEMM (0: none do)
 };
 const Tuning& tuning();

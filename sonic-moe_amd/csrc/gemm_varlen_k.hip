@@ -577,27 +577,44 @@ static int launch_varlen_k(const VarlenKParams& pin, hipStream_t st, void* works
     const int64_t s_rows = C::S_GATHER ? p.gather_rows : p.total_rows + 8 * C::BK;
     const bool fits = p.off != nullptr && p.gidx != nullptr && p.gather_rows > 0 && (r_rows + 1) * p.r_stride * 2 < lim &&
                       (s_rows + 1) * p.s_stride * 2 < lim && (p.total_rows + 8 * C::BK) * 4 < lim;
-    // What a stream saves is the turnaround between the tiles of a workgroup and, per stage, the hand-scheduled loop; it
-    // costs a launch that sorts the experts.  With at most one tile per workgroup and short experts nothing of that is
-    // left (H = 512, I = 256, E = 8, 32 tiles: 256 rows per expert 12.7 us one-tile, 14.1 + 3.2 stream; 1024 rows 27.3 /
-    // 29.2; 4096 rows 85 / 77.  H = 768, E = 32, 192 tiles: 1024 rows 36 / 31, 4096 rows 144 / 103).
-    const bool long_enough = total > 256 || p.total_rows >= 1024ll * p.E;
-    if (tuning().gemm_asm && fits && long_enough && p.E <= SCHED_MAX_E && total < (1ll << 30) && workspace != nullptr &&
-        (size_t)p.E * sizeof(int32_t) <= workspace_bytes) {
-      // a block is ba x bb tiles with ba * bb = 32, as square as the tile counts allow (fewest operand panels per block)
-      UnitShape us = {0, 0, 0, 0, 0, 0};
-      if (total >= 256) {
-        for (int bb : {8, 4, 16, 2, 32, 1}) {
-          if (p.tiles_b % bb == 0 && p.tiles_a % (32 / bb) == 0) {
-            us.bb = bb;
-            us.ba = 32 / bb;
-            us.nbj = p.tiles_b / us.bb;
-            us.nb = (p.tiles_a / us.ba) * us.nbj;
-            us.units = us.nb * p.E;
-            break;
-          }
+    // a block is ba x bb tiles with ba * bb = 32, as square as the tile counts allow (fewest operand panels per block)
+    UnitShape us = {0, 0, 0, 0, 0, 0};
+    if (total >= 256) {
+      for (int bb : {8, 4, 16, 2, 32, 1}) {
+        if (p.tiles_b % bb == 0 && p.tiles_a % (32 / bb) == 0) {
+          us.bb = bb;
+          us.ba = 32 / bb;
+          us.nbj = p.tiles_b / us.bb;
+          us.nb = (p.tiles_a / us.ba) * us.nbj;
+          break;
         }
       }
+    }
+    // Where the line lies, in rows per expert on average.  A stream saves the turnaround between the tiles of a workgroup
+    // and, per stage, has the hand-scheduled loop; it costs a launch that sorts the experts (3 us), runs three stages for
+    // any shorter expert, and its loads wait behind the stores of the tile before.  With few rows all there is to do is to
+    // store the gradients, and the eight-wavefront kernel, one tile per workgroup, does that faster.  dW1, dW2 in us,
+    // one-tile kernel / stream, (H, I), E, even load and, last, popularity by Zipf's law:
+    //   blocks             16 rows           48 rows           70 rows           512 rows, Zipf
+    //   (4096, 1024) 128   390/489 219/252   414/487 232/253   506/494 269/252
+    //   (4096, 1024)  64   205/250 112/132   223/252 122/132   267/251 140/134   778/566 494/306
+    //   (4096, 1536) 128   569/726 284/370   604/727 311/370   739/735 358/374
+    //   (2048, 2048)  32   108/134  61/71    115/133  61/73    138/133  74/74
+    //   (2048, 1024)  16    35/42   20/26     34/42   20/26     40/43   22/26    123/94   84/70
+    //   chunks             16 rows           64 rows           256 rows          256 rows, Zipf
+    //   (1536,  256) 128    45/60   26/36     51/62   28/37     96/79   52/47    132/123 102/95
+    //   (1472,  704)  48    46/63   28/41     53/63   33/41    102/81   61/52    112/108  77/74
+    //   (3072,  640)  32    57/71   32/47     57/72   37/47    104/99   69/59     95/102  69/76
+    // With at most one tile per workgroup more rows are needed: (512, 256), 8, 32 tiles: 256 rows 12.7/17.3, 1024 rows
+    // 27.3/29.2, 4096 rows 85/77; (768, 256), 32, 192 tiles: 1024 rows 36/31.  A schedule that is fixed in advance loses
+    // where all tokens pick the same K experts, because the empty experts' tiles are dealt to the workgroups that hold the
+    // long ones too: (1536, 256) at 384 rows 136/182 129/133, (4096, 1024) at 256 rows 371/405 184/207.
+    const int64_t least = tuning().varlen_k_stream_rows >= 0 ? tuning().varlen_k_stream_rows
+                          : total <= 256 ? 1024 : us.nb > 0 ? 64 : 256;
+    const bool long_enough = p.total_rows >= least * p.E;
+    if (tuning().gemm_asm && fits && long_enough && p.E <= SCHED_MAX_E && total < (1ll << 30) && workspace != nullptr &&
+        (size_t)p.E * sizeof(int32_t) <= workspace_bytes) {
+      us.units = us.nb * p.E;
       if (us.nb == 0) {
         us.chunk = total < 256 ? (int)ceil_div(total, 8) : 32;
         us.units = (int)ceil_div(total, us.chunk);

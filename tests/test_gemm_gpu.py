@@ -332,6 +332,7 @@ def test_weight_gradients_in_chunks(dev, tuning, T, H, I, E, K, skew, empty):
     """Outputs that do not split into blocks of 32 tiles run as tile streams over chunks of tiles of several experts:
     against the oracle (bf16 rounding of the stored result, as everywhere) and, bit for bit, against the one-tile kernel,
     which adds the same products in the same order."""
+    tuning("varlen_k_stream_rows", 0)
     _, bwd = _ops()
     _, w1, w2 = make_weights(E, H, I, dev, seed=T)
     idx, scores, meta, md = make_tc_routing(T, E, K, dev, seed=T + 1, skew=skew, empty=empty)
@@ -364,6 +365,29 @@ def test_weight_gradients_in_chunks(dev, tuning, T, H, I, E, K, skew, empty):
     tuning("gemm_asm", 0)
     for a, b in zip((dw1, dw2), run()):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("H,I,E,rows,streams", [
+    (768, 256, 48, 255, (False, False)), (768, 256, 48, 256, (True, False)),   # chunks (288 tiles), too few tiles (144)
+    (2048, 1024, 9, 63, (False, False)), (2048, 1024, 9, 64, (True, True)),    # blocks of 32 tiles
+])
+def test_weight_gradients_of_few_rows(dev, monkeypatch, H, I, E, rows, streams):
+    """Where the line between the one-tile kernel and the streams lies: only a stream writes (the experts' order) into the
+    workspace."""
+    _, bwd = _ops()
+    TK = E * rows
+    off = torch.arange(0, TK + 1, rows, dtype=torch.int32, device=dev)
+    gidx = torch.arange(TK, dtype=torch.int32, device=dev) % 100
+    x, dout = (torch.randn(100, H, device=dev).to(torch.bfloat16) for _ in range(2))
+    dz, y1s = torch.randn(TK, 2 * I, device=dev).to(torch.bfloat16), torch.randn(TK, I, device=dev).to(torch.bfloat16)
+    w1, dw1 = (torch.empty(E, 2 * I, H, dtype=torch.bfloat16, device=dev).permute(1, 2, 0) for _ in range(2))
+    dw2 = torch.empty(E, H, I, dtype=torch.bfloat16, device=dev).permute(1, 2, 0)
+    stream = torch.cuda.current_stream().cuda_stream
+    make, workspaces = bwd._gemm_workspace, []
+    monkeypatch.setattr(bwd, "_gemm_workspace", lambda *a: workspaces.append(make(*a).fill_(0xEE)) or workspaces[-1])
+    bwd._up_projection_backward(x, w1, None, dw1, dz, None, off, None, gidx, gidx, True, stream)
+    bwd._down_projection_weight_grad(dout, y1s, dw2, None, torch.zeros(TK, device=dev), off, None, gidx, gidx, stream)
+    assert tuple(not w[:4].eq(0xEE).all().item() for w in workspaces) == streams
 
 
 @pytest.mark.parametrize("stream_kernels", [1, 0])
