@@ -9,8 +9,8 @@ namespace smoe {
 // A workgroup owns 64 weight rows (output columns) of one expert and up to 32 of its token rows.  Its four
 // wavefronts split the contraction: wavefront w takes the pieces w, w + 4, ... of 64 elements (128 bytes of every row), so
 // that together they walk through each weight row front to back.  A wavefront loads the matrix-core fragments of weights
-// and tokens straight from memory into registers, DEPTH pieces ahead, and the partial sums of the four are added in LDS
-// in a fixed order.
+// and tokens straight from memory into registers, DEPTH - 1 pieces ahead (two or three, one for blocks of more than 16
+// rows), and the partial sums of the four are added in LDS in a fixed order.
 constexpr int SK_NW = 4, SK_FN = 4, SK_BN = 16 * SK_FN, SK_PIECE = 64, SK_FM_MAX = 2;
 
 constexpr int SK_ROWS = 16 * SK_FM_MAX;
@@ -195,15 +195,29 @@ __global__ __launch_bounds__(SK_NW * 64, DEPTH >= 4 ? 2 : 3) void skinny_gemm_ke
 // the most blocks that TK rows of E experts can make
 static int64_t skinny_blocks(const SkinnyGemm& g, int64_t TK) { return TK / SK_ROWS + (TK < g.E ? TK : g.E); }
 
-// Where the line to the 256 x 256 tile streams lies, in token rows per expert on average.  A tile of those costs the same
-// for one row as for 256, and they need some tiles per compute unit; but they read the weights of an expert with many
-// rows once, where this kernel reads them from the caches again for every 32 rows.  SwiGLU, up + down in us (this kernel /
-// tile streams with their tile map), even load and, behind "|", popularity by Zipf's law:
-//   H = 4096, I = 1024, E = 128   1 token 37 / 104   4 rows 534 / 566 | 245 / 266   8 rows 559 / 576 | 336 / 295
-//   H = 4096, I =  256, E = 256   1 token 29 / 92    8 rows 318 / 342 | 203 / 198   16 rows 341 / 345
-//   H = 1536, I =  256, E = 128   1 token 13 / 50    8 rows 50 / 76 | 45 / 63       16 rows 55 / 77 | 60 / 64
-//   H = 1472, I =  704, E = 48    1 token 14 / 56    11 rows 57 / 103 | 53 / 62
-//   H = 512,  I =  256, E = 8     1 token 8 / 34     16 rows 10 / 34
+// Where the line to the tile kernels lies, in token rows per expert on average.  A tile costs the same for one row as for
+// 128 or 256, and a kernel of tiles needs some of them per compute unit; but it reads the weights of an expert with many
+// rows once, where this kernel reads them from the caches again for every 32 rows.  SwiGLU, us, the tile kernel that would
+// run / this kernel: even load, popularity by Zipf's law, all tokens with the same K experts.
+//   (H, I)        E    rows   up                             down
+//   (4096, 1024)  128   1     275/250  171/116   74/24       157/119   83/55    29/14
+//                       4     368/360  174/174   76/50       209/176   96/86    29/28
+//                       8     369/374  190/237   78/92       210/182  111/118   29/50
+//   (4096,  256)  256   2     183/176   82/79    73/26       111/80    43/34    15/18
+//                       4     194/188   86/103   73/48       120/91    55/46    15/26
+//                       8     194/192  109/136   74/49       124/99    66/68    16/41
+//                      16     195/200  177/190   74/94       130/117   84/108   22/71
+//   (3072, 1408)  256   2     689/649  203/185   62/58       367/319  103/91    34/36
+//                       4     761/729  216/263   64/108      400/357  111/128   33/52
+//   (2048,  512)  256   4     209/187   65/69    44/30       109/93    33/32    13/18
+//                      16     208/200  101/155   45/99       114/109   56/81    18/58
+//   (1536,  256)  128   4      44/38    26/28    21/21        30/20    17/14    10/10
+//                      16      45/43    37/42    22/29        31/23    22/24    10/16
+//   (1472,  704)   48  16      54/44    40/46    21/29        31/24    24/27    14/17
+//   (512,   256)    8  16      12/6     12/7     11/7          9/5      9/5      9/5
+// Where the matrices fill the chip (512 tiles and more) the gain at an even load is small, and how many rows the most
+// popular experts get grows with the rows of the launch: there the line is also drawn by those, sooner for a long
+// contraction, whose workgroups take longer over a second block of rows.
 bool skinny_gemm_takes(const SkinnyGemm& g, int64_t TK) {
   const int64_t lim = 1ll << 31;
   const int most = tuning().gemm_skinny_rows;
@@ -211,6 +225,7 @@ bool skinny_gemm_takes(const SkinnyGemm& g, int64_t TK) {
   if (g.E * ceil_div(g.N, 256) >= 512) {
     rows = (16ll << 20) / ((int64_t)g.N * g.Kdim);
     rows = rows < most / 4 ? most / 4 : rows > most ? most : rows;
+    if (TK > (g.Kdim >= 1024 ? 32ll : 128ll) * most) return false;
   }
   return TK <= rows * g.E && skinny_blocks(g, TK) <= 65535 && g.N % SK_BN == 0 && g.Kdim % SK_PIECE == 0 &&
          g.q_stride_row > 0 && g.N * g.q_stride_row * 2 < lim && g.p_rows * g.p_stride * 2 < lim;

@@ -56,6 +56,27 @@ def test_rows_and_contractions(dev, tuning, counts, H, I, dtype):
         assert (t[TK:] == guard).all()
 
 
+@pytest.mark.parametrize("H,I,E,rows,skinny", [
+    (512, 256, 8, 128, (True, True)), (512, 256, 8, 129, (False, False)),  # 16 rows per expert
+    # matrices that fill the chip: by the number of rows, sooner where the contraction is long
+    (4096, 256, 256, 512, (True, True)), (4096, 256, 256, 513, (False, True)),
+    (4096, 256, 256, 2048, (False, True)), (4096, 256, 256, 2049, (False, False)),
+])
+def test_where_the_line_lies(dev, monkeypatch, H, I, E, rows, skinny):
+    """Only the other kernels write (a tile map) into the workspace."""
+    fwd = _ops()
+    off = (torch.arange(E + 1, device=dev) * rows // E).to(torch.int32)
+    gidx = torch.zeros(rows, dtype=torch.int32, device=dev)
+    x, y1, y2 = (torch.zeros(n, c, dtype=torch.bfloat16, device=dev) for n, c in ((1, H), (rows, I), (rows, H)))
+    w1, w2 = (torch.zeros(E, *s, dtype=torch.bfloat16, device=dev).permute(1, 2, 0) for s in ((2 * I, H), (H, I)))
+    stream = torch.cuda.current_stream().cuda_stream
+    make, workspaces = fwd._gemm_workspace, []
+    monkeypatch.setattr(fwd, "_gemm_workspace", lambda *a: workspaces.append(make(*a).fill_(0xEE)) or workspaces[-1])
+    fwd._up_projection_forward(x, w1, None, y1, None, off, None, gidx, stream, "swiglu", True, True)
+    fwd._down_projection_forward(w2, y1, y2, None, off, None, gidx, stream)
+    assert tuple(w.eq(0xEE).all().item() for w in workspaces) == skinny
+
+
 @pytest.mark.parametrize("act", ["swiglu", "geglu", "reglu", "relu_sq", "relu", "gelu", "silu"])
 def test_epilogues_against_the_tile_streams(dev, tuning, act):
     """Every activation with biases, and z not stored: the same values as the other kernel of the operator up to the order
