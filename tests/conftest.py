@@ -36,3 +36,11 @@ def tuning():
     yield set_knob
     for name in touched:
         _lib.set_tuning(name, -1)
+
+
+@pytest.fixture
+def tile_streams(tuning):
+    """The bf16 / fp16 grouped GEMMs as tile streams whatever the sizes are, for tests that are about those kernels: their
+    problems are small, and on their own would take the kernels for few rows and few tiles."""
+    for knob in ("gemm_small_tiles", "gemm_skinny_rows", "varlen_k_stream_rows"):
+        tuning(knob, 0)

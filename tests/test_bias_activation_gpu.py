@@ -34,10 +34,13 @@ def _problem(dev, T, H, I, E, K, activation, seed, skew=0.0, empty=()):
 
 @pytest.mark.parametrize("activation", ACTIVATIONS)
 @pytest.mark.parametrize("with_bias", [False, True])
-def test_operators_bias_activation(dev, activation, with_bias):
+@pytest.mark.parametrize("kernels", ["by_size", "streams"])
+def test_operators_bias_activation(dev, request, activation, with_bias, kernels):
     from sonicmoe.functional import backward as bwd
     from sonicmoe.functional import forward as fwd
 
+    if kernels == "streams":
+        request.getfixturevalue("tile_streams")
     T, H, I, E, K = 1500, 320, 192, 8, 2  # ragged tiles in every dimension, one empty expert
     glu, N1, w1, w2, b1, b2, x, dout, s_flat, md = _problem(dev, T, H, I, E, K, activation, 7, skew=0.7, empty=(5,))
     if not with_bias:

@@ -32,7 +32,7 @@ SHAPES = [
 
 @pytest.mark.parametrize("gemm_asm", [1, 0])
 @pytest.mark.parametrize("T,H,I,E,K,skew,empty,bias", SHAPES)
-def test_fp16_operator_chain(dev, tuning, gemm_asm, T, H, I, E, K, skew, empty, bias):
+def test_fp16_operator_chain(dev, tuning, tile_streams, gemm_asm, T, H, I, E, K, skew, empty, bias):
     """Every GEMM-side operator of a training step on fp16 tensors, each against the oracle on the operator's own
     inputs, with the hand-scheduled loops and with the compiler-scheduled kernels."""
     from sonicmoe.functional import backward as bwd

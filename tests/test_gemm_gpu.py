@@ -75,7 +75,7 @@ def test_forward_ops(dev, T, H, I, E, K, skew, empty):
 
 
 @pytest.mark.parametrize("rows_short_of_4gib", [2, 1])
-def test_token_tensor_ending_next_to_4gib(dev, rows_short_of_4gib):
+def test_token_tensor_ending_next_to_4gib(dev, tile_streams, rows_short_of_4gib):
     """The tile streams address the gathered token operand with 32-bit byte offsets from the tensor's start, and drop the
     loads of rows behind an expert's end by giving them the tensor's end as offset - unless that end plus a stage offset
     could wrap around 32 bits, in which case they re-read the expert's last row.  A token tensor of 4 GiB less two rows
@@ -104,7 +104,7 @@ def test_token_tensor_ending_next_to_4gib(dev, rows_short_of_4gib):
 
 
 @pytest.mark.parametrize("pad_short", [0, 64])
-def test_weight_view_with_rows_4gib_apart(dev, pad_short):
+def test_weight_view_with_rows_4gib_apart(dev, tile_streams, pad_short):
     """The C ABI takes any weight row stride; the tile streams form weight addresses as 32-bit byte offsets from the
     expert's matrix.  A (N1, E, padded H) storage whose (N1, H, E) view spans exactly 4 GiB per expert must be sent to the
     kernels with 64-bit pointers; 64 columns less, the offsets just fit and the tile stream takes it."""
@@ -216,7 +216,7 @@ STREAM_SHAPES = [
 
 @pytest.mark.parametrize("grid", [8, 24])
 @pytest.mark.parametrize("T,H,I,E,K,skew,empty", STREAM_SHAPES)
-def test_tile_streams(dev, tuning, grid, T, H, I, E, K, skew, empty):
+def test_tile_streams(dev, tuning, tile_streams, grid, T, H, I, E, K, skew, empty):
     """The grouped GEMMs whose workgroups walk through several tiles each: few workgroups (8 = one per XCD, 24) force
     long streams on small problems, so tile switches, the parked epilogue and the last tile of a stream are all hit."""
     tuning("gemm_stream_grid", grid)
@@ -280,7 +280,7 @@ def test_tile_streams(dev, tuning, grid, T, H, I, E, K, skew, empty):
                                         ("varlen_k_tile_order", 0), ("varlen_k_tile_order", 1),
                                         ("gemm_group_tiles", 1), ("gemm_group_tiles", 3), ("gemm_group_tiles", 127),
                                         ("gemm_group_snake", 0)])
-def test_kernel_selection_knobs(dev, tuning, knob, value):
+def test_kernel_selection_knobs(dev, tuning, tile_streams, knob, value):
     """The alternative kernels / tile orders a tuning knob selects give the same results as the defaults
     (bit-identical: the arithmetic of a tile does not depend on who computes it or when; the score gradient is a sum of
     per-wave partial sums over the wave tile's columns, so kernels with different wave tiles agree to fp32 rounding)."""
@@ -314,6 +314,8 @@ def test_kernel_selection_knobs(dev, tuning, knob, value):
 
     base = run()
     tuning(knob, value)
+    if knob == "varlen_k_tile_order":
+        tuning("gemm_asm", 0)  # the weight-gradient streams have a schedule of their own
     other = run()
     for name, a, b in zip(["z", "y1", "y2", "dw1", "dx_expanded", "dz", "ds"], base, other):
         if name == "ds":
@@ -328,11 +330,10 @@ def test_kernel_selection_knobs(dev, tuning, knob, value):
     (2000, 768, 320, 43, 3, 1.2, (0, 42)),   # 387 and 258 tiles of ragged width: whole chunks and a short last one
     (3000, 1472, 704, 16, 4, 0.5, (7,)),     # 36 and 18 tiles per expert
 ])
-def test_weight_gradients_in_chunks(dev, tuning, T, H, I, E, K, skew, empty):
+def test_weight_gradients_in_chunks(dev, tuning, tile_streams, T, H, I, E, K, skew, empty):
     """Outputs that do not split into blocks of 32 tiles run as tile streams over chunks of tiles of several experts:
     against the oracle (bf16 rounding of the stored result, as everywhere) and, bit for bit, against the one-tile kernel,
     which adds the same products in the same order."""
-    tuning("varlen_k_stream_rows", 0)
     _, bwd = _ops()
     _, w1, w2 = make_weights(E, H, I, dev, seed=T)
     idx, scores, meta, md = make_tc_routing(T, E, K, dev, seed=T + 1, skew=skew, empty=empty)
@@ -392,7 +393,7 @@ def test_weight_gradients_of_few_rows(dev, monkeypatch, H, I, E, rows, streams):
 
 @pytest.mark.parametrize("stream_kernels", [1, 0])
 @pytest.mark.parametrize("order_kind", ["reversed", "largest_first", "random"])
-def test_expert_schedule_order(dev, tuning, order_kind, stream_kernels):
+def test_expert_schedule_order(dev, tuning, tile_streams, order_kind, stream_kernels):
     """The four grouped-GEMM operators with an expert_schedule_order (the reference operators' argument,
     sonicmoe/functional/forward.py:61, backward.py:204, :298): every permutation of the experts gives the results of
     the default order bit for bit -- only the order in which the tiles are taken up changes."""

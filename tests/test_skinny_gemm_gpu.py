@@ -109,5 +109,6 @@ def test_epilogues_against_the_tile_streams(dev, tuning, act):
     mine, again = run(True), run(False)
     assert torch.equal(mine[1], again[0]) and torch.equal(mine[2], again[1])
     tuning("gemm_skinny_rows", 0)
+    tuning("gemm_small_tiles", 0)
     for a, b in zip(mine, run(True)):
         assert rel_l2(a, b) < 1e-3
