@@ -227,8 +227,11 @@ __global__ __launch_bounds__(256) void softmax_topk_bwd_kernel(T* __restrict__ d
 // The whole gradient of the router logits: the scatter above onto whatever gradient reached the logits from outside (the
 // load-balancing loss), or onto zeros, in one pass that writes every row.  As a zero fill, the scatter and an add it was
 // three launches and five passes over (T, E); T = 6001, E = 128, K = 8: 11.2 -> 4.0 us, T = 40960: 17.5 -> 10.0.
-// A thread owns VEC columns of a row and looks for the row's K winners among them.
-template <typename T, int VEC>
+// A thread owns VEC columns of a row and looks for the row's K winners among them.  WIDE: they are one aligned piece of 16
+// bytes.  Otherwise they are read and written one by one and lie `pieces` apart, so that neighbouring lanes have
+// neighbouring columns; still VEC to a thread, because the search costs the same for one column as for eight (E = 100,
+// K = 5, T = 40960, bf16: three launches 12.8 us, one column to a thread 32, eight adjacent ones 15.2, eight apart 12.6).
+template <typename T, int VEC, bool WIDE>
 __global__ __launch_bounds__(256) void router_logit_grad_kernel(T* __restrict__ dlogits, int64_t row_stride,
                                                                 const T* __restrict__ outside, int64_t outside_stride,
                                                                 const float* __restrict__ dscores,
@@ -245,22 +248,38 @@ __global__ __launch_bounds__(256) void router_logit_grad_kernel(T* __restrict__ 
   const int32_t* ix = indices + row * K;
   float dot = 0.f;
   for (int k = 0; k < K; k++) dot += g[k] * s[k];
-  for (int piece = threadIdx.x % pieces; piece * VEC < E; piece += pieces) {
-    const int c0 = piece * VEC;
+  constexpr int FIRST = WIDE ? VEC : 1;
+  const int gap = WIDE ? 1 : pieces;  // from one of a thread's columns to the next
+  for (int c0 = (int)threadIdx.x % pieces * FIRST; c0 < E; c0 += pieces * VEC) {
     float v[VEC];
     Pack p;
-    if (outside != nullptr) p = *(const Pack*)(outside + row * outside_stride + c0);
+    if (outside != nullptr) {
+      const T* src = outside + row * outside_stride;
+      if constexpr (WIDE) {
+        p = *(const Pack*)(src + c0);
+      } else {
+#pragma unroll
+        for (int j = 0; j < VEC; j++) p.e[j] = src[c0 + j * gap < E ? c0 + j * gap : E - 1];
+      }
+    }
 #pragma unroll
     for (int j = 0; j < VEC; j++) v[j] = outside != nullptr ? __uint_as_float(load_as_f32_bits<T>(&p.e[j])) : 0.f;
     for (int k = 0; k < K; k++) {
       const int c = ix[k] - c0;
       const float add = s[k] * (g[k] - dot);
 #pragma unroll
-      for (int j = 0; j < VEC; j++) v[j] = c == j ? v[j] + add : v[j];
+      for (int j = 0; j < VEC; j++) v[j] = c == j * gap ? v[j] + add : v[j];
     }
 #pragma unroll
     for (int j = 0; j < VEC; j++) store_from_f32<T>(&p.e[j], v[j]);
-    *(Pack*)(dlogits + row * row_stride + c0) = p;
+    T* dst = dlogits + row * row_stride + c0;
+    if constexpr (WIDE) {
+      *(Pack*)dst = p;
+    } else {
+#pragma unroll
+      for (int j = 0; j < VEC; j++)
+        if (c0 + j * gap < E) dst[j * gap] = p.e[j];
+    }
   }
 }
 
@@ -271,16 +290,16 @@ static void launch_router_logit_grad(void* dlogits, int64_t row_stride, const vo
   constexpr int VEC = 16 / sizeof(T);
   const bool wide = E % VEC == 0 && row_stride % VEC == 0 && aligned16(dlogits) &&
                     (outside == nullptr || (outside_stride % VEC == 0 && aligned16(outside)));
-  const int pieces = (int)ceil_div(E, wide ? VEC : 1);
+  const int pieces = (int)ceil_div(E, VEC);
   const int columns = pieces < 256 ? pieces : 256;  // threads of a row
   const int rows_per_block = 256 / columns;
   const dim3 grid((unsigned)ceil_div(T_, rows_per_block)), block(256);
   if (wide)
-    hipLaunchKernelGGL((router_logit_grad_kernel<T, VEC>), grid, block, 0, st, (T*)dlogits, row_stride, (const T*)outside,
-                       outside_stride, dscores, scores, indices, T_, E, K, columns, rows_per_block);
+    hipLaunchKernelGGL((router_logit_grad_kernel<T, VEC, true>), grid, block, 0, st, (T*)dlogits, row_stride,
+                       (const T*)outside, outside_stride, dscores, scores, indices, T_, E, K, columns, rows_per_block);
   else
-    hipLaunchKernelGGL((router_logit_grad_kernel<T, 1>), grid, block, 0, st, (T*)dlogits, row_stride, (const T*)outside,
-                       outside_stride, dscores, scores, indices, T_, E, K, columns, rows_per_block);
+    hipLaunchKernelGGL((router_logit_grad_kernel<T, VEC, false>), grid, block, 0, st, (T*)dlogits, row_stride,
+                       (const T*)outside, outside_stride, dscores, scores, indices, T_, E, K, columns, rows_per_block);
 }
 
 // Backward of the un-fused top-K (values without softmax): the gradient of a selected logit is the gradient of its
