@@ -722,7 +722,7 @@ extern "C" int smoe_down_projection_backward(const void* dout, const void* z, co
   p.order = expert_schedule_order;
   p.total_rows = TK;
   p.gather_rows = T;
-  // the schedule table may take the place of the tile map: the activation-gradient GEMM that used it ran before
+  // the sorted experts may take the place of the tile map: the activation-gradient GEMM that used it ran before
   return launch_varlen_k_variant<true, false>(p, st, workspace, workspace_bytes);
 }
 
@@ -768,7 +768,7 @@ extern "C" int smoe_up_projection_backward(const void* x, const void* w1, int64_
     p.order = expert_schedule_order;
     p.total_rows = TK;
     p.gather_rows = T;
-    // the schedule table shares the workspace with the tile map the dx GEMM builds afterwards, in stream order
+    // the sorted experts share the workspace with the tile map the dx GEMM builds afterwards, in stream order
     rc = launch_varlen_k_variant<false, true>(p, st, workspace, workspace_bytes);
     if (rc) return rc;
   }

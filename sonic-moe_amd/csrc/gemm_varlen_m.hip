@@ -740,9 +740,14 @@ using SmallCfg = Cfg<128, 128, 2, 2, QMN, 64, 2>;
 //   128 x 32 of (768, 256)     36/28 27/20 42/25 39/30        128 x 512   80/91 48/58 95/76 74/88
 //   128 x 64 of (1536, 256)    56/49 38/34 59/36 59/53        128 x 128   59/73 39/42 64/53 65/69
 //   128 x 32 of (4096, 1024)   383/550 210/222 223/227 399/522
+// and, with popularity by Zipf's law, 256 / as the rule has it:
+//   48 x 65 of (1472, 704)     77/64 44/36 64/47 68/58        128 x 32 of (768, 256)     34/26 28/19 50/26 38/28
+//   128 x 64 of (1536, 256)    52/52 38/34 64/45 55/54        48 x 171 of (1472, 704)    82/82 45/47 68/68 70/70
 // The terms: 256-row tiles come in rounds of one per compute unit, a round that is not full costs most of a full one, and
 // the epilogue of dz costs as much as 15 stages; of the 128-row tiles an unfilled chip runs any number in the time of its
-// latencies; 4.3 TB/s is what that kernel draws from memory.  A small margin goes to the 256-row tiles.
+// latencies; 4.3 TB/s is what that kernel draws from memory.  A small margin goes to the 256-row tiles.  Known misses: up of
+// 128 x 64 of (1536, 256) is priced 52/55 and stays on 256; where all tokens pick the same K experts, (1472, 704) at 171 rows
+// on average takes 49 instead of 44 for up.
 static bool small_tiles_pay(const VarlenMParams& p, int role, int64_t TK, int E, int cus) {
   const Tuning& tune = tuning();
   if (tune.gemm_small_tiles != 1) return tune.gemm_small_tiles == 2;

@@ -554,7 +554,7 @@ class _SwitchLossFunction(torch.autograd.Function):
 def switch_loss(router_logits: torch.Tensor, expert_frequency: torch.Tensor) -> torch.Tensor:
     """Load-balancing loss of the reference's MoE._compute_switch_loss (sonicmoe/moe.py:261-274) from the router
     logits (..., E) and the per-expert token counts (E): the softmax, its column sums, both normalisations and the dot
-    product in two launches forward and one backward, without a (T, E) fp32 tensor."""
+    product in two launches forward (one for up to 64 tokens) and one backward, without a (T, E) fp32 tensor."""
     if router_logits.numel() == 0:  # no tokens: both normalisations clamp and the loss is 0, as in the reference
         acc = F.softmax(router_logits.reshape(-1, router_logits.size(-1)), dim=-1, dtype=torch.float32).sum(0)
         f = F.normalize(expert_frequency.float(), p=1, dim=0)
