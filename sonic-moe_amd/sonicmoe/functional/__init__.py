@@ -511,7 +511,8 @@ class _TCLayerFunction(torch.autograd.Function):
             has_b1, ctx.order, ctx.fp8_backward,
         )
         dlogits = torch.empty(T, E, dtype=logits_dtype, device=x.device)
-        if dlogits_outside is not None and dlogits_outside.layout != torch.strided:
+        # (a compiled backward pass knows dense gradients only, and refuses the question)
+        if not torch.compiler.is_compiling() and dlogits_outside is not None and dlogits_outside.layout != torch.strided:
             dlogits_outside = dlogits_outside.to_dense()
         run(_router_logit_grad, dlogits, dlogits_outside, ds.view(T, K), scores, indices)
         dwr = _router_wgrad(dlogits, x, router_w) if ctx.needs_input_grad[1] else None

@@ -109,5 +109,9 @@ def test_sparse_gradient_from_outside(dev, layer_grads):
     """A sparse gradient (an embedding lookup on the logits, say) counts as the dense one."""
     rows = torch.tensor([5, 9, 5], device=dev)
     grad = torch.sparse_coo_tensor(rows[None], torch.randn(3, 16, device=dev).to(torch.bfloat16), (64, 16))
-    for a, b in zip(layer_grads(grad), layer_grads(grad.to_dense())):
+    dense = layer_grads(grad.to_dense())
+    for a, b in zip(layer_grads(grad), dense):
         assert torch.equal(a, b)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]):  # through the dispatcher
+        for a, b in zip(layer_grads(grad), dense):
+            assert torch.equal(a, b)
