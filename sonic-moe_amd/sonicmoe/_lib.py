@@ -140,8 +140,18 @@ def set_tuning(name: str, value: int) -> None:
     _TUNING[name] = int(value)
 
 
+class NoMemory(RuntimeError):
+    """A tensor with elements but without memory (a zero tensor that nothing has filled)."""
+
+
+def _null(t: torch.Tensor) -> int:
+    if t.numel():
+        raise NoMemory("a tensor without memory reached the HIP library")
+    return 0
+
+
 def ptr(t: torch.Tensor | None):
-    return None if t is None else t.data_ptr()
+    return None if t is None else t.data_ptr() or _null(t)
 
 
 def require_device(*tensors: torch.Tensor | None) -> None:

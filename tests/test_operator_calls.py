@@ -6,6 +6,7 @@ from torch._subclasses.fake_tensor import FakeTensorMode
 from torch.overrides import TorchFunctionMode
 from torch.utils._python_dispatch import TorchDispatchMode
 
+from sonicmoe import _lib
 from sonicmoe._operator import operator, run
 
 BODY_CALLS = []
@@ -155,14 +156,20 @@ def test_lazily_negated_views_are_resolved():
 
 
 def test_zero_tensors_without_memory_are_filled():
-    out, seen = torch.ones(3), []
-    body = _test_copy.body
-    _test_copy.body = lambda *args: seen.append(args)
-    try:
-        run(_test_copy, torch._efficientzerotensor((3,)), out, 2.0)
-    finally:
-        _test_copy.body = body
-    assert not seen and not out.any()
+    pointers = []
+
+    @operator("_test_pointers", mutates_args={"out"})
+    def op(x: torch.Tensor, out: torch.Tensor) -> None:
+        pointers.append((_lib.ptr(x), _lib.ptr(out)))
+        out.copy_(x)
+
+    out = torch.ones(3)
+    run(op, torch._efficientzerotensor((3,)), out)
+    assert len(pointers) == 1 and all(pointers[0]) and not out.any()
+    run(op, torch.empty(0), torch.empty(0))
+    assert len(pointers) == 2
+    with pytest.raises(_lib.NoMemory):
+        _lib.ptr(torch._efficientzerotensor((3,)))
 
 
 def test_layer_shapes_on_the_meta_device():
