@@ -107,4 +107,19 @@ SMOE_DEV uint32_t opaque(uint32_t v) {
 // 1 / (1 + e^-x) with the hardware reciprocal (1 ulp): a correctly rounded division is a dozen instructions per value
 SMOE_DEV float fast_sigmoid(float x) { return __builtin_amdgcn_rcpf(1.0f + __expf(-x)); }
 
+// Raise a kernel's dynamic-LDS limit once per device (the attribute is per device; a repeated call is harmless, so the
+// flags need no lock).
+struct LdsLimitOnce {
+  bool done[64] = {};
+  int ensure(const void* kernel, int bytes) {
+    int dev = 0;
+    SMOE_HIP_CHECK(hipGetDevice(&dev));
+    if (dev < 0 || dev >= 64 || !done[dev]) {
+      SMOE_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+      if (dev >= 0 && dev < 64) done[dev] = true;
+    }
+    return SMOE_OK;
+  }
+};
+
 }  // namespace smoe

@@ -380,44 +380,45 @@ __global__ __launch_bounds__(1024) void inclusive_scan_kernel(const int32_t* __r
 // ============================================================================================================
 // routing metadata: stable counting sort of TK expert ids
 // ============================================================================================================
-// A "segment" is SEG consecutive flat slots, owned by ONE wavefront so that the order inside a segment is the
-// lane / iteration order.  Pass A: per-segment histogram -> hist_t[e][s].  Pass B: one wavefront per expert scans
-// its row of hist_t -> base_t[e][s] (slots of expert e that precede segment s) and freq[e].  Pass C: every
-// segment rebuilds off[] from freq, seeds a cursor per expert and assigns positions with ballot-based ranking.
+// A "segment" is SEG consecutive flat slots, owned by ONE workgroup, whose wavefronts own consecutive quarters of it, so
+// that the order inside a segment is the wavefront / lane / iteration order.  Pass A: per-segment histogram ->
+// hist_t[e][s].  Pass B: one wavefront per expert scans its row of hist_t -> base_t[e][s] (slots of expert e that precede
+// segment s) and freq[e].  Pass C: every segment rebuilds off[] from freq, seeds a cursor per wavefront and expert and
+// assigns positions with ballot-based ranking.
+// All three wait for memory and for chains of dependent instructions, so the ranking is spread over four wavefronts (four
+// steps of 64 slots each instead of sixteen in a row) and takes a slot's token by ONE 32-bit division (two 64-bit ones
+// were half of its instructions).  The three passes, us, one wavefront per segment -> four: 16384 slots, E = 128 22.7 -> 10.9;
+// 48008 23.1 -> 11.4; 327680 26.2 -> 16.5; 10000 slots, E = 4096 77 -> 28.
 constexpr int SEG = 1024;
 constexpr int META_WAVES = 4;
-constexpr int SEG_STEPS = SEG / 64;
+constexpr int SEG_STEPS = SEG / 64 / META_WAVES;  // steps of one wavefront
 
-// The expert ids of a wavefront's segment, -1 past the end: all loads before the first use (taken one step at a time, and
-// under a condition each, every step of the histogram and of the ranking began with a round trip to memory; the three
-// passes at TK = 48008, E = 128: 25.2 -> 22.8 us).
-SMOE_DEV void load_segment(const int32_t* __restrict__ expert_idx, int64_t lo, int64_t TK, int lane, int (&ids)[SEG_STEPS]) {
+// The expert ids of a wavefront's quarter of a segment, -1 past the end: all loads before the first use (taken one step at
+// a time, and under a condition each, every step of the histogram and of the ranking began with a round trip to memory).
+SMOE_DEV void load_segment(const int32_t* __restrict__ expert_idx, int lo, int TK, int lane, int (&ids)[SEG_STEPS]) {
 #pragma unroll
   for (int i = 0; i < SEG_STEPS; i++) {
-    const int64_t j = lo + i * 64 + lane;
-    ids[i] = TK > 0 ? expert_idx[j < TK ? j : TK - 1] : -1;
+    const uint32_t j = (uint32_t)lo + i * 64 + lane;
+    ids[i] = TK > 0 ? expert_idx[j < (uint32_t)TK ? j : TK - 1] : -1;
   }
 #pragma unroll
-  for (int i = 0; i < SEG_STEPS; i++) ids[i] = lo + i * 64 + lane < TK ? (int)opaque(ids[i]) : -1;
+  for (int i = 0; i < SEG_STEPS; i++) ids[i] = (uint32_t)lo + i * 64 + lane < (uint32_t)TK ? (int)opaque(ids[i]) : -1;
 }
 
-__global__ __launch_bounds__(64 * META_WAVES) void meta_hist_kernel(const int32_t* __restrict__ expert_idx,
-                                                                    int64_t TK, int E, int NS,
-                                                                    int32_t* __restrict__ hist_t) {
-  extern __shared__ int32_t lds[];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  int32_t* hist = lds + (size_t)wave * E;
-  const int s = blockIdx.x * META_WAVES + wave;
-  if (s >= NS) return;
+__global__ __launch_bounds__(64 * META_WAVES) void meta_hist_kernel(const int32_t* __restrict__ expert_idx, int TK, int E,
+                                                                    int NS, int32_t* __restrict__ hist_t) {
+  extern __shared__ int32_t hist[];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int s = blockIdx.x;
   int ids[SEG_STEPS];
-  load_segment(expert_idx, (int64_t)s * SEG, TK, lane, ids);
-  for (int e = lane; e < E; e += 64) hist[e] = 0;
-  __builtin_amdgcn_wave_barrier();
+  load_segment(expert_idx, s * SEG + wave * (SEG / META_WAVES), TK, lane, ids);
+  for (int e = tid; e < E; e += 64 * META_WAVES) hist[e] = 0;
+  __syncthreads();
 #pragma unroll
   for (int i = 0; i < SEG_STEPS; i++)
     if (ids[i] >= 0 && ids[i] < E) atomicAdd(&hist[ids[i]], 1);
-  __builtin_amdgcn_wave_barrier();
-  for (int e = lane; e < E; e += 64) hist_t[(size_t)e * NS + s] = hist[e];
+  __syncthreads();
+  for (int e = tid; e < E; e += 64 * META_WAVES) hist_t[(size_t)e * NS + s] = hist[e];
 }
 
 __global__ __launch_bounds__(256) void meta_scan_kernel(const int32_t* __restrict__ hist_t, int E, int NS,
@@ -442,7 +443,7 @@ __global__ __launch_bounds__(256) void meta_scan_kernel(const int32_t* __restric
 
 // One step of the counting sort for a wavefront: lane l holds slot j (consecutive over the lanes, `valid` a prefix of them)
 // of expert e.  Slots of the same expert take consecutive positions from that expert's cursor, in lane order.
-SMOE_DEV void place_slots(int e, int64_t j, bool valid, int lane, const int32_t* __restrict__ token_idx, int64_t TK,
+SMOE_DEV void place_slots(int e, int j, bool valid, int lane, const int32_t* __restrict__ token_idx, int TK,
                           int64_t T, int E, int K, int ebits, int32_t* cursor, int32_t* __restrict__ gidx,
                           int32_t* __restrict__ sidx, int32_t* __restrict__ ridx, int32_t* __restrict__ tok_off) {
   const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
@@ -460,75 +461,100 @@ SMOE_DEV void place_slots(int e, int64_t j, bool valid, int lane, const int32_t*
   __builtin_amdgcn_wave_barrier();
   if (in_range && (peers >> lane) >> 1 == 0) cursor[e] = pos + 1;  // highest peer lane advances the cursor
   __builtin_amdgcn_wave_barrier();
+  // (past the end j may not fit a token: nothing is read or written for it)
+  int32_t t = 0;
+  if (token_idx == nullptr)
+    t = (int32_t)((uint32_t)j / (uint32_t)K);
+  else if (valid)
+    t = token_idx[j];
   if (in_range) {
-    sidx[pos] = (int32_t)j;
+    sidx[pos] = j;
     ridx[j] = pos;
-    gidx[pos] = token_idx ? token_idx[j] : (int32_t)(j / K);
+    gidx[pos] = t;
   }
   if (tok_off && valid) {
     if (token_idx) {
-      const int32_t t = token_idx[j];
       const int32_t tprev = j == 0 ? -1 : token_idx[j - 1];
-      for (int32_t u = tprev + 1; u <= t; u++) tok_off[u] = (int32_t)j;
+      for (int32_t u = tprev + 1; u <= t; u++) tok_off[u] = j;
       if (j == TK - 1)
-        for (int64_t u = (int64_t)t + 1; u <= T; u++) tok_off[u] = (int32_t)TK;
+        for (int64_t u = (int64_t)t + 1; u <= T; u++) tok_off[u] = TK;
     } else {
-      if (j % K == 0) tok_off[j / K] = (int32_t)j;
-      if (j == TK - 1) tok_off[T] = (int32_t)TK;
+      if (j == t * K) tok_off[t] = j;
+      if (j == TK - 1) tok_off[T] = TK;
     }
   }
 }
 
 __global__ __launch_bounds__(64 * META_WAVES) void meta_scatter_kernel(
-    const int32_t* __restrict__ expert_idx, const int32_t* __restrict__ token_idx, int64_t TK, int64_t T, int E,
+    const int32_t* __restrict__ expert_idx, const int32_t* __restrict__ token_idx, int TK, int64_t T, int E,
     int K, int NS, int ebits, const int32_t* __restrict__ freq, const int32_t* __restrict__ base_t,
     int32_t* __restrict__ off, int32_t* __restrict__ gidx, int32_t* __restrict__ sidx, int32_t* __restrict__ ridx,
     int32_t* __restrict__ tok_off) {
-  extern __shared__ int32_t lds[];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  extern __shared__ int32_t lds[];  // META_WAVES x E, then a word per wavefront
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   int32_t* cursor = lds + (size_t)wave * E;
-  const int s = blockIdx.x * META_WAVES + wave;
-  if (s >= NS) return;
-  const int64_t lo = (int64_t)s * SEG;
+  int32_t* wave_total = lds + (size_t)META_WAVES * E;
+  const int s = blockIdx.x;
+  const int lo = s * SEG + wave * (SEG / META_WAVES);
   int ids[SEG_STEPS];
   load_segment(expert_idx, lo, TK, lane, ids);
+  for (int e = lane; e < E; e += 64) cursor[e] = 0;
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int i = 0; i < SEG_STEPS; i++)
+    if (ids[i] >= 0 && ids[i] < E) atomicAdd(&cursor[ids[i]], 1);
 
-  // exclusive scan of freq -> off (every segment needs it; segment 0 also publishes it)
+  // exclusive scan of freq -> off (every segment needs it; segment 0 also publishes it), 256 experts at a time; thread e
+  // turns the wavefronts' counts of expert e into their cursors
   int32_t carry = 0;
-  for (int e0 = 0; e0 < E; e0 += 64) {
-    const int e = e0 + lane;
+  for (int e0 = 0; e0 < E; e0 += 64 * META_WAVES) {
+    const int e = e0 + tid;
     const int32_t f = e < E ? freq[e] : 0;
+    const int32_t base = e < E ? base_t[(size_t)e * NS + s] : 0;
     int32_t v = f;
     for (int d = 1; d < 64; d <<= 1) {
       int32_t o = __shfl_up(v, d, 64);
       if (lane >= d) v += o;
     }
+    if (lane == 63) wave_total[wave] = v;
+    __syncthreads();  // (the first one also: every wavefront's counts are there)
+    int32_t excl = carry + v - f;
+#pragma unroll
+    for (int w = 0; w < META_WAVES; w++) {
+      if (w < wave) excl += wave_total[w];
+      carry += wave_total[w];
+    }
     if (e < E) {
-      const int32_t excl = carry + v - f;
-      cursor[e] = excl + base_t[(size_t)e * NS + s];
+      int32_t at = excl + base;
+#pragma unroll
+      for (int w = 0; w < META_WAVES; w++) {
+        const int32_t n = lds[(size_t)w * E + e];
+        lds[(size_t)w * E + e] = at;
+        at += n;
+      }
       if (s == 0) off[e] = excl;
     }
-    carry += __shfl(v, 63, 64);
+    __syncthreads();
   }
-  if (s == 0 && lane == 0) off[E] = carry;
-  __builtin_amdgcn_wave_barrier();
+  if (s == 0 && tid == 0) off[E] = carry;
 
 #pragma unroll
   for (int i = 0; i < SEG_STEPS; i++) {
-    const int64_t j = lo + i * 64 + lane;
-    if (lo + i * 64 < TK)
-      place_slots(ids[i], j, j < TK, lane, token_idx, TK, T, E, K, ebits, cursor, gidx, sidx, ridx, tok_off);
+    const uint32_t j0 = (uint32_t)lo + i * 64;
+    if (j0 < (uint32_t)TK)
+      place_slots(ids[i], (int)(j0 + lane), j0 + lane < (uint32_t)TK, lane, token_idx, TK, T, E, K, ebits, cursor, gidx,
+                  sidx, ridx, tok_off);
   }
   if (tok_off && TK == 0 && s == 0)
-    for (int64_t u = lane; u <= T; u += 64) tok_off[u] = 0;
+    for (int64_t u = tid; u <= T; u += 64 * META_WAVES) tok_off[u] = 0;
 }
 
 // The three passes as one workgroup, for few slots: what they cost there is launches and one round trip to memory after
 // the other.  Wavefront w owns M1_STEPS * 64 consecutive slots at most, whose expert ids it reads once, all at the start;
 // histograms, scan and cursors stay in LDS.  The line at M1_SLOTS: one compute unit ranks 64 slots of each of its 16
-// wavefronts in about a microsecond, the three launches and their dependent reads take 20.  Three passes -> one, us:
-// 8 slots, E = 128 7.5 -> 4.5; 512 slots 14.7 -> 4.7; 3108 slots, E = 48 21.8 -> 7.3; 8192 slots, E = 128 24.6 -> 12.8.
-constexpr int M1_WAVES = 16, M1_STEPS = 8, M1_SLOTS = M1_WAVES * M1_STEPS * 64, M1_MAX_E = 512;
+// wavefronts in about a microsecond, the three launches and their dependent reads take 10 to 11 us: one workgroup takes 4.7
+// for 512 slots, 7.6 for 3108 (E = 48), 13.5 for 8192.
+constexpr int M1_WAVES = 16, M1_STEPS = 4, M1_SLOTS = M1_WAVES * M1_STEPS * 64, M1_MAX_E = 512;
 
 __global__ __launch_bounds__(64 * M1_WAVES) void meta_one_kernel(
     const int32_t* __restrict__ expert_idx, const int32_t* __restrict__ token_idx, int TK, int64_t T, int E, int K,
@@ -779,13 +805,17 @@ static int launch_routing_metadata(const int32_t* expert_idx, const int32_t* tok
     SMOE_LAUNCH_CHECK();
     return SMOE_OK;
   }
-  const dim3 grid_seg((unsigned)ceil_div(NS, META_WAVES)), block_seg(64 * META_WAVES);
-  const size_t smem = (size_t)META_WAVES * E * sizeof(int32_t);
-  hipLaunchKernelGGL(meta_hist_kernel, grid_seg, block_seg, smem, st, expert_idx, TK, E, NS, hist_t);
+  const dim3 grid_seg((unsigned)NS), block_seg(64 * META_WAVES);
+  const size_t smem = (size_t)META_WAVES * (E + 1) * sizeof(int32_t);
+  static LdsLimitOnce lds_limit;  // E = 4096 is the first size beyond 64 KiB
+  const int rc_attr = lds_limit.ensure((const void*)meta_scatter_kernel, META_WAVES * (4096 + 1) * (int)sizeof(int32_t));
+  if (rc_attr) return rc_attr;
+  hipLaunchKernelGGL(meta_hist_kernel, grid_seg, block_seg, (size_t)E * sizeof(int32_t), st, expert_idx, (int)TK, E, NS,
+                     hist_t);
   SMOE_LAUNCH_CHECK();
   hipLaunchKernelGGL(meta_scan_kernel, dim3((unsigned)ceil_div(E, 4)), dim3(256), 0, st, hist_t, E, NS, base_t, freq);
   SMOE_LAUNCH_CHECK();
-  hipLaunchKernelGGL(meta_scatter_kernel, grid_seg, block_seg, smem, st, expert_idx, token_idx, TK, T, E, K, NS, ebits,
+  hipLaunchKernelGGL(meta_scatter_kernel, grid_seg, block_seg, smem, st, expert_idx, token_idx, (int)TK, T, E, K, NS, ebits,
                      freq, base_t, off, x_gather_idx, s_scatter_idx, s_reverse_scatter_idx, tok_off);
   SMOE_LAUNCH_CHECK();
   return SMOE_OK;

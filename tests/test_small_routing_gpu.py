@@ -31,3 +31,18 @@ def test_metadata_borders(dev, TK, E):
     ref = R.tc_topk_router_metadata(experts.reshape(-1, K), E)
     for key, got in zip(KEYS, choice):
         np.testing.assert_array_equal(got.cpu().numpy(), ref[key], err_msg=key)
+
+
+@pytest.mark.parametrize("E", [8, 256, 257, 4096])
+@pytest.mark.parametrize("TK", [1, 8193, 9216, 9471, 33333])
+def test_metadata_segments(dev, TK, E):
+    """The three passes: segments of 1024 slots, wavefronts of 256, scans of 256 experts, LDS beyond 64 KiB at E = 4096."""
+    from sonicmoe.functional import _build_metadata
+
+    rng = np.random.default_rng(TK + E)
+    experts = (E * rng.random(TK) ** 2).astype(np.int32)
+    K = next(k for k in (7, 3, 1) if TK % k == 0)
+    choice = _build_metadata(torch.from_numpy(experts).to(dev), None, TK // K, E, K)
+    ref = R.tc_topk_router_metadata(experts.reshape(-1, K), E)
+    for key, got in zip(KEYS, choice):
+        np.testing.assert_array_equal(got.cpu().numpy(), ref[key], err_msg=key)
