@@ -400,6 +400,54 @@ int smoe_down_projection_backward_fp8(const void* doutq, const void* dout_scales
 int smoe_score_grad_bias_term(const void* dout, const void* b2, const int32_t* off, const int32_t* x_gather_idx,
                               const int32_t* s_scatter_idx, float* ds, int64_t TK, int H, int E, void* stream);
 
+/* ---------------------------------------------------------------------------------------------------------
+ * The token-choice layer behind its router GEMM, one call per direction (_TC_Softmax_Topk_Router / _UpProjection /
+ * _DownProjection of the reference, sonicmoe/functional/__init__.py:85-420, :437-490): the entry points above in the order
+ * of the operators, on one workspace.  For callers whose time goes into calls rather than kernels.  Every field of the two
+ * structs is 8 bytes wide.  Shapes and limits are those of the entry points; T >= 1; experts in index order.
+ *   smoe_topk_softmax_fwd -> smoe_routing_metadata -> smoe_up_projection_forward -> smoe_down_projection_forward ->
+ *   smoe_gather_sum -> smoe_switch_loss_fwd (loss != NULL)
+ *   smoe_down_projection_backward -> smoe_up_projection_backward -> smoe_gather_sum -> smoe_switch_loss_bwd (loss_grad !=
+ *   NULL) -> smoe_router_logit_grad -> smoe_router_weight_grad and smoe_sum_chunks (router_chunks > 0)
+ * The caller adds the router's share of dx (dlogits Wr) itself. */
+typedef struct {
+  const void *x, *logits, *w1, *b1, *w2, *b2; /* b1, b2: nullable */
+  int64_t w1_stride_e, w1_stride_row, w2_stride_e, w2_stride_row;
+  int64_t logits_dtype, logits_row_stride; /* smoe_dtype; elements */
+  int64_t T, H, I, E, K, activation;
+  void *z, *o; /* z: nullable (not kept) */
+  float* scores;
+  int32_t *indices, *freq, *off, *x_gather_idx, *s_scatter_idx, *s_reverse_scatter_idx, *tok_off;
+  float *loss_acc, *loss; /* loss: nullable */
+  void* workspace;
+  int64_t workspace_bytes;
+} smoe_layer_forward_args;
+size_t smoe_layer_forward_workspace_bytes(int64_t T, int H, int I, int E, int K);
+int smoe_layer_forward(const smoe_layer_forward_args* args, void* stream);
+
+typedef struct {
+  const void *x, *dout, *z, *w1, *w2, *b2; /* b2: nullable */
+  int64_t w1_stride_e, w1_stride_row, w2_stride_e, w2_stride_row;
+  const float* scores;
+  const int32_t *indices, *freq, *off, *x_gather_idx, *s_scatter_idx, *s_reverse_scatter_idx;
+  const void* logits; /* with loss_grad only, as freq and loss_acc */
+  int64_t logits_dtype, logits_row_stride;
+  const float *loss_acc, *loss_grad; /* loss_grad: nullable, one float */
+  const void* outside;               /* nullable: gradient of the logits from outside, in their type */
+  int64_t outside_row_stride;
+  int64_t T, H, I, E, K, activation;
+  void *dw1, *dw2;
+  int64_t dw1_stride_e, dw1_stride_row, dw2_stride_e, dw2_stride_row;
+  void *db1, *db2; /* nullable */
+  void *dx, *dlogits;
+  void* dwr; /* (E, H), router_chunks > 0 only */
+  int64_t router_chunks;
+  void* workspace;
+  int64_t workspace_bytes;
+} smoe_layer_backward_args;
+size_t smoe_layer_backward_workspace_bytes(int64_t T, int H, int I, int E, int K, int activation, int chunks);
+int smoe_layer_backward(const smoe_layer_backward_args* args, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

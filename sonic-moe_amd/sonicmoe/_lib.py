@@ -81,6 +81,10 @@ _SIGNATURES = {
         [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L, _L, _I, _I, _I, _I, _P, _Z, _P],
     ),
     "smoe_down_projection_forward_fp8": (c_int, [_P, _P, _P, _P, _P, _P, _P, _L, _I, _I, _I, _P, _Z, _P]),
+    "smoe_layer_forward_workspace_bytes": (c_size_t, [_L, _I, _I, _I, _I]),
+    "smoe_layer_forward": (c_int, [c_char_p, _P]),  # (the packed struct)
+    "smoe_layer_backward_workspace_bytes": (c_size_t, [_L, _I, _I, _I, _I, _I, _I]),
+    "smoe_layer_backward": (c_int, [c_char_p, _P]),
     "smoe_score_grad_bias_term": (c_int, [_P, _P, _P, _P, _P, _P, _L, _I, _I, _P]),
 }
 

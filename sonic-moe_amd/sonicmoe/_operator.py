@@ -40,6 +40,30 @@ def operator(name: str, mutates_args: set[str]):
     return register
 
 
+def elsewhere(*ops) -> frozenset:
+    """The names under which somebody else may register an implementation of one of these operators."""
+    return frozenset().union(*(op.elsewhere for op in ops))
+
+
+def unobserved(names: frozenset, *tensors) -> bool:
+    """Whether nobody looks on the calls of the operators behind `names` (`elsewhere`) on these tensors (or None) in a row:
+    the questions of `run`, asked once.  For eager code only."""
+    if not (
+        torch._C._len_torch_dispatch_stack() == 0
+        and torch._C._functorch.peek_interpreter_stack() is None
+        and not torch._C._is_torch_function_mode_enabled()
+        and torch._C._get_tracing_state() is None
+        and not torch.autograd._profiler_enabled()
+        and _REGISTERED is not None
+        and _REGISTERED.isdisjoint(names)
+    ):
+        return False
+    for t in tensors:
+        if t is not None and (type(t) not in _TENSORS or not t.is_cuda or t.is_neg()):
+            return False
+    return True
+
+
 def run(op, *args) -> None:
     """op(*args) for outputs that were allocated for this call and that nothing has saved yet (the dispatcher would also
     count the mutation in their version counters)."""

@@ -58,6 +58,7 @@ from .fp8 import (
     quantize_expert_weight_both,
     quantize_expert_weight_transposed,
 )
+from . import layer_call
 from .utils import enable_quack_gemm, is_using_quack_gemm
 
 
@@ -441,14 +442,19 @@ class _ExpertsFunction(torch.autograd.Function):
         return dx, dw1, db1, dw2, db2, ds, None, None, None, None, None, None, None, None, None, None
 
 
+def _router_wgrad_takes(dlogits: torch.Tensor, x: torch.Tensor) -> bool:
+    (T, E), H = dlogits.shape, x.size(1)
+    fast = (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and dlogits.dtype == x.dtype and E % 8 == 0
+            and H % 8 == 0)
+    return fast and T >= 256 and os.environ.get("SMOE_ROUTER_WGRAD", "1") != "0"
+
+
 def _router_wgrad(dlogits: torch.Tensor, x: torch.Tensor, like: torch.Tensor) -> torch.Tensor:
     """dWr = dlogits^T x: a token-split GEMM where the kernel supports the shape (it has only E output rows and T
     contraction elements, which a library GEMM without a split runs on an eighth of the chip), torch otherwise."""
     T, E = dlogits.shape
     H = x.size(1)
-    fast = (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and dlogits.dtype == x.dtype and E % 8 == 0
-            and H % 8 == 0)
-    if fast and T >= 256 and os.environ.get("SMOE_ROUTER_WGRAD", "1") != "0":
+    if _router_wgrad_takes(dlogits, x):
         partial = torch.empty(router_weight_grad_chunks(T, E, H), E, H, dtype=x.dtype, device=x.device)
         run(_router_weight_grad, dlogits.contiguous(), x.contiguous(), partial)
         if partial.size(0) == 1:
@@ -505,22 +511,79 @@ class _TCLayerFunction(torch.autograd.Function):
         if inference:
             raise RuntimeError("backward through an inference-mode MoE forward: z was not stored")
         x, router_w, w1, w2, b2, z, scores, indices, off, gidx, sidx, ridx, tok_off = ctx.saved_tensors
-        T, E = x.size(0), router_w.size(0)
-        dx, dw1, db1, dw2, db2, ds = _experts_backward(
-            dout, x, w1, w2, b2, z, scores.view(-1), off, gidx, sidx, ridx, tok_off, K, False, activation_type, stream_id,
-            has_b1, ctx.order, ctx.fp8_backward,
-        )
-        dlogits = torch.empty(T, E, dtype=logits_dtype, device=x.device)
-        # (a compiled backward pass knows dense gradients only, and refuses the question)
-        if not torch.compiler.is_compiling() and dlogits_outside is not None and dlogits_outside.layout != torch.strided:
-            dlogits_outside = dlogits_outside.to_dense()
-        run(_router_logit_grad, dlogits, dlogits_outside, ds.view(T, K), scores, indices)
-        dwr = _router_wgrad(dlogits, x, router_w) if ctx.needs_input_grad[1] else None
-        if ctx.needs_input_grad[0]:
-            dx.addmm_(dlogits, router_w)  # dx_experts + dlogits Wr in the GEMM's epilogue
-        else:
-            dx = None
-        return dx, dwr, dw1, db1, dw2, db2, None, None, None, None
+        return _tc_layer_backward(ctx, dout, dlogits_outside, x, router_w, w1, w2, b2, z, scores, indices, off, gidx, sidx, ridx,
+                                  tok_off, K, activation_type, stream_id, logits_dtype, has_b1, ctx.order, ctx.fp8_backward)
+
+
+def _tc_layer_backward(ctx, dout, dlogits_outside, x, router_w, w1, w2, b2, z, scores, indices, off, gidx, sidx, ridx, tok_off,
+                       K, activation_type, stream_id, logits_dtype, has_b1, order, fp8):
+    T, E = x.size(0), router_w.size(0)
+    dx, dw1, db1, dw2, db2, ds = _experts_backward(
+        dout, x, w1, w2, b2, z, scores.view(-1), off, gidx, sidx, ridx, tok_off, K, False, activation_type, stream_id,
+        has_b1, order, fp8,
+    )
+    dlogits = torch.empty(T, E, dtype=logits_dtype, device=x.device)
+    # (a compiled backward pass knows dense gradients only, and refuses the question)
+    if not torch.compiler.is_compiling() and dlogits_outside is not None and dlogits_outside.layout != torch.strided:
+        dlogits_outside = dlogits_outside.to_dense()
+    run(_router_logit_grad, dlogits, dlogits_outside, ds.view(T, K), scores, indices)
+    dwr = _router_wgrad(dlogits, x, router_w) if ctx.needs_input_grad[1] else None
+    if ctx.needs_input_grad[0]:
+        dx.addmm_(dlogits, router_w)  # dx_experts + dlogits Wr in the GEMM's epilogue
+    else:
+        dx = None
+    return dx, dwr, dw1, db1, dw2, db2, None, None, None, None
+
+
+class _OneCallLayerFunction(torch.autograd.Function):
+    """_TCLayerFunction whose operators behind the router GEMM run as one call of the library per direction
+    (layer_call.py), with the load-balancing loss as a fourth output if `with_loss`."""
+
+    @staticmethod
+    def forward(ctx, x, router_w, w1, b1, w2, b2, K: int, activation_type: ActivationType, stream_id: int, with_loss: bool):
+        x = x.contiguous()
+        logits = F.linear(x, router_w)
+        done = layer_call.forward(x, logits, w1, b1, w2, b2, K, activation_type, stream_id, True, with_loss)
+        if done is None:
+            raise layer_call.Refused
+        o, z, freq, ints, loss = done
+        ctx.save_for_backward(x, router_w, w1, w2, b2, z, ints, freq, logits)
+        ctx.cfg = (K, activation_type, stream_id, b1 is not None)
+        ctx.set_materialize_grads(False)  # (zeros for the token counts and the logits nobody used would be two launches)
+        ctx.mark_non_differentiable(freq)
+        return o, logits, freq, loss
+
+    @staticmethod
+    def backward(ctx, dout, dlogits_outside, _dfreq, daux):
+        K, activation_type, stream_id, has_b1 = ctx.cfg
+        x, router_w, w1, w2, b2, z, ints, freq, logits = ctx.saved_tensors
+        T, H = x.shape
+        E = router_w.size(0)
+        if dout is None:
+            dout = torch.zeros(T, H, dtype=x.dtype, device=x.device)
+        fast_router = (ctx.needs_input_grad[1] and _router_wgrad_takes(logits, x))
+        chunks = router_weight_grad_chunks(T, E, H) if fast_router else 0
+        done = None
+        if (_down_projection_backward, _up_projection_backward, _token_broadcast_backward, _switch_loss_bwd,
+                _router_logit_grad, _router_weight_grad, _sum_chunks) == layer_call._BACKWARD_OPERATORS:
+            done = layer_call.backward(x, dout, z, w1, w2, b2, has_b1, ints, freq, logits, K, activation_type, stream_id, daux,
+                                       dlogits_outside, chunks)
+        if done is not None:
+            dx, dlogits, dwr, dw1, db1, dw2, db2 = done
+            if dwr is None and ctx.needs_input_grad[1]:
+                dwr = dlogits.t() @ x
+            if ctx.needs_input_grad[0]:
+                dx.addmm_(dlogits, router_w)
+            else:
+                dx = None
+            return dx, dwr, dw1, db1, dw2, db2, None, None, None, None
+        scores, indices, gidx, sidx, ridx, off, tok_off, acc = layer_call.Indices(T, E, K).views(ints)
+        if daux is not None:
+            dlogits = torch.empty_like(logits, memory_format=torch.contiguous_format)
+            run(_switch_loss_bwd, logits, freq, acc, daux.reshape(1).float().contiguous(), dlogits)
+            dlogits_outside = dlogits if dlogits_outside is None else dlogits_outside + dlogits
+        return _tc_layer_backward(ctx, dout, dlogits_outside, x, router_w, w1, w2, b2, z, scores, indices, off, gidx, sidx, ridx,
+                                  tok_off, K, activation_type, stream_id, logits.dtype, has_b1, None, False)
 
 
 class _SwitchLossFunction(torch.autograd.Function):
@@ -596,8 +659,43 @@ def moe_TC_softmax_topk_layer(
     x (T, H); router_w (E, H); w1 (2I, H, E) and w2 (H, I, E) are permuted views of the (E, out, in) parameters.
     Returns (o (T, H), router_logits (T, E), expert_frequency (E,) int32).
     """
+    return layer_with_loss(x, router_w, w1, b1, w2, b2, K, stream_id, activation_type, is_inference_mode_enabled, False)[:3]
+
+
+_ONE_CALL_NAMES = layer_call.forward_names(_routing_metadata)
+_ONE_CALL_OPERATORS = (_softmax_topk_fwd, _routing_metadata, _up_projection_forward, _down_projection_forward, _router_forward,
+                       _switch_loss_fwd)
+
+
+def layer_with_loss(x, router_w, w1, b1, w2, b2, K: int, stream_id: int, activation_type, is_inference_mode_enabled: bool,
+                    with_loss: bool):
+    """moe_TC_softmax_topk_layer, and its load-balancing loss: (o, router_logits, expert_frequency, loss).  loss is None where
+    it is not asked for, and where the layer runs operator by operator: switch_loss computes it from the other two."""
     b1, b2 = _check_bias(b1, b2)
     activation_type = _as_activation(activation_type)
+    if (
+        not torch.compiler.is_compiling()
+        and not (_FUSED_ROUTER or _FUSED_COMBINE or is_using_fp8_forward() or is_using_fp8_backward())
+        and _SCHEDULE_POLICY == "expert_index"
+        and (_softmax_topk_fwd, _routing_metadata, _up_projection_forward, _down_projection_forward, _router_forward,
+             _switch_loss_fwd) == _ONE_CALL_OPERATORS
+        and layer_call.takes(x, router_w, w1, b1, w2, b2, K, activation_type, stream_id, _ONE_CALL_NAMES)
+        and os.environ.get("SMOE_FUSED_TC_LAYER", "1") != "0"
+    ):
+        needs_grad = torch.is_grad_enabled() and (
+            x.requires_grad or router_w.requires_grad or w1.requires_grad or w2.requires_grad
+            or (b1 is not None and (b1.requires_grad or b2.requires_grad)))
+        if not needs_grad:
+            x = x.contiguous()
+            logits = F.linear(x, router_w)
+            done = layer_call.forward(x, logits, w1, b1, w2, b2, K, activation_type, stream_id, False, with_loss)
+            if done is not None:
+                return done[0], logits, done[2], done[4]
+        elif not is_inference_mode_enabled:
+            try:
+                return _OneCallLayerFunction.apply(x, router_w, w1, b1, w2, b2, K, activation_type, stream_id, with_loss)
+            except layer_call.Refused:
+                pass
     if os.environ.get("SMOE_FUSED_TC_LAYER", "1") == "0":  # the layer as three autograd nodes, as the reference builds it
         T, E = x.size(0), router_w.size(0)
         router_logits = _RouterLinearFunction.apply(x, router_w)
@@ -607,10 +705,10 @@ def moe_TC_softmax_topk_layer(
             x, w1, b1, w2, b2, topk_scores.view(-1), off, gidx, sidx, ridx, tok_off, K, False, activation_type,
             stream_id, is_inference_mode_enabled,
         )
-        return o, router_logits, freq
-    return _TCLayerFunction.apply(
+        return o, router_logits, freq, None
+    return *_TCLayerFunction.apply(
         x, router_w, w1, b1, w2, b2, K, activation_type, stream_id, is_inference_mode_enabled
-    )
+    ), None
 
 
 def moe_general_routing_inputs(

@@ -15,7 +15,7 @@ import torch.nn.functional as F
 
 from .count_cumsum import count_cumsum
 from .enums import ActivationType, KernelBackendMoE, is_glu
-from .functional import moe_TC_softmax_topk_layer, switch_loss
+from .functional import layer_with_loss, switch_loss
 
 
 def _split_gate_up(h: torch.Tensor):
@@ -108,7 +108,7 @@ class MoE(nn.Module):
         x = hidden_states.view(-1, self.hidden_size)
 
         if kernel_backend_moe == KernelBackendMoE.sonicmoe:
-            out, router_logits, expert_frequency = moe_TC_softmax_topk_layer(
+            out, router_logits, expert_frequency, aux_loss = layer_with_loss(
                 x,
                 self.router.weight,
                 self.c_fc.weight.permute(1, 2, 0),
@@ -119,6 +119,7 @@ class MoE(nn.Module):
                 self.stream_id,
                 self.activation_function,
                 is_inference_mode or not self.training,
+                True,
             )
         elif kernel_backend_moe == KernelBackendMoE.torch:
             router_logits, gates, selected = self._compute_routing_weights(x)
@@ -131,7 +132,8 @@ class MoE(nn.Module):
         out = out.view(shape)
         if kernel_backend_moe == KernelBackendMoE.sonicmoe:
             # same value as _compute_switch_loss below, one pass over the logits instead of six torch kernels
-            aux_loss = switch_loss(router_logits, expert_frequency)
+            if aux_loss is None:
+                aux_loss = switch_loss(router_logits, expert_frequency)
         else:
             aux_loss = self._compute_switch_loss(
                 logits=router_logits,

@@ -1,0 +1,198 @@
+"""The layer as one call of the library per direction: the packed arguments against the declared structs, and the same bits
+as operator by operator."""
+
+import re
+
+import pytest
+import torch
+
+from test_abi import HEADER
+
+
+@pytest.mark.parametrize("name, packed", [("smoe_layer_forward_args", "_FORWARD"), ("smoe_layer_backward_args", "_BACKWARD")])
+def test_packed_arguments_fill_the_struct(name, packed):
+    from sonicmoe.functional import layer_call
+
+    text = re.sub(r"/\*.*?\*/", "", HEADER.read_text(), flags=re.S)
+    fields = re.search(r"typedef struct \{([^}]*)\} " + name, text).group(1)
+    assert getattr(layer_call, packed).size == 8 * sum(decl.count(",") + 1 for decl in fields.split(";") if decl.strip())
+
+
+@pytest.mark.parametrize("T, E, K", [(1, 8, 1), (63, 5, 3), (777, 48, 4), (64, 4096, 64)])
+def test_index_views_do_not_overlap(T, E, K):
+    from sonicmoe.functional.layer_call import Indices
+
+    where = Indices(T, E, K)
+    spans = sorted((v.storage_offset(), v.storage_offset() + v.numel())
+                   for v in where.views(torch.zeros(where.words, dtype=torch.int32)))
+    assert all(a[1] <= b[0] for a, b in zip(spans, spans[1:])) and spans[-1][1] <= where.words
+    assert all(a % 64 == 0 for a, _ in spans)
+
+
+def _module(T, H, I, E, K, act, bias, dtype, dev):
+    from sonicmoe import MoE
+    from sonicmoe.enums import ActivationType
+
+    torch.manual_seed(T + H)
+    moe = MoE(E, K, H, I, ActivationType(act), bias, 0.02).to(device=dev, dtype=dtype)
+    if bias:
+        for p in (moe.c_fc.bias, moe.c_proj.bias):
+            torch.nn.init.normal_(p, 0, 0.1)
+    return moe, torch.randn(T, H, device=dev).to(dtype), torch.randn(T, H, device=dev).to(dtype)
+
+
+def _both(monkeypatch, step):
+    """step() in one call per direction and operator by operator; how often the library was asked for the whole"""
+    from sonicmoe.functional import layer_call
+
+    asked = []
+    for name in ("forward", "backward"):
+        real = getattr(layer_call, name)
+        monkeypatch.setattr(layer_call, name, lambda *a, _n=name, _r=real: (r := _r(*a), asked.append((_n, r is not None)))[0])
+    one = step()
+    calls = list(asked)
+    monkeypatch.setattr(layer_call, "MAX_TRANSIENT_BYTES", -1)
+    asked.clear()
+    each = step()
+    assert not asked
+    for a, b in zip(one, each):
+        assert (a is None) == (b is None) and (a is None or torch.equal(a, b))
+    return calls
+
+
+# one token; few rows and an idle expert; borders of the token chunks of the router's gradient; odd expert counts
+SHAPES = [(1, 128, 64, 8, 2), (37, 192, 128, 16, 5), (255, 256, 64, 12, 3), (512, 512, 192, 8, 2), (1000, 320, 256, 33, 4)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("act, bias, dtype", [("swiglu", False, torch.bfloat16), ("geglu", True, torch.float16),
+                                              ("relu_sq", True, torch.bfloat16), ("silu", False, torch.float16)])
+def test_module_step(dev, monkeypatch, shape, act, bias, dtype):
+    moe, x, dy = _module(*shape, act, bias, dtype, dev)
+
+    def step():
+        xx = x.clone().requires_grad_()
+        out, aux = moe(xx)
+        grads = torch.autograd.grad([out, aux], [xx, *moe.parameters()], grad_outputs=[dy, torch.tensor(0.3, device=dev)])
+        with torch.no_grad():
+            still, aux2 = moe(x)
+            moe.eval()
+            quiet, aux3 = moe(x)
+            moe.train()
+        return [out.detach(), aux.detach(), *grads, still, aux2, quiet, aux3]
+
+    assert _both(monkeypatch, step) == [("forward", True), ("backward", True), ("forward", True), ("forward", True)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", ["loss only", "output only", "logits too", "logits transposed", "router frozen", "x frozen",
+                                  "x strided", "dout strided", "weights strided", "hooks", "twice"])
+def test_functional_forms(dev, monkeypatch, case):
+    from sonicmoe.functional import moe_TC_softmax_topk_layer, switch_loss
+
+    T, H, I, E, K = 300, 256, 128, 16, 4
+    moe, x, dy = _module(T, H, I, E, K, "swiglu", False, torch.bfloat16, dev)
+    parts = [p.detach() for p in moe.parameters()]
+    if case == "weights strided":  # every other row of wider matrices
+        parts[1:] = [torch.stack([p, p], 2).flatten(1, 2)[:, ::2] for p in parts[1:]]
+    if case == "x strided":
+        x = torch.stack([x, x], 1).flatten(0, 1)[::2]
+    if case == "dout strided":
+        dy = dy.t().contiguous().t()
+    dl = (torch.randn(E, T, device=dev) * 0.01).bfloat16()
+
+    def step():
+        xx = x.detach().requires_grad_(case != "x frozen")
+        ps = [p.detach().requires_grad_(case != "router frozen" or i > 0) for i, p in enumerate(parts)]
+        ins = [t for t in [xx, *ps] if t.requires_grad]
+
+        def forward():
+            return moe_TC_softmax_topk_layer(xx, ps[0], ps[1].permute(1, 2, 0), None, ps[2].permute(1, 2, 0), None, K,
+                                             torch.cuda.current_stream().cuda_stream)
+
+        if case == "hooks":
+            with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.to(dev)):
+                o, logits, freq = forward()
+        else:
+            o, logits, freq = forward()
+        outs, grads = [o], [dy]
+        if case == "loss only":
+            outs, grads = [switch_loss(logits, freq)], [torch.tensor(2.0, device=dev)]
+        elif case.startswith("logits"):
+            outs.append(logits)
+            grads.append(dl.t() if case == "logits transposed" else dl.t().contiguous())
+        got = torch.autograd.grad(outs, ins, grad_outputs=grads, retain_graph=case == "twice")
+        again = torch.autograd.grad(outs, ins, grad_outputs=grads) if case == "twice" else ()
+        return [o.detach(), logits.detach(), freq, *got, *again]
+
+    calls = _both(monkeypatch, step)
+    assert calls[0] == ("forward", True)
+    assert all(done == (case != "logits transposed") for name, done in calls[1:]) and len(calls) == 2 + (case == "twice")
+
+
+@pytest.mark.gpu
+def test_module_gradient_of_one_output(dev, monkeypatch):
+    moe, x, dy = _module(200, 256, 128, 16, 4, "swiglu", False, torch.bfloat16, dev)
+
+    def step():
+        out = []
+        for which in (0, 1):
+            xx = x.clone().requires_grad_()
+            got = moe(xx)[which]
+            out += torch.autograd.grad(got, [xx, *moe.parameters()], grad_outputs=dy if which == 0 else None)
+        return out
+
+    _both(monkeypatch, step)
+
+
+@pytest.mark.gpu
+def test_what_is_left_to_the_operators(dev, monkeypatch):
+    """Profilers, autocast, another stream, forward-mode derivatives, odd sizes: as operator by operator, errors included."""
+    from sonicmoe.functional import layer_call, moe_TC_softmax_topk_layer
+
+    moe, x, _ = _module(64, 128, 64, 8, 2, "swiglu", False, torch.bfloat16, dev)
+    real = layer_call.forward
+    done = []
+    monkeypatch.setattr(layer_call, "forward", lambda *a: (r := real(*a), done.append(r is not None))[0])
+    with torch.no_grad():
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as profile:
+            moe(x)
+        assert any("_up_projection_forward" in e.key for e in profile.key_averages()) and not done
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            moe(x)
+        assert not done
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side), pytest.raises(RuntimeError, match="stream"):
+            moe(x)
+        torch.cuda.current_stream().wait_stream(side)
+        w = moe.c_fc.weight[:, :, :96].contiguous()  # H = 96 is no multiple of 64: told by the operator
+        with pytest.raises(RuntimeError, match="multiple of 64"):
+            moe_TC_softmax_topk_layer(x[:, :96].contiguous(), moe.router.weight[:, :96].contiguous(), w.permute(1, 2, 0), None,
+                                      moe.c_proj.weight[:, :96].contiguous().permute(1, 2, 0), None, 2, moe.stream_id)
+        assert not any(done)
+
+
+@pytest.mark.gpu
+def test_under_capture(dev):
+    moe, x, _ = _module(16, 256, 128, 16, 4, "swiglu", False, torch.bfloat16, dev)
+    moe.eval()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side), torch.no_grad():
+        moe.stream_id = side.cuda_stream
+        moe(x)
+        side.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            out, aux = moe(x)
+    torch.cuda.current_stream().wait_stream(side)
+    moe.stream_id = torch.cuda.current_stream().cuda_stream
+    for seed in range(3):
+        x.copy_(torch.randn(x.shape, device=dev, generator=torch.Generator(dev).manual_seed(seed)))
+        graph.replay()
+        torch.cuda.synchronize()
+        with torch.no_grad():
+            want, want_aux = moe(x)
+        assert torch.equal(out, want) and torch.equal(aux, want_aux)
