@@ -1319,6 +1319,48 @@ static inline TileMap carve_tile_map(void* ws, int64_t TK, int E, int BM) {
 }
 
 int launch_build_tile_map(const int32_t* off, const int32_t* order, int E, int BM, TileMap tm, hipStream_t st);
+
+// Scratch memory of the bf16 grouped GEMMs of ONE routing (one off, no schedule order or the same one): the tile map of the
+// token-grouped kernels and the experts' order of the weight-gradient streams.  An entry point makes one for its call, on
+// its workspace, where the two share the memory; the layer's calls keep one for all GEMMs of a direction, with memory for
+// both, so that the map is built and the experts are sorted once (a launch of 4 to 6 us each).
+struct GemmScratch {
+  void* map;
+  void* sorted;
+  size_t sorted_bytes;
+  int map_rows = 0;            // token rows per tile of the map in `map` (0: none)
+  bool sorted_valid = false;
+  GemmScratch(void* map_, void* sorted_, size_t sorted_bytes_) : map(map_), sorted(sorted_), sorted_bytes(sorted_bytes_) {}
+  GemmScratch(void* workspace, size_t bytes) : GemmScratch(workspace, workspace, bytes) {}
+};
+
+// The tile map for tiles of BM rows: the one that is there, or a new one
+static inline int tile_map_in(GemmScratch& ws, const int32_t* off, const int32_t* order, int64_t TK, int E, int BM, TileMap& tm,
+                              hipStream_t st) {
+  tm = carve_tile_map(ws.map, TK, E, BM);
+  if (ws.map_rows == BM) return SMOE_OK;
+  if (ws.map == ws.sorted) ws.sorted_valid = false;
+  ws.map_rows = BM;
+  return launch_build_tile_map(off, order, E, BM, tm, st);
+}
+
+// The entry points' bodies on such a scratch (their own checks of the workspace's size are the entry points')
+int up_projection_forward(const void* x, const void* w1, int64_t w1_stride_e, int64_t w1_stride_row, const void* b1, void* z,
+                          void* y1, const int32_t* off, const int32_t* expert_schedule_order, const int32_t* x_gather_idx,
+                          int64_t T, int64_t TK, int H, int I, int E, int activation, GemmScratch& ws, void* stream);
+int down_projection_forward(const void* y1, const void* w2, int64_t w2_stride_e, int64_t w2_stride_row, const void* b2,
+                            void* y2, const int32_t* off, const int32_t* expert_schedule_order, int64_t TK, int H, int I,
+                            int E, GemmScratch& ws, void* stream);
+int down_projection_backward(const void* dout, const void* z, const void* w2, int64_t w2_stride_e, int64_t w2_stride_row,
+                             const void* b2, void* dw2, int64_t dw2_stride_e, int64_t dw2_stride_row, void* db2, void* dz,
+                             void* y1s, float* ds, float* ds_partial, const float* scores, const int32_t* off,
+                             const int32_t* expert_schedule_order, const int32_t* x_gather_idx,
+                             const int32_t* s_scatter_idx, int64_t T, int64_t TK, int H, int I, int E, int activation,
+                             GemmScratch& ws, void* stream);
+int up_projection_backward(const void* x, const void* w1, int64_t w1_stride_e, int64_t w1_stride_row, const void* dz,
+                           void* dw1, int64_t dw1_stride_e, int64_t dw1_stride_row, void* db1, void* dx_expanded,
+                           const int32_t* off, const int32_t* expert_schedule_order, const int32_t* x_gather_idx, int64_t T,
+                           int64_t TK, int H, int I, int E, int activation, GemmScratch& ws, void* stream);
 // entries of a tile map index 24 bits of group[]
 static inline bool tile_map_fits(int64_t TK, int E, int BM) { return max_token_tiles(TK, E, BM) < (1ll << 24); }
 

@@ -10,7 +10,6 @@
 #include "tile_loop_gen.h"
 
 namespace smoe {
-
 struct VarlenKParams {
   const uint16_t* R;
   int64_t r_stride;
@@ -542,7 +541,7 @@ __global__ __launch_bounds__(256) void varlen_k_stream_kernel(const VarlenKParam
 }
 
 template <class C>
-static int launch_varlen_k(const VarlenKParams& pin, hipStream_t st, void* workspace = nullptr, size_t workspace_bytes = 0) {
+static int launch_varlen_k(const VarlenKParams& pin, hipStream_t st, GemmScratch* ws) {
   static LdsLimitOnce lds_limit;
   auto kern = varlen_k_kernel<C>;
   {
@@ -612,8 +611,8 @@ static int launch_varlen_k(const VarlenKParams& pin, hipStream_t st, void* works
     const int64_t least = tuning().varlen_k_stream_rows >= 0 ? tuning().varlen_k_stream_rows
                           : total <= 256 ? 1024 : us.nb > 0 ? 64 : 256;
     const bool long_enough = p.total_rows >= least * p.E;
-    if (tuning().gemm_asm && fits && long_enough && p.E <= SCHED_MAX_E && total < (1ll << 30) && workspace != nullptr &&
-        (size_t)p.E * sizeof(int32_t) <= workspace_bytes) {
+    if (tuning().gemm_asm && fits && long_enough && p.E <= SCHED_MAX_E && total < (1ll << 30) && ws != nullptr &&
+        ws->sorted != nullptr && (size_t)p.E * sizeof(int32_t) <= ws->sorted_bytes) {
       us.units = us.nb * p.E;
       if (us.nb == 0) {
         us.chunk = total < 256 ? (int)ceil_div(total, 8) : 32;
@@ -623,9 +622,13 @@ static int launch_varlen_k(const VarlenKParams& pin, hipStream_t st, void* works
       auto akern = varlen_k_stream_kernel<C::R_GATHER, C::S_GATHER>;
       const int rc_a = lds_limit_asm.ensure((const void*)akern, 160 * 1024);
       if (rc_a) return rc_a;
-      hipLaunchKernelGGL(sort_experts_kernel, dim3(1), dim3(1024), 0, st, p.off, p.order, p.E, (int32_t*)workspace);
-      SMOE_LAUNCH_CHECK();
-      hipLaunchKernelGGL(akern, dim3(256), dim3(256), 160 * 1024, st, p, us, (const int32_t*)workspace);
+      if (!ws->sorted_valid) {
+        if (ws->map == ws->sorted) ws->map_rows = 0;
+        ws->sorted_valid = true;
+        hipLaunchKernelGGL(sort_experts_kernel, dim3(1), dim3(1024), 0, st, p.off, p.order, p.E, (int32_t*)ws->sorted);
+        SMOE_LAUNCH_CHECK();
+      }
+      hipLaunchKernelGGL(akern, dim3(256), dim3(256), 160 * 1024, st, p, us, (const int32_t*)ws->sorted);
       SMOE_LAUNCH_CHECK();
       return SMOE_OK;
     }
@@ -637,41 +640,45 @@ static int launch_varlen_k(const VarlenKParams& pin, hipStream_t st, void* works
 
 // 256 x 256 output tile, 8 wavefronts as 2 x 4, 64 token rows per stage, double buffer
 template <bool RG, bool SG>
-static int launch_varlen_k_variant(const VarlenKParams& p, hipStream_t st, void* workspace = nullptr,
-                                   size_t workspace_bytes = 0) {
-  return launch_varlen_k<KCfg<256, 256, 2, 4, RG, SG, 64, 2>>(p, st, workspace, workspace_bytes);
+static int launch_varlen_k_variant(const VarlenKParams& p, hipStream_t st, GemmScratch* ws = nullptr) {
+  return launch_varlen_k<KCfg<256, 256, 2, 4, RG, SG, 64, 2>>(p, st, ws);
 }
 
 int launch_dz(const void* dout, const void* z, const void* w2, int64_t w2_stride_e, int64_t w2_stride_row, void* dz,
               void* y1s, float* ds_partial, const float* scores, const int32_t* off, const int32_t* order,
               const int32_t* gidx, const int32_t* sidx, int64_t T, int64_t TK, int H, int I, int E,
-              int activation, void* workspace, hipStream_t st);
+              int activation, GemmScratch& ws, hipStream_t st);
 int launch_dx(const void* dz, const void* w1, int64_t w1_stride_e, int64_t w1_stride_row, void* dx_expanded,
-              const int32_t* off, const int32_t* order, int64_t TK, int H, int N1, int E, void* workspace,
+              const int32_t* off, const int32_t* order, int64_t TK, int H, int N1, int E, GemmScratch& ws,
               hipStream_t st);
 
 }  // namespace smoe
 
 using namespace smoe;
 
-static int check_bwd(int64_t TK, int H, int I, int E, const void* ws, size_t ws_bytes, const char* who) {
+static int check_sizes(int64_t TK, int H, int I, int E, const char* who) {
   SMOE_REQUIRE(TK >= 0 && TK < (1ll << 31), SMOE_ERR_INVALID, "%s: TK out of range", who);
   SMOE_REQUIRE(E >= 1, SMOE_ERR_INVALID, "%s: E must be >= 1", who);
   SMOE_REQUIRE(H >= 64 && H % 64 == 0, SMOE_ERR_UNSUPPORTED, "%s: H=%d must be a multiple of 64", who, H);
   SMOE_REQUIRE(I >= 64 && I % 64 == 0, SMOE_ERR_UNSUPPORTED, "%s: I=%d must be a multiple of 64", who, I);
+  return SMOE_OK;
+}
+
+static int check_bwd(int64_t TK, int H, int I, int E, const void* ws, size_t ws_bytes, const char* who) {
+  const int rc = check_sizes(TK, H, I, E, who);
+  if (rc) return rc;
   SMOE_REQUIRE(ws != nullptr && ws_bytes >= smoe_gemm_workspace_bytes(TK, E), SMOE_ERR_WORKSPACE,
                "%s: workspace too small", who);
   return SMOE_OK;
 }
 
-extern "C" int smoe_down_projection_backward(const void* dout, const void* z, const void* w2, int64_t w2_stride_e,
-                                             int64_t w2_stride_row, const void* b2, void* dw2, int64_t dw2_stride_e,
-                                             int64_t dw2_stride_row, void* db2, void* dz, void* y1s, float* ds,
-                                             float* ds_partial, const float* scores, const int32_t* off,
-                                             const int32_t* expert_schedule_order, const int32_t* x_gather_idx,
-                                             const int32_t* s_scatter_idx, int64_t T, int64_t TK, int H, int I, int E,
-                                             int activation, void* workspace, size_t workspace_bytes, void* stream) {
-  int rc = check_bwd(TK, H, I, E, workspace, workspace_bytes, "down_projection_backward");
+int smoe::down_projection_backward(const void* dout, const void* z, const void* w2, int64_t w2_stride_e,
+                                   int64_t w2_stride_row, const void* b2, void* dw2, int64_t dw2_stride_e,
+                                   int64_t dw2_stride_row, void* db2, void* dz, void* y1s, float* ds, float* ds_partial,
+                                   const float* scores, const int32_t* off, const int32_t* expert_schedule_order,
+                                   const int32_t* x_gather_idx, const int32_t* s_scatter_idx, int64_t T, int64_t TK, int H,
+                                   int I, int E, int activation, GemmScratch& ws, void* stream) {
+  int rc = check_sizes(TK, H, I, E, "down_projection_backward");
   if (rc) return rc;
   SMOE_REQUIRE(activation >= SMOE_ACT_SWIGLU && activation <= SMOE_ACT_SILU, SMOE_ERR_INVALID,
                "down_projection_backward: unknown activation code %d", activation);
@@ -690,7 +697,7 @@ extern "C" int smoe_down_projection_backward(const void* dout, const void* z, co
   hipStream_t st = (hipStream_t)stream;
   if (TK > 0 && dz) {
     rc = launch_dz(dout, z, w2, w2_stride_e, w2_stride_row, dz, y1s, ds_partial, scores, off, expert_schedule_order,
-                   x_gather_idx, s_scatter_idx, T, TK, H, I, E, activation, workspace, st);
+                   x_gather_idx, s_scatter_idx, T, TK, H, I, E, activation, ws, st);
     if (rc) return rc;
     rc = launch_ds_finalize(ds_partial, smoe_dz_partial_cols(I), s_scatter_idx, ds, TK, st);
     if (rc) return rc;
@@ -722,17 +729,31 @@ extern "C" int smoe_down_projection_backward(const void* dout, const void* z, co
   p.order = expert_schedule_order;
   p.total_rows = TK;
   p.gather_rows = T;
-  // the sorted experts may take the place of the tile map: the activation-gradient GEMM that used it ran before
-  return launch_varlen_k_variant<true, false>(p, st, workspace, workspace_bytes);
+  // (on one workspace the sorted experts take the place of the tile map: the GEMM that used it ran before)
+  return launch_varlen_k_variant<true, false>(p, st, &ws);
 }
 
-extern "C" int smoe_up_projection_backward(const void* x, const void* w1, int64_t w1_stride_e, int64_t w1_stride_row,
-                                           const void* dz, void* dw1, int64_t dw1_stride_e, int64_t dw1_stride_row,
-                                           void* db1, void* dx_expanded, const int32_t* off,
-                                           const int32_t* expert_schedule_order, const int32_t* x_gather_idx,
-                                           int64_t T, int64_t TK, int H, int I, int E, int activation, void* workspace,
-                                           size_t workspace_bytes, void* stream) {
-  int rc = check_bwd(TK, H, I, E, workspace, workspace_bytes, "up_projection_backward");
+extern "C" int smoe_down_projection_backward(const void* dout, const void* z, const void* w2, int64_t w2_stride_e,
+                                             int64_t w2_stride_row, const void* b2, void* dw2, int64_t dw2_stride_e,
+                                             int64_t dw2_stride_row, void* db2, void* dz, void* y1s, float* ds,
+                                             float* ds_partial, const float* scores, const int32_t* off,
+                                             const int32_t* expert_schedule_order, const int32_t* x_gather_idx,
+                                             const int32_t* s_scatter_idx, int64_t T, int64_t TK, int H, int I, int E,
+                                             int activation, void* workspace, size_t workspace_bytes, void* stream) {
+  int rc = check_bwd(TK, H, I, E, workspace, workspace_bytes, "down_projection_backward");
+  if (rc) return rc;
+  GemmScratch ws(workspace, workspace_bytes);
+  return smoe::down_projection_backward(dout, z, w2, w2_stride_e, w2_stride_row, b2, dw2, dw2_stride_e, dw2_stride_row, db2,
+                                        dz, y1s, ds, ds_partial, scores, off, expert_schedule_order, x_gather_idx,
+                                        s_scatter_idx, T, TK, H, I, E, activation, ws, stream);
+}
+
+int smoe::up_projection_backward(const void* x, const void* w1, int64_t w1_stride_e, int64_t w1_stride_row, const void* dz,
+                                 void* dw1, int64_t dw1_stride_e, int64_t dw1_stride_row, void* db1, void* dx_expanded,
+                                 const int32_t* off, const int32_t* expert_schedule_order, const int32_t* x_gather_idx,
+                                 int64_t T, int64_t TK, int H, int I, int E, int activation, GemmScratch& ws,
+                                 void* stream) {
+  int rc = check_sizes(TK, H, I, E, "up_projection_backward");
   if (rc) return rc;
   SMOE_REQUIRE(activation >= SMOE_ACT_SWIGLU && activation <= SMOE_ACT_SILU, SMOE_ERR_INVALID,
                "up_projection_backward: unknown activation code %d", activation);
@@ -768,16 +789,30 @@ extern "C" int smoe_up_projection_backward(const void* x, const void* w1, int64_
     p.order = expert_schedule_order;
     p.total_rows = TK;
     p.gather_rows = T;
-    // the sorted experts share the workspace with the tile map the dx GEMM builds afterwards, in stream order
-    rc = launch_varlen_k_variant<false, true>(p, st, workspace, workspace_bytes);
+    // (on one workspace the tile map of the dx GEMM then takes the place of the sorted experts, in stream order)
+    rc = launch_varlen_k_variant<false, true>(p, st, &ws);
     if (rc) return rc;
   }
   if (TK > 0 && dx_expanded) {
-    rc = launch_dx(dz, w1, w1_stride_e, w1_stride_row, dx_expanded, off, expert_schedule_order, TK, H, N1, E, workspace,
+    rc = launch_dx(dz, w1, w1_stride_e, w1_stride_row, dx_expanded, off, expert_schedule_order, TK, H, N1, E, ws,
                    st);
     if (rc) return rc;
   }
   return SMOE_OK;
+}
+
+extern "C" int smoe_up_projection_backward(const void* x, const void* w1, int64_t w1_stride_e, int64_t w1_stride_row,
+                                           const void* dz, void* dw1, int64_t dw1_stride_e, int64_t dw1_stride_row,
+                                           void* db1, void* dx_expanded, const int32_t* off,
+                                           const int32_t* expert_schedule_order, const int32_t* x_gather_idx,
+                                           int64_t T, int64_t TK, int H, int I, int E, int activation, void* workspace,
+                                           size_t workspace_bytes, void* stream) {
+  int rc = check_bwd(TK, H, I, E, workspace, workspace_bytes, "up_projection_backward");
+  if (rc) return rc;
+  GemmScratch ws(workspace, workspace_bytes);
+  return smoe::up_projection_backward(x, w1, w1_stride_e, w1_stride_row, dz, dw1, dw1_stride_e, dw1_stride_row, db1,
+                                      dx_expanded, off, expert_schedule_order, x_gather_idx, T, TK, H, I, E, activation, ws,
+                                      stream);
 }
 
 extern "C" int smoe_router_weight_grad(const void* dlogits, const void* x, void* partial, int64_t T, int E, int H,

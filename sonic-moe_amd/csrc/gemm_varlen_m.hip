@@ -11,7 +11,6 @@
 #include <math.h>
 
 namespace smoe {
-
 // ROLE_COMBINE: the down-projection forward that adds its score-weighted rows onto the tokens' output rows instead of
 // storing y2 (opt-in, atomic: combine_epilogue_batch)
 enum Role { ROLE_UP_FWD = 0, ROLE_PLAIN = 1, ROLE_DZ = 2, ROLE_COMBINE = 3 };
@@ -767,13 +766,12 @@ static bool small_tiles_pay(const VarlenMParams& p, int role, int64_t TK, int E,
 }
 
 template <class C, int ROLE, int ACT>
-static int launch_small_tiles(VarlenMParams& p, const int32_t* off, void* workspace, int64_t TK, int E, hipStream_t st) {
+static int launch_small_tiles(VarlenMParams& p, const int32_t* off, GemmScratch& ws, int64_t TK, int E, hipStream_t st) {
   static LdsLimitOnce lds_limit;
   auto kern = varlen_m_kernel<C, ROLE, ACT>;
   const int rc_attr = lds_limit.ensure((const void*)kern, C::SMEM);
   if (rc_attr) return rc_attr;
-  p.tm = carve_tile_map(workspace, TK, E, C::BM);
-  const int rc = launch_build_tile_map(off, p.order, E, C::BM, p.tm, st);
+  const int rc = tile_map_in(ws, off, p.order, TK, E, C::BM, p.tm, st);
   if (rc) return rc;
   p.n_tiles = (int)ceil_div(p.N, C::BN);
   if (ROLE == ROLE_DZ) p.ds_cols = (int)ceil_div(p.N, 256) * DS_COLS_PER_TILE;
@@ -785,7 +783,7 @@ static int launch_small_tiles(VarlenMParams& p, const int32_t* off, void* worksp
 }
 
 template <class C, int ROLE, int ACT>
-static int launch_varlen_m(VarlenMParams& p, const int32_t* off, void* workspace, int64_t TK, int E, hipStream_t st) {
+static int launch_varlen_m(VarlenMParams& p, const int32_t* off, GemmScratch& ws, int64_t TK, int E, hipStream_t st) {
   if constexpr (!C::QMN && (ROLE == ROLE_UP_FWD || ROLE == ROLE_PLAIN)) {
     SkinnyGemm g = {};
     g.P = p.P;
@@ -810,7 +808,7 @@ static int launch_varlen_m(VarlenMParams& p, const int32_t* off, void* workspace
     int cus = 0;
     const int rc_cu = device_compute_units(&cus);
     if (rc_cu) return rc_cu;
-    if (small_tiles_pay(p, ROLE, TK, E, cus)) return launch_small_tiles<SmallCfg<C::QMN>, ROLE, ACT>(p, off, workspace, TK, E, st);
+    if (small_tiles_pay(p, ROLE, TK, E, cus)) return launch_small_tiles<SmallCfg<C::QMN>, ROLE, ACT>(p, off, ws, TK, E, st);
   }
   static LdsLimitOnce lds_limit;
   auto kern = varlen_m_kernel<C, ROLE, ACT>;
@@ -819,8 +817,7 @@ static int launch_varlen_m(VarlenMParams& p, const int32_t* off, void* workspace
     if (rc_attr) return rc_attr;
   }
   if (p.gidx == nullptr) p.p_rows = TK;
-  p.tm = carve_tile_map(workspace, TK, E, C::BM);
-  int rc = launch_build_tile_map(off, p.order, E, C::BM, p.tm, st);
+  const int rc = tile_map_in(ws, off, p.order, TK, E, C::BM, p.tm, st);
   if (rc) return rc;
   p.n_tiles = (int)ceil_div(p.N, C::BN);
   static_assert(C::WN == DS_COLS_PER_TILE, "pitch of the score-gradient partials");
@@ -873,16 +870,16 @@ using TileCfg = Cfg<256, 256, 2, 4, QMN, 64, 2>;
 
 // one kernel per activation: the epilogue math and (gated or not) the tile geometry of z / y1 depend on it
 template <bool QMN, int ROLE>
-static int launch_by_activation(int act, VarlenMParams& p, const int32_t* off, void* workspace, int64_t TK, int E,
+static int launch_by_activation(int act, VarlenMParams& p, const int32_t* off, GemmScratch& ws, int64_t TK, int E,
                                 hipStream_t st) {
   switch (act) {
-    case SMOE_ACT_SWIGLU: return launch_varlen_m<TileCfg<QMN>, ROLE, SMOE_ACT_SWIGLU>(p, off, workspace, TK, E, st);
-    case SMOE_ACT_GEGLU: return launch_varlen_m<TileCfg<QMN>, ROLE, SMOE_ACT_GEGLU>(p, off, workspace, TK, E, st);
-    case SMOE_ACT_REGLU: return launch_varlen_m<TileCfg<QMN>, ROLE, SMOE_ACT_REGLU>(p, off, workspace, TK, E, st);
-    case SMOE_ACT_RELU_SQ: return launch_varlen_m<TileCfg<QMN>, ROLE, SMOE_ACT_RELU_SQ>(p, off, workspace, TK, E, st);
-    case SMOE_ACT_RELU: return launch_varlen_m<TileCfg<QMN>, ROLE, SMOE_ACT_RELU>(p, off, workspace, TK, E, st);
-    case SMOE_ACT_GELU: return launch_varlen_m<TileCfg<QMN>, ROLE, SMOE_ACT_GELU>(p, off, workspace, TK, E, st);
-    case SMOE_ACT_SILU: return launch_varlen_m<TileCfg<QMN>, ROLE, SMOE_ACT_SILU>(p, off, workspace, TK, E, st);
+    case SMOE_ACT_SWIGLU: return launch_varlen_m<TileCfg<QMN>, ROLE, SMOE_ACT_SWIGLU>(p, off, ws, TK, E, st);
+    case SMOE_ACT_GEGLU: return launch_varlen_m<TileCfg<QMN>, ROLE, SMOE_ACT_GEGLU>(p, off, ws, TK, E, st);
+    case SMOE_ACT_REGLU: return launch_varlen_m<TileCfg<QMN>, ROLE, SMOE_ACT_REGLU>(p, off, ws, TK, E, st);
+    case SMOE_ACT_RELU_SQ: return launch_varlen_m<TileCfg<QMN>, ROLE, SMOE_ACT_RELU_SQ>(p, off, ws, TK, E, st);
+    case SMOE_ACT_RELU: return launch_varlen_m<TileCfg<QMN>, ROLE, SMOE_ACT_RELU>(p, off, ws, TK, E, st);
+    case SMOE_ACT_GELU: return launch_varlen_m<TileCfg<QMN>, ROLE, SMOE_ACT_GELU>(p, off, ws, TK, E, st);
+    case SMOE_ACT_SILU: return launch_varlen_m<TileCfg<QMN>, ROLE, SMOE_ACT_SILU>(p, off, ws, TK, E, st);
   }
   set_error("unknown activation code %d", act);
   return SMOE_ERR_INVALID;
@@ -895,11 +892,17 @@ int dz_tile_cols() { return TileCfg<true>::BN; }
 
 using namespace smoe;
 
-static int check_common(int64_t TK, int H, int I, int E, const void* ws, size_t ws_bytes, const char* who) {
+static int check_sizes(int64_t TK, int H, int I, int E, const char* who) {
   SMOE_REQUIRE(TK >= 0 && TK < (1ll << 31), SMOE_ERR_INVALID, "%s: TK out of range", who);
   SMOE_REQUIRE(E >= 1, SMOE_ERR_INVALID, "%s: E must be >= 1", who);
   SMOE_REQUIRE(H >= 64 && H % 64 == 0, SMOE_ERR_UNSUPPORTED, "%s: H=%d must be a multiple of 64", who, H);
   SMOE_REQUIRE(I >= 64 && I % 64 == 0, SMOE_ERR_UNSUPPORTED, "%s: I=%d must be a multiple of 64", who, I);
+  return SMOE_OK;
+}
+
+static int check_common(int64_t TK, int H, int I, int E, const void* ws, size_t ws_bytes, const char* who) {
+  const int rc = check_sizes(TK, H, I, E, who);
+  if (rc) return rc;
   SMOE_REQUIRE(ws != nullptr && ws_bytes >= smoe_gemm_workspace_bytes(TK, E), SMOE_ERR_WORKSPACE,
                "%s: workspace too small", who);
   return SMOE_OK;
@@ -912,12 +915,11 @@ extern "C" size_t smoe_gemm_workspace_bytes(int64_t TK, int E) {
 
 extern "C" int smoe_dz_partial_cols(int I) { return (int)ceil_div(I, dz_tile_cols()) * dz_wave_cols(); }
 
-extern "C" int smoe_up_projection_forward(const void* x, const void* w1, int64_t w1_stride_e, int64_t w1_stride_row,
-                                          const void* b1, void* z, void* y1, const int32_t* off,
-                                          const int32_t* expert_schedule_order, const int32_t* x_gather_idx, int64_t T,
-                                          int64_t TK, int H, int I, int E, int activation, void* workspace,
-                                          size_t workspace_bytes, void* stream) {
-  int rc = check_common(TK, H, I, E, workspace, workspace_bytes, "up_projection_forward");
+int smoe::up_projection_forward(const void* x, const void* w1, int64_t w1_stride_e, int64_t w1_stride_row, const void* b1,
+                                void* z, void* y1, const int32_t* off, const int32_t* expert_schedule_order,
+                                const int32_t* x_gather_idx, int64_t T, int64_t TK, int H, int I, int E, int activation,
+                                GemmScratch& ws, void* stream) {
+  const int rc = check_sizes(TK, H, I, E, "up_projection_forward");
   if (rc) return rc;
   SMOE_REQUIRE(activation >= SMOE_ACT_SWIGLU && activation <= SMOE_ACT_SILU, SMOE_ERR_INVALID,
                "up_projection_forward: unknown activation code %d", activation);
@@ -945,14 +947,25 @@ extern "C" int smoe_up_projection_forward(const void* x, const void* w1, int64_t
   p.out0_stride = p.N;
   p.out1 = (uint16_t*)y1;
   p.out1_stride = I;
-  return launch_by_activation<false, ROLE_UP_FWD>(activation, p, off, workspace, TK, E, st);
+  return launch_by_activation<false, ROLE_UP_FWD>(activation, p, off, ws, TK, E, st);
 }
 
-extern "C" int smoe_down_projection_forward(const void* y1, const void* w2, int64_t w2_stride_e, int64_t w2_stride_row,
-                                            const void* b2, void* y2, const int32_t* off,
-                                            const int32_t* expert_schedule_order, int64_t TK, int H, int I, int E,
-                                            void* workspace, size_t workspace_bytes, void* stream) {
-  int rc = check_common(TK, H, I, E, workspace, workspace_bytes, "down_projection_forward");
+extern "C" int smoe_up_projection_forward(const void* x, const void* w1, int64_t w1_stride_e, int64_t w1_stride_row,
+                                          const void* b1, void* z, void* y1, const int32_t* off,
+                                          const int32_t* expert_schedule_order, const int32_t* x_gather_idx, int64_t T,
+                                          int64_t TK, int H, int I, int E, int activation, void* workspace,
+                                          size_t workspace_bytes, void* stream) {
+  int rc = check_common(TK, H, I, E, workspace, workspace_bytes, "up_projection_forward");
+  if (rc) return rc;
+  GemmScratch ws(workspace, workspace_bytes);
+  return smoe::up_projection_forward(x, w1, w1_stride_e, w1_stride_row, b1, z, y1, off, expert_schedule_order, x_gather_idx,
+                                     T, TK, H, I, E, activation, ws, stream);
+}
+
+int smoe::down_projection_forward(const void* y1, const void* w2, int64_t w2_stride_e, int64_t w2_stride_row,
+                                  const void* b2, void* y2, const int32_t* off, const int32_t* expert_schedule_order,
+                                  int64_t TK, int H, int I, int E, GemmScratch& ws, void* stream) {
+  const int rc = check_sizes(TK, H, I, E, "down_projection_forward");
   if (rc) return rc;
   if (TK == 0) return SMOE_OK;
   SMOE_REQUIRE(y1 && w2 && y2 && off, SMOE_ERR_INVALID, "down_projection_forward: null pointer");
@@ -973,7 +986,18 @@ extern "C" int smoe_down_projection_forward(const void* y1, const void* w2, int6
   p.bias = (const uint16_t*)b2;
   p.out0 = (uint16_t*)y2;
   p.out0_stride = H;
-  return launch_varlen_m<TileCfg<false>, ROLE_PLAIN, SMOE_ACT_SWIGLU>(p, off, workspace, TK, E, st);
+  return launch_varlen_m<TileCfg<false>, ROLE_PLAIN, SMOE_ACT_SWIGLU>(p, off, ws, TK, E, st);
+}
+
+extern "C" int smoe_down_projection_forward(const void* y1, const void* w2, int64_t w2_stride_e, int64_t w2_stride_row,
+                                            const void* b2, void* y2, const int32_t* off,
+                                            const int32_t* expert_schedule_order, int64_t TK, int H, int I, int E,
+                                            void* workspace, size_t workspace_bytes, void* stream) {
+  int rc = check_common(TK, H, I, E, workspace, workspace_bytes, "down_projection_forward");
+  if (rc) return rc;
+  GemmScratch ws(workspace, workspace_bytes);
+  return smoe::down_projection_forward(y1, w2, w2_stride_e, w2_stride_row, b2, y2, off, expert_schedule_order, TK, H, I, E,
+                                       ws, stream);
 }
 
 extern "C" int smoe_down_projection_forward_combine(const void* y1, const void* w2, int64_t w2_stride_e,
@@ -1008,16 +1032,16 @@ extern "C" int smoe_down_projection_forward_combine(const void* y1, const void* 
   p.out_rows = x_gather_idx;
   p.scores = scores;
   p.sidx = s_scatter_idx;
-  return launch_varlen_m<TileCfg<false>, ROLE_COMBINE, SMOE_ACT_SWIGLU>(p, off, workspace, TK, E, st);
+  GemmScratch ws(workspace, workspace_bytes);
+  return launch_varlen_m<TileCfg<false>, ROLE_COMBINE, SMOE_ACT_SWIGLU>(p, off, ws, TK, E, st);
 }
 
 // activation-gradient halves of the two backward operators; the weight-gradient halves live in gemm_varlen_k.hip
 namespace smoe {
-
 int launch_dz(const void* dout, const void* z, const void* w2, int64_t w2_stride_e, int64_t w2_stride_row, void* dz,
               void* y1s, float* ds_partial, const float* scores, const int32_t* off, const int32_t* order,
               const int32_t* gidx, const int32_t* sidx, int64_t T, int64_t TK, int H, int I, int E,
-              int activation, void* workspace, hipStream_t st) {
+              int activation, GemmScratch& ws, hipStream_t st) {
   const int zw = act_is_glu(activation) ? 2 : 1;
   VarlenMParams p = {};
   p.P = (const uint16_t*)dout;
@@ -1040,11 +1064,11 @@ int launch_dz(const void* dout, const void* z, const void* w2, int64_t w2_stride
   p.scores = scores;
   p.sidx = sidx;
   p.ds_partial = ds_partial;
-  return launch_by_activation<true, ROLE_DZ>(activation, p, off, workspace, TK, E, st);
+  return launch_by_activation<true, ROLE_DZ>(activation, p, off, ws, TK, E, st);
 }
 
 int launch_dx(const void* dz, const void* w1, int64_t w1_stride_e, int64_t w1_stride_row, void* dx_expanded,
-              const int32_t* off, const int32_t* order, int64_t TK, int H, int N1, int E, void* workspace,
+              const int32_t* off, const int32_t* order, int64_t TK, int H, int N1, int E, GemmScratch& ws,
               hipStream_t st) {
   VarlenMParams p = {};
   p.P = (const uint16_t*)dz;
@@ -1058,7 +1082,7 @@ int launch_dx(const void* dz, const void* w1, int64_t w1_stride_e, int64_t w1_st
   p.Kdim = N1;
   p.out0 = (uint16_t*)dx_expanded;
   p.out0_stride = H;
-  return launch_varlen_m<TileCfg<true>, ROLE_PLAIN, SMOE_ACT_SWIGLU>(p, off, workspace, TK, E, st);
+  return launch_varlen_m<TileCfg<true>, ROLE_PLAIN, SMOE_ACT_SWIGLU>(p, off, ws, TK, E, st);
 }
 
 }  // namespace smoe

@@ -1,8 +1,9 @@
 // The token-choice layer's launches behind the router GEMM as one call per direction: the entry points of this library in
 // the order in which the operators of the Python layer call them, on scratch memory that is carved here out of one buffer.
-// No kernel of its own.  What it is for: a call of an operator from Python (argument checks, allocations, ctypes) costs 8 to
-// 15 us of host time, more than most of the kernels take on a few tokens; a launch from here costs 3.
-#include "common.h"
+// No kernel of its own; the GEMMs of a direction share one tile map and one order of the experts (GemmScratch).  What it is
+// for: a call of an operator from Python (argument checks, allocations, ctypes) costs 8 to 15 us of host time, more than
+// most of the kernels take on a few tokens; a launch from here costs 3.
+#include "gemm_common.h"
 
 namespace smoe {
 
@@ -36,14 +37,15 @@ struct ForwardScratch {
 };
 
 struct BackwardScratch {
-  void *dz, *y1s, *dx_expanded, *partial, *loss_dlogits, *gemm;
+  void *dz, *y1s, *dx_expanded, *partial, *loss_dlogits, *map, *sorted;
   float *ds, *ds_partial;
-  size_t gemm_bytes, total;
+  size_t sorted_bytes, total;
   BackwardScratch(void* base, int64_t T, int H, int I, int E, int K, int N1, int64_t chunks) {
     Carver c{(char*)base};
     const int64_t TK = T * K;
-    gemm_bytes = smoe_gemm_workspace_bytes(TK, E);
-    gemm = c.take(gemm_bytes);
+    map = c.take(smoe_gemm_workspace_bytes(TK, E));
+    sorted_bytes = (size_t)E * sizeof(int32_t);
+    sorted = c.take(sorted_bytes);
     ds = (float*)c.take((size_t)TK * 4);
     loss_dlogits = c.take((size_t)T * E * 4);
     partial = c.take((size_t)(chunks > 1 ? chunks : 0) * E * H * 2);  // (one chunk is the gradient itself)
@@ -87,11 +89,12 @@ extern "C" int smoe_layer_forward(const smoe_layer_forward_args* a, void* stream
   rc = smoe_routing_metadata(a->indices, nullptr, TK, T, E, K, a->freq, a->off, a->x_gather_idx, a->s_scatter_idx,
                              a->s_reverse_scatter_idx, a->tok_off, s.metadata, s.metadata_bytes, stream);
   if (rc) return rc;
-  rc = smoe_up_projection_forward(a->x, a->w1, a->w1_stride_e, a->w1_stride_row, a->b1, a->z, s.y1, a->off, nullptr,
-                                  a->x_gather_idx, T, TK, H, I, E, (int)a->activation, s.gemm, s.gemm_bytes, stream);
+  GemmScratch ws(s.gemm, s.gemm_bytes);
+  rc = up_projection_forward(a->x, a->w1, a->w1_stride_e, a->w1_stride_row, a->b1, a->z, s.y1, a->off, nullptr,
+                             a->x_gather_idx, T, TK, H, I, E, (int)a->activation, ws, stream);
   if (rc) return rc;
-  rc = smoe_down_projection_forward(s.y1, a->w2, a->w2_stride_e, a->w2_stride_row, a->b2, s.y2, a->off, nullptr, TK, H, I, E,
-                                    s.gemm, s.gemm_bytes, stream);
+  rc = down_projection_forward(s.y1, a->w2, a->w2_stride_e, a->w2_stride_row, a->b2, s.y2, a->off, nullptr, TK, H, I, E, ws,
+                               stream);
   if (rc) return rc;
   rc = smoe_gather_sum(s.y2, a->o, a->scores, a->s_reverse_scatter_idx, nullptr, T, K, H, stream);
   if (rc || a->loss == nullptr) return rc;
@@ -115,14 +118,15 @@ extern "C" int smoe_layer_backward(const smoe_layer_backward_args* a, void* stre
   const BackwardScratch s(a->workspace, T, H, I, E, K, act <= SMOE_ACT_REGLU ? 2 * I : I, a->router_chunks);
   SMOE_REQUIRE(a->workspace != nullptr && a->workspace_bytes >= (int64_t)s.total, SMOE_ERR_WORKSPACE,
                "layer_backward: workspace too small");
-  int rc = smoe_down_projection_backward(a->dout, a->z, a->w2, a->w2_stride_e, a->w2_stride_row, a->b2, a->dw2,
+  GemmScratch ws(s.map, s.sorted, s.sorted_bytes);
+  int rc = down_projection_backward(a->dout, a->z, a->w2, a->w2_stride_e, a->w2_stride_row, a->b2, a->dw2,
                                          a->dw2_stride_e, a->dw2_stride_row, a->db2, s.dz, s.y1s, s.ds, s.ds_partial,
                                          a->scores, a->off, nullptr, a->x_gather_idx, a->s_scatter_idx, T, TK, H, I, E, act,
-                                         s.gemm, s.gemm_bytes, stream);
+                                         ws, stream);
   if (rc) return rc;
-  rc = smoe_up_projection_backward(a->x, a->w1, a->w1_stride_e, a->w1_stride_row, s.dz, a->dw1, a->dw1_stride_e,
+  rc = up_projection_backward(a->x, a->w1, a->w1_stride_e, a->w1_stride_row, s.dz, a->dw1, a->dw1_stride_e,
                                    a->dw1_stride_row, a->db1, s.dx_expanded, a->off, nullptr, a->x_gather_idx, T, TK, H, I, E,
-                                   act, s.gemm, s.gemm_bytes, stream);
+                                   act, ws, stream);
   if (rc) return rc;
   rc = smoe_gather_sum(s.dx_expanded, a->dx, nullptr, a->s_reverse_scatter_idx, nullptr, T, K, H, stream);
   if (rc) return rc;
