@@ -253,6 +253,11 @@ int smoe_router_weight_grad(const void* dlogits, const void* x, void* partial, i
 /* That sum: out[i] = sum of partial[c][i] over the chunks, in fp32 and chunk order, i < n; n a multiple of 8, bf16. */
 int smoe_sum_chunks(const void* partial, int chunks, int64_t n, void* out, void* stream);
 
+/* logits (T, E) = x (T, H) Wr (E, H)^T, 16-bit elements, fp32 accumulation: router_logits = F.linear(x, router_w)
+ * (sonicmoe/functional/__init__.py:438) for few tokens, where a library GEMM is latencies of host and device.  All
+ * contiguous, x and wr 16-byte aligned, H % 32 == 0. */
+int smoe_router_logits(const void* x, const void* wr, int64_t T, int H, int E, void* logits, void* stream);
+
 /* The router in one pass over x (bf16): logits = x Wr^T, the top-K winners of every row with their softmax scores, and
  * optionally the column sums of the full row softmax, all from the GEMM's accumulators.  Replaces the chain
  * router_logits = F.linear(x, router_w) -> sonicmoe::_softmax_topk_fwd (sonicmoe/functional/__init__.py:438-439,
@@ -401,17 +406,19 @@ int smoe_score_grad_bias_term(const void* dout, const void* b2, const int32_t* o
                               const int32_t* s_scatter_idx, float* ds, int64_t TK, int H, int E, void* stream);
 
 /* ---------------------------------------------------------------------------------------------------------
- * The token-choice layer behind its router GEMM, one call per direction (_TC_Softmax_Topk_Router / _UpProjection /
+ * The token-choice layer behind (of few tokens: with) its router GEMM, one call per direction (_TC_Softmax_Topk_Router / _UpProjection /
  * _DownProjection of the reference, sonicmoe/functional/__init__.py:85-420, :437-490): the entry points above in the order
  * of the operators, on one workspace.  For callers whose time goes into calls rather than kernels.  Every field of the two
  * structs is 8 bytes wide.  Shapes and limits are those of the entry points; T >= 1; experts in index order.
- *   smoe_topk_softmax_fwd -> smoe_routing_metadata -> smoe_up_projection_forward -> smoe_down_projection_forward ->
+ *   (smoe_router_logits ->) smoe_topk_softmax_fwd -> smoe_routing_metadata -> smoe_up_projection_forward -> smoe_down_projection_forward ->
  *   smoe_gather_sum -> smoe_switch_loss_fwd (loss != NULL)
  *   smoe_down_projection_backward -> smoe_up_projection_backward -> smoe_gather_sum -> smoe_switch_loss_bwd (loss_grad !=
  *   NULL) -> smoe_router_logit_grad -> smoe_router_weight_grad and smoe_sum_chunks (router_chunks > 0)
  * The caller adds the router's share of dx (dlogits Wr) itself. */
 typedef struct {
-  const void *x, *logits, *w1, *b1, *w2, *b2; /* b1, b2: nullable */
+  const void *x, *router_w; /* router_w: nullable; given, the call begins with smoe_router_logits into logits */
+  void* logits;
+  const void *w1, *b1, *w2, *b2; /* b1, b2: nullable */
   int64_t w1_stride_e, w1_stride_row, w2_stride_e, w2_stride_row;
   int64_t logits_dtype, logits_row_stride; /* smoe_dtype; elements */
   int64_t T, H, I, E, K, activation;

@@ -4,6 +4,7 @@
 // for: a call of an operator from Python (argument checks, allocations, ctypes) costs 8 to 15 us of host time, more than
 // most of the kernels take on a few tokens; a launch from here costs 3.
 #include "gemm_common.h"
+#include "routing_common.h"
 
 namespace smoe {
 
@@ -19,7 +20,7 @@ struct Carver {
 };
 
 struct ForwardScratch {
-  void *y1, *y2, *gemm, *metadata, *loss;
+  void *y1, *y2, *gemm, *metadata, *loss, *few;
   size_t gemm_bytes, metadata_bytes, loss_bytes, total;
   ForwardScratch(void* base, int64_t T, int H, int I, int E, int K) {
     Carver c{(char*)base};
@@ -30,6 +31,7 @@ struct ForwardScratch {
     gemm = c.take(gemm_bytes);
     metadata = c.take(metadata_bytes);
     loss = c.take(loss_bytes);
+    few = c.take(route_few_workspace_bytes(T, E));
     y1 = c.take((size_t)TK * I * 2);
     y2 = c.take((size_t)TK * H * 2);
     total = c.used;
@@ -61,6 +63,12 @@ struct BackwardScratch {
   }
 };
 
+#ifdef SMOE_ELEM_F16
+constexpr int ELEM_DTYPE = SMOE_DT_F16;
+#else
+constexpr int ELEM_DTYPE = SMOE_DT_BF16;
+#endif
+
 static bool layer_sizes_ok(int64_t T, int64_t H, int64_t I, int64_t E, int64_t K) {
   const int64_t lim = 1ll << 31;
   return T > 0 && T < lim && H > 0 && H < (1 << 24) && I > 0 && I < (1 << 24) && E > 0 && E <= 4096 && K > 0 && K <= E &&
@@ -83,12 +91,27 @@ extern "C" int smoe_layer_forward(const smoe_layer_forward_args* a, void* stream
   const ForwardScratch s(a->workspace, T, H, I, E, K);
   SMOE_REQUIRE(a->workspace != nullptr && a->workspace_bytes >= (int64_t)s.total, SMOE_ERR_WORKSPACE,
                "layer_forward: workspace too small");
-  int rc = smoe_topk_softmax_fwd(a->logits, (int)a->logits_dtype, T, E, K, a->logits_row_stride, a->scores, a->indices, 1,
-                                 stream);
-  if (rc) return rc;
-  rc = smoe_routing_metadata(a->indices, nullptr, TK, T, E, K, a->freq, a->off, a->x_gather_idx, a->s_scatter_idx,
-                             a->s_reverse_scatter_idx, a->tok_off, s.metadata, s.metadata_bytes, stream);
-  if (rc) return rc;
+  int rc = SMOE_OK;
+  SMOE_REQUIRE(a->router_w == nullptr || (a->logits_row_stride == E && a->logits_dtype == ELEM_DTYPE), SMOE_ERR_INVALID,
+               "layer_forward: logits to be computed are contiguous, of the library's type");
+  const bool few = a->router_w != nullptr && route_few_takes(T, H, E, K);
+  if (few) {  // logits, top-K, metadata and loss in two launches, the same results
+    rc = launch_route_few(a->x, a->router_w, T, H, E, K, a->logits, a->scores, a->indices, a->freq, a->off, a->x_gather_idx,
+                          a->s_scatter_idx, a->s_reverse_scatter_idx, a->tok_off, a->loss_acc, a->loss, s.few,
+                          (hipStream_t)stream);
+    if (rc) return rc;
+  } else {
+    if (a->router_w != nullptr) {
+      rc = smoe_router_logits(a->x, a->router_w, T, H, E, a->logits, stream);
+      if (rc) return rc;
+    }
+    rc = smoe_topk_softmax_fwd(a->logits, (int)a->logits_dtype, T, E, K, a->logits_row_stride, a->scores, a->indices, 1,
+                               stream);
+    if (rc) return rc;
+    rc = smoe_routing_metadata(a->indices, nullptr, TK, T, E, K, a->freq, a->off, a->x_gather_idx, a->s_scatter_idx,
+                               a->s_reverse_scatter_idx, a->tok_off, s.metadata, s.metadata_bytes, stream);
+    if (rc) return rc;
+  }
   GemmScratch ws(s.gemm, s.gemm_bytes);
   rc = up_projection_forward(a->x, a->w1, a->w1_stride_e, a->w1_stride_row, a->b1, a->z, s.y1, a->off, nullptr,
                              a->x_gather_idx, T, TK, H, I, E, (int)a->activation, ws, stream);
@@ -97,7 +120,7 @@ extern "C" int smoe_layer_forward(const smoe_layer_forward_args* a, void* stream
                                stream);
   if (rc) return rc;
   rc = smoe_gather_sum(s.y2, a->o, a->scores, a->s_reverse_scatter_idx, nullptr, T, K, H, stream);
-  if (rc || a->loss == nullptr) return rc;
+  if (rc || few || a->loss == nullptr) return rc;
   return smoe_switch_loss_fwd(a->logits, (int)a->logits_dtype, a->logits_row_stride, T, E, a->freq, a->loss_acc, a->loss,
                               s.loss, s.loss_bytes, stream);
 }

@@ -4,7 +4,7 @@
 
 #include <mutex>
 
-#include "common.h"
+#include "routing_common.h"
 
 namespace smoe {
 
@@ -18,66 +18,6 @@ namespace smoe {
 // values, the lowest column.  K rounds of "group arg-max, then retire the winner" give the winners in descending order.
 // A round is a chain of maxima, one instruction each on 32-bit keys and three on 64-bit ones (one row, E = 128, K = 8:
 // 8.3 -> 5.8 us; T = 40960, E = 256: 32 -> 26 us).
-
-SMOE_DEV uint32_t orderable(uint32_t bits) { return bits ^ ((bits >> 31) ? 0xffffffffu : 0x80000000u); }
-SMOE_DEV uint32_t unorderable(uint32_t o) { return o ^ ((o >> 31) ? 0x80000000u : 0xffffffffu); }
-
-SMOE_DEV uint64_t shfl_xor_u64(uint64_t v, int mask) {
-  uint32_t lo = (uint32_t)v, hi = (uint32_t)(v >> 32);
-  lo = __shfl_xor(lo, mask, 64);
-  hi = __shfl_xor(hi, mask, 64);
-  return ((uint64_t)hi << 32) | lo;
-}
-
-template <typename T>
-SMOE_DEV uint32_t load_as_f32_bits(const T* p);
-template <>
-__device__ __forceinline__ uint32_t load_as_f32_bits<uint16_t>(const uint16_t* p) {  // bf16
-  return (uint32_t)(*p) << 16;
-}
-template <>
-__device__ __forceinline__ uint32_t load_as_f32_bits<__half>(const __half* p) {
-  return __float_as_uint(__half2float(*p));
-}
-template <>
-__device__ __forceinline__ uint32_t load_as_f32_bits<float>(const float* p) {
-  return __float_as_uint(*p);
-}
-
-template <typename T>
-struct TopkKey;
-template <>
-struct TopkKey<float> {
-  typedef uint64_t Key;
-  static __device__ __forceinline__ uint32_t load(const float* p, uint32_t clear_mask) {
-    return __float_as_uint(*p) & clear_mask;
-  }
-  static __device__ __forceinline__ Key make(uint32_t bits, int col) {
-    return ((uint64_t)orderable(bits) << 32) | (uint64_t)(0xffffffffu - (uint32_t)col);
-  }
-  static __device__ __forceinline__ float value(Key k) { return __uint_as_float(unorderable((uint32_t)(k >> 32))); }
-  static __device__ __forceinline__ int column(Key k) { return (int)(0xffffffffu - (uint32_t)k); }
-  static __device__ __forceinline__ Key shfl_xor(Key k, int m) { return shfl_xor_u64(k, m); }
-};
-// (clearing the low bits of the fp32 image, log2(E) <= 12 of them, does not touch a 16-bit value)
-template <typename T>
-struct TopkKey16 {
-  typedef uint32_t Key;
-  static __device__ __forceinline__ uint32_t load(const T* p, uint32_t) { return *(const uint16_t*)p; }
-  static __device__ __forceinline__ Key make(uint32_t bits, int col) {
-    return (bits ^ ((bits >> 15) ? 0xffffu : 0x8000u)) << 16 | (0xffffu - (uint32_t)col);
-  }
-  static __device__ __forceinline__ float value(Key k) {
-    const uint16_t o = (uint16_t)(k >> 16), bits = o ^ ((o >> 15) ? 0x8000u : 0xffffu);
-    return __uint_as_float(load_as_f32_bits<T>((const T*)&bits));
-  }
-  static __device__ __forceinline__ int column(Key k) { return (int)(0xffffu - (k & 0xffffu)); }
-  static __device__ __forceinline__ Key shfl_xor(Key k, int m) { return __shfl_xor(k, m, 64); }
-};
-template <>
-struct TopkKey<uint16_t> : TopkKey16<uint16_t> {};
-template <>
-struct TopkKey<__half> : TopkKey16<__half> {};
 
 template <typename T, int VPL>
 __global__ __launch_bounds__(256) void topk_softmax_kernel(const T* __restrict__ logits, int64_t row_stride,
@@ -118,10 +58,7 @@ __global__ __launch_bounds__(256) void topk_softmax_kernel(const T* __restrict__
     Key best = key[0];
 #pragma unroll
     for (int i = 1; i < VPL; i++) best = key[i] > best ? key[i] : best;
-    for (int m = 1; m < G; m <<= 1) {
-      const Key o = TK::shfl_xor(best, m);
-      best = o > best ? o : best;
-    }
+    best = TK::max_over(best, G);
 #pragma unroll
     for (int i = 0; i < VPL; i++) key[i] = (key[i] == best) ? 0 : key[i];
     if (g == 0 && row_ok) {
@@ -439,50 +376,6 @@ __global__ __launch_bounds__(256) void meta_scan_kernel(const int32_t* __restric
     carry += __shfl(v, 63, 64);
   }
   if (lane == 0) freq[e] = carry;
-}
-
-// One step of the counting sort for a wavefront: lane l holds slot j (consecutive over the lanes, `valid` a prefix of them)
-// of expert e.  Slots of the same expert take consecutive positions from that expert's cursor, in lane order.
-SMOE_DEV void place_slots(int e, int j, bool valid, int lane, const int32_t* __restrict__ token_idx, int TK,
-                          int64_t T, int E, int K, int ebits, int32_t* cursor, int32_t* __restrict__ gidx,
-                          int32_t* __restrict__ sidx, int32_t* __restrict__ ridx, int32_t* __restrict__ tok_off) {
-  const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-  const bool in_range = valid && e >= 0 && e < E;
-  if (!in_range) e = 0;
-  uint64_t peers = __ballot(in_range);
-  for (int b = 0; b < ebits; b++) {
-    const uint64_t bal = __ballot((e >> b) & 1);
-    peers &= ((e >> b) & 1) ? bal : ~bal;
-  }
-  int32_t pos = 0;
-  if (in_range) {
-    pos = cursor[e] + __popcll(peers & lt_mask);
-  }
-  __builtin_amdgcn_wave_barrier();
-  if (in_range && (peers >> lane) >> 1 == 0) cursor[e] = pos + 1;  // highest peer lane advances the cursor
-  __builtin_amdgcn_wave_barrier();
-  // (past the end j may not fit a token: nothing is read or written for it)
-  int32_t t = 0;
-  if (token_idx == nullptr)
-    t = (int32_t)((uint32_t)j / (uint32_t)K);
-  else if (valid)
-    t = token_idx[j];
-  if (in_range) {
-    sidx[pos] = j;
-    ridx[j] = pos;
-    gidx[pos] = t;
-  }
-  if (tok_off && valid) {
-    if (token_idx) {
-      const int32_t tprev = j == 0 ? -1 : token_idx[j - 1];
-      for (int32_t u = tprev + 1; u <= t; u++) tok_off[u] = j;
-      if (j == TK - 1)
-        for (int64_t u = (int64_t)t + 1; u <= T; u++) tok_off[u] = TK;
-    } else {
-      if (j == t * K) tok_off[t] = j;
-      if (j == TK - 1) tok_off[T] = TK;
-    }
-  }
 }
 
 __global__ __launch_bounds__(64 * META_WAVES) void meta_scatter_kernel(

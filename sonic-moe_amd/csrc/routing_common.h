@@ -1,0 +1,241 @@
+// What the routing kernels and the load-balancing loss share: sort keys of the top-K, one step of the counting sort, row
+// softmax and sums over a wavefront or workgroup.
+#pragma once
+#include <hip/hip_fp16.h>
+
+#include "common.h"
+
+namespace smoe {
+
+// ---- reductions ----------------------------------------------------------------------------------------------------------
+// Reductions over a wavefront in six steps of the vector pipe: neighbours, pairs and quads inside rows of 16 lanes by DPP,
+// the rows by lane swaps.  Through __shfl_xor each step is a round trip to LDS of some 60 cycles, and a top-K of 8 is 48 of
+// them in a row.  Every lane gets the result.
+template <int CTRL>
+SMOE_DEV uint32_t dpp(uint32_t v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+constexpr int DPP_XOR1 = 0xb1, DPP_XOR2 = 0x4e, DPP_HALF_MIRROR = 0x141, DPP_MIRROR = 0x140;
+// op over lanes whose numbers differ in the bits below G (a power of two up to 64, the same for all lanes)
+template <class V, class Op>
+SMOE_DEV V group_reduce(V v, int G, Op op) {
+  auto bits = [](V x) { return __builtin_bit_cast(uint32_t, x); };
+  auto value = [](uint32_t x) { return __builtin_bit_cast(V, x); };
+  if (G > 1) v = op(v, value(dpp<DPP_XOR1>(bits(v))));
+  if (G > 2) v = op(v, value(dpp<DPP_XOR2>(bits(v))));
+  if (G > 4) v = op(v, value(dpp<DPP_HALF_MIRROR>(bits(v))));  // (a quad's lanes agree by now: any lane of the other one)
+  if (G > 8) v = op(v, value(dpp<DPP_MIRROR>(bits(v))));
+  if (G > 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(bits(v), bits(v), false, false);
+    v = op(value(r[0]), value(r[1]));
+  }
+  if (G > 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(bits(v), bits(v), false, false);
+    v = op(value(r[0]), value(r[1]));
+  }
+  return v;
+}
+SMOE_DEV uint32_t group_max(uint32_t v, int G) {
+  return group_reduce(v, G, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
+}
+SMOE_DEV float wave_max(float v) {
+  return group_reduce(v, 64, [](float a, float b) { return fmaxf(a, b); });
+}
+SMOE_DEV float wave_sum(float v) {
+  return group_reduce(v, 64, [](float a, float b) { return a + b; });
+}
+
+// ---- top-K keys (layout: routing.hip) ------------------------------------------------------------------------------------
+SMOE_DEV uint32_t orderable(uint32_t bits) { return bits ^ ((bits >> 31) ? 0xffffffffu : 0x80000000u); }
+SMOE_DEV uint32_t unorderable(uint32_t o) { return o ^ ((o >> 31) ? 0x80000000u : 0xffffffffu); }
+
+SMOE_DEV uint64_t shfl_xor_u64(uint64_t v, int mask) {
+  uint32_t lo = (uint32_t)v, hi = (uint32_t)(v >> 32);
+  lo = __shfl_xor(lo, mask, 64);
+  hi = __shfl_xor(hi, mask, 64);
+  return ((uint64_t)hi << 32) | lo;
+}
+
+template <typename T>
+SMOE_DEV uint32_t load_as_f32_bits(const T* p);
+template <>
+__device__ __forceinline__ uint32_t load_as_f32_bits<uint16_t>(const uint16_t* p) {  // bf16
+  return (uint32_t)(*p) << 16;
+}
+template <>
+__device__ __forceinline__ uint32_t load_as_f32_bits<__half>(const __half* p) {
+  return __float_as_uint(__half2float(*p));
+}
+template <>
+__device__ __forceinline__ uint32_t load_as_f32_bits<float>(const float* p) {
+  return __float_as_uint(*p);
+}
+
+template <typename T>
+struct TopkKey;
+template <>
+struct TopkKey<float> {
+  typedef uint64_t Key;
+  static __device__ __forceinline__ uint32_t load(const float* p, uint32_t clear_mask) {
+    return __float_as_uint(*p) & clear_mask;
+  }
+  static __device__ __forceinline__ Key make(uint32_t bits, int col) {
+    return ((uint64_t)orderable(bits) << 32) | (uint64_t)(0xffffffffu - (uint32_t)col);
+  }
+  static __device__ __forceinline__ float value(Key k) { return __uint_as_float(unorderable((uint32_t)(k >> 32))); }
+  static __device__ __forceinline__ int column(Key k) { return (int)(0xffffffffu - (uint32_t)k); }
+  static __device__ __forceinline__ Key max_over(Key k, int G) {
+    for (int m = 1; m < G; m <<= 1) {
+      const Key o = shfl_xor_u64(k, m);
+      k = o > k ? o : k;
+    }
+    return k;
+  }
+};
+// (clearing the low bits of the fp32 image, log2(E) <= 12 of them, does not touch a 16-bit value)
+template <typename T>
+struct TopkKey16 {
+  typedef uint32_t Key;
+  static __device__ __forceinline__ uint32_t load(const T* p, uint32_t) { return *(const uint16_t*)p; }
+  static __device__ __forceinline__ Key make(uint32_t bits, int col) {
+    return (bits ^ ((bits >> 15) ? 0xffffu : 0x8000u)) << 16 | (0xffffu - (uint32_t)col);
+  }
+  static __device__ __forceinline__ float value(Key k) {
+    const uint16_t o = (uint16_t)(k >> 16), bits = o ^ ((o >> 15) ? 0x8000u : 0xffffu);
+    return __uint_as_float(load_as_f32_bits<T>((const T*)&bits));
+  }
+  static __device__ __forceinline__ int column(Key k) { return (int)(0xffffu - (k & 0xffffu)); }
+  static __device__ __forceinline__ Key max_over(Key k, int G) { return group_max(k, G); }
+};
+template <>
+struct TopkKey<uint16_t> : TopkKey16<uint16_t> {};
+template <>
+struct TopkKey<__half> : TopkKey16<__half> {};
+
+// ---- counting sort ---------------------------------------------------------------------------------------------------------
+// One step of the counting sort for a wavefront: lane l holds slot j (consecutive over the lanes, `valid` a prefix of them)
+// of expert e.  Slots of the same expert take consecutive positions from that expert's cursor, in lane order.
+SMOE_DEV void place_slots(int e, int j, bool valid, int lane, const int32_t* __restrict__ token_idx, int TK,
+                          int64_t T, int E, int K, int ebits, int32_t* cursor, int32_t* __restrict__ gidx,
+                          int32_t* __restrict__ sidx, int32_t* __restrict__ ridx, int32_t* __restrict__ tok_off) {
+  const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+  const bool in_range = valid && e >= 0 && e < E;
+  if (!in_range) e = 0;
+  uint64_t peers = __ballot(in_range);
+  for (int b = 0; b < ebits; b++) {
+    const uint64_t bal = __ballot((e >> b) & 1);
+    peers &= ((e >> b) & 1) ? bal : ~bal;
+  }
+  int32_t pos = 0;
+  if (in_range) {
+    pos = cursor[e] + __popcll(peers & lt_mask);
+  }
+  __builtin_amdgcn_wave_barrier();
+  if (in_range && (peers >> lane) >> 1 == 0) cursor[e] = pos + 1;  // highest peer lane advances the cursor
+  __builtin_amdgcn_wave_barrier();
+  // (past the end j may not fit a token: nothing is read or written for it)
+  int32_t t = 0;
+  if (token_idx == nullptr)
+    t = (int32_t)((uint32_t)j / (uint32_t)K);
+  else if (valid)
+    t = token_idx[j];
+  if (in_range) {
+    sidx[pos] = j;
+    ridx[j] = pos;
+    gidx[pos] = t;
+  }
+  if (tok_off && valid) {
+    if (token_idx) {
+      const int32_t tprev = j == 0 ? -1 : token_idx[j - 1];
+      for (int32_t u = tprev + 1; u <= t; u++) tok_off[u] = j;
+      if (j == TK - 1)
+        for (int64_t u = (int64_t)t + 1; u <= T; u++) tok_off[u] = TK;
+    } else {
+      if (j == t * K) tok_off[t] = j;
+      if (j == TK - 1) tok_off[T] = TK;
+    }
+  }
+}
+
+// ---- softmax of a row, sums --------------------------------------------------------------------------------------------------
+template <typename T>
+SMOE_DEV float sl_load(const T* p);
+template <>
+__device__ __forceinline__ float sl_load<uint16_t>(const uint16_t* p) {  // bf16
+  return __uint_as_float((uint32_t)(*p) << 16);
+}
+template <>
+__device__ __forceinline__ float sl_load<__half>(const __half* p) {
+  return __half2float(*p);
+}
+template <>
+__device__ __forceinline__ float sl_load<float>(const float* p) {
+  return *p;
+}
+
+// softmax of one row held as VPL values per lane (columns lane + 64 i); columns >= E hold -inf and come out as 0
+template <int VPL>
+SMOE_DEV void row_softmax(float (&v)[VPL]) {
+  float m = v[0];
+#pragma unroll
+  for (int i = 1; i < VPL; i++) m = fmaxf(m, v[i]);
+  m = wave_max(m);
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < VPL; i++) {
+    v[i] = __expf(v[i] - m);
+    s += v[i];
+  }
+  s = wave_sum(s);
+  const float inv = 1.0f / s;
+#pragma unroll
+  for (int i = 0; i < VPL; i++) v[i] *= inv;
+}
+
+template <typename T, int VPL>
+SMOE_DEV void load_row(const T* row, int E, int lane, float (&v)[VPL]) {
+#pragma unroll
+  for (int i = 0; i < VPL; i++) {
+    const int c = lane + 64 * i;
+    v[i] = sl_load<T>(row + (c < E ? c : E - 1));
+  }
+}
+// the columns past the end, once all of a wavefront's loads are under way
+template <int VPL>
+SMOE_DEV void mask_row(int E, int lane, float (&v)[VPL]) {
+#pragma unroll
+  for (int i = 0; i < VPL; i++) {
+    const float x = __uint_as_float(opaque(__float_as_uint(v[i])));
+    v[i] = lane + 64 * i < E ? x : -INFINITY;
+  }
+}
+
+// block-wide sum of three values; every thread gets the totals
+SMOE_DEV void block_sum3(float& a, float& b, float& c, float* scratch /* 3 * 16 floats */) {
+  a = wave_sum(a);
+  b = wave_sum(b);
+  c = wave_sum(c);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  if (lane == 0) {
+    scratch[wave] = a;
+    scratch[16 + wave] = b;
+    scratch[32 + wave] = c;
+  }
+  __syncthreads();
+  a = b = c = 0.f;
+  for (int w = 0; w < nw; w++) {
+    a += scratch[w];
+    b += scratch[16 + w];
+    c += scratch[32 + w];
+  }
+  __syncthreads();
+}
+
+// router_logits, top-K, metadata and loss of few tokens: route_few.hip
+bool route_few_takes(int64_t T, int H, int E, int K);
+size_t route_few_workspace_bytes(int64_t T, int E);
+int launch_route_few(const void* x, const void* wr, int64_t T, int H, int E, int K, void* logits, float* scores,
+                     int32_t* indices, int32_t* freq, int32_t* off, int32_t* gidx, int32_t* sidx, int32_t* ridx,
+                     int32_t* tok_off, float* loss_acc, float* loss, void* workspace, hipStream_t st);
+
+}  // namespace smoe

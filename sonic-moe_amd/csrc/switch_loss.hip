@@ -9,24 +9,10 @@
 // logits' dtype, with dacc[j] = E / (S F) * (freq[j] - D / S), S = |acc|_1, F = |freq|_1, D = <acc, freq>.
 #include <hip/hip_fp16.h>
 
-#include "common.h"
+#include "routing_common.h"
 
 namespace smoe {
 
-template <typename T>
-SMOE_DEV float sl_load(const T* p);
-template <>
-__device__ __forceinline__ float sl_load<uint16_t>(const uint16_t* p) {  // bf16
-  return __uint_as_float((uint32_t)(*p) << 16);
-}
-template <>
-__device__ __forceinline__ float sl_load<__half>(const __half* p) {
-  return __half2float(*p);
-}
-template <>
-__device__ __forceinline__ float sl_load<float>(const float* p) {
-  return *p;
-}
 template <typename T>
 SMOE_DEV void sl_store(T* p, float v);
 template <>
@@ -42,38 +28,8 @@ __device__ __forceinline__ void sl_store<float>(float* p, float v) {
   *p = v;
 }
 
-SMOE_DEV float wave_max(float v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v = fmaxf(v, __shfl_xor(v, m, 64));
-  return v;
-}
-SMOE_DEV float wave_sum(float v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
-  return v;
-}
-
 constexpr int SL_WAVES = 4;            // wavefronts per workgroup of the backward pass
 constexpr int SL_MAX_PARTIALS = 256;  // workgroups of the forward pass
-
-// softmax of one row held as VPL values per lane (columns lane + 64 i); columns >= E hold -inf and come out as 0
-template <int VPL>
-SMOE_DEV void row_softmax(float (&v)[VPL]) {
-  float m = v[0];
-#pragma unroll
-  for (int i = 1; i < VPL; i++) m = fmaxf(m, v[i]);
-  m = wave_max(m);
-  float s = 0.f;
-#pragma unroll
-  for (int i = 0; i < VPL; i++) {
-    v[i] = __expf(v[i] - m);
-    s += v[i];
-  }
-  s = wave_sum(s);
-  const float inv = 1.0f / s;
-#pragma unroll
-  for (int i = 0; i < VPL; i++) v[i] *= inv;
-}
 
 // R rows at once: the R wave reductions are independent chains the hardware overlaps (one row at a time leaves a
 // wavefront waiting on 12 dependent cross-lane moves per row)
@@ -87,9 +43,7 @@ SMOE_DEV void rows_softmax(float (&v)[R][VPL]) {
     for (int i = 1; i < VPL; i++) m[r] = fmaxf(m[r], v[r][i]);
   }
 #pragma unroll
-  for (int k = 32; k >= 1; k >>= 1)
-#pragma unroll
-    for (int r = 0; r < R; r++) m[r] = fmaxf(m[r], __shfl_xor(m[r], k, 64));
+  for (int r = 0; r < R; r++) m[r] = wave_max(m[r]);
 #pragma unroll
   for (int r = 0; r < R; r++) {
     s[r] = 0.f;
@@ -100,9 +54,7 @@ SMOE_DEV void rows_softmax(float (&v)[R][VPL]) {
     }
   }
 #pragma unroll
-  for (int k = 32; k >= 1; k >>= 1)
-#pragma unroll
-    for (int r = 0; r < R; r++) s[r] += __shfl_xor(s[r], k, 64);
+  for (int r = 0; r < R; r++) s[r] = wave_sum(s[r]);
 #pragma unroll
   for (int r = 0; r < R; r++) {
     const float inv = 1.0f / s[r];
@@ -116,45 +68,6 @@ template <int VPL>
 struct RowsAtOnce {
   static constexpr int value = VPL <= 4 ? 4 : (VPL <= 16 ? 2 : 1);
 };
-
-template <typename T, int VPL>
-SMOE_DEV void load_row(const T* row, int E, int lane, float (&v)[VPL]) {
-#pragma unroll
-  for (int i = 0; i < VPL; i++) {
-    const int c = lane + 64 * i;
-    v[i] = sl_load<T>(row + (c < E ? c : E - 1));
-  }
-}
-// the columns past the end, once all of a wavefront's loads are under way
-template <int VPL>
-SMOE_DEV void mask_row(int E, int lane, float (&v)[VPL]) {
-#pragma unroll
-  for (int i = 0; i < VPL; i++) {
-    const float x = __uint_as_float(opaque(__float_as_uint(v[i])));
-    v[i] = lane + 64 * i < E ? x : -INFINITY;
-  }
-}
-
-// block-wide sum of three values; every thread gets the totals
-SMOE_DEV void block_sum3(float& a, float& b, float& c, float* scratch /* 3 * 16 floats */) {
-  a = wave_sum(a);
-  b = wave_sum(b);
-  c = wave_sum(c);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  if (lane == 0) {
-    scratch[wave] = a;
-    scratch[16 + wave] = b;
-    scratch[32 + wave] = c;
-  }
-  __syncthreads();
-  a = b = c = 0.f;
-  for (int w = 0; w < nw; w++) {
-    a += scratch[w];
-    b += scratch[16 + w];
-    c += scratch[32 + w];
-  }
-  __syncthreads();
-}
 
 template <typename T, int VPL>
 __global__ __launch_bounds__(VPL <= 16 ? 1024 : 256) void softmax_colsum_kernel(const T* __restrict__ logits,

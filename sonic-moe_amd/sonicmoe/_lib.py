@@ -58,6 +58,7 @@ _SIGNATURES = {
     ),
     "smoe_router_weight_grad": (c_int, [_P, _P, _P, _L, _I, _I, _I, _P]),
     "smoe_sum_chunks": (c_int, [_P, _I, _L, _P, _P]),
+    "smoe_router_logits": (c_int, [_P, _P, _L, _I, _I, _P, _P]),
     "smoe_router_fused_partials": (ctypes.c_int64, [_L, _I]),
     "smoe_router_forward_fused": (c_int, [_P, _P, _L, _I, _I, _I, _P, _P, _P, _P, _P]),
     "smoe_switch_loss_from_partials": (c_int, [_P, _L, _I, _P, _P, _P, _P]),

@@ -43,6 +43,7 @@ from .forward import (
     _up_projection_forward,
     router_fused_partials,
     router_fused_supported,
+    router_linear,
 )
 from .fp8 import (
     _down_projection_backward_fp8,
@@ -161,7 +162,7 @@ class _RouterLinearFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x: torch.Tensor, router_w: torch.Tensor):
         ctx.save_for_backward(x, router_w)
-        return F.linear(x, router_w)
+        return router_linear(x, router_w)
 
     @staticmethod
     def backward(ctx, dlogits: torch.Tensor):
@@ -490,7 +491,7 @@ class _TCLayerFunction(torch.autograd.Function):
             if not torch.compiler.is_compiling():
                 router_logits._smoe_softmax_colsum_partials = (colsum, router_logits._version)
         else:
-            router_logits = F.linear(x, router_w)
+            router_logits = router_linear(x, router_w)
             run(_softmax_topk_fwd, router_logits, scores, indices, E, K)
         freq, off, gidx, sidx, ridx, tok_off = _build_metadata(indices.view(-1), None, T, E, K)
         scores_flat = scores.view(-1)
@@ -542,11 +543,10 @@ class _OneCallLayerFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, router_w, w1, b1, w2, b2, K: int, activation_type: ActivationType, stream_id: int, with_loss: bool):
         x = x.contiguous()
-        logits = F.linear(x, router_w)
-        done = layer_call.forward(x, logits, w1, b1, w2, b2, K, activation_type, stream_id, True, with_loss)
+        done = layer_call.forward(x, router_w, w1, b1, w2, b2, K, activation_type, stream_id, True, with_loss)
         if done is None:
             raise layer_call.Refused
-        o, z, freq, ints, loss = done
+        o, logits, z, freq, ints, loss = done
         ctx.save_for_backward(x, router_w, w1, w2, b2, z, ints, freq, logits)
         ctx.cfg = (K, activation_type, stream_id, b1 is not None)
         ctx.set_materialize_grads(False)  # (zeros for the token counts and the logits nobody used would be two launches)
@@ -686,11 +686,9 @@ def layer_with_loss(x, router_w, w1, b1, w2, b2, K: int, stream_id: int, activat
             x.requires_grad or router_w.requires_grad or w1.requires_grad or w2.requires_grad
             or (b1 is not None and (b1.requires_grad or b2.requires_grad)))
         if not needs_grad:
-            x = x.contiguous()
-            logits = F.linear(x, router_w)
-            done = layer_call.forward(x, logits, w1, b1, w2, b2, K, activation_type, stream_id, False, with_loss)
+            done = layer_call.forward(x.contiguous(), router_w, w1, b1, w2, b2, K, activation_type, stream_id, False, with_loss)
             if done is not None:
-                return done[0], logits, done[2], done[4]
+                return done[0], done[1], done[3], done[5]
         elif not is_inference_mode_enabled:
             try:
                 return _OneCallLayerFunction.apply(x, router_w, w1, b1, w2, b2, K, activation_type, stream_id, with_loss)

@@ -315,6 +315,48 @@ def _switch_loss_fwd(router_logits: torch.Tensor, expert_frequency: torch.Tensor
     _lib.check(rc, "_switch_loss_fwd")
 
 
+@operator("_router_logits", mutates_args={"logits"})
+def _router_logits(x: torch.Tensor, router_w: torch.Tensor, logits: torch.Tensor) -> None:
+    """logits (T, E) = x router_w^T: the reference's F.linear (sonicmoe/functional/__init__.py:438) for few tokens."""
+    _lib.require_device(x, router_w, logits)
+    dt = _elem_dtype(("x", x), ("router_w", router_w), ("logits", logits))
+    T, H = x.shape
+    E = router_w.size(0)
+    assert x.is_contiguous() and router_w.is_contiguous() and logits.is_contiguous()
+    assert router_w.shape == (E, H) and logits.shape == (T, E)
+    rc = _lib.lib(dt).smoe_router_logits(_lib.ptr(x), _lib.ptr(router_w), T, H, E, _lib.ptr(logits),
+                                         _lib.current_stream_handle())
+    _lib.check(rc, "_router_logits")
+
+
+# Where the router GEMM is `_router_logits` and not the library's.  The library's call takes 20 us on the host.  Up to 64
+# tokens a layer waits for its launches, and there the kernel is half of a fused routing (csrc/route_few.hip); up to 1024 that
+# holds for the smallest layers, whose few experts leave the kernel one workgroup per 16 tokens (6.4 us at E = 8, H = 512,
+# 3.5 the library's); with more tokens or experts the GPU is busy, and the library's kernel is the faster one: 777 tokens,
+# E = 48, H = 1472 9.1 against 6.0 us, 1024 tokens, E = 128, H = 4096 19 against 8.
+ROUTER_LOGITS_MAX_TOKENS, ROUTER_LOGITS_MAX_TOKENS_FEW_EXPERTS, FEW_EXPERTS = 64, 1024, 16
+
+
+def router_logits_takes(x: torch.Tensor, router_w: torch.Tensor) -> bool:
+    """Whether `_router_logits` stands in for F.linear(x, router_w) (eager code; compiled code keeps the library GEMM, whose
+    call it can see through)."""
+    return (not torch.compiler.is_compiling() and x.is_cuda and x.dtype == router_w.dtype
+            and x.dtype in (torch.bfloat16, torch.float16) and x.dim() == 2
+            and 0 < x.size(0) <= (ROUTER_LOGITS_MAX_TOKENS_FEW_EXPERTS if router_w.size(0) <= FEW_EXPERTS
+                                  else ROUTER_LOGITS_MAX_TOKENS)
+            and x.size(1) % 32 == 0 and x.size(1) == router_w.size(1) and x.is_contiguous() and router_w.is_contiguous()
+            and x.data_ptr() % 16 == 0 and router_w.data_ptr() % 16 == 0 and not torch.is_autocast_enabled("cuda"))
+
+
+def router_linear(x: torch.Tensor, router_w: torch.Tensor) -> torch.Tensor:
+    """F.linear(x, router_w) (nothing of it is differentiated through: the layer's own nodes call it)"""
+    if not router_logits_takes(x, router_w):
+        return torch.nn.functional.linear(x, router_w)
+    logits = torch.empty(x.size(0), router_w.size(0), dtype=x.dtype, device=x.device)
+    run(_router_logits, x, router_w, logits)
+    return logits
+
+
 def router_fused_supported(x: torch.Tensor, router_w: torch.Tensor) -> bool:
     """Shapes and dtypes `_router_forward_fused` takes: bf16, E a multiple of 16 up to 256, H a multiple of 256."""
     E, H = router_w.shape

@@ -1,4 +1,4 @@
-"""The token-choice layer behind its router GEMM as one call of the HIP library per direction (smoe_layer_forward /
+"""The token-choice layer behind (of few tokens: with) its router GEMM as one call of the HIP library per direction (smoe_layer_forward /
 smoe_layer_backward: the operators' entry points in the operators' order, so the same kernels and the same results).
 
 For the common case only: plain 16-bit tensors of one type, nobody looking on the operators, no autocast, no tensor of a
@@ -24,9 +24,9 @@ from . import forward as _f
 # step takes milliseconds, to which the calls (0.1 ms) add nothing, and memory is what counts.
 MAX_TRANSIENT_BYTES = 1 << 30
 
-_FORWARD = struct.Struct("32q")
+_FORWARD = struct.Struct("33q")
 _BACKWARD = struct.Struct("44q")
-_FORWARD_OPERATORS = (_f._softmax_topk_fwd, _f._topk_fwd, _f._up_projection_forward, _f._down_projection_forward,
+_FORWARD_OPERATORS = (_f._router_logits, _f._softmax_topk_fwd, _f._topk_fwd, _f._up_projection_forward, _f._down_projection_forward,
                       _f._router_forward, _f._switch_loss_fwd)
 _BACKWARD_OPERATORS = (_b._down_projection_backward, _b._up_projection_backward, _b._token_broadcast_backward,
                        _b._switch_loss_bwd, _b._router_logit_grad, _b._router_weight_grad, _b._sum_chunks)
@@ -94,13 +94,18 @@ def takes(x, router_w, w1, b1, w2, b2, K: int, activation, stream_id: int, names
             and b1.is_contiguous() and b2.is_contiguous() and b1.data_ptr() != 0 and b2.data_ptr() != 0)
 
 
-def forward(x, logits, w1, b1, w2, b2, K: int, activation, stream_id: int, keep_z: bool, with_loss: bool):
-    """(o, z or None, freq, the routing's int32 tensor, loss or None), or None where the library refuses."""
+def forward(x, router_w, w1, b1, w2, b2, K: int, activation, stream_id: int, keep_z: bool, with_loss: bool):
+    """(o, logits, z or None, freq, the routing's int32 tensor, loss or None), or None where the library refuses."""
     T, H = x.shape
-    E, I = logits.size(1), w2.size(1)
+    E, I = router_w.size(0), w2.size(1)
     dev, dtype = x.device, x.dtype
-    if logits.dtype != dtype or logits.stride(1) != 1:
-        return None
+    own_logits = _f.router_logits_takes(x, router_w)
+    if own_logits:
+        logits = torch.empty(T, E, dtype=dtype, device=dev)
+    else:
+        logits = torch.nn.functional.linear(x, router_w)
+        if logits.dtype != dtype or logits.stride(1) != 1:
+            return None
     L = _lib.lib(dtype)
     where = Indices(T, E, K)
     need = L.smoe_layer_forward_workspace_bytes(T, H, I, E, K)
@@ -115,7 +120,7 @@ def forward(x, logits, w1, b1, w2, b2, K: int, activation, stream_id: int, keep_
     s1, s2, base, at = w1.stride(), w2.stride(), ints.data_ptr(), where.at
     rc = L.smoe_layer_forward(
         _FORWARD.pack(
-            x.data_ptr(), logits.data_ptr(), w1.data_ptr(), 0 if b1 is None else b1.data_ptr(), w2.data_ptr(),
+            x.data_ptr(), router_w.data_ptr() if own_logits else 0, logits.data_ptr(), w1.data_ptr(), 0 if b1 is None else b1.data_ptr(), w2.data_ptr(),
             0 if b2 is None else b2.data_ptr(),
             s1[2], s1[0], s2[2], s2[0], _lib.DT_CODE[dtype], logits.stride(0), T, H, I, E, K, ACTIVATION_CODE[activation],
             z.data_ptr() if keep_z else 0, o.data_ptr(),
@@ -125,7 +130,7 @@ def forward(x, logits, w1, b1, w2, b2, K: int, activation, stream_id: int, keep_
         ),
         stream_id,
     )
-    return None if rc else (o, z, freq, ints, loss)
+    return None if rc else (o, logits, z, freq, ints, loss)
 
 
 def backward(x, dout, z, w1, w2, b2, has_b1: bool, ints, freq, logits, K: int, activation, stream_id: int, loss_grad,
