@@ -90,49 +90,6 @@ typedef __half route_t;
 typedef uint16_t route_t;  // bf16 bits
 #endif
 
-// Top-K softmax of the rows in LDS; LANES lanes own a row of at most COLS * LANES columns, a wavefront 64 / LANES rows
-template <int COLS, int LANES>
-SMOE_DEV void pick_winners(const uint16_t* rows, int Trows, int E, int K, int wave, int lane, float* __restrict__ scores,
-                           int32_t* __restrict__ indices, int32_t* picks) {
-  typedef TopkKey<route_t> Top;
-  constexpr int PER_WAVE = 64 / LANES;
-  if (wave * PER_WAVE >= Trows) return;
-  const int g = lane & (LANES - 1), lane0 = lane - g, row = wave * PER_WAVE + lane / LANES;
-  const bool row_ok = row < Trows;
-  const uint16_t* src = rows + (row_ok ? row : Trows - 1) * E;
-  uint32_t key[COLS];
-#pragma unroll
-  for (int i = 0; i < COLS; i++) {
-    const int c = g + LANES * i;
-    key[i] = c < E ? Top::make(src[c], c) : 0;
-  }
-  float vmax = 0.f, esum = 0.f;
-  for (int r0 = 0; r0 < K; r0 += LANES) {  // lane g keeps winner r0 + g, its score unnormalised until the sum is known
-    const int n = K - r0 < LANES ? K - r0 : LANES;
-    uint32_t mine = 0;
-    for (int r = 0; r < n; r++) {
-      uint32_t best = key[0];
-#pragma unroll
-      for (int i = 1; i < COLS; i++) best = key[i] > best ? key[i] : best;
-      best = group_max(best, LANES);
-#pragma unroll
-      for (int i = 0; i < COLS; i++) key[i] = key[i] == best ? 0 : key[i];
-      mine = g == r ? best : mine;
-    }
-    if (r0 == 0) vmax = Top::value(__shfl(mine, lane0, 64));
-    const float ex = expf(Top::value(mine) - vmax);
-    for (int r = 0; r < n; r++) esum += __shfl(ex, lane0 + r, 64);
-    if (row_ok && g < n) {
-      const int slot = row * K + r0 + g;
-      picks[slot] = Top::column(mine);
-      indices[slot] = Top::column(mine);
-      scores[slot] = ex;
-    }
-  }
-  if (row_ok)
-    for (int r = g; r < K; r += LANES) scores[row * K + r] = scores[row * K + r] / esum;  // (the lane's own stores)
-}
-
 // VPL: columns per lane of a wavefront that owns a row (E <= 64 * VPL)
 template <int VPL>
 __global__ __launch_bounds__(64 * RF_WAVES) void route_few_kernel(
@@ -187,7 +144,19 @@ __global__ __launch_bounds__(64 * RF_WAVES) void route_few_kernel(
     if (c < E) sums[wave * E + c] = acc[i];
   }
   __syncthreads();
-  pick_winners<4 * VPL, 16>(rows, Trows, E, K, wave, lane, scores, indices, picks);
+  if (wave * 4 < Trows) {  // (the same for all lanes of a wavefront)
+    const int g = lane & 15, row = wave * 4 + lane / 16;
+    const bool row_ok = row < Trows;
+    const uint16_t* src = rows + (row_ok ? row : Trows - 1) * E;
+    typedef TopkKey<route_t> Top;
+    uint32_t key[4 * VPL];
+#pragma unroll
+    for (int i = 0; i < 4 * VPL; i++) {
+      const int c = g + 16 * i;
+      key[i] = c < E ? Top::make(src[c], c) : 0;
+    }
+    pick_winners<Top>(key, 16, g, lane, row_ok, K, true, scores + row * K, indices + row * K, picks + row * K);
+  }
   __syncthreads();
   for (int e = lane; e < E; e += 64) cursor[e] = 0;
   __syncthreads();

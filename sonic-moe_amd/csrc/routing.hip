@@ -16,16 +16,14 @@ namespace smoe {
 //     key = (order-preserving image of the value's bits) << W | (2^W - 1 - column)
 // with W = 32 for fp32 and W = 16 for the 16-bit types, so that the maximum key is the largest value and, among equal
 // values, the lowest column.  K rounds of "group arg-max, then retire the winner" give the winners in descending order.
-// A round is a chain of maxima, one instruction each on 32-bit keys and three on 64-bit ones (one row, E = 128, K = 8:
-// 8.3 -> 5.8 us; T = 40960, E = 256: 32 -> 26 us).
+// A round is a chain of maxima, one instruction each on 32-bit keys and three on 64-bit ones, and the winners' exponentials
+// are taken behind the rounds (one row, E = 128, K = 8: 3.0 us; 40960 rows, E = 256: 22).
 
 template <typename T, int VPL>
 __global__ __launch_bounds__(256) void topk_softmax_kernel(const T* __restrict__ logits, int64_t row_stride,
                                                            int64_t Trows, int E, int K, int G, uint32_t clear_mask,
                                                            float* __restrict__ scores, int32_t* __restrict__ indices,
                                                            int do_softmax) {
-  // the winners' scores, K per row of the workgroup, until their sum is known
-  extern __shared__ float won[];
   const int lane_in_block = threadIdx.x;
   const int rows_per_block = 256 / G;
   const int g = lane_in_block % G;
@@ -53,54 +51,27 @@ __global__ __launch_bounds__(256) void topk_softmax_kernel(const T* __restrict__
     key[i] = col < E ? TK::make(v, col) : 0;
   }
 
-  float vmax = 0.f, esum = 0.f;
-  for (int r = 0; r < K; r++) {
-    Key best = key[0];
-#pragma unroll
-    for (int i = 1; i < VPL; i++) best = key[i] > best ? key[i] : best;
-    best = TK::max_over(best, G);
-#pragma unroll
-    for (int i = 0; i < VPL; i++) key[i] = (key[i] == best) ? 0 : key[i];
-    if (g == 0 && row_ok) {
-      const float v = TK::value(best);
-      const int col = TK::column(best);
-      float outv = v;
-      if (do_softmax) {
-        if (r == 0) vmax = v;
-        outv = expf(v - vmax);
-        esum += outv;
-      }
-      if (do_softmax) {
-        won[lane_in_block / G * K + r] = outv;
-      } else {
-        scores[row * K + r] = outv;
-      }
-      indices[row * K + r] = col;
-    }
-  }
-  if (do_softmax) {  // the row's lanes are lanes of one wavefront
-    const float sum = __shfl(esum, lane_in_block & 63 & -G, 64);
-    __builtin_amdgcn_wave_barrier();
-    if (row_ok)
-      for (int r = g; r < K; r += G) scores[row * K + r] = won[lane_in_block / G * K + r] / sum;
-  }
+  pick_winners<TK>(key, G, g, lane_in_block & 63, row_ok, K, do_softmax != 0, scores + rrow * K, indices + rrow * K, nullptr);
 }
 
 template <typename T>
 static int launch_topk(const void* logits, int64_t T_, int E, int K, int64_t row_stride, float* scores,
                        int32_t* indices, int softmax, uint32_t clear_mask, hipStream_t st) {
+  // Columns per lane.  With 4 a round is a short chain and many lanes run; with 16 it takes fewer instructions in all, which
+  // counts once the chip is full.  The two meet near T E K = 2^25; us, 16 / 4 columns, bf16: E = 128, K = 8 256 rows 5.5/3.4,
+  // 8192 5.7/4.6, 40960 13.1/12.4; E = 256, K = 8 1024 rows 5.6/3.5, 16384 11.1/11.0, 40960 21.8/23.1; K = 16 4096 rows
+  // 7.5/6.6, 16384 13.5/16.8.  (64-bit keys go through LDS from lane to lane: as few lanes as possible.)
+  const int cols = sizeof(T) == 2 && T_ * E <= (1ll << 25) / K ? 4 : 16;
   int G = 1;
-  while (G < 64 && G * 16 < E) G <<= 1;
+  while (G < 64 && G * cols < E) G <<= 1;
   int vpl = 1;
   while (vpl * G < E) vpl <<= 1;
   const int rows_per_block = 256 / G;
   const dim3 grid((unsigned)ceil_div(T_, rows_per_block)), block(256);
-  // at most 16 KiB: G < 64 lanes own at most 16 G columns, so K <= 16 G; G = 64 makes 4 rows of K <= 64
-  const size_t won_bytes = softmax ? (size_t)rows_per_block * K * sizeof(float) : 0;
   const T* p = (const T*)logits;
 #define SMOE_TOPK_CASE(V)                                                                                          \
   case V:                                                                                                          \
-    hipLaunchKernelGGL((topk_softmax_kernel<T, V>), grid, block, won_bytes, st, p, row_stride, T_, E, K, G, clear_mask,    \
+    hipLaunchKernelGGL((topk_softmax_kernel<T, V>), grid, block, 0, st, p, row_stride, T_, E, K, G, clear_mask,    \
                        scores, indices, softmax);                                                                  \
     break;
   switch (vpl) {

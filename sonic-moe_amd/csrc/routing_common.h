@@ -112,6 +112,44 @@ struct TopkKey<uint16_t> : TopkKey16<uint16_t> {};
 template <>
 struct TopkKey<__half> : TopkKey16<__half> {};
 
+// The K winners of a row whose keys G consecutive lanes hold (G a power of two up to 64, the same for all lanes of the
+// wavefront; g = the lane's number in its row): K rounds of "arg-max over the row, retire the winner".  Lane g keeps the
+// winners g, G + g, ...: their softmax, which needs one exponential per winner, is evaluated outside the rounds.  picks:
+// nullable, the columns once more.
+template <class Top, int COLS>
+SMOE_DEV void pick_winners(typename Top::Key (&key)[COLS], int G, int g, int lane, bool row_ok, int K, bool softmax,
+                           float* scores, int32_t* indices, int32_t* picks) {
+  typedef typename Top::Key Key;
+  float vmax = 0.f, esum = 0.f;
+  for (int r0 = 0; r0 < K; r0 += G) {
+    const int n = K - r0 < G ? K - r0 : G;
+    Key mine = 0;
+    for (int r = 0; r < n; r++) {
+      Key best = key[0];
+#pragma unroll
+      for (int i = 1; i < COLS; i++) best = key[i] > best ? key[i] : best;
+      best = Top::max_over(best, G);
+#pragma unroll
+      for (int i = 0; i < COLS; i++) key[i] = key[i] == best ? 0 : key[i];
+      mine = g == r ? best : mine;
+    }
+    float out = Top::value(mine);
+    if (softmax) {
+      if (r0 == 0) vmax = __shfl(out, lane - g, 64);
+      out = expf(out - vmax);
+      for (int r = 0; r < n; r++) esum += __shfl(out, lane - g + r, 64);  // one after the other, as the winners come
+    }
+    if (row_ok && g < n) {
+      const int col = Top::column(mine);
+      indices[r0 + g] = col;
+      if (picks != nullptr) picks[r0 + g] = col;
+      scores[r0 + g] = out;  // (still to be divided by the sum)
+    }
+  }
+  if (softmax && row_ok)
+    for (int r = g; r < K; r += G) scores[r] = scores[r] / esum;  // the lane's own stores
+}
+
 // ---- counting sort ---------------------------------------------------------------------------------------------------------
 // One step of the counting sort for a wavefront: lane l holds slot j (consecutive over the lanes, `valid` a prefix of them)
 // of expert e.  Slots of the same expert take consecutive positions from that expert's cursor, in lane order.
