@@ -76,8 +76,10 @@ int device_compute_units(int* out) {
 
 // order == nullptr: experts are listed 0, 1, ...; otherwise position i of the list holds expert order[i]
 __global__ __launch_bounds__(1024) void build_tile_map_kernel(const int32_t* __restrict__ off,
-                                                              const int32_t* __restrict__ order, int E, int BM,
-                                                              int gmax, int snake, TileMap tm) {
+                                                              const int32_t* __restrict__ order, int E, int BM_,
+                                                              int gmax, int snake, TileMap tm_, TileMap tm2, int BM2) {
+  const TileMap tm = blockIdx.x == 0 ? tm_ : tm2;
+  const int BM = blockIdx.x == 0 ? BM_ : BM2;
   __shared__ int32_t wave_tot[16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int32_t base = 0;
@@ -129,10 +131,11 @@ __global__ __launch_bounds__(1024) void build_tile_map_kernel(const int32_t* __r
   if (tid == 0) tm.header[0] = base;
 }
 
-int launch_build_tile_map(const int32_t* off, const int32_t* order, int E, int BM, TileMap tm, hipStream_t st) {
+int launch_build_tile_map(const int32_t* off, const int32_t* order, int E, int BM, TileMap tm, hipStream_t st,
+                          const TileMap* tm2, int BM2) {
   const Tuning& tune = tuning();
-  hipLaunchKernelGGL(build_tile_map_kernel, dim3(1), dim3(1024), 0, st, off, order, E, BM, tune.gemm_group_tiles,
-                     tune.gemm_group_snake, tm);
+  hipLaunchKernelGGL(build_tile_map_kernel, dim3(tm2 != nullptr ? 2 : 1), dim3(1024), 0, st, off, order, E, BM,
+                     tune.gemm_group_tiles, tune.gemm_group_snake, tm, tm2 != nullptr ? *tm2 : tm, BM2);
   SMOE_LAUNCH_CHECK();
   return SMOE_OK;
 }

@@ -1318,25 +1318,37 @@ static inline TileMap carve_tile_map(void* ws, int64_t TK, int E, int BM) {
   return t;
 }
 
-int launch_build_tile_map(const int32_t* off, const int32_t* order, int E, int BM, TileMap tm, hipStream_t st);
+// tm2 (nullable): a second map, for tiles of BM2 rows, by a second workgroup of the same launch
+int launch_build_tile_map(const int32_t* off, const int32_t* order, int E, int BM, TileMap tm, hipStream_t st,
+                          const TileMap* tm2 = nullptr, int BM2 = 0);
 
 // Scratch memory of the bf16 grouped GEMMs of ONE routing (one off, no schedule order or the same one): the tile map of the
 // token-grouped kernels and the experts' order of the weight-gradient streams.  An entry point makes one for its call, on
 // its workspace, where the two share the memory; the layer's calls keep one for all GEMMs of a direction, with memory for
-// both, so that the map is built and the experts are sorted once (a launch of 4 to 6 us each).
+// a map of either tile height (256 and 128 rows) and for the order, so that the maps are built and the experts are sorted
+// once (a launch of 4 to 6 us each).
 struct GemmScratch {
   void* map;
+  void* small_map;  // nullable: no memory for a second map
   void* sorted;
   size_t sorted_bytes;
-  int map_rows = 0;            // token rows per tile of the map in `map` (0: none)
+  int map_rows = 0;            // token rows per tile of the map in `map` (0: none); with small_map 256, and 128 there
   bool sorted_valid = false;
-  GemmScratch(void* map_, void* sorted_, size_t sorted_bytes_) : map(map_), sorted(sorted_), sorted_bytes(sorted_bytes_) {}
-  GemmScratch(void* workspace, size_t bytes) : GemmScratch(workspace, workspace, bytes) {}
+  GemmScratch(void* map_, void* small_map_, void* sorted_, size_t sorted_bytes_)
+      : map(map_), small_map(small_map_), sorted(sorted_), sorted_bytes(sorted_bytes_) {}
+  GemmScratch(void* workspace, size_t bytes) : GemmScratch(workspace, nullptr, workspace, bytes) {}
 };
 
 // The tile map for tiles of BM rows: the one that is there, or a new one
 static inline int tile_map_in(GemmScratch& ws, const int32_t* off, const int32_t* order, int64_t TK, int E, int BM, TileMap& tm,
                               hipStream_t st) {
+  if (ws.small_map != nullptr && (BM == 256 || BM == 128)) {
+    const TileMap tall = carve_tile_map(ws.map, TK, E, 256), low = carve_tile_map(ws.small_map, TK, E, 128);
+    tm = BM == 256 ? tall : low;
+    if (ws.map_rows != 0) return SMOE_OK;
+    ws.map_rows = 256;
+    return launch_build_tile_map(off, order, E, 256, tall, st, &low, 128);
+  }
   tm = carve_tile_map(ws.map, TK, E, BM);
   if (ws.map_rows == BM) return SMOE_OK;
   if (ws.map == ws.sorted) ws.sorted_valid = false;

@@ -20,15 +20,15 @@ struct Carver {
 };
 
 struct ForwardScratch {
-  void *y1, *y2, *gemm, *metadata, *loss, *few;
-  size_t gemm_bytes, metadata_bytes, loss_bytes, total;
+  void *y1, *y2, *map, *small_map, *metadata, *loss, *few;
+  size_t metadata_bytes, loss_bytes, total;
   ForwardScratch(void* base, int64_t T, int H, int I, int E, int K) {
     Carver c{(char*)base};
     const int64_t TK = T * K;
-    gemm_bytes = smoe_gemm_workspace_bytes(TK, E);
     metadata_bytes = smoe_routing_metadata_workspace_bytes(TK, E);
     loss_bytes = smoe_switch_loss_workspace_bytes(T, E);
-    gemm = c.take(gemm_bytes);
+    map = c.take(smoe_gemm_workspace_bytes(TK, E));
+    small_map = c.take(smoe_gemm_workspace_bytes(TK, E));
     metadata = c.take(metadata_bytes);
     loss = c.take(loss_bytes);
     few = c.take(route_few_workspace_bytes(T, E));
@@ -39,13 +39,14 @@ struct ForwardScratch {
 };
 
 struct BackwardScratch {
-  void *dz, *y1s, *dx_expanded, *partial, *loss_dlogits, *map, *sorted;
+  void *dz, *y1s, *dx_expanded, *partial, *loss_dlogits, *map, *small_map, *sorted;
   float *ds, *ds_partial;
   size_t sorted_bytes, total;
   BackwardScratch(void* base, int64_t T, int H, int I, int E, int K, int N1, int64_t chunks) {
     Carver c{(char*)base};
     const int64_t TK = T * K;
     map = c.take(smoe_gemm_workspace_bytes(TK, E));
+    small_map = c.take(smoe_gemm_workspace_bytes(TK, E));
     sorted_bytes = (size_t)E * sizeof(int32_t);
     sorted = c.take(sorted_bytes);
     ds = (float*)c.take((size_t)TK * 4);
@@ -112,7 +113,7 @@ extern "C" int smoe_layer_forward(const smoe_layer_forward_args* a, void* stream
                                a->s_reverse_scatter_idx, a->tok_off, s.metadata, s.metadata_bytes, stream);
     if (rc) return rc;
   }
-  GemmScratch ws(s.gemm, s.gemm_bytes);
+  GemmScratch ws(s.map, s.small_map, nullptr, 0);
   rc = up_projection_forward(a->x, a->w1, a->w1_stride_e, a->w1_stride_row, a->b1, a->z, s.y1, a->off, nullptr,
                              a->x_gather_idx, T, TK, H, I, E, (int)a->activation, ws, stream);
   if (rc) return rc;
@@ -141,7 +142,7 @@ extern "C" int smoe_layer_backward(const smoe_layer_backward_args* a, void* stre
   const BackwardScratch s(a->workspace, T, H, I, E, K, act <= SMOE_ACT_REGLU ? 2 * I : I, a->router_chunks);
   SMOE_REQUIRE(a->workspace != nullptr && a->workspace_bytes >= (int64_t)s.total, SMOE_ERR_WORKSPACE,
                "layer_backward: workspace too small");
-  GemmScratch ws(s.map, s.sorted, s.sorted_bytes);
+  GemmScratch ws(s.map, s.small_map, s.sorted, s.sorted_bytes);
   int rc = down_projection_backward(a->dout, a->z, a->w2, a->w2_stride_e, a->w2_stride_row, a->b2, a->dw2,
                                          a->dw2_stride_e, a->dw2_stride_row, a->db2, s.dz, s.y1s, s.ds, s.ds_partial,
                                          a->scores, a->off, nullptr, a->x_gather_idx, a->s_scatter_idx, T, TK, H, I, E, act,
