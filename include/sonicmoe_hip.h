@@ -212,6 +212,12 @@ int smoe_down_projection_forward_combine(const void* y1, const void* w2, int64_t
 int smoe_gather_sum(const void* src, void* out, const float* w, const int32_t* ridx, const int32_t* tok_off,
                     int64_t T, int K, int H, void* stream);
 
+/* out[t] = sum_{j < K} src[ridx[t K + j]] + dlogits[t] wr, fp32 accumulation, one rounding: the dx reduction above with the
+ * router's share of dx, which the reference leaves to autograd (a GEMM and an addition, sonicmoe/functional/__init__.py:438).
+ * dlogits (T, E), wr (E, H) contiguous; E % 8 == 0, H % 8 == 0, K <= 16. */
+int smoe_gather_sum_router(const void* src, void* out, const int32_t* ridx, int64_t T, int K, int H, const void* dlogits,
+                           int E, const void* wr, void* stream);
+
 /* Backward of down projection + combine.  Replaces sonicmoe::_down_projection_backward
  * (sonicmoe/functional/backward.py:286-461; bias part backward.py:31-107; epilogue math
  * sonicmoe/functional/grouped_gemm.py:1154-1271, :1311-1333, :2536-2561).
@@ -414,7 +420,7 @@ int smoe_score_grad_bias_term(const void* dout, const void* b2, const int32_t* o
  *   smoe_gather_sum -> smoe_switch_loss_fwd (loss != NULL)
  *   smoe_down_projection_backward -> smoe_up_projection_backward -> smoe_gather_sum -> smoe_switch_loss_bwd (loss_grad !=
  *   NULL) -> smoe_router_logit_grad -> smoe_router_weight_grad and smoe_sum_chunks (router_chunks > 0)
- * The caller adds the router's share of dx (dlogits Wr) itself. */
+ * Without router_w the caller adds the router's share of dx (dlogits Wr) itself. */
 typedef struct {
   const void *x, *router_w; /* router_w: nullable; given, the call begins with smoe_router_logits into logits */
   void* logits;
@@ -447,6 +453,7 @@ typedef struct {
   int64_t dw1_stride_e, dw1_stride_row, dw2_stride_e, dw2_stride_row;
   void *db1, *db2; /* nullable */
   void *dx, *dlogits;
+  const void* router_w; /* nullable; given, dx includes dlogits router_w (smoe_gather_sum_router) */
   void* dwr; /* (E, H), router_chunks > 0 only */
   int64_t router_chunks;
   void* workspace;

@@ -54,6 +54,111 @@ __global__ __launch_bounds__(512) void gather_sum_kernel(const uint16_t* __restr
   }
 }
 
+// dx[t] = sum of the token's K routed rows of dx_expanded + dlogits[t] Wr: the reduction with the router's share of the gradient
+// formed in place, so that dx is written once and rounded once instead of read, added to and written again.
+// A workgroup owns 64 tokens x 128 columns, a wavefront 16 of the tokens: the product runs on matrix instructions, Wr through
+// LDS 64 experts at a time (read transposed), dlogits straight into registers; the fp32 tile then goes through LDS into the
+// layout of the row loads, 16 lanes to the 256 bytes of a row.  Bound by the gathered rows like gather_sum_kernel.
+// gather_sum_kernel and a library GEMM that adds onto dx / this kernel, us: 1024 x 1536, E = 128, K = 8 25/12; 6001 x 1536
+// 52/40; 40960 x 768 131/113; 32768 x 4096 553/487; 4096 x 4096, E = 256, K = 16 121/121.  Distance from 64 bits 2.3e-3 -> 1.7e-3.
+constexpr int GR_T = 64, GR_C = 128, GR_E = 64, GR_PITCH = GR_C + 4, GR_MAX_K = 16;
+
+template <int ROWS>
+__global__ __launch_bounds__(256) void gather_sum_router_kernel(const uint16_t* __restrict__ src,
+                                                                uint16_t* __restrict__ out,
+                                                                const int32_t* __restrict__ ridx, int T, int K, int H,
+                                                                const uint16_t* __restrict__ dlogits, int E,
+                                                                const uint16_t* __restrict__ wr) {
+  __shared__ __attribute__((aligned(16))) char smem[GR_T * GR_PITCH * 4];
+  __shared__ int32_t idx[GR_T * GR_MAX_K];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h0 = blockIdx.x * GR_C, t0 = blockIdx.y * GR_T;
+  for (int i = tid; i < GR_T * K; i += 256) {
+    const int64_t j = (int64_t)t0 * K + i;
+    idx[i] = ridx[j < (int64_t)T * K ? j : (int64_t)T * K - 1];
+  }
+  const int grp = lane >> 4, i16 = lane & 15;
+  const int trow = t0 + wave * 16 + i16;
+  const uint16_t* dl = dlogits + (int64_t)(trow < T ? trow : T - 1) * E + 8 * grp;
+  const u32x4 zero4 = {0, 0, 0, 0};
+  f32x4 acc[8];
+#pragma unroll
+  for (int fn = 0; fn < 8; fn++) acc[fn] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int k0 = 0; k0 < E; k0 += GR_E) {
+    u32x4 stage[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int at = tid + 256 * i, k = k0 + (at >> 4), col = h0 + (at & 15) * 8;
+      const u32x4 v = *(const u32x4*)(wr + (int64_t)(k < E ? k : E - 1) * H + (col < H ? col : H - 8));
+      stage[i] = k < E && col < H ? v : zero4;
+    }
+    elemx8 p[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) {
+      const int k = k0 + ks * 32 + 8 * grp;  // (E is a multiple of 8)
+      const u32x4 v = *(const u32x4*)(dl + (k < E ? k0 + ks * 32 : E - 8 - 8 * grp));
+      p[ks] = __builtin_bit_cast(elemx8, k < E ? v : zero4);
+    }
+    __syncthreads();  // the products of the experts before have read their stage
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int at = tid + 256 * i, k = at >> 4, piece = at & 15;
+      *(u32x4*)(smem + k * (GR_C * 2) + (((piece >> 1) ^ mnswz(k)) << 5) + ((piece & 1) << 4)) = stage[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) {
+#pragma unroll
+      for (int fn = 0; fn < 8; fn++) {
+        const char* at[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          const int k = ks * 32 + 8 * grp + (i16 >> 2) + 4 * h;
+          at[h] = smem + k * (GR_C * 2) + ((fn ^ mnswz(k)) << 5) + ((i16 & 3) << 3);
+        }
+        acc[fn] = ElemMma16::run(lds_read_tr2(at[0], at[1]), p[ks], acc[fn]);
+      }
+    }
+  }
+  __syncthreads();
+  float* tile = (float*)smem;
+#pragma unroll
+  for (int fn = 0; fn < 8; fn++) *(f32x4*)(tile + (wave * 16 + i16) * GR_PITCH + fn * 16 + 4 * grp) = acc[fn];
+  __syncthreads();
+  const int col = h0 + i16 * 8;
+  if (col >= H) return;
+#pragma unroll 1
+  for (int pass = 0; pass < 4; pass++) {
+    const int r = wave * 16 + pass * 4 + grp, t = t0 + r;
+    if (t >= T) break;  // (rows ascend with the pass)
+    float sum[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) sum[q] = 0.f;
+    for (int j0 = 0; j0 < K; j0 += ROWS) {
+      u32x4 v[ROWS];
+#pragma unroll
+      for (int u = 0; u < ROWS; u++) {
+        const int j = j0 + u < K ? j0 + u : K - 1;
+        v[u] = __builtin_nontemporal_load((const u32x4*)(src + (int64_t)idx[r * K + j] * H + col));
+      }
+#pragma unroll
+      for (int u = 0; u < ROWS; u++) {
+        if (j0 + u < K) {
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            sum[2 * q] += elem_lo(v[u][q]);
+            sum[2 * q + 1] += elem_hi(v[u][q]);
+          }
+        }
+      }
+    }
+    const f32x4 lo = *(const f32x4*)(tile + r * GR_PITCH + i16 * 8), hi = *(const f32x4*)(tile + r * GR_PITCH + i16 * 8 + 4);
+    const u32x4 o = {pack_elem2(sum[0] + lo[0], sum[1] + lo[1]), pack_elem2(sum[2] + lo[2], sum[3] + lo[3]),
+                     pack_elem2(sum[4] + hi[0], sum[5] + hi[1]), pack_elem2(sum[6] + hi[2], sum[7] + hi[3])};
+    __builtin_nontemporal_store(o, (u32x4*)(out + (int64_t)t * H + col));
+  }
+}
+
 // ds[sidx[m]] = sum_n ds_partial[m][n]
 __global__ __launch_bounds__(256) void ds_finalize_kernel(const float* __restrict__ ds_partial, int ncols,
                                                           const int32_t* __restrict__ sidx, float* __restrict__ ds,
@@ -178,6 +283,23 @@ int launch_ds_bias_term(const uint16_t* dout, const uint16_t* b2, const int32_t*
 }  // namespace smoe
 
 using namespace smoe;
+
+extern "C" int smoe_gather_sum_router(const void* src, void* out, const int32_t* ridx, int64_t T, int K, int H,
+                                      const void* dlogits, int E, const void* wr, void* stream) {
+  SMOE_REQUIRE(T >= 0 && T < (1ll << 31) / GR_MAX_K, SMOE_ERR_UNSUPPORTED, "gather_sum_router: T out of range");
+  if (T == 0) return SMOE_OK;
+  SMOE_REQUIRE(src && out && ridx && dlogits && wr, SMOE_ERR_INVALID, "gather_sum_router: null pointer");
+  SMOE_REQUIRE(H >= 8 && H % 8 == 0 && E >= 8 && E % 8 == 0 && K >= 1 && K <= GR_MAX_K, SMOE_ERR_UNSUPPORTED,
+               "gather_sum_router: H=%d and E=%d must be multiples of 8, K=%d at most %d", H, E, K, GR_MAX_K);
+  SMOE_REQUIRE(ceil_div(T, GR_T) < 65536, SMOE_ERR_UNSUPPORTED, "gather_sum_router: too many tokens");
+  SMOE_REQUIRE_ALIGNED("gather_sum_router", src, out, dlogits, wr);
+  const dim3 grid((unsigned)ceil_div(H, GR_C), (unsigned)ceil_div(T, GR_T));
+  auto kernel = K <= 2 ? gather_sum_router_kernel<2> : K <= 4 ? gather_sum_router_kernel<4> : gather_sum_router_kernel<8>;
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, (hipStream_t)stream, (const uint16_t*)src, (uint16_t*)out, ridx, (int)T, K, H,
+                     (const uint16_t*)dlogits, E, (const uint16_t*)wr);
+  SMOE_LAUNCH_CHECK();
+  return SMOE_OK;
+}
 
 extern "C" int smoe_gather_sum(const void* src, void* out, const float* w, const int32_t* ridx, const int32_t* tok_off,
                                int64_t T, int K, int H, void* stream) {

@@ -152,8 +152,10 @@ extern "C" int smoe_layer_backward(const smoe_layer_backward_args* a, void* stre
                                    a->dw1_stride_row, a->db1, s.dx_expanded, a->off, nullptr, a->x_gather_idx, T, TK, H, I, E,
                                    act, ws, stream);
   if (rc) return rc;
-  rc = smoe_gather_sum(s.dx_expanded, a->dx, nullptr, a->s_reverse_scatter_idx, nullptr, T, K, H, stream);
-  if (rc) return rc;
+  if (a->router_w == nullptr) {
+    rc = smoe_gather_sum(s.dx_expanded, a->dx, nullptr, a->s_reverse_scatter_idx, nullptr, T, K, H, stream);
+    if (rc) return rc;
+  }
   const void* outside = a->outside;
   int64_t outside_stride = a->outside_row_stride;
   if (a->loss_grad != nullptr) {
@@ -165,7 +167,12 @@ extern "C" int smoe_layer_backward(const smoe_layer_backward_args* a, void* stre
   }
   rc = smoe_router_logit_grad(a->dlogits, (int)a->logits_dtype, E, outside, outside_stride, s.ds, a->scores, a->indices, T, E,
                               K, stream);
-  if (rc || a->router_chunks == 0) return rc;
+  if (rc) return rc;
+  if (a->router_w != nullptr) {
+    rc = smoe_gather_sum_router(s.dx_expanded, a->dx, a->s_reverse_scatter_idx, T, K, H, a->dlogits, E, a->router_w, stream);
+    if (rc) return rc;
+  }
+  if (a->router_chunks == 0) return rc;
   if (a->router_chunks == 1) return smoe_router_weight_grad(a->dlogits, a->x, a->dwr, T, E, H, 1, stream);
   rc = smoe_router_weight_grad(a->dlogits, a->x, s.partial, T, E, H, (int)a->router_chunks, stream);
   if (rc) return rc;

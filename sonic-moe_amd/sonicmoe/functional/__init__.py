@@ -29,7 +29,9 @@ from .backward import (
     _sum_chunks,
     _switch_loss_bwd,
     _token_broadcast_backward,
+    _token_broadcast_backward_router,
     _up_projection_backward,
+    router_dx_takes,
     router_weight_grad_chunks,
 )
 from .forward import (
@@ -322,9 +324,9 @@ def _experts_forward(x, w1, b1, w2, b2, scores_flat, off, gidx, ridx, tok_off, K
 
 
 def _experts_backward(dout, x, w1, w2, b2, z, scores_flat, off, gidx, sidx, ridx, tok_off, K_or_maxK, is_varlen_K,
-                      activation_type, stream_id, has_b1, order=None, fp8=False):
-    """Returns (dx, dw1, db1, dw2, db2, ds) of _experts_forward; `has_b1` says whether the forward pass had an
-    up-projection bias (b1 itself is not needed for any gradient and is not kept)."""
+                      activation_type, stream_id, has_b1, order=None, fp8=False, reduce=True):
+    """Returns (dx, dw1, db1, dw2, db2, ds) of _experts_forward, without `reduce` dx_expanded in the place of dx; `has_b1`
+    says whether the forward pass had an up-projection bias (b1 itself is not needed for any gradient and is not kept)."""
     T, H = x.shape
     TK = gidx.numel()
     glu = is_glu(activation_type)
@@ -332,7 +334,7 @@ def _experts_backward(dout, x, w1, w2, b2, z, scores_flat, off, gidx, sidx, ridx
 
     if fp8:
         return _experts_backward_fp8(dout, x, w1, w2, b2, z, scores_flat, off, gidx, sidx, ridx, tok_off, K_or_maxK,
-                                     is_varlen_K, activation_type, stream_id, has_b1, order)
+                                     is_varlen_K, activation_type, stream_id, has_b1, order, reduce)
 
     dw2 = torch.empty_like(w2)  # keeps the (E, H, I)-contiguous layout of the parameter view
     db2 = None if b2 is None else torch.empty_like(b2)
@@ -347,13 +349,15 @@ def _experts_backward(dout, x, w1, w2, b2, z, scores_flat, off, gidx, sidx, ridx
     dx_expanded = torch.empty(TK, H, dtype=x.dtype, device=x.device)
     run(_up_projection_backward, x, w1, dx_expanded, dw1, dz, db1, off, order, gidx, sidx, glu, stream_id)
     del dz
+    if not reduce:
+        return dx_expanded, dw1, db1, dw2, db2, ds
     dx = torch.empty(T, H, dtype=x.dtype, device=x.device)
     run(_token_broadcast_backward, dx, dx_expanded, ridx, tok_off, K_or_maxK, H, is_varlen_K)
     return dx, dw1, db1, dw2, db2, ds
 
 
 def _experts_backward_fp8(dout, x, w1, w2, b2, z, scores_flat, off, gidx, sidx, ridx, tok_off, K_or_maxK, is_varlen_K,
-                          activation_type, stream_id, has_b1, order):
+                          activation_type, stream_id, has_b1, order, reduce=True):
     """_experts_backward with the two activation-gradient GEMMs on fp8 operands: dout and W2^T are quantised for dz,
     the dz kernel leaves dz in bf16 (for dW1 and db1) and quantised (for dx), W1^T is quantised for dx; dW2 and dW1
     are the bf16 weight-gradient GEMMs, and the bias gradients and the bias term of ds are the bf16 step's kernels."""
@@ -386,6 +390,8 @@ def _experts_backward_fp8(dout, x, w1, w2, b2, z, scores_flat, off, gidx, sidx, 
     db1 = torch.empty(w1.size(2), w1.size(0), dtype=x.dtype, device=x.device) if has_b1 else None
     run(_up_projection_backward, x, w1, None, dw1, dz, db1, off, order, gidx, sidx, glu, stream_id)
     del dz
+    if not reduce:
+        return dx_expanded, dw1, db1, dw2, db2, ds
     dx = torch.empty(T, H, dtype=x.dtype, device=x.device)
     run(_token_broadcast_backward, dx, dx_expanded, ridx, tok_off, K_or_maxK, H, is_varlen_K)
     return dx, dw1, db1, dw2, db2, ds
@@ -519,17 +525,24 @@ class _TCLayerFunction(torch.autograd.Function):
 def _tc_layer_backward(ctx, dout, dlogits_outside, x, router_w, w1, w2, b2, z, scores, indices, off, gidx, sidx, ridx, tok_off,
                        K, activation_type, stream_id, logits_dtype, has_b1, order, fp8):
     T, E = x.size(0), router_w.size(0)
+    with_router = ctx.needs_input_grad[0] and router_dx_takes(x, router_w, logits_dtype, K)
     dx, dw1, db1, dw2, db2, ds = _experts_backward(
         dout, x, w1, w2, b2, z, scores.view(-1), off, gidx, sidx, ridx, tok_off, K, False, activation_type, stream_id,
-        has_b1, order, fp8,
+        has_b1, order, fp8, not with_router,
     )
     dlogits = torch.empty(T, E, dtype=logits_dtype, device=x.device)
     # (a compiled backward pass knows dense gradients only, and refuses the question)
     if not torch.compiler.is_compiling() and dlogits_outside is not None and dlogits_outside.layout != torch.strided:
         dlogits_outside = dlogits_outside.to_dense()
     run(_router_logit_grad, dlogits, dlogits_outside, ds.view(T, K), scores, indices)
+    if with_router:
+        dx_expanded, dx = dx, torch.empty_like(x)
+        run(_token_broadcast_backward_router, dx, dx_expanded, ridx, dlogits, router_w, K)
+        del dx_expanded
     dwr = _router_wgrad(dlogits, x, router_w) if ctx.needs_input_grad[1] else None
-    if ctx.needs_input_grad[0]:
+    if with_router:
+        pass
+    elif ctx.needs_input_grad[0]:
         dx.addmm_(dlogits, router_w)  # dx_experts + dlogits Wr in the GEMM's epilogue
     else:
         dx = None
@@ -564,18 +577,19 @@ class _OneCallLayerFunction(torch.autograd.Function):
         fast_router = (ctx.needs_input_grad[1] and _router_wgrad_takes(logits, x))
         chunks = router_weight_grad_chunks(T, E, H) if fast_router else 0
         done = None
-        if (_down_projection_backward, _up_projection_backward, _token_broadcast_backward, _switch_loss_bwd,
-                _router_logit_grad, _router_weight_grad, _sum_chunks) == layer_call._BACKWARD_OPERATORS:
+        with_router = ctx.needs_input_grad[0] and router_dx_takes(x, router_w, logits.dtype, K)
+        if (_down_projection_backward, _up_projection_backward, _token_broadcast_backward, _token_broadcast_backward_router,
+                _switch_loss_bwd, _router_logit_grad, _router_weight_grad, _sum_chunks) == layer_call._BACKWARD_OPERATORS:
             done = layer_call.backward(x, dout, z, w1, w2, b2, has_b1, ints, freq, logits, K, activation_type, stream_id, daux,
-                                       dlogits_outside, chunks)
+                                       dlogits_outside, chunks, router_w if with_router else None)
         if done is not None:
             dx, dlogits, dwr, dw1, db1, dw2, db2 = done
             if dwr is None and ctx.needs_input_grad[1]:
                 dwr = dlogits.t() @ x
-            if ctx.needs_input_grad[0]:
-                dx.addmm_(dlogits, router_w)
-            else:
+            if not ctx.needs_input_grad[0]:
                 dx = None
+            elif not with_router:
+                dx.addmm_(dlogits, router_w)
             return dx, dwr, dw1, db1, dw2, db2, None, None, None, None
         scores, indices, gidx, sidx, ridx, off, tok_off, acc = layer_call.Indices(T, E, K).views(ints)
         if daux is not None:

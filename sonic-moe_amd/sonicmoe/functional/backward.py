@@ -201,6 +201,35 @@ def _token_broadcast_backward(
     )
 
 
+@operator("_token_broadcast_backward_router", mutates_args={"dx"})
+def _token_broadcast_backward_router(
+    dx: torch.Tensor, dx_expanded: torch.Tensor, s_reverse_scatter_idx: torch.Tensor, dlogits: torch.Tensor,
+    router_w: torch.Tensor, K: int
+) -> None:
+    """`_token_broadcast_backward` for K slots per token with the router's share of dx: dx[t] = sum of the token's rows of
+    dx_expanded + dlogits[t] router_w, one rounding (the reference leaves the second term to autograd)."""
+    _lib.require_device(dx, dx_expanded, s_reverse_scatter_idx, dlogits, router_w)
+    dt = _elem_dtype(("dx", dx), ("dx_expanded", dx_expanded), ("dlogits", dlogits), ("router_w", router_w))
+    T, H = dx.shape
+    E = router_w.size(0)
+    assert dx.is_contiguous() and dx_expanded.is_contiguous() and dlogits.is_contiguous() and router_w.is_contiguous()
+    assert dlogits.shape == (T, E) and router_w.shape == (E, H) and dx_expanded.shape == (T * K, H)
+    assert s_reverse_scatter_idx.dtype == torch.int32 and s_reverse_scatter_idx.numel() == T * K
+    rc = _lib.lib(dt).smoe_gather_sum_router(
+        _lib.ptr(dx_expanded), _lib.ptr(dx), _lib.ptr(s_reverse_scatter_idx), T, K, H, _lib.ptr(dlogits), E,
+        _lib.ptr(router_w), _lib.current_stream_handle(),
+    )
+    _lib.check(rc, "_token_broadcast_backward_router")
+
+
+def router_dx_takes(x: torch.Tensor, router_w: torch.Tensor, logits_dtype: torch.dtype, K: int) -> bool:
+    """Whether `_token_broadcast_backward_router` forms dx (eager code; compiled code keeps the GEMM it can see through)"""
+    return (not torch.compiler.is_compiling() and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16)
+            and router_w.dtype == x.dtype and logits_dtype == x.dtype and x.size(0) > 0 and 1 <= K <= 16
+            and router_w.size(0) % 8 == 0 and x.size(1) % 8 == 0 and router_w.is_contiguous()
+            and router_w.data_ptr() % 16 == 0)
+
+
 @operator("_softmax_topk_bwd", mutates_args={"dlogits_full"})
 def _softmax_topk_bwd(
     dlogits_full: torch.Tensor,

@@ -25,10 +25,10 @@ from . import forward as _f
 MAX_TRANSIENT_BYTES = 1 << 30
 
 _FORWARD = struct.Struct("33q")
-_BACKWARD = struct.Struct("44q")
+_BACKWARD = struct.Struct("45q")
 _FORWARD_OPERATORS = (_f._router_logits, _f._softmax_topk_fwd, _f._topk_fwd, _f._up_projection_forward, _f._down_projection_forward,
                       _f._router_forward, _f._switch_loss_fwd)
-_BACKWARD_OPERATORS = (_b._down_projection_backward, _b._up_projection_backward, _b._token_broadcast_backward,
+_BACKWARD_OPERATORS = (_b._down_projection_backward, _b._up_projection_backward, _b._token_broadcast_backward, _b._token_broadcast_backward_router,
                        _b._switch_loss_bwd, _b._router_logit_grad, _b._router_weight_grad, _b._sum_chunks)
 _BACKWARD_NAMES = elsewhere(*_BACKWARD_OPERATORS)
 _ELEMENTS = (torch.bfloat16, torch.float16)
@@ -134,9 +134,9 @@ def forward(x, router_w, w1, b1, w2, b2, K: int, activation, stream_id: int, kee
 
 
 def backward(x, dout, z, w1, w2, b2, has_b1: bool, ints, freq, logits, K: int, activation, stream_id: int, loss_grad,
-             outside, chunks: int):
-    """(dx of the experts, dlogits, dwr or None, dw1, db1, dw2, db2), or None where the operators have to do it.  chunks:
-    token chunks of the router's weight gradient (0: the caller forms it)."""
+             outside, chunks: int, router_w):
+    """(dx, dlogits, dwr or None, dw1, db1, dw2, db2), or None where the operators have to do it.  chunks: token chunks of the
+    router's weight gradient (0: the caller forms it).  router_w: None leaves the router's share of dx to the caller."""
     dtype = x.dtype
     if torch.compiler.is_compiling() or not (
         unobserved(_BACKWARD_NAMES, x, dout, z, w1, w2, b2, ints, freq, logits, loss_grad, outside)
@@ -188,6 +188,7 @@ def backward(x, dout, z, w1, w2, b2, has_b1: bool, ints, freq, logits, K: int, a
             0 if outside is None else outside.stride(0), T, H, I, E, K, code,
             dw1.data_ptr(), dw2.data_ptr(), d1[2], d1[0], d2[2], d2[0],
             0 if db1 is None else db1.data_ptr(), 0 if db2 is None else db2.data_ptr(), dx.data_ptr(), dlogits.data_ptr(),
+            0 if router_w is None else router_w.data_ptr(),
             0 if dwr is None else dwr.data_ptr(), chunks, scratch.data_ptr(), need,
         ),
         stream_id,
