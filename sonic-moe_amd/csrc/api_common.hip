@@ -74,68 +74,27 @@ int device_compute_units(int* out) {
   return SMOE_OK;
 }
 
-// order == nullptr: experts are listed 0, 1, ...; otherwise position i of the list holds expert order[i]
+// workgroup 0 and, with a pair, 1: the maps; 2: the experts' order
 __global__ __launch_bounds__(1024) void build_tile_map_kernel(const int32_t* __restrict__ off,
-                                                              const int32_t* __restrict__ order, int E, int BM_,
-                                                              int gmax, int snake, TileMap tm_, TileMap tm2, int BM2) {
-  const TileMap tm = blockIdx.x == 0 ? tm_ : tm2;
-  const int BM = blockIdx.x == 0 ? BM_ : BM2;
-  __shared__ int32_t wave_tot[16];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  int32_t base = 0;
-  for (int e0 = 0; e0 < E; e0 += 1024) {
-    int e = e0 + tid;
-    int32_t lo = 0, cnt = 0;
-    if (e < E) {
-      if (order != nullptr) e = order[e];
-      lo = off[e];
-      cnt = off[e + 1] - lo;
-    }
-    const int32_t tiles = (cnt + BM - 1) / BM;
-    int32_t v = tiles;
-    for (int d = 1; d < 64; d <<= 1) {
-      int32_t o = __shfl_up(v, d, 64);
-      if (lane >= d) v += o;
-    }
-    __syncthreads();  // wave_tot reuse across iterations
-    if (lane == 63) wave_tot[wave] = v;
-    __syncthreads();
-    int32_t wbase = 0, tot = 0;
-    for (int w = 0; w < 16; w++) {
-      if (w < wave) wbase += wave_tot[w];
-      tot += wave_tot[w];
-    }
-    const int32_t start = base + wbase + v - tiles;
-    // groups of nearly equal height: the first `taller` of them have one token tile more
-    const int32_t ngroups = (tiles + gmax - 1) / gmax;
-    const int32_t hbase = ngroups ? tiles / ngroups : 0, taller = ngroups ? tiles % ngroups : 0;
-    const int32_t split = taller * (hbase + 1);
-    for (int32_t i = 0; i < tiles; i++) {
-      tm.expert[start + i] = e;
-      tm.row0[start + i] = lo + i * BM;
-      int32_t g, first, h;
-      if (i < split) {
-        h = hbase + 1;
-        g = i / h;
-        first = g * h;
-      } else {
-        h = hbase;
-        g = (i - split) / h;
-        first = split + g * h;
-        g += taller;
-      }
-      tm.group[start + i] = (int32_t)((uint32_t)(start + first) | (uint32_t)h << 24 | (uint32_t)(snake & g & 1) << 31);
-    }
-    base += tot;
+                                                              const int32_t* __restrict__ order, int E, int BM,
+                                                              const TileMapPair maps, int32_t* __restrict__ sorted) {
+  __shared__ int32_t lds[TILE_SORT_MAX_E];
+  static_assert(TILE_SORT_MAX_E >= 32, "write_tile_map's words");
+  const int which = blockIdx.x;
+  if (which == 2) {
+    sort_experts(off, order, E, sorted, lds);
+    return;
   }
-  if (tid == 0) tm.header[0] = base;
+  write_tile_map<16, false>(nullptr, off, order, E, which == 0 ? BM : tile_map_rows(1), maps.gmax, maps.snake,
+                            which == 0 ? maps.map[0] : maps.map[1], lds);
 }
 
 int launch_build_tile_map(const int32_t* off, const int32_t* order, int E, int BM, TileMap tm, hipStream_t st,
-                          const TileMap* tm2, int BM2) {
-  const Tuning& tune = tuning();
-  hipLaunchKernelGGL(build_tile_map_kernel, dim3(tm2 != nullptr ? 2 : 1), dim3(1024), 0, st, off, order, E, BM,
-                     tune.gemm_group_tiles, tune.gemm_group_snake, tm, tm2 != nullptr ? *tm2 : tm, BM2);
+                          const TileMapPair* pair, int32_t* sorted) {
+  const TileMapPair one = {{tm, tm}, tuning().gemm_group_tiles, tuning().gemm_group_snake};
+  const int grid = pair == nullptr ? 1 : sorted == nullptr ? 2 : 3;
+  hipLaunchKernelGGL(build_tile_map_kernel, dim3(grid), dim3(1024), 0, st, off, order, E, BM,
+                     pair ? *pair : one, sorted);
   SMOE_LAUNCH_CHECK();
   return SMOE_OK;
 }

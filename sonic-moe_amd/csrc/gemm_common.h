@@ -24,6 +24,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "tile_map.h"
 
 namespace smoe {
 
@@ -1288,45 +1289,22 @@ const Tuning& tuning();
 // number of compute units of the current device (looked up once per device)
 int device_compute_units(int* out);
 
-// ---- tile map ------------------------------------------------------------------------------------------------
-// Built on the device from the expert offsets; header[0] = number of token tiles.  Entry i = (expert, first row) and
-// the group of token tiles entry i belongs to: the token tiles of an expert are cut into groups of nearly equal height
-// (at most gemm_group_tiles), and a group's tiles are walked feature tile by feature tile, so that the workgroups of an
-// XCD that run at the same time share few operand panels.  group[i] = first entry of the group | height << 24 |
-// (sweep direction) << 31.
-struct TileMap {
-  int32_t* header;  // [4]
-  int32_t* expert;  // [max_tiles]
-  int32_t* row0;    // [max_tiles]
-  int32_t* group;   // [max_tiles]
-};
-constexpr int TILE_GROUP_MAX = 127;  // 7 bits of height
-
-static inline int64_t max_token_tiles(int64_t TK, int E, int BM) { return TK / BM + E; }
-
-static inline size_t tile_map_bytes(int64_t TK, int E) {
-  // sized for the smallest token tile any kernel uses (64 rows)
-  return (size_t)(4 + 3 * max_token_tiles(TK, E, 64)) * sizeof(int32_t);
-}
-
-static inline TileMap carve_tile_map(void* ws, int64_t TK, int E, int BM) {
-  TileMap t;
-  t.header = (int32_t*)ws;
-  t.expert = t.header + 4;
-  t.row0 = t.expert + max_token_tiles(TK, E, BM);
-  t.group = t.row0 + max_token_tiles(TK, E, BM);
-  return t;
-}
-
-// tm2 (nullable): a second map, for tiles of BM2 rows, by a second workgroup of the same launch
+// pair (nullable): maps for both heights instead of tm's.  sorted (nullable, with pair): the experts' order too, which
+// sort_experts would write; E <= TILE_SORT_MAX_E
 int launch_build_tile_map(const int32_t* off, const int32_t* order, int E, int BM, TileMap tm, hipStream_t st,
-                          const TileMap* tm2 = nullptr, int BM2 = 0);
+                          const TileMapPair* pair = nullptr, int32_t* sorted = nullptr);
+
+static inline TileMapPair tile_map_pair(void* map, void* small_map, int64_t TK, int E) {
+  return {{carve_tile_map(map, TK, E, 256), carve_tile_map(small_map, TK, E, 128)}, tuning().gemm_group_tiles,
+          tuning().gemm_group_snake};
+}
 
 // Scratch memory of the bf16 grouped GEMMs of ONE routing (one off, no schedule order or the same one): the tile map of the
 // token-grouped kernels and the experts' order of the weight-gradient streams.  An entry point makes one for its call, on
 // its workspace, where the two share the memory; the layer's calls keep one for all GEMMs of a direction, with memory for
 // a map of either tile height (256 and 128 rows) and for the order, so that the maps are built and the experts are sorted
-// once (a launch of 4 to 6 us each).
+// once, in one launch or with the routing metadata.  E = 128, 6001 tokens, K = 8, forward and backward: 654 us with a launch
+// of 4 to 6 us for each of the three, 641 so.
 struct GemmScratch {
   void* map;
   void* small_map;  // nullable: no memory for a second map
@@ -1343,11 +1321,16 @@ struct GemmScratch {
 static inline int tile_map_in(GemmScratch& ws, const int32_t* off, const int32_t* order, int64_t TK, int E, int BM, TileMap& tm,
                               hipStream_t st) {
   if (ws.small_map != nullptr && (BM == 256 || BM == 128)) {
-    const TileMap tall = carve_tile_map(ws.map, TK, E, 256), low = carve_tile_map(ws.small_map, TK, E, 128);
-    tm = BM == 256 ? tall : low;
+    const TileMapPair pair = tile_map_pair(ws.map, ws.small_map, TK, E);
+    tm = pair.map[BM == 256 ? 0 : 1];
     if (ws.map_rows != 0) return SMOE_OK;
     ws.map_rows = 256;
-    return launch_build_tile_map(off, order, E, 256, tall, st, &low, 128);
+    // the order as well where a weight-gradient stream may follow (none takes fewer than 64 rows per expert unless it is
+    // tuned to, and then sorts itself)
+    const bool sort = ws.sorted != nullptr && !ws.sorted_valid && E <= TILE_SORT_MAX_E && TK >= 64ll * E &&
+                      (size_t)E * sizeof(int32_t) <= ws.sorted_bytes;
+    if (sort) ws.sorted_valid = true;
+    return launch_build_tile_map(off, order, E, 256, tm, st, &pair, sort ? (int32_t*)ws.sorted : nullptr);
   }
   tm = carve_tile_map(ws.map, TK, E, BM);
   if (ws.map_rows == BM) return SMOE_OK;

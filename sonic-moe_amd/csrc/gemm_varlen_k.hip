@@ -319,20 +319,7 @@ __global__ __launch_bounds__(1024) void sort_experts_kernel(const int32_t* __res
                                                             const int32_t* __restrict__ order, int E,
                                                             int32_t* __restrict__ sorted) {
   __shared__ int32_t cost[SCHED_MAX_E];
-  const int tid = threadIdx.x;
-  for (int e = tid; e < E; e += 1024) cost[e] = off[e + 1] - off[e];
-  __syncthreads();
-  for (int e = tid; e < E; e += 1024) {
-    if (order != nullptr) {
-      sorted[e] = order[e];
-    } else {
-      int pos = 0;
-      const int c = cost[e];
-#pragma unroll 8
-      for (int o = 0; o < E; o++) pos += (cost[o] > c || (cost[o] == c && o < e)) ? 1 : 0;
-      sorted[pos] = e;
-    }
-  }
+  sort_experts(off, order, E, sorted, cost);
 }
 
 // Four wavefronts as 2 x 2 wave tiles of 128 x 128; the contraction of a tile is the weight-gradient statement of

@@ -93,6 +93,7 @@ extern "C" int smoe_layer_forward(const smoe_layer_forward_args* a, void* stream
   SMOE_REQUIRE(a->workspace != nullptr && a->workspace_bytes >= (int64_t)s.total, SMOE_ERR_WORKSPACE,
                "layer_forward: workspace too small");
   int rc = SMOE_OK;
+  bool maps_written = false;
   SMOE_REQUIRE(a->router_w == nullptr || (a->logits_row_stride == E && a->logits_dtype == ELEM_DTYPE), SMOE_ERR_INVALID,
                "layer_forward: logits to be computed are contiguous, of the library's type");
   const bool few = a->router_w != nullptr && route_few_takes(T, H, E, K);
@@ -109,11 +110,13 @@ extern "C" int smoe_layer_forward(const smoe_layer_forward_args* a, void* stream
     rc = smoe_topk_softmax_fwd(a->logits, (int)a->logits_dtype, T, E, K, a->logits_row_stride, a->scores, a->indices, 1,
                                stream);
     if (rc) return rc;
-    rc = smoe_routing_metadata(a->indices, nullptr, TK, T, E, K, a->freq, a->off, a->x_gather_idx, a->s_scatter_idx,
-                               a->s_reverse_scatter_idx, a->tok_off, s.metadata, s.metadata_bytes, stream);
+    rc = routing_metadata_and_maps(a->indices, TK, T, E, K, a->freq, a->off, a->x_gather_idx, a->s_scatter_idx,
+                                   a->s_reverse_scatter_idx, a->tok_off, s.metadata, s.metadata_bytes,
+                                   tile_map_pair(s.map, s.small_map, TK, E), &maps_written, (hipStream_t)stream);
     if (rc) return rc;
   }
   GemmScratch ws(s.map, s.small_map, nullptr, 0);
+  if (maps_written) ws.map_rows = 256;
   rc = up_projection_forward(a->x, a->w1, a->w1_stride_e, a->w1_stride_row, a->b1, a->z, s.y1, a->off, nullptr,
                              a->x_gather_idx, T, TK, H, I, E, (int)a->activation, ws, stream);
   if (rc) return rc;

@@ -85,6 +85,24 @@ def test_module_step(dev, monkeypatch, shape, act, bias, dtype):
     assert _both(monkeypatch, step) == [("forward", True), ("backward", True), ("forward", True), ("forward", True)]
 
 
+# tile maps from the metadata's last launch (above 4096 slots, to 256 experts) and the experts' order from the backward's
+# (from 64 rows per expert): either side of each line, one expert, remainders, and weight-gradient streams that walk it
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(4097, 128, 64, 1, 1), (1366, 128, 64, 63, 3), (1100, 128, 64, 65, 4), (8191, 128, 128, 256, 2),
+                                   (8192, 128, 128, 256, 2), (8230, 128, 64, 257, 2), (8200, 256, 128, 8, 2),
+                                   (4100, 768, 256, 128, 8)])
+def test_maps_written_on_the_way(dev, monkeypatch, shape):
+    moe, x, dy = _module(*shape, "swiglu", False, torch.bfloat16, dev)
+
+    def step():
+        xx = x.clone().requires_grad_()
+        out, aux = moe(xx)
+        return [out.detach(), *torch.autograd.grad([out, aux], [xx, *moe.parameters()],
+                                                   grad_outputs=[dy, torch.tensor(0.3, device=dev)])]
+
+    assert _both(monkeypatch, step) == [("forward", True), ("backward", True)]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", ["loss only", "output only", "logits too", "logits transposed", "router frozen", "x frozen",
                                   "x strided", "dout strided", "weights strided", "hooks", "twice"])
