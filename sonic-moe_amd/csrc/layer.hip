@@ -110,9 +110,12 @@ extern "C" int smoe_layer_forward(const smoe_layer_forward_args* a, void* stream
     rc = smoe_topk_softmax_fwd(a->logits, (int)a->logits_dtype, T, E, K, a->logits_row_stride, a->scores, a->indices, 1,
                                stream);
     if (rc) return rc;
+    // (to that many rows per expert the GEMMs may be the ones that walk no map)
+    const TileMapPair maps = tile_map_pair(s.map, s.small_map, TK, E);
+    const bool want_maps = TK > (int64_t)tuning().gemm_skinny_rows * E;
     rc = routing_metadata_and_maps(a->indices, TK, T, E, K, a->freq, a->off, a->x_gather_idx, a->s_scatter_idx,
                                    a->s_reverse_scatter_idx, a->tok_off, s.metadata, s.metadata_bytes,
-                                   tile_map_pair(s.map, s.small_map, TK, E), &maps_written, (hipStream_t)stream);
+                                   want_maps ? &maps : nullptr, &maps_written, (hipStream_t)stream);
     if (rc) return rc;
   }
   GemmScratch ws(s.map, s.small_map, nullptr, 0);

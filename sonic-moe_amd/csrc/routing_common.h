@@ -277,10 +277,11 @@ int launch_route_few(const void* x, const void* wr, int64_t T, int H, int E, int
                      int32_t* indices, int32_t* freq, int32_t* off, int32_t* gidx, int32_t* sidx, int32_t* ridx,
                      int32_t* tok_off, float* loss_acc, float* loss, void* workspace, hipStream_t st);
 
-// smoe_routing_metadata of a top-K router's picks; the tile maps too where they cost no launch of their own: routing.hip
+// smoe_routing_metadata of a top-K router's picks; the tile maps (nullable) too where they cost no launch of their
+// own: routing.hip
 int routing_metadata_and_maps(const int32_t* expert_idx, int64_t TK, int64_t T, int E, int K, int32_t* freq, int32_t* off,
                               int32_t* x_gather_idx, int32_t* s_scatter_idx, int32_t* s_reverse_scatter_idx,
-                              int32_t* tok_off, void* workspace, size_t workspace_bytes, const TileMapPair& maps,
+                              int32_t* tok_off, void* workspace, size_t workspace_bytes, const TileMapPair* maps,
                               bool* maps_written, hipStream_t st);
 
 }  // namespace smoe

@@ -85,10 +85,12 @@ def test_module_step(dev, monkeypatch, shape, act, bias, dtype):
     assert _both(monkeypatch, step) == [("forward", True), ("backward", True), ("forward", True), ("forward", True)]
 
 
-# tile maps from the metadata's last launch (above 4096 slots, to 256 experts) and the experts' order from the backward's
-# (from 64 rows per expert): either side of each line, one expert, remainders, and weight-gradient streams that walk it
+# tile maps from the metadata's last launch (above 4096 slots, to 256 experts; above 16 rows per expert) and the experts'
+# order from the backward's (from 64 rows per expert): either side of each line, one expert, remainders, and
+# weight-gradient streams that walk it
 @pytest.mark.gpu
-@pytest.mark.parametrize("shape", [(4097, 128, 64, 1, 1), (1366, 128, 64, 63, 3), (1100, 128, 64, 65, 4), (8191, 128, 128, 256, 2),
+@pytest.mark.parametrize("shape", [(4096, 128, 64, 1, 1), (1020, 128, 64, 255, 4), (1021, 128, 64, 255, 4),
+                                   (4097, 128, 64, 1, 1), (1366, 128, 64, 63, 3), (1100, 128, 64, 65, 4), (8191, 128, 128, 256, 2),
                                    (8192, 128, 128, 256, 2), (8230, 128, 64, 257, 2), (8200, 256, 128, 8, 2),
                                    (4100, 768, 256, 128, 8)])
 def test_maps_written_on_the_way(dev, monkeypatch, shape):
