@@ -27,3 +27,11 @@ def test_gather_sum_router(dev, T, H, E, K, dtype):
     size = picked.abs().sum(1) + dlogits.double().abs() @ wr.double().abs()
     bound = torch.finfo(dtype).eps / 2 * want.abs() + (K + E) * 2.0 ** -24 * size + torch.finfo(dtype).tiny
     assert ((dx[:T].double().cpu() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("T, takes", [(0, False), (1, True), (65535 * 64, True), (65535 * 64 + 1, False)])
+def test_token_counts_the_launch_takes(dev, T, takes):
+    from sonicmoe.functional.backward import router_dx_takes
+
+    x = torch.zeros(1, 64, dtype=torch.bfloat16, device=dev).expand(T, 64)
+    assert router_dx_takes(x, torch.zeros(8, 64, dtype=x.dtype, device=dev), x.dtype, 2) == takes
