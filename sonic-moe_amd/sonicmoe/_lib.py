@@ -166,6 +166,18 @@ def require_device(*tensors: torch.Tensor | None) -> None:
             raise RuntimeError("sonicmoe HIP operators need tensors on the GPU (got a CPU tensor)")
 
 
+def require_one_device(*tensors: torch.Tensor) -> None:
+    """require_device for the kernels that stand in for a torch operation, which refuses tensors of several GPUs."""
+    require_device(*tensors)
+    if len({t.get_device() for t in tensors}) > 1:
+        raise RuntimeError(f"expected all tensors to be on one GPU, got {', '.join(str(t.device) for t in tensors)}")
+
+
+def current_gpu() -> int | None:
+    """Number of the GPU that kernels are launched on now; None before the first use of one."""
+    return torch._C._cuda_getDevice() if torch.cuda.is_initialized() else None
+
+
 def current_stream_handle() -> int:
     if torch.cuda.is_initialized():  # the Stream object behind current_stream() costs several us
         return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())

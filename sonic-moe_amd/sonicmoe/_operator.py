@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import torch
 
+from . import _lib
 from ._lib import NoMemory
 from .enums import LIBRARY_NAME
 
@@ -47,7 +48,9 @@ def elsewhere(*ops) -> frozenset:
 
 def unobserved(names: frozenset, *tensors) -> bool:
     """Whether nobody looks on the calls of the operators behind `names` (`elsewhere`) on these tensors (or None) in a row:
-    the questions of `run`, asked once.  For eager code only."""
+    the questions of `run`, asked once, and whether a kernel launched now may be given all of them: memory of the current
+    GPU (the caller's own torch operations would refuse tensors of several, and run where theirs are).  For eager code
+    only."""
     if not (
         torch._C._len_torch_dispatch_stack() == 0
         and torch._C._functorch.peek_interpreter_stack() is None
@@ -58,8 +61,9 @@ def unobserved(names: frozenset, *tensors) -> bool:
         and _REGISTERED.isdisjoint(names)
     ):
         return False
+    gpu = _lib.current_gpu()
     for t in tensors:
-        if t is not None and (type(t) not in _TENSORS or not t.is_cuda or t.is_neg()):
+        if t is not None and (type(t) not in _TENSORS or t.get_device() != gpu or t.is_neg()):
             return False
     return True
 

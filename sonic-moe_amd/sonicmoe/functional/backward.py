@@ -208,7 +208,7 @@ def _token_broadcast_backward_router(
 ) -> None:
     """`_token_broadcast_backward` for K slots per token with the router's share of dx: dx[t] = sum of the token's rows of
     dx_expanded + dlogits[t] router_w, one rounding (the reference leaves the second term to autograd)."""
-    _lib.require_device(dx, dx_expanded, s_reverse_scatter_idx, dlogits, router_w)
+    _lib.require_one_device(dx, dx_expanded, s_reverse_scatter_idx, dlogits, router_w)
     dt = _elem_dtype(("dx", dx), ("dx_expanded", dx_expanded), ("dlogits", dlogits), ("router_w", router_w))
     T, H = dx.shape
     E = router_w.size(0)
@@ -224,8 +224,8 @@ def _token_broadcast_backward_router(
 
 def router_dx_takes(x: torch.Tensor, router_w: torch.Tensor, logits_dtype: torch.dtype, K: int) -> bool:
     """Whether `_token_broadcast_backward_router` forms dx (eager code; compiled code keeps the GEMM it can see through)"""
-    return (not torch.compiler.is_compiling() and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16)
-            and router_w.dtype == x.dtype and logits_dtype == x.dtype and 1 <= K <= 16
+    return (not torch.compiler.is_compiling() and x.get_device() == router_w.get_device() == _lib.current_gpu()
+            and x.dtype in (torch.bfloat16, torch.float16) and router_w.dtype == x.dtype and logits_dtype == x.dtype and 1 <= K <= 16
             and 0 < x.size(0) < 65536 * 64 - 63  # (64 tokens to a workgroup, 65535 of them)
             and router_w.size(0) % 8 == 0 and x.size(1) % 8 == 0 and router_w.is_contiguous()
             and router_w.data_ptr() % 16 == 0)

@@ -318,7 +318,7 @@ def _switch_loss_fwd(router_logits: torch.Tensor, expert_frequency: torch.Tensor
 @operator("_router_logits", mutates_args={"logits"})
 def _router_logits(x: torch.Tensor, router_w: torch.Tensor, logits: torch.Tensor) -> None:
     """logits (T, E) = x router_w^T: the reference's F.linear (sonicmoe/functional/__init__.py:438) for few tokens."""
-    _lib.require_device(x, router_w, logits)
+    _lib.require_one_device(x, router_w, logits)
     dt = _elem_dtype(("x", x), ("router_w", router_w), ("logits", logits))
     T, H = x.shape
     E = router_w.size(0)
@@ -340,7 +340,8 @@ ROUTER_LOGITS_MAX_TOKENS, ROUTER_LOGITS_MAX_TOKENS_FEW_EXPERTS, FEW_EXPERTS = 64
 def router_logits_takes(x: torch.Tensor, router_w: torch.Tensor) -> bool:
     """Whether `_router_logits` stands in for F.linear(x, router_w) (eager code; compiled code keeps the library GEMM, whose
     call it can see through)."""
-    return (not torch.compiler.is_compiling() and x.is_cuda and x.dtype == router_w.dtype
+    return (not torch.compiler.is_compiling() and x.get_device() == router_w.get_device() == _lib.current_gpu()
+            and x.dtype == router_w.dtype
             and x.dtype in (torch.bfloat16, torch.float16) and x.dim() == 2
             and 0 < x.size(0) <= (ROUTER_LOGITS_MAX_TOKENS_FEW_EXPERTS if router_w.size(0) <= FEW_EXPERTS
                                   else ROUTER_LOGITS_MAX_TOKENS)

@@ -2,7 +2,7 @@
 
 import pytest
 import torch
-from torch._subclasses.fake_tensor import FakeTensorMode
+from torch._subclasses.fake_tensor import FakeTensor, FakeTensorMode
 from torch.overrides import TorchFunctionMode
 from torch.utils._python_dispatch import TorchDispatchMode
 
@@ -182,3 +182,33 @@ def test_layer_shapes_on_the_meta_device():
     out, aux = moe(x)
     (dx,) = torch.autograd.grad(out, [x], torch.empty_like(out))
     assert out.shape == dx.shape == (32, 128) and aux.shape == () and out.is_meta
+
+
+def _on_gpus(monkeypatch, *numbers, current=0):
+    """Tensors that say they are on these GPUs, taken for ordinary ones (8 tokens; 16 router rows)"""
+    from sonicmoe import _operator
+
+    monkeypatch.setattr(_operator, "_TENSORS", (FakeTensor,))
+    monkeypatch.setattr(_lib, "current_gpu", lambda: current)
+    with FakeTensorMode():
+        return [torch.empty(rows, 128, dtype=torch.bfloat16, device=f"cuda:{n}") for rows, n in zip((8, 16), numbers)]
+
+
+@pytest.mark.filterwarnings("ignore:Accessing the data pointer")
+@pytest.mark.parametrize("gpus, current, taken", [((0, 0), 0, True), ((0, 1), 0, False), ((1, 0), 0, False), ((1, 1), 0, False),
+                                                  ((1, 1), 1, True)])
+def test_kernels_in_the_place_of_torch_operations_stay_on_one_gpu(monkeypatch, gpus, current, taken):
+    """F.linear refuses tensors of two GPUs and runs on theirs, not on the current one."""
+    from sonicmoe._operator import unobserved
+    from sonicmoe.functional.backward import _token_broadcast_backward_router, router_dx_takes
+    from sonicmoe.functional.forward import _router_logits, router_logits_takes
+
+    x, w = _on_gpus(monkeypatch, *gpus, current=current)
+    assert unobserved(frozenset(), x, None, w) == taken
+    assert router_logits_takes(x, w) == taken
+    assert router_dx_takes(x, w, x.dtype, 2) == taken
+    if gpus[0] != gpus[1]:
+        with pytest.raises(RuntimeError, match="one GPU"):
+            _router_logits.body(x, w, x)
+        with pytest.raises(RuntimeError, match="one GPU"):
+            _token_broadcast_backward_router.body(x, x, x, x, w, 2)
