@@ -449,9 +449,9 @@ class _ExpertsFunction(torch.autograd.Function):
         return dx, dw1, db1, dw2, db2, ds, None, None, None, None, None, None, None, None, None, None
 
 
-def _router_wgrad_takes(dlogits: torch.Tensor, x: torch.Tensor) -> bool:
-    (T, E), H = dlogits.shape, x.size(1)
-    fast = (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and dlogits.dtype == x.dtype and E % 8 == 0
+def _router_wgrad_takes(logits_dtype: torch.dtype, E: int, x: torch.Tensor) -> bool:
+    T, H = x.shape
+    fast = (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and logits_dtype == x.dtype and E % 8 == 0
             and H % 8 == 0)
     return fast and T >= 256 and os.environ.get("SMOE_ROUTER_WGRAD", "1") != "0"
 
@@ -461,7 +461,7 @@ def _router_wgrad(dlogits: torch.Tensor, x: torch.Tensor, like: torch.Tensor) ->
     contraction elements, which a library GEMM without a split runs on an eighth of the chip), torch otherwise."""
     T, E = dlogits.shape
     H = x.size(1)
-    if _router_wgrad_takes(dlogits, x):
+    if _router_wgrad_takes(dlogits.dtype, E, x):
         partial = torch.empty(router_weight_grad_chunks(T, E, H), E, H, dtype=x.dtype, device=x.device)
         run(_router_weight_grad, dlogits.contiguous(), x.contiguous(), partial)
         if partial.size(0) == 1:
@@ -560,7 +560,9 @@ class _OneCallLayerFunction(torch.autograd.Function):
         if done is None:
             raise layer_call.Refused
         o, logits, z, freq, ints, loss = done
-        ctx.save_for_backward(x, router_w, w1, w2, b2, z, ints, freq, logits)
+        # the counts and the logits belong to the caller, who may change them in place: they are kept only for the loss, which
+        # is formed from them (as switch_loss keeps them)
+        ctx.save_for_backward(x, router_w, w1, w2, b2, z, ints, *((freq, logits) if with_loss else (None, None)))
         ctx.cfg = (K, activation_type, stream_id, b1 is not None)
         ctx.set_materialize_grads(False)  # (zeros for the token counts and the logits nobody used would be two launches)
         ctx.mark_non_differentiable(freq)
@@ -574,10 +576,10 @@ class _OneCallLayerFunction(torch.autograd.Function):
         E = router_w.size(0)
         if dout is None:
             dout = torch.zeros(T, H, dtype=x.dtype, device=x.device)
-        fast_router = (ctx.needs_input_grad[1] and _router_wgrad_takes(logits, x))
+        fast_router = ctx.needs_input_grad[1] and _router_wgrad_takes(x.dtype, E, x)  # (the logits have x's type)
         chunks = router_weight_grad_chunks(T, E, H) if fast_router else 0
         done = None
-        with_router = ctx.needs_input_grad[0] and router_dx_takes(x, router_w, logits.dtype, K)
+        with_router = ctx.needs_input_grad[0] and router_dx_takes(x, router_w, x.dtype, K)
         if (_down_projection_backward, _up_projection_backward, _token_broadcast_backward, _token_broadcast_backward_router,
                 _switch_loss_bwd, _router_logit_grad, _router_weight_grad, _sum_chunks) == layer_call._BACKWARD_OPERATORS:
             done = layer_call.backward(x, dout, z, w1, w2, b2, has_b1, ints, freq, logits, K, activation_type, stream_id, daux,
@@ -597,7 +599,7 @@ class _OneCallLayerFunction(torch.autograd.Function):
             run(_switch_loss_bwd, logits, freq, acc, daux.reshape(1).float().contiguous(), dlogits)
             dlogits_outside = dlogits if dlogits_outside is None else dlogits_outside + dlogits
         return _tc_layer_backward(ctx, dout, dlogits_outside, x, router_w, w1, w2, b2, z, scores, indices, off, gidx, sidx, ridx,
-                                  tok_off, K, activation_type, stream_id, logits.dtype, has_b1, None, False)
+                                  tok_off, K, activation_type, stream_id, x.dtype, has_b1, None, False)
 
 
 class _SwitchLossFunction(torch.autograd.Function):

@@ -136,7 +136,8 @@ def forward(x, router_w, w1, b1, w2, b2, K: int, activation, stream_id: int, kee
 def backward(x, dout, z, w1, w2, b2, has_b1: bool, ints, freq, logits, K: int, activation, stream_id: int, loss_grad,
              outside, chunks: int, router_w):
     """(dx, dlogits, dwr or None, dw1, db1, dw2, db2), or None where the operators have to do it.  chunks: token chunks of the
-    router's weight gradient (0: the caller forms it).  router_w: None leaves the router's share of dx to the caller."""
+    router's weight gradient (0: the caller forms it).  router_w: None leaves the router's share of dx to the caller.  freq
+    and logits: with loss_grad only."""
     dtype = x.dtype
     if torch.compiler.is_compiling() or not (
         unobserved(_BACKWARD_NAMES, x, dout, z, w1, w2, b2, ints, freq, logits, loss_grad, outside)
@@ -146,20 +147,20 @@ def backward(x, dout, z, w1, w2, b2, has_b1: bool, ints, freq, logits, K: int, a
         return None
     dout = dout.contiguous()
     T, H = x.shape
-    E, I = logits.size(1), w2.size(1)
+    _, I, E = w2.shape
     if loss_grad is not None:
         loss_grad = loss_grad.reshape(1).float()
     elif outside is not None and not (outside.layout == torch.strided and outside.dtype == dtype
-                                      and outside.shape == logits.shape and outside.stride(1) == 1
+                                      and outside.shape == (T, E) and outside.stride(1) == 1
                                       and outside.stride(0) >= E):
         return None
-    tensors = (x, dout, z, w1, w2, ints, freq, logits)
+    loss = () if loss_grad is None else (loss_grad, freq, logits)
     # (saved tensors may come back from hooks in other memory)
-    if not (x.is_contiguous() and z.is_contiguous() and ints.is_contiguous() and freq.is_contiguous()
-            and w1.stride(1) == 1 and w2.stride(1) == 1 and logits.stride(1) == 1
+    if not (x.is_contiguous() and z.is_contiguous() and ints.is_contiguous() and w1.stride(1) == 1 and w2.stride(1) == 1
             and (b2 is None or (b2.is_contiguous() and b2.data_ptr() != 0))
-            and all(t.data_ptr() != 0 for t in tensors)
-            and (loss_grad is None or loss_grad.data_ptr() != 0) and (outside is None or outside.data_ptr() != 0)):
+            and (not loss or (freq.is_contiguous() and logits.stride(1) == 1))
+            and all(t.data_ptr() != 0 for t in (x, dout, z, w1, w2, ints, *loss))
+            and (outside is None or outside.data_ptr() != 0)):
         return None
     where = Indices(T, E, K)
     L = _lib.lib(dtype)
@@ -182,9 +183,9 @@ def backward(x, dout, z, w1, w2, b2, has_b1: bool, ints, freq, logits, K: int, a
         _BACKWARD.pack(
             x.data_ptr(), dout.data_ptr(), z.data_ptr(), w1.data_ptr(), w2.data_ptr(), 0 if b2 is None else b2.data_ptr(),
             s1[2], s1[0], s2[2], s2[0],
-            base, base + 4 * at[1], freq.data_ptr(), base + 4 * at[5], base + 4 * at[2], base + 4 * at[3], base + 4 * at[4],
-            logits.data_ptr(), _lib.DT_CODE[dtype], logits.stride(0), base + 4 * at[7],
-            0 if loss_grad is None else loss_grad.data_ptr(), 0 if outside is None else outside.data_ptr(),
+            base, base + 4 * at[1], freq.data_ptr() if loss else 0, base + 4 * at[5], base + 4 * at[2], base + 4 * at[3],
+            base + 4 * at[4], logits.data_ptr() if loss else 0, _lib.DT_CODE[dtype], logits.stride(0) if loss else 0,
+            base + 4 * at[7], loss_grad.data_ptr() if loss else 0, 0 if outside is None else outside.data_ptr(),
             0 if outside is None else outside.stride(0), T, H, I, E, K, code,
             dw1.data_ptr(), dw2.data_ptr(), d1[2], d1[0], d2[2], d2[0],
             0 if db1 is None else db1.data_ptr(), 0 if db2 is None else db2.data_ptr(), dx.data_ptr(), dlogits.data_ptr(),

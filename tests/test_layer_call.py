@@ -29,6 +29,38 @@ def test_index_views_do_not_overlap(T, E, K):
     assert all(a % 64 == 0 for a, _ in spans)
 
 
+@pytest.mark.parametrize("with_loss", [False, True])
+def test_what_the_layer_keeps_for_its_backward(monkeypatch, with_loss):
+    """Counts and logits are the caller's to change in place: without the loss the backward pass does without them."""
+    from sonicmoe.enums import ActivationType
+    from sonicmoe.functional import layer_call, layer_with_loss
+
+    T, H, I, E, K = 6, 16, 8, 4, 2
+    asked = []
+
+    def forward(x, router_w, w1, b1, w2, b2, K, activation, stream_id, keep_z, loss):
+        return (torch.zeros(T, H), torch.zeros(T, E), torch.zeros(T * K, 2 * I), torch.zeros(E, dtype=torch.int32),
+                torch.zeros(layer_call.Indices(T, E, K).words, dtype=torch.int32), torch.zeros(()) if loss else None)
+
+    def backward(x, dout, z, w1, w2, b2, has_b1, ints, freq, logits, *rest):
+        asked.append((freq is not None, logits is not None))
+        return torch.zeros(T, H), torch.zeros(T, E), torch.zeros(E, H), torch.empty_like(w1), None, torch.empty_like(w2), None
+
+    monkeypatch.setattr(layer_call, "takes", lambda *a: True)
+    monkeypatch.setattr(layer_call, "forward", forward)
+    monkeypatch.setattr(layer_call, "backward", backward)
+    x, wr = torch.randn(T, H, requires_grad=True), torch.randn(E, H, requires_grad=True)
+    w1, w2 = torch.randn(E, 2 * I, H, requires_grad=True), torch.randn(E, H, I, requires_grad=True)
+    o, logits, freq, loss = layer_with_loss(x, wr, w1.permute(1, 2, 0), None, w2.permute(1, 2, 0), None, K, 0,
+                                            ActivationType.SWIGLU, False, with_loss)
+    assert (loss is not None) == with_loss
+    if not with_loss:
+        logits.mul_(2)
+        freq.add_(1)
+    torch.autograd.grad([o, logits], [x, wr, w1, w2], [torch.ones_like(o), torch.ones_like(logits)])
+    assert asked == [(with_loss, with_loss)]
+
+
 def _module(T, H, I, E, K, act, bias, dtype, dev):
     from sonicmoe import MoE
     from sonicmoe.enums import ActivationType
@@ -107,7 +139,7 @@ def test_maps_written_on_the_way(dev, monkeypatch, shape):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", ["loss only", "output only", "logits too", "logits transposed", "router frozen", "x frozen",
-                                  "x strided", "dout strided", "weights strided", "hooks", "twice"])
+                                  "x strided", "dout strided", "weights strided", "hooks", "twice", "outputs changed"])
 def test_functional_forms(dev, monkeypatch, case):
     from sonicmoe.functional import moe_TC_softmax_topk_layer, switch_loss
 
@@ -139,6 +171,11 @@ def test_functional_forms(dev, monkeypatch, case):
         outs, grads = [o], [dy]
         if case == "loss only":
             outs, grads = [switch_loss(logits, freq)], [torch.tensor(2.0, device=dev)]
+        elif case == "outputs changed":
+            logits.mul_(2)
+            freq.add_(1)
+            outs.append(logits)
+            grads.append(dl.t().contiguous())
         elif case.startswith("logits"):
             outs.append(logits)
             grads.append(dl.t() if case == "logits transposed" else dl.t().contiguous())
