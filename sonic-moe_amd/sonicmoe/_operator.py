@@ -46,26 +46,43 @@ def elsewhere(*ops) -> frozenset:
     return frozenset().union(*(op.elsewhere for op in ops))
 
 
-def unobserved(names: frozenset, *tensors) -> bool:
-    """Whether nobody looks on the calls of the operators behind `names` (`elsewhere`) on these tensors (or None) in a row:
-    the questions of `run`, asked once, and whether a kernel launched now may be given all of them: memory of the current
-    GPU (the caller's own torch operations would refuse tensors of several, and run where theirs are).  For eager code
-    only."""
-    if not (
-        torch._C._len_torch_dispatch_stack() == 0
-        and torch._C._functorch.peek_interpreter_stack() is None
+def untraced() -> bool:
+    """Whether no mode, transformation or trace stands between a torch call and its tensors.  For eager code only."""
+    return (
+        torch._C._len_torch_dispatch_stack() == 0  # dispatch modes: fake tensors, make_fx, profiling counters
+        and torch._C._functorch.peek_interpreter_stack() is None  # vmap, grad, functionalization
         and not torch._C._is_torch_function_mode_enabled()
-        and torch._C._get_tracing_state() is None
-        and not torch.autograd._profiler_enabled()
-        and _REGISTERED is not None
-        and _REGISTERED.isdisjoint(names)
-    ):
-        return False
+        and torch._C._get_tracing_state() is None  # torch.jit.trace
+    )
+
+
+def in_memory(*tensors) -> bool:
+    """Whether a kernel launched now may be given the addresses of all these tensors (or None): plain ones, which have an
+    address that means something, in memory of the current GPU (the torch operation that the kernel stands in for would refuse
+    tensors of several, and run where theirs are)."""
     gpu = _lib.current_gpu()
     for t in tensors:
         if t is not None and (type(t) not in _TENSORS or t.get_device() != gpu or t.is_neg()):
             return False
     return True
+
+
+def unobserved(names: frozenset, *tensors) -> bool:
+    """Whether nobody looks on the calls of the operators behind `names` (`elsewhere`) in a row and these tensors are
+    `in_memory`: the questions of `run`, asked once.  For eager code only."""
+    return (
+        untraced()
+        and not torch.autograd._profiler_enabled()
+        and _REGISTERED is not None
+        and _REGISTERED.isdisjoint(names)
+        and in_memory(*tensors)
+    )
+
+
+def stands_in(*tensors) -> bool:
+    """Whether an operator may stand in for a torch operation on these tensors: whoever traces or transforms torch calls keeps
+    the operation, which they can see through, and so do tensors without an address to ask for.  (Profilers see the operator.)"""
+    return not torch.compiler.is_compiling() and untraced() and in_memory(*tensors)
 
 
 def run(op, *args) -> None:
@@ -75,10 +92,7 @@ def run(op, *args) -> None:
         op(*args)
         return
     if (
-        torch._C._len_torch_dispatch_stack() == 0  # dispatch modes: fake tensors, make_fx, profiling counters
-        and torch._C._functorch.peek_interpreter_stack() is None  # vmap, grad, functionalization
-        and not torch._C._is_torch_function_mode_enabled()
-        and torch._C._get_tracing_state() is None  # torch.jit.trace
+        untraced()
         and not torch.autograd._profiler_enabled()  # its rows come from the dispatcher
         and not args[0].is_meta  # (every operator's first argument is a tensor, and all of one call are on one device)
     ):

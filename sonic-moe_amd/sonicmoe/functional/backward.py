@@ -7,7 +7,7 @@ from typing import Optional
 import torch
 
 from .. import _lib
-from .._operator import operator
+from .._operator import operator, stands_in
 from ..enums import ACTIVATION_CODE, ActivationType
 from ..utils import expert_major_strides
 from .forward import _check_schedule_order, _elem_dtype, _gather_sum, _gemm_workspace
@@ -223,9 +223,9 @@ def _token_broadcast_backward_router(
 
 
 def router_dx_takes(x: torch.Tensor, router_w: torch.Tensor, logits_dtype: torch.dtype, K: int) -> bool:
-    """Whether `_token_broadcast_backward_router` forms dx (eager code; compiled code keeps the GEMM it can see through)"""
-    return (not torch.compiler.is_compiling() and x.get_device() == router_w.get_device() == _lib.current_gpu()
-            and x.dtype in (torch.bfloat16, torch.float16) and router_w.dtype == x.dtype and logits_dtype == x.dtype and 1 <= K <= 16
+    """Whether `_token_broadcast_backward_router` forms dx, in the place of a reduction and an addmm_"""
+    return (stands_in(x, router_w) and x.dtype in (torch.bfloat16, torch.float16)
+            and router_w.dtype == x.dtype and logits_dtype == x.dtype and 1 <= K <= 16
             and 0 < x.size(0) < 65536 * 64 - 63  # (64 tokens to a workgroup, 65535 of them)
             and router_w.size(0) % 8 == 0 and x.size(1) % 8 == 0 and router_w.is_contiguous()
             and router_w.data_ptr() % 16 == 0)

@@ -199,16 +199,48 @@ def _on_gpus(monkeypatch, *numbers, current=0):
                                                   ((1, 1), 1, True)])
 def test_kernels_in_the_place_of_torch_operations_stay_on_one_gpu(monkeypatch, gpus, current, taken):
     """F.linear refuses tensors of two GPUs and runs on theirs, not on the current one."""
-    from sonicmoe._operator import unobserved
+    from sonicmoe._operator import stands_in, unobserved
     from sonicmoe.functional.backward import _token_broadcast_backward_router, router_dx_takes
-    from sonicmoe.functional.forward import _router_logits, router_logits_takes
+    from sonicmoe.functional.forward import _router_logits
 
     x, w = _on_gpus(monkeypatch, *gpus, current=current)
     assert unobserved(frozenset(), x, None, w) == taken
-    assert router_logits_takes(x, w) == taken
+    assert stands_in(x, w) == taken
     assert router_dx_takes(x, w, x.dtype, 2) == taken
     if gpus[0] != gpus[1]:
         with pytest.raises(RuntimeError, match="one GPU"):
             _router_logits.body(x, w, x)
         with pytest.raises(RuntimeError, match="one GPU"):
             _token_broadcast_backward_router.body(x, x, x, x, w, 2)
+
+
+@pytest.mark.filterwarnings("error:Accessing the data pointer")
+@pytest.mark.parametrize("tracer", ["fake tensors", "aot_function", "make_fx"])
+def test_tracers_keep_the_router_gemm(monkeypatch, tracer):
+    """Outside torch.compile too: no address is asked for, and the trace holds the torch operation."""
+    from torch._functorch.aot_autograd import aot_function
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    from sonicmoe.functional import moe_TC_softmax_topk_layer
+    from sonicmoe.functional.backward import router_dx_takes
+
+    def layer(x, wr, w1, w2):
+        return moe_TC_softmax_topk_layer(x, wr, w1.permute(1, 2, 0), None, w2.permute(1, 2, 0), None, 2, 0)
+
+    monkeypatch.setattr(_lib, "current_gpu", lambda: 0)
+    T, H, I, E = 8, 128, 64, 16
+    graphs = []
+    with FakeTensorMode(), torch.no_grad():
+        args = [torch.empty(s, dtype=torch.bfloat16, device="cuda:0") for s in ((T, H), (E, H), (E, 2 * I, H), (E, H, I))]
+        assert not router_dx_takes(args[0], args[1], torch.bfloat16, 2)
+        if tracer == "aot_function":
+            got = aot_function(layer, fw_compiler=lambda gm, _: (graphs.append(gm), gm)[1])(*args)
+        elif tracer == "make_fx":
+            graphs.append(make_fx(layer)(*args))
+            got = layer(*args)
+        else:
+            got = layer(*args)
+    assert [t.shape for t in got] == [(T, H), (T, E), (E,)]
+    for graph in graphs:
+        called = [str(n.target) for n in graph.graph.nodes if n.op == "call_function"]
+        assert "aten.mm.default" in called and not any("_router_logits" in t for t in called)
