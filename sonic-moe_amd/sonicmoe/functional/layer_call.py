@@ -140,7 +140,7 @@ def backward(x, dout, z, w1, w2, b2, has_b1: bool, ints, freq, logits, K: int, a
     and logits: with loss_grad only."""
     dtype = x.dtype
     if torch.compiler.is_compiling() or not (
-        unobserved(_BACKWARD_NAMES, x, dout, z, w1, w2, b2, ints, freq, logits, loss_grad, outside)
+        unobserved(_BACKWARD_NAMES, x, dout, z, w1, w2, b2, ints, freq, logits, loss_grad, outside, router_w)
         and dout.dtype == dtype and dout.layout == torch.strided and stream_id == _lib.current_stream_handle()
         and (loss_grad is None or outside is None)
     ):
@@ -155,14 +155,23 @@ def backward(x, dout, z, w1, w2, b2, has_b1: bool, ints, freq, logits, K: int, a
                                       and outside.stride(0) >= E):
         return None
     loss = () if loss_grad is None else (loss_grad, freq, logits)
-    # (saved tensors may come back from hooks in other memory)
+    where = Indices(T, E, K)
+    # (saved tensors may come back from hooks in other memory, of another type or shape)
+    if not (z.dtype == w1.dtype == w2.dtype == dtype and (b2 is None or b2.dtype == dtype)
+            and (router_w is None or router_w.dtype == dtype and router_w.shape == (E, H))
+            and dout.shape == (T, H) and w1.shape == (z.size(1), H, E) and w2.size(0) == H
+            and z.shape == (T * K, 2 * I if is_glu(activation) else I)
+            and (b2 is None or b2.shape == (E, H)) and ints.dtype == torch.int32 and ints.shape == (where.words,)
+            and (not loss or (freq.dtype == torch.int32 and freq.shape == (E,) and logits.dtype == dtype
+                              and logits.shape == (T, E)))):
+        return None
     if not (x.is_contiguous() and z.is_contiguous() and ints.is_contiguous() and w1.stride(1) == 1 and w2.stride(1) == 1
             and (b2 is None or (b2.is_contiguous() and b2.data_ptr() != 0))
+            and (router_w is None or (router_w.is_contiguous() and router_w.data_ptr() != 0))
             and (not loss or (freq.is_contiguous() and logits.stride(1) == 1))
             and all(t.data_ptr() != 0 for t in (x, dout, z, w1, w2, ints, *loss))
             and (outside is None or outside.data_ptr() != 0)):
         return None
-    where = Indices(T, E, K)
     L = _lib.lib(dtype)
     code, dev = ACTIVATION_CODE[activation], x.device
     need = L.smoe_layer_backward_workspace_bytes(T, H, I, E, K, code, chunks)

@@ -61,6 +61,52 @@ def test_what_the_layer_keeps_for_its_backward(monkeypatch, with_loss):
     assert asked == [(with_loss, with_loss)]
 
 
+@pytest.mark.parametrize("what", ["plain", "lazily negated", "without memory", "subclass", "other GPU", "wider type",
+                                  "longer"])
+def test_the_backward_asks_about_every_tensor_it_passes_on(monkeypatch, what):
+    """Saved-tensor hooks decide what comes back: for each tensor that is not as the library needs it, the operators do it."""
+    from sonicmoe import _lib, _operator
+    from sonicmoe.enums import ActivationType
+    from sonicmoe.functional import layer_call
+
+    class Asked(Exception):
+        pass
+
+    class Tagged(torch.Tensor):
+        pass
+
+    def reached(dtype):
+        raise Asked
+
+    class Elsewhere(torch.Tensor):
+        def get_device(self):
+            return 1
+
+    # (on the CPU, which is number -1)
+    monkeypatch.setattr(_lib, "current_gpu", lambda: -1)
+    monkeypatch.setattr(_lib, "current_stream_handle", lambda: 0)
+    monkeypatch.setattr(_lib, "lib", reached)
+    monkeypatch.setattr(_operator, "_TENSORS", (torch.Tensor, Elsewhere))
+    T, H, I, E, K = 6, 16, 8, 4, 2
+    bf16 = lambda *shape: torch.zeros(*shape, dtype=torch.bfloat16)
+    given = dict(x=bf16(T, H), dout=bf16(T, H), z=bf16(T * K, 2 * I), w1=bf16(E, 2 * I, H).permute(1, 2, 0),
+                 w2=bf16(E, H, I).permute(1, 2, 0), b2=bf16(E, H), has_b1=True,
+                 ints=torch.zeros(layer_call.Indices(T, E, K).words, dtype=torch.int32), freq=torch.zeros(E, dtype=torch.int32),
+                 logits=bf16(T, E), K=K, activation=ActivationType.SWIGLU, stream_id=0, loss_grad=torch.zeros(()), outside=None,
+                 chunks=0, router_w=bf16(E, H))
+    if what == "plain":
+        with pytest.raises(Asked):
+            layer_call.backward(**given)
+        return
+    changed = {"lazily negated": torch._neg_view, "subclass": lambda t: t.as_subclass(Tagged),
+               "other GPU": lambda t: t.as_subclass(Elsewhere), "wider type": lambda t: t.double(),
+               "longer": lambda t: torch.cat([t, t]),
+               "without memory": lambda t: torch._efficientzerotensor(t.shape, dtype=t.dtype)}[what]
+    for name, t in given.items():
+        if isinstance(t, torch.Tensor) and (name != "loss_grad" or what not in ("wider type", "longer")):
+            assert layer_call.backward(**{**given, name: changed(t)}) is None, name
+
+
 def _module(T, H, I, E, K, act, bias, dtype, dev):
     from sonicmoe import MoE
     from sonicmoe.enums import ActivationType
