@@ -38,6 +38,18 @@ class Refused(Exception):
     """The library does not take the layer: the operators tell why."""
 
 
+# smoe_status of arguments or shapes that the kernels do not take (bad argument, unsupported)
+_NOT_TAKEN = (1, 2)
+
+
+def _taken(rc: int, what: str) -> bool:
+    """Whether the library did it; a launch that failed or a workspace that does not suffice is told, and not tried again."""
+    if rc in _NOT_TAKEN:
+        return False
+    _lib.check(rc, what)
+    return True
+
+
 def forward_names(routing_metadata) -> frozenset:
     return elsewhere(*_FORWARD_OPERATORS, routing_metadata)
 
@@ -130,7 +142,7 @@ def forward(x, router_w, w1, b1, w2, b2, K: int, activation, stream_id: int, kee
         ),
         stream_id,
     )
-    return None if rc else (o, logits, z, freq, ints, loss)
+    return (o, logits, z, freq, ints, loss) if _taken(rc, "layer_forward") else None
 
 
 def backward(x, dout, z, w1, w2, b2, has_b1: bool, ints, freq, logits, K: int, activation, stream_id: int, loss_grad,
@@ -203,4 +215,4 @@ def backward(x, dout, z, w1, w2, b2, has_b1: bool, ints, freq, logits, K: int, a
         ),
         stream_id,
     )
-    return None if rc else (dx, dlogits, dwr, dw1, db1, dw2, db2)
+    return (dx, dlogits, dwr, dw1, db1, dw2, db2) if _taken(rc, "layer_backward") else None

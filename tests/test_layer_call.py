@@ -61,12 +61,62 @@ def test_what_the_layer_keeps_for_its_backward(monkeypatch, with_loss):
     assert asked == [(with_loss, with_loss)]
 
 
+@pytest.fixture
+def on_the_cpu(monkeypatch):
+    """layer_call with CPU tensors (device number -1), as far as the library: on_the_cpu(library)"""
+    from sonicmoe import _lib
+
+    monkeypatch.setattr(_lib, "current_gpu", lambda: -1)
+    monkeypatch.setattr(_lib, "current_stream_handle", lambda: 0)
+    return lambda library: monkeypatch.setattr(_lib, "lib", library)
+
+
+def _arguments():
+    """(of the forward call, of the backward call)"""
+    from sonicmoe.enums import ActivationType
+    from sonicmoe.functional import layer_call
+
+    T, H, I, E, K = 6, 32, 8, 4, 2
+    bf16 = lambda *shape: torch.zeros(*shape, dtype=torch.bfloat16)
+    both = dict(x=bf16(T, H), router_w=bf16(E, H), w1=bf16(E, 2 * I, H).permute(1, 2, 0), w2=bf16(E, H, I).permute(1, 2, 0),
+                b2=bf16(E, H), K=K, activation=ActivationType.SWIGLU, stream_id=0)
+    return (dict(both, b1=bf16(E, 2 * I), keep_z=True, with_loss=True),
+            dict(both, dout=bf16(T, H), z=bf16(T * K, 2 * I), has_b1=True, logits=bf16(T, E), loss_grad=torch.zeros(()),
+                 ints=torch.zeros(layer_call.Indices(T, E, K).words, dtype=torch.int32), freq=torch.zeros(E, dtype=torch.int32),
+                 outside=None, chunks=0))
+
+
+@pytest.mark.parametrize("status, told", [(0, False), (1, False), (2, False), (3, True), (4, True)])
+def test_status_of_the_library(on_the_cpu, status, told):
+    """What the kernels do not take goes to the operators, which tell why; a failed launch or a workspace that does not suffice
+    is told at once."""
+    from sonicmoe.functional import layer_call
+
+    class Library:
+        smoe_last_error = staticmethod(lambda: b"planted")
+
+        def __getattr__(self, name):
+            return lambda *args: 256 if name.endswith("workspace_bytes") else status
+
+    from sonicmoe import _lib
+
+    on_the_cpu(lambda *dtype: setattr(_lib._TLS, "last", Library()) or Library())
+    try:
+        for call, given in zip((layer_call.forward, layer_call.backward), _arguments()):
+            if told:
+                with pytest.raises(RuntimeError, match="planted"):
+                    call(**given)
+            else:
+                assert (call(**given) is None) == (status != 0)
+    finally:
+        del _lib._TLS.last
+
+
 @pytest.mark.parametrize("what", ["plain", "lazily negated", "without memory", "subclass", "other GPU", "wider type",
                                   "longer"])
-def test_the_backward_asks_about_every_tensor_it_passes_on(monkeypatch, what):
+def test_the_backward_asks_about_every_tensor_it_passes_on(monkeypatch, on_the_cpu, what):
     """Saved-tensor hooks decide what comes back: for each tensor that is not as the library needs it, the operators do it."""
-    from sonicmoe import _lib, _operator
-    from sonicmoe.enums import ActivationType
+    from sonicmoe import _operator
     from sonicmoe.functional import layer_call
 
     class Asked(Exception):
@@ -75,25 +125,16 @@ def test_the_backward_asks_about_every_tensor_it_passes_on(monkeypatch, what):
     class Tagged(torch.Tensor):
         pass
 
-    def reached(dtype):
-        raise Asked
-
     class Elsewhere(torch.Tensor):
         def get_device(self):
             return 1
 
-    # (on the CPU, which is number -1)
-    monkeypatch.setattr(_lib, "current_gpu", lambda: -1)
-    monkeypatch.setattr(_lib, "current_stream_handle", lambda: 0)
-    monkeypatch.setattr(_lib, "lib", reached)
+    def reached(dtype):
+        raise Asked
+
+    on_the_cpu(reached)
     monkeypatch.setattr(_operator, "_TENSORS", (torch.Tensor, Elsewhere))
-    T, H, I, E, K = 6, 16, 8, 4, 2
-    bf16 = lambda *shape: torch.zeros(*shape, dtype=torch.bfloat16)
-    given = dict(x=bf16(T, H), dout=bf16(T, H), z=bf16(T * K, 2 * I), w1=bf16(E, 2 * I, H).permute(1, 2, 0),
-                 w2=bf16(E, H, I).permute(1, 2, 0), b2=bf16(E, H), has_b1=True,
-                 ints=torch.zeros(layer_call.Indices(T, E, K).words, dtype=torch.int32), freq=torch.zeros(E, dtype=torch.int32),
-                 logits=bf16(T, E), K=K, activation=ActivationType.SWIGLU, stream_id=0, loss_grad=torch.zeros(()), outside=None,
-                 chunks=0, router_w=bf16(E, H))
+    given = _arguments()[1]
     if what == "plain":
         with pytest.raises(Asked):
             layer_call.backward(**given)
