@@ -597,7 +597,7 @@ class _OneCallLayerFunction(torch.autograd.Function):
         if daux is not None:
             dlogits = torch.empty_like(logits, memory_format=torch.contiguous_format)
             run(_switch_loss_bwd, logits, freq, acc, daux.reshape(1).float().contiguous(), dlogits)
-            dlogits_outside = dlogits if dlogits_outside is None else dlogits_outside + dlogits
+            dlogits_outside = dlogits if dlogits_outside is None else dlogits + dlogits_outside  # (which may be sparse)
         return _tc_layer_backward(ctx, dout, dlogits_outside, x, router_w, w1, w2, b2, z, scores, indices, off, gidx, sidx, ridx,
                                   tok_off, K, activation_type, stream_id, x.dtype, has_b1, None, False)
 

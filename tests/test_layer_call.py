@@ -148,6 +148,28 @@ def test_the_backward_asks_about_every_tensor_it_passes_on(monkeypatch, on_the_c
             assert layer_call.backward(**{**given, name: changed(t)}) is None, name
 
 
+@pytest.mark.parametrize("sparse", [False, True])
+def test_gradients_of_the_loss_and_of_the_logits_add_up(monkeypatch, sparse):
+    """Operator by operator: the logits' own gradient may be a sparse one (an embedding lookup in the logits)."""
+    from types import SimpleNamespace
+
+    from sonicmoe import functional
+    from sonicmoe.enums import ActivationType
+
+    T, H, I, E, K = 6, 16, 8, 4, 2
+    seen = []
+    monkeypatch.setattr(functional, "run", lambda op, *args: args[-1].fill_(3.0))
+    monkeypatch.setattr(functional.layer_call, "backward", lambda *a: None)
+    monkeypatch.setattr(functional, "_tc_layer_backward", lambda ctx, dout, dlogits, *a: seen.append(dlogits))
+    ints = torch.zeros(functional.layer_call.Indices(T, E, K).words, dtype=torch.int32)
+    ctx = SimpleNamespace(cfg=(K, ActivationType.SWIGLU, 0, False), needs_input_grad=(True,) * 6, saved_tensors=(
+        torch.zeros(T, H), torch.zeros(E, H), None, torch.zeros(H, I, E), None, None, ints, torch.zeros(E, dtype=torch.int32),
+        torch.zeros(T, E)))
+    own = torch.eye(T, E)
+    functional._OneCallLayerFunction.backward(ctx, torch.zeros(T, H), own.to_sparse() if sparse else own, None, torch.ones(()))
+    assert torch.equal(seen[0], own + 3)
+
+
 def _module(T, H, I, E, K, act, bias, dtype, dev):
     from sonicmoe import MoE
     from sonicmoe.enums import ActivationType
