@@ -29,13 +29,17 @@ _KEYS = ("CUDA", "AutogradCUDA", "AutocastCUDA", "CPU", "AutogradCPU", "Autocast
 _REGISTERED = getattr(torch.library, "_impls", None)
 
 
+def _names(library: str, *names: str) -> frozenset:
+    return frozenset(f"{library}/{name}/{key}" for name in names for key in _KEYS)
+
+
 def operator(name: str, mutates_args: set[str]):
     """torch.library.custom_op in this package's namespace; the undecorated function is kept as `.body`."""
 
     def register(body):
         op = torch.library.custom_op(f"{LIBRARY_NAME}::{name}", mutates_args=mutates_args)(body)
         op.body = body
-        op.elsewhere = frozenset(f"{LIBRARY_NAME}/{name}/{key}" for key in _KEYS)
+        op.elsewhere = _names(LIBRARY_NAME, name)
         return op
 
     return register
@@ -44,6 +48,16 @@ def operator(name: str, mutates_args: set[str]):
 def elsewhere(*ops) -> frozenset:
     """The names under which somebody else may register an implementation of one of these operators."""
     return frozenset().union(*(op.elsewhere for op in ops))
+
+
+def torch_elsewhere(*names: str) -> frozenset:
+    """The same of these torch operations."""
+    return _names("aten", *names)
+
+
+def registered(names: frozenset) -> bool:
+    """Whether somebody has registered an implementation under one of these names (or nobody can say)."""
+    return _REGISTERED is None or not _REGISTERED.isdisjoint(names)
 
 
 def untraced() -> bool:
@@ -73,16 +87,16 @@ def unobserved(names: frozenset, *tensors) -> bool:
     return (
         untraced()
         and not torch.autograd._profiler_enabled()
-        and _REGISTERED is not None
-        and _REGISTERED.isdisjoint(names)
+        and not registered(names)
         and in_memory(*tensors)
     )
 
 
-def stands_in(*tensors) -> bool:
-    """Whether an operator may stand in for a torch operation on these tensors: whoever traces or transforms torch calls keeps
-    the operation, which they can see through, and so do tensors without an address to ask for.  (Profilers see the operator.)"""
-    return not torch.compiler.is_compiling() and untraced() and in_memory(*tensors)
+def stands_in(replaced: frozenset, *tensors) -> bool:
+    """Whether an operator may stand in for the operations behind `replaced` (`elsewhere`, `torch_elsewhere`) on these tensors:
+    whoever traces or transforms torch calls keeps them, and can see through them, as does who has registered an
+    implementation of one; and so do tensors without an address to ask for.  (Profilers see the operator.)"""
+    return not torch.compiler.is_compiling() and untraced() and not registered(replaced) and in_memory(*tensors)
 
 
 def run(op, *args) -> None:
@@ -102,7 +116,7 @@ def run(op, *args) -> None:
                 break
         else:
             # (a plain function put in an operator's place is called as it is)
-            if hasattr(op, "body") and _REGISTERED is not None and _REGISTERED.isdisjoint(op.elsewhere):
+            if hasattr(op, "body") and not registered(op.elsewhere):
                 try:
                     return op.body(*args)
                 except NoMemory:

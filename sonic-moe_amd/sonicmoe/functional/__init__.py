@@ -522,10 +522,19 @@ class _TCLayerFunction(torch.autograd.Function):
                                   tok_off, K, activation_type, stream_id, logits_dtype, has_b1, ctx.order, ctx.fp8_backward)
 
 
+_REDUCTION = _token_broadcast_backward
+
+
+def _dx_with_router(ctx, x, router_w, logits_dtype, K) -> bool:
+    # (a plain function put in the reduction's place is called as it is)
+    return (ctx.needs_input_grad[0] and _token_broadcast_backward is _REDUCTION
+            and router_dx_takes(x, router_w, logits_dtype, K))
+
+
 def _tc_layer_backward(ctx, dout, dlogits_outside, x, router_w, w1, w2, b2, z, scores, indices, off, gidx, sidx, ridx, tok_off,
                        K, activation_type, stream_id, logits_dtype, has_b1, order, fp8):
     T, E = x.size(0), router_w.size(0)
-    with_router = ctx.needs_input_grad[0] and router_dx_takes(x, router_w, logits_dtype, K)
+    with_router = _dx_with_router(ctx, x, router_w, logits_dtype, K)
     dx, dw1, db1, dw2, db2, ds = _experts_backward(
         dout, x, w1, w2, b2, z, scores.view(-1), off, gidx, sidx, ridx, tok_off, K, False, activation_type, stream_id,
         has_b1, order, fp8, not with_router,
@@ -579,7 +588,7 @@ class _OneCallLayerFunction(torch.autograd.Function):
         fast_router = ctx.needs_input_grad[1] and _router_wgrad_takes(x.dtype, E, x)  # (the logits have x's type)
         chunks = router_weight_grad_chunks(T, E, H) if fast_router else 0
         done = None
-        with_router = ctx.needs_input_grad[0] and router_dx_takes(x, router_w, x.dtype, K)
+        with_router = _dx_with_router(ctx, x, router_w, x.dtype, K)
         if (_down_projection_backward, _up_projection_backward, _token_broadcast_backward, _token_broadcast_backward_router,
                 _switch_loss_bwd, _router_logit_grad, _router_weight_grad, _sum_chunks) == layer_call._BACKWARD_OPERATORS:
             done = layer_call.backward(x, dout, z, w1, w2, b2, has_b1, ints, freq, logits, K, activation_type, stream_id, daux,

@@ -7,7 +7,7 @@ from typing import Optional
 import torch
 
 from .. import _lib
-from .._operator import operator, stands_in
+from .._operator import elsewhere, operator, stands_in, torch_elsewhere
 from ..enums import ACTIVATION_CODE, ActivationType
 from ..utils import expert_major_strides
 from .forward import _check_schedule_order, _elem_dtype, _gather_sum, _gemm_workspace
@@ -222,9 +222,12 @@ def _token_broadcast_backward_router(
     _lib.check(rc, "_token_broadcast_backward_router")
 
 
+_DX = elsewhere(_token_broadcast_backward) | torch_elsewhere("addmm_", "addmm", "addmm.out")
+
+
 def router_dx_takes(x: torch.Tensor, router_w: torch.Tensor, logits_dtype: torch.dtype, K: int) -> bool:
     """Whether `_token_broadcast_backward_router` forms dx, in the place of a reduction and an addmm_"""
-    return (stands_in(x, router_w) and x.dtype in (torch.bfloat16, torch.float16)
+    return (stands_in(_DX, x, router_w) and x.dtype in (torch.bfloat16, torch.float16)
             and router_w.dtype == x.dtype and logits_dtype == x.dtype and 1 <= K <= 16
             and 0 < x.size(0) < 65536 * 64 - 63  # (64 tokens to a workgroup, 65535 of them)
             and router_w.size(0) % 8 == 0 and x.size(1) % 8 == 0 and router_w.is_contiguous()

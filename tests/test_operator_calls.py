@@ -205,7 +205,7 @@ def test_kernels_in_the_place_of_torch_operations_stay_on_one_gpu(monkeypatch, g
 
     x, w = _on_gpus(monkeypatch, *gpus, current=current)
     assert unobserved(frozenset(), x, None, w) == taken
-    assert stands_in(x, w) == taken
+    assert stands_in(frozenset(), x, w) == taken
     assert router_dx_takes(x, w, x.dtype, 2) == taken
     if gpus[0] != gpus[1]:
         with pytest.raises(RuntimeError, match="one GPU"):
@@ -244,3 +244,33 @@ def test_tracers_keep_the_router_gemm(monkeypatch, tracer):
     for graph in graphs:
         called = [str(n.target) for n in graph.graph.nodes if n.op == "call_function"]
         assert "aten.mm.default" in called and not any("_router_logits" in t for t in called)
+
+
+@pytest.mark.filterwarnings("ignore:Accessing the data pointer")
+@pytest.mark.filterwarnings("ignore:Warning only once for all operators")
+@pytest.mark.parametrize("name, linear, dx", [("aten::mm", False, True), ("aten::linear", False, True), ("aten::addmm_", True, False),
+                                              ("aten::addmm.out", True, False), ("aten::tanh", True, True),
+                                              ("sonicmoe::_token_broadcast_backward", True, False)])
+def test_implementations_registered_for_what_a_kernel_stands_in_for_are_called(monkeypatch, name, linear, dx):
+    from sonicmoe._operator import stands_in
+    from sonicmoe.functional.backward import router_dx_takes
+    from sonicmoe.functional.forward import _LINEAR, router_logits_takes
+
+    x, w = _on_gpus(monkeypatch, 0, 0)
+    with torch.library._scoped_library(name.split("::")[0], "IMPL") as lib:
+        lib.impl(name.split("::")[1], lambda *args, **kwargs: pytest.fail("called"), "CUDA")
+        assert router_logits_takes(x, w) == stands_in(_LINEAR, x, w) == linear
+        assert router_dx_takes(x, w, x.dtype, 2) == dx
+    assert router_logits_takes(x, w) and router_dx_takes(x, w, x.dtype, 2)
+
+
+def test_a_function_in_the_place_of_the_reduction_is_called(monkeypatch):
+    from types import SimpleNamespace
+
+    from sonicmoe import functional
+
+    ctx = SimpleNamespace(needs_input_grad=(True,))
+    monkeypatch.setattr(functional, "router_dx_takes", lambda *args: True)
+    assert functional._dx_with_router(ctx, None, None, None, 2)
+    monkeypatch.setattr(functional, "_token_broadcast_backward", lambda *args: None)
+    assert not functional._dx_with_router(ctx, None, None, None, 2)
