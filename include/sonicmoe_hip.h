@@ -114,8 +114,8 @@ int smoe_softmax_topk_bwd(void* dlogits, int dtype, int64_t row_stride, const vo
 
 /* The whole gradient of the router logits, every element written: dlogits[t, e] = outside[t, e] (0 when outside is NULL)
  * + s_k (ds_k - sum_j ds_j s_j) where e = idx[t, k], added in fp32 and rounded once.  smoe_softmax_topk_bwd onto a zero
- * fill and an addition, in one pass.  outside has dlogits' dtype, its rows outside_stride elements apart; it is not
- * dlogits itself. */
+ * fill and an addition, in one pass.  outside has dlogits' dtype, its rows outside_stride elements apart; it may be
+ * dlogits itself, with row_stride. */
 int smoe_router_logit_grad(void* dlogits, int dtype, int64_t row_stride, const void* outside, int64_t outside_stride,
                            const float* dscores, const float* scores, const int32_t* indices, int64_t T, int E, int K,
                            void* stream);

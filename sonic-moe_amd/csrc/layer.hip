@@ -39,7 +39,7 @@ struct ForwardScratch {
 };
 
 struct BackwardScratch {
-  void *dz, *y1s, *dx_expanded, *partial, *loss_dlogits, *map, *small_map, *sorted;
+  void *dz, *y1s, *dx_expanded, *partial, *map, *small_map, *sorted;
   float *ds, *ds_partial;
   size_t sorted_bytes, total;
   BackwardScratch(void* base, int64_t T, int H, int I, int E, int K, int N1, int64_t chunks) {
@@ -50,9 +50,13 @@ struct BackwardScratch {
     sorted_bytes = (size_t)E * sizeof(int32_t);
     sorted = c.take(sorted_bytes);
     ds = (float*)c.take((size_t)TK * 4);
-    loss_dlogits = c.take((size_t)T * E * 4);
-    partial = c.take((size_t)(chunks > 1 ? chunks : 0) * E * H * 2);  // (one chunk is the gradient itself)
+    // dz is done with when the chunks of the router's weight gradient are written (one chunk is the gradient itself)
+    const size_t at_dz = c.used;
+    partial = c.take((size_t)(chunks > 1 ? chunks : 0) * E * H * 2);
+    const size_t behind_partial = c.used;
+    c.used = at_dz;
     dz = c.take((size_t)TK * N1 * 2);
+    if (c.used < behind_partial) c.used = behind_partial;
     // y1s and the score gradient's partial sums are done with when dx_expanded is written
     const size_t shared = c.used;
     y1s = c.take((size_t)TK * I * 2);
@@ -166,9 +170,9 @@ extern "C" int smoe_layer_backward(const smoe_layer_backward_args* a, void* stre
   int64_t outside_stride = a->outside_row_stride;
   if (a->loss_grad != nullptr) {
     rc = smoe_switch_loss_bwd(a->logits, (int)a->logits_dtype, a->logits_row_stride, T, E, a->freq, a->loss_acc, a->loss_grad,
-                              s.loss_dlogits, E, stream);
+                              a->dlogits, E, stream);
     if (rc) return rc;
-    outside = s.loss_dlogits;
+    outside = a->dlogits;  // (the top-K's share is added in place)
     outside_stride = E;
   }
   rc = smoe_router_logit_grad(a->dlogits, (int)a->logits_dtype, E, outside, outside_stride, s.ds, a->scores, a->indices, T, E,

@@ -139,9 +139,11 @@ __global__ __launch_bounds__(256) void softmax_topk_bwd_kernel(T* __restrict__ d
 // bytes.  Otherwise they are read and written one by one and lie `pieces` apart, so that neighbouring lanes have
 // neighbouring columns; still VEC to a thread, because the search costs the same for one column as for eight (E = 100,
 // K = 5, T = 40960, bf16: three launches 12.8 us, one column to a thread 32, eight adjacent ones 15.2, eight apart 12.6).
+// outside may be dlogits itself, with the same stride: a thread reads its columns before it writes them (and what it reads of
+// another's, past the end of a row, it does not use).
 template <typename T, int VEC, bool WIDE>
-__global__ __launch_bounds__(256) void router_logit_grad_kernel(T* __restrict__ dlogits, int64_t row_stride,
-                                                                const T* __restrict__ outside, int64_t outside_stride,
+__global__ __launch_bounds__(256) void router_logit_grad_kernel(T* dlogits, int64_t row_stride,
+                                                                const T* outside, int64_t outside_stride,
                                                                 const float* __restrict__ dscores,
                                                                 const float* __restrict__ scores,
                                                                 const int32_t* __restrict__ indices, int64_t Trows, int E,

@@ -20,8 +20,8 @@ from . import backward as _b
 from . import forward as _f
 
 # All of a step's operators run in one call, so nothing it needs for a while can be given back in between: the gathered
-# rows of both GEMMs are held while the output is written.  Up to this many bytes of them that is no matter; beyond it a
-# step takes milliseconds, to which the calls (0.1 ms) add nothing, and memory is what counts.
+# rows of both GEMMs are held while the output is written, the logits while all gradients are.  Up to this many bytes of them
+# that is no matter; beyond it a step takes milliseconds, to which the calls (0.1 ms) add nothing, and memory is what counts.
 MAX_TRANSIENT_BYTES = 1 << 30
 
 _FORWARD = struct.Struct("33q")
@@ -94,7 +94,7 @@ def takes(x, router_w, w1, b1, w2, b2, K: int, activation, stream_id: int, names
     I = w2.size(1)
     N1 = 2 * I if is_glu(activation) else I
     if not (
-        T > 0 and 0 < K <= E and T * K * (H + I) * 2 <= MAX_TRANSIENT_BYTES
+        T > 0 and 0 < K <= E and (T * K * (H + I) + T * E) * 2 <= MAX_TRANSIENT_BYTES
         and router_w.size(1) == H and w1.shape == (N1, H, E) and w2.shape == (H, I, E)
         and w1.stride(1) == 1 and w2.stride(1) == 1
         and x.data_ptr() != 0 and w1.data_ptr() != 0 and w2.data_ptr() != 0 and router_w.data_ptr() != 0

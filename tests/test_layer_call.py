@@ -61,6 +61,20 @@ def test_what_the_layer_keeps_for_its_backward(monkeypatch, with_loss):
     assert asked == [(with_loss, with_loss)]
 
 
+@pytest.mark.parametrize("T, H, I, E, K, chunks", [(300000, 128, 64, 1024, 1, 4), (65536, 768, 256, 4096, 1, 8),
+                                                   (6001, 1536, 256, 128, 8, 12), (64, 512, 64, 4096, 2, 0)])
+def test_scratch_of_the_backward_does_not_grow_with_the_logits(T, H, I, E, K, chunks):
+    """dz or the chunks of the router's gradient, y1 or dx_expanded beside it; the loss's share of the logits' gradient is
+    formed where that gradient goes."""
+    from sonicmoe import _lib
+
+    need = _lib.lib().smoe_layer_backward_workspace_bytes(T, H, I, E, K, 0, chunks)
+    TK = T * K
+    rows = max(TK * 2 * I, chunks * E * H) * 2 + TK * max(2 * H, 2 * I + 4 * _lib.lib().smoe_dz_partial_cols(I))
+    small = 2 * _lib.lib().smoe_gemm_workspace_bytes(TK, E) + 4 * (TK + E)
+    assert need <= rows + small + 8 * 256
+
+
 @pytest.fixture
 def on_the_cpu(monkeypatch):
     """layer_call with CPU tensors (device number -1), as far as the library: on_the_cpu(library)"""
@@ -295,6 +309,31 @@ def test_functional_forms(dev, monkeypatch, case):
     calls = _both(monkeypatch, step)
     assert calls[0] == ("forward", True)
     assert all(done == (case != "logits transposed") for name, done in calls[1:]) and len(calls) == 2 + (case == "twice")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(20000, 128, 64, 1024, 1), (20000, 128, 64, 1000, 2), (2000, 1024, 64, 16, 8)])
+def test_memory_of_a_step(dev, monkeypatch, shape):
+    """What the one call holds longer than the operators is counted: the rows of both GEMMs, and the logits."""
+    T, H, I, E, K = shape
+    moe, x, dy = _module(*shape, "swiglu", False, torch.bfloat16, dev)
+    xx = x.clone().requires_grad_()
+    peaks = []
+
+    def step():
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        out, aux = moe(xx)
+        grads = torch.autograd.grad([out, aux], [xx, *moe.parameters()], grad_outputs=[dy, torch.tensor(0.3, device=dev)])
+        peaks.append(torch.cuda.max_memory_allocated() - before)
+        return [out.detach(), aux.detach(), *grads]
+
+    step()  # (workspaces that libraries keep)
+    peaks.clear()
+    _both(monkeypatch, step)
+    # (sizes are rounded up to 512 bytes each, large ones to 2 MiB)
+    assert peaks[0] - peaks[1] <= (T * K * (H + I) + T * E) * 2 + (16 << 20), peaks
 
 
 @pytest.mark.gpu
