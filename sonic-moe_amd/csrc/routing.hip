@@ -14,10 +14,10 @@ namespace smoe {
 // One row is owned by a group of G consecutive lanes (G a power of two <= 64); lane g of the group holds the
 // VPL consecutive columns [g*VPL, (g+1)*VPL) as keys
 //     key = (order-preserving image of the value's bits) << W | (2^W - 1 - column)
-// with W = 32 for fp32 and W = 16 for the 16-bit types, so that the maximum key is the largest value and, among equal
-// values, the lowest column.  K rounds of "group arg-max, then retire the winner" give the winners in descending order.
-// A round is a chain of maxima, one instruction each on 32-bit keys and three on 64-bit ones, and the winners' exponentials
-// are taken behind the rounds (one row, E = 128, K = 8: 3.0 us; 40960 rows, E = 256: 22).
+// with W = 32 for fp32 (two words) and W = 16 for the 16-bit types, so that the maximum key is the largest value and, among
+// equal values, the lowest column.  K rounds of "group arg-max, then retire the winner" give the winners in descending order.
+// A round is a chain of maxima, and the winners' exponentials are taken behind the rounds (bf16, one row, E = 128, K = 8:
+// 3.8 us; 40960 rows, E = 256: 18; fp32 5.2 and 29).
 
 template <typename T, int VPL>
 __global__ __launch_bounds__(256) void topk_softmax_kernel(const T* __restrict__ logits, int64_t row_stride,
@@ -48,7 +48,7 @@ __global__ __launch_bounds__(256) void topk_softmax_kernel(const T* __restrict__
     const int col = g * VPL + i;
     // 0 = retired / out of range: below every real key (real keys have a non-zero column part)
     const uint32_t v = opaque(bits[i]);
-    key[i] = col < E ? TK::make(v, col) : 0;
+    key[i] = col < E ? TK::make(v, col) : TK::none();
   }
 
   pick_winners<TK>(key, G, g, lane_in_block & 63, row_ok, K, do_softmax != 0, scores + rrow * K, indices + rrow * K, nullptr);
@@ -57,11 +57,13 @@ __global__ __launch_bounds__(256) void topk_softmax_kernel(const T* __restrict__
 template <typename T>
 static int launch_topk(const void* logits, int64_t T_, int E, int K, int64_t row_stride, float* scores,
                        int32_t* indices, int softmax, uint32_t clear_mask, hipStream_t st) {
-  // Columns per lane.  With 4 a round is a short chain and many lanes run; with 16 it takes fewer instructions in all, which
-  // counts once the chip is full.  The two meet near T E K = 2^25; us, 16 / 4 columns, bf16: E = 128, K = 8 256 rows 5.5/3.4,
-  // 8192 5.7/4.6, 40960 13.1/12.4; E = 256, K = 8 1024 rows 5.6/3.5, 16384 11.1/11.0, 40960 21.8/23.1; K = 16 4096 rows
-  // 7.5/6.6, 16384 13.5/16.8.  (64-bit keys go through LDS from lane to lane: as few lanes as possible.)
-  const int cols = sizeof(T) == 2 && T_ * E <= (1ll << 25) / K ? 4 : 16;
+  // Columns per lane.  With few a round is a short chain and many lanes run; with many it takes fewer instructions in all,
+  // which counts once the chip is full.  us, 4 / 8 / 16 columns: bf16 E = 128, K = 8 8192 rows 5.0/5.3/6.2, 16384 7.0/6.7/8.2,
+  // 40960 13.0/11.2/14.1; E = 100, K = 5 8192 4.9/5.1/4.7, 40960 11.4/9.7/8.4; E = 256, K = 16 4096 7.3/7.1/8.1, 40960
+  // 38/27/27.  fp32, whose keys are two words, E = 128, K = 8 8192 7.7/7.8/9.1, 16384 11.1/10.5/11.3, 40960 22/19/18;
+  // E = 256, K = 16 4096 13/12/14, 40960 74/53/45.
+  const int64_t logits_count = T_ * E;
+  const int cols = logits_count <= 1 << 20 ? 4 : sizeof(T) == 2 || logits_count <= 1 << 21 ? 8 : 16;
   int G = 1;
   while (G < 64 && G * cols < E) G <<= 1;
   int vpl = 1;

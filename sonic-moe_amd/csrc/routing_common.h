@@ -50,13 +50,6 @@ SMOE_DEV float wave_sum(float v) {
 SMOE_DEV uint32_t orderable(uint32_t bits) { return bits ^ ((bits >> 31) ? 0xffffffffu : 0x80000000u); }
 SMOE_DEV uint32_t unorderable(uint32_t o) { return o ^ ((o >> 31) ? 0x80000000u : 0xffffffffu); }
 
-SMOE_DEV uint64_t shfl_xor_u64(uint64_t v, int mask) {
-  uint32_t lo = (uint32_t)v, hi = (uint32_t)(v >> 32);
-  lo = __shfl_xor(lo, mask, 64);
-  hi = __shfl_xor(hi, mask, 64);
-  return ((uint64_t)hi << 32) | lo;
-}
-
 template <typename T>
 SMOE_DEV uint32_t load_as_f32_bits(const T* p);
 template <>
@@ -76,22 +69,33 @@ template <typename T>
 struct TopkKey;
 template <>
 struct TopkKey<float> {
-  typedef uint64_t Key;
+  // Two words, compared one after the other.  As one 64-bit key a maximum was a compare and two selects, each waiting for the
+  // one before, and went from lane to lane through LDS; us, that / this: E = 16, K = 16, 8192 rows 16.8/10.0; E = 256, K = 16
+  // one row 17.7/8.3, 8192 rows 26.6/16.7; E = 4096, K = 32, 1000 rows 104/58.
+  struct Key {
+    uint32_t hi, lo;
+  };
   static __device__ __forceinline__ uint32_t load(const float* p, uint32_t clear_mask) {
     return __float_as_uint(*p) & clear_mask;
   }
-  static __device__ __forceinline__ Key make(uint32_t bits, int col) {
-    return ((uint64_t)orderable(bits) << 32) | (uint64_t)(0xffffffffu - (uint32_t)col);
-  }
-  static __device__ __forceinline__ float value(Key k) { return __uint_as_float(unorderable((uint32_t)(k >> 32))); }
-  static __device__ __forceinline__ int column(Key k) { return (int)(0xffffffffu - (uint32_t)k); }
-  static __device__ __forceinline__ Key max_over(Key k, int G) {
-    for (int m = 1; m < G; m <<= 1) {
-      const Key o = shfl_xor_u64(k, m);
-      k = o > k ? o : k;
+  static __device__ __forceinline__ Key make(uint32_t bits, int col) { return {orderable(bits), 0xffffffffu - (uint32_t)col}; }
+  static __device__ __forceinline__ Key none() { return {0, 0}; }
+  static __device__ __forceinline__ float value(Key k) { return __uint_as_float(unorderable(k.hi)); }
+  static __device__ __forceinline__ int column(Key k) { return (int)(0xffffffffu - k.lo); }
+  template <int COLS>
+  static __device__ __forceinline__ Key best(const Key (&key)[COLS], int G) {
+    uint32_t hi = key[0].hi, lo = 0;
+#pragma unroll
+    for (int i = 1; i < COLS; i++) hi = key[i].hi > hi ? key[i].hi : hi;
+    hi = group_max(hi, G);
+#pragma unroll
+    for (int i = 0; i < COLS; i++) {
+      const uint32_t c = key[i].hi == hi ? key[i].lo : 0;
+      lo = c > lo ? c : lo;
     }
-    return k;
+    return {hi, group_max(lo, G)};
   }
+  static __device__ __forceinline__ bool same(Key a, Key b) { return a.lo == b.lo; }  // (columns of a row differ)
 };
 // (clearing the low bits of the fp32 image, log2(E) <= 12 of them, does not touch a 16-bit value)
 template <typename T>
@@ -106,7 +110,15 @@ struct TopkKey16 {
     return __uint_as_float(load_as_f32_bits<T>((const T*)&bits));
   }
   static __device__ __forceinline__ int column(Key k) { return (int)(0xffffu - (k & 0xffffu)); }
-  static __device__ __forceinline__ Key max_over(Key k, int G) { return group_max(k, G); }
+  static __device__ __forceinline__ Key none() { return 0; }
+  template <int COLS>
+  static __device__ __forceinline__ Key best(const Key (&key)[COLS], int G) {
+    Key k = key[0];
+#pragma unroll
+    for (int i = 1; i < COLS; i++) k = key[i] > k ? key[i] : k;
+    return group_max(k, G);
+  }
+  static __device__ __forceinline__ bool same(Key a, Key b) { return a == b; }
 };
 template <>
 struct TopkKey<uint16_t> : TopkKey16<uint16_t> {};
@@ -124,14 +136,11 @@ SMOE_DEV void pick_winners(typename Top::Key (&key)[COLS], int G, int g, int lan
   float vmax = 0.f, esum = 0.f;
   for (int r0 = 0; r0 < K; r0 += G) {
     const int n = K - r0 < G ? K - r0 : G;
-    Key mine = 0;
+    Key mine = Top::none();
     for (int r = 0; r < n; r++) {
-      Key best = key[0];
+      const Key best = Top::best(key, G);
 #pragma unroll
-      for (int i = 1; i < COLS; i++) best = key[i] > best ? key[i] : best;
-      best = Top::max_over(best, G);
-#pragma unroll
-      for (int i = 0; i < COLS; i++) key[i] = key[i] == best ? 0 : key[i];
+      for (int i = 0; i < COLS; i++) key[i] = Top::same(key[i], best) ? Top::none() : key[i];
       mine = g == r ? best : mine;
     }
     float out = Top::value(mine);

@@ -51,6 +51,32 @@ def test_topk_softmax_matches_oracle(dev, T, E, K, dtype):
     np.testing.assert_array_equal(v, v_ref)
 
 
+# columns per lane: 4 up to 2^20 logits, then 8, of fp32 16 above 2^21; more winners than lanes of a row, one lane, padded lanes
+@pytest.mark.parametrize("T, E, K", [(1, 1, 1), (8192, 128, 8), (8193, 128, 8), (16384, 128, 3), (16385, 128, 3), (65537, 16, 16),
+                                     (21001, 100, 64), (30000, 72, 4), (5003, 257, 33), (600, 4096, 5)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
+def test_topk_columns_per_lane(dev, T, E, K, dtype):
+    """Bit for bit the first K of a row sorted by the values' bits and, among equal ones, by column: ties, infinities, the
+    lowest value as a mask, NaN and both zeros included."""
+    g = torch.Generator().manual_seed(T + E)
+    logits = (torch.randn(T, E, generator=g) * 2).round(decimals=1).to(dtype)
+    special = torch.tensor([float("inf"), -float("inf"), float("nan"), -float("nan"), 0.0, -0.0, torch.finfo(dtype).min]).to(dtype)
+    where = torch.randint(0, 40, (T, E), generator=g)
+    logits = torch.where(where < len(special), special[where.clamp(max=len(special) - 1)], logits)
+    logits[::7] = torch.finfo(dtype).min
+    if dtype == torch.float32:
+        bits = logits.numpy().view(np.uint32) & ~np.uint32((1 << (E - 1).bit_length()) - 1)
+        numbers = bits.view(np.float32)
+    else:  # (of the 16 bits: conversions on the CPU keep a NaN's sign or do not)
+        bits = logits.view(torch.int16).numpy().view(np.uint16).astype(np.uint32) << 16
+        numbers = logits.float().numpy()
+    order = np.where(bits >> 31, ~bits, bits | np.uint32(1 << 31)).astype(np.int64)
+    want = np.argsort(-order, axis=1, kind="stable")[:, :K]
+    values, indices = _topk(dev, logits.to(dev), K, softmax=False)
+    np.testing.assert_array_equal(indices, want)
+    np.testing.assert_array_equal(values, np.take_along_axis(numbers, want, 1))
+
+
 def test_topk_fp32_low_bit_ties(dev):
     """fp32 logits that differ only in the mantissa bits the reference overwrites must tie towards the lower column."""
     E, K = 128, 4
