@@ -329,12 +329,31 @@ def _router_logits(x: torch.Tensor, router_w: torch.Tensor, logits: torch.Tensor
     _lib.check(rc, "_router_logits")
 
 
-# Where the router GEMM is `_router_logits` and not the library's.  The library's call takes 20 us on the host.  Up to 64
-# tokens a layer waits for its launches, and there the kernel is half of a fused routing (csrc/route_few.hip); up to 1024 that
-# holds for the smallest layers, whose few experts leave the kernel one workgroup per 16 tokens (6.4 us at E = 8, H = 512,
-# 3.5 the library's); with more tokens or experts the GPU is busy, and the library's kernel is the faster one: 777 tokens,
-# E = 48, H = 1472 9.1 against 6.0 us, 1024 tokens, E = 128, H = 4096 19 against 8.
-ROUTER_LOGITS_MAX_TOKENS, ROUTER_LOGITS_MAX_TOKENS_FEW_EXPERTS, FEW_EXPERTS = 64, 1024, 16
+# Where the router GEMM is `_router_logits` and not the library's, whose call takes 20 us on the host.  Passes of whole layers
+# (H, I, E, K), eager and replayed from a graph, us, library / kernel:
+#   Up to 64 tokens and 256 experts the kernel is half of a fused routing (csrc/route_few.hip): (4096, 1024, 128, 8) 16 tokens
+#   387/370 and 385/372; (8192, 256, 64, 4) 64 tokens 181/171 and 180/170.
+#   With more experts it stands alone, 16 tokens x 16 experts to a workgroup, and pays while every compute unit has one at
+#   most and a part of the contraction is one batch of loads (H <= 4096): (4096, 64, 1024, 8) 64 tokens 314/309 and 313/309;
+#   (512, 64, 2048, 8) 16 tokens 78/69 and 64/68, 64 tokens (512 workgroups) 113/120 and 112/119; (512, 64, 4096, 8) 16 tokens
+#   100/102, 64 172/190; (8192, 64, 512, 8) 16 tokens 146/151.
+#   With few experts there are few workgroups, and the layer waits for its calls up to a few thousand tokens: (512, 256, 8, 2)
+#   1024 tokens 74/51 and 39/42, with backward 321/288 and 128/129; 4096 73/53 and 50/52; (1024, 256, 16, 4) 3000 tokens 74/72
+#   and 69/72, 4096 90/92; (4096, 1024, 16, 2) 2048 tokens 189/184 and 189/185, 8192 444/452; (8192, 512, 16, 2) 1024 tokens
+#   176/182.  (What the kernel costs there shows in a replay alone, which runs it all the same: it gives the eager call's
+#   bits.)
+ROUTER_LOGITS_MAX_TOKENS, ROUTER_LOGITS_MAX_EXPERTS, ROUTER_LOGITS_MAX_TILES, FUSED_MAX_EXPERTS = 64, 2048, 256, 256
+ROUTER_LOGITS_MAX_TOKENS_FEW_EXPERTS, FEW_EXPERTS, ROUTER_LOGITS_MAX_HIDDEN = 2048, 16, 4096
+
+
+def _router_logits_pays(T: int, H: int, E: int) -> bool:
+    if T <= ROUTER_LOGITS_MAX_TOKENS and E <= FUSED_MAX_EXPERTS:
+        return True
+    if T <= ROUTER_LOGITS_MAX_TOKENS:
+        few = E <= ROUTER_LOGITS_MAX_EXPERTS and (T + 15) // 16 * ((E + 15) // 16) <= ROUTER_LOGITS_MAX_TILES
+    else:
+        few = E <= FEW_EXPERTS and T <= ROUTER_LOGITS_MAX_TOKENS_FEW_EXPERTS
+    return few and H <= ROUTER_LOGITS_MAX_HIDDEN
 
 
 _LINEAR = torch_elsewhere("linear", "matmul", "mm")
@@ -343,9 +362,9 @@ _LINEAR = torch_elsewhere("linear", "matmul", "mm")
 def router_logits_takes(x: torch.Tensor, router_w: torch.Tensor) -> bool:
     """Whether `_router_logits` takes these tensors, and is the better one; for tensors that it may be given (`stands_in`)."""
     return (x.dtype == router_w.dtype and x.dtype in (torch.bfloat16, torch.float16) and x.dim() == 2
-            and not registered(_LINEAR) and 0 < x.size(0) <= (ROUTER_LOGITS_MAX_TOKENS_FEW_EXPERTS if router_w.size(0) <= FEW_EXPERTS
-                                  else ROUTER_LOGITS_MAX_TOKENS)
-            and x.size(1) % 32 == 0 and x.size(1) == router_w.size(1) and x.is_contiguous() and router_w.is_contiguous()
+            and x.size(0) > 0 and _router_logits_pays(x.size(0), x.size(1), router_w.size(0))
+            and not registered(_LINEAR) and x.size(1) % 32 == 0 and x.size(1) == router_w.size(1)
+            and x.is_contiguous() and router_w.is_contiguous()
             and x.data_ptr() % 16 == 0 and router_w.data_ptr() % 16 == 0 and not torch.is_autocast_enabled("cuda"))
 
 

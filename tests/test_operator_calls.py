@@ -274,3 +274,14 @@ def test_a_function_in_the_place_of_the_reduction_is_called(monkeypatch):
     assert functional._dx_with_router(ctx, None, None, None, 2)
     monkeypatch.setattr(functional, "_token_broadcast_backward", lambda *args: None)
     assert not functional._dx_with_router(ctx, None, None, None, 2)
+
+
+@pytest.mark.parametrize("T, H, E, taken", [
+    (0, 512, 8, False), (1, 32, 1, True), (64, 8192, 256, True), (65, 512, 17, False), (64, 4096, 1024, True),
+    (64, 4096, 1025, False), (32, 4096, 2048, True), (33, 512, 2048, False), (1, 512, 2049, False), (1, 4128, 257, False),
+    (2048, 4096, 16, True), (2049, 512, 16, False), (65, 4128, 16, False), (64, 500, 8, False)])
+def test_sizes_of_the_router_kernel(T, H, E, taken):
+    from sonicmoe.functional.forward import router_logits_takes
+
+    x, w = (torch.empty(n, H, dtype=torch.bfloat16, device="meta") for n in (T, E))
+    assert router_logits_takes(x, w) == taken
