@@ -59,8 +59,9 @@ __global__ __launch_bounds__(512) void gather_sum_kernel(const uint16_t* __restr
 // A workgroup owns 64 tokens x 128 columns, a wavefront 16 of the tokens: the product runs on matrix instructions, Wr through
 // LDS 64 experts at a time (read transposed), dlogits straight into registers; the fp32 tile then goes through LDS into the
 // layout of the row loads, 16 lanes to the 256 bytes of a row.  Bound by the gathered rows like gather_sum_kernel.
-// gather_sum_kernel and a library GEMM that adds onto dx / this kernel, us: 1024 x 1536, E = 128, K = 8 25/12; 6001 x 1536
-// 52/40; 40960 x 768 131/113; 32768 x 4096 553/487; 4096 x 4096, E = 256, K = 16 121/121.  Distance from 64 bits 2.3e-3 -> 1.7e-3.
+// gather_sum_kernel and a library GEMM that adds onto dx / this kernel, us: 1024 x 1536, E = 128, K = 8 13.4/12.7; 6001 x 1536
+// 53/42; 40960 x 768 131/113; 32768 x 4096 557/495; 4096 x 4096, E = 256, K = 16 121/121 (the caller draws the line).  Distance
+// from 64 bits 2.3e-3 -> 1.7e-3.
 constexpr int GR_T = 64, GR_C = 128, GR_E = 64, GR_PITCH = GR_C + 4, GR_MAX_K = 16;
 
 template <int ROWS>

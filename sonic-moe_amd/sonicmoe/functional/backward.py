@@ -224,14 +224,24 @@ def _token_broadcast_backward_router(
 
 _DX = elsewhere(_token_broadcast_backward) | torch_elsewhere("addmm_", "addmm", "addmm.out")
 
+# Where dx is formed by `_token_broadcast_backward_router` and not by the reduction and addmm_ (20 us of host time).  Its
+# workgroups read all of the router's weights and add a token's K rows in batches of eight, so the line is by E and E K.
+# Kernels alone, us, two launches / one: E = 128, K = 8, H = 1536 64 tokens 8.6/10.8, 1024 13.4/12.7, 6001 53.5/41.5; E = 256,
+# K = 8, H = 4096 64 tokens 9.5/12.2, 6001 111/104; E = 512, K = 2, H = 4096 64 10.4/13.0, 32768 338/338; above it E = 256,
+# K = 16, H = 1536 64 10.4/18.3, 6001 72/78; E = 512, K = 8, H = 1536 64 10.4/14.6, 6001 52/56; E = 1024, K = 2, H = 4096
+# 32768 424/525; E = 4096, K = 1 972/1643.  With few tokens the launch is a chain of latencies, but there a step waits for its
+# calls: (H, I, E, K) = (512, 256, 128, 8), 256 tokens, forward and backward 331/306, replayed from a graph 152/155.
+ROUTER_DX_MAX_E, ROUTER_DX_MAX_EK = 512, 2048
+
 
 def router_dx_takes(x: torch.Tensor, router_w: torch.Tensor, logits_dtype: torch.dtype, K: int) -> bool:
     """Whether `_token_broadcast_backward_router` forms dx, in the place of a reduction and an addmm_"""
+    E = router_w.size(0)
     return (stands_in(_DX, x, router_w) and x.dtype in (torch.bfloat16, torch.float16)
             and router_w.dtype == x.dtype and logits_dtype == x.dtype and 1 <= K <= 16
+            and E <= ROUTER_DX_MAX_E and E * K <= ROUTER_DX_MAX_EK
             and 0 < x.size(0) < 65536 * 64 - 63  # (64 tokens to a workgroup, 65535 of them)
-            and router_w.size(0) % 8 == 0 and x.size(1) % 8 == 0 and router_w.is_contiguous()
-            and router_w.data_ptr() % 16 == 0)
+            and E % 8 == 0 and x.size(1) % 8 == 0 and router_w.is_contiguous() and router_w.data_ptr() % 16 == 0)
 
 
 @operator("_softmax_topk_bwd", mutates_args={"dlogits_full"})

@@ -285,3 +285,17 @@ def test_sizes_of_the_router_kernel(T, H, E, taken):
 
     x, w = (torch.empty(n, H, dtype=torch.bfloat16, device="meta") for n in (T, E))
     assert router_logits_takes(x, w) == taken
+
+
+@pytest.mark.filterwarnings("ignore:Accessing the data pointer")
+@pytest.mark.parametrize("E, K, taken", [(8, 1, True), (128, 16, True), (136, 16, False), (256, 8, True), (512, 4, True),
+                                         (512, 5, False), (520, 1, False), (8, 17, False), (12, 2, False)])
+def test_sizes_of_the_dx_kernel(monkeypatch, E, K, taken):
+    from sonicmoe import _operator
+    from sonicmoe.functional.backward import router_dx_takes
+
+    monkeypatch.setattr(_operator, "_TENSORS", (FakeTensor,))
+    monkeypatch.setattr(_lib, "current_gpu", lambda: 0)
+    with FakeTensorMode():
+        x, w = (torch.empty(n, 128, dtype=torch.bfloat16, device="cuda:0") for n in (8, E))
+    assert router_dx_takes(x, w, x.dtype, K) == taken
