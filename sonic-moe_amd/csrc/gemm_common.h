@@ -1339,6 +1339,23 @@ static inline int tile_map_in(GemmScratch& ws, const int32_t* off, const int32_t
   return launch_build_tile_map(off, order, E, BM, tm, st);
 }
 
+// Sizes that the 16-bit grouped GEMMs take
+static inline int check_gemm_sizes(int64_t TK, int H, int I, int E, const char* who) {
+  SMOE_REQUIRE(TK >= 0 && TK < (1ll << 31), SMOE_ERR_INVALID, "%s: TK out of range", who);
+  SMOE_REQUIRE(E >= 1, SMOE_ERR_INVALID, "%s: E must be >= 1", who);
+  SMOE_REQUIRE(H >= 64 && H % 64 == 0, SMOE_ERR_UNSUPPORTED, "%s: H=%d must be a multiple of 64", who, H);
+  SMOE_REQUIRE(I >= 64 && I % 64 == 0, SMOE_ERR_UNSUPPORTED, "%s: I=%d must be a multiple of 64", who, I);
+  return SMOE_OK;
+}
+
+static inline int check_gemm_call(int64_t TK, int H, int I, int E, const void* ws, size_t ws_bytes, const char* who) {
+  const int rc = check_gemm_sizes(TK, H, I, E, who);
+  if (rc) return rc;
+  SMOE_REQUIRE(ws != nullptr && ws_bytes >= smoe_gemm_workspace_bytes(TK, E), SMOE_ERR_WORKSPACE,
+               "%s: workspace too small", who);
+  return SMOE_OK;
+}
+
 // The entry points' bodies on such a scratch (their own checks of the workspace's size are the entry points')
 int up_projection_forward(const void* x, const void* w1, int64_t w1_stride_e, int64_t w1_stride_row, const void* b1, void* z,
                           void* y1, const int32_t* off, const int32_t* expert_schedule_order, const int32_t* x_gather_idx,

@@ -643,29 +643,13 @@ int launch_dx(const void* dz, const void* w1, int64_t w1_stride_e, int64_t w1_st
 
 using namespace smoe;
 
-static int check_sizes(int64_t TK, int H, int I, int E, const char* who) {
-  SMOE_REQUIRE(TK >= 0 && TK < (1ll << 31), SMOE_ERR_INVALID, "%s: TK out of range", who);
-  SMOE_REQUIRE(E >= 1, SMOE_ERR_INVALID, "%s: E must be >= 1", who);
-  SMOE_REQUIRE(H >= 64 && H % 64 == 0, SMOE_ERR_UNSUPPORTED, "%s: H=%d must be a multiple of 64", who, H);
-  SMOE_REQUIRE(I >= 64 && I % 64 == 0, SMOE_ERR_UNSUPPORTED, "%s: I=%d must be a multiple of 64", who, I);
-  return SMOE_OK;
-}
-
-static int check_bwd(int64_t TK, int H, int I, int E, const void* ws, size_t ws_bytes, const char* who) {
-  const int rc = check_sizes(TK, H, I, E, who);
-  if (rc) return rc;
-  SMOE_REQUIRE(ws != nullptr && ws_bytes >= smoe_gemm_workspace_bytes(TK, E), SMOE_ERR_WORKSPACE,
-               "%s: workspace too small", who);
-  return SMOE_OK;
-}
-
 int smoe::down_projection_backward(const void* dout, const void* z, const void* w2, int64_t w2_stride_e,
                                    int64_t w2_stride_row, const void* b2, void* dw2, int64_t dw2_stride_e,
                                    int64_t dw2_stride_row, void* db2, void* dz, void* y1s, float* ds, float* ds_partial,
                                    const float* scores, const int32_t* off, const int32_t* expert_schedule_order,
                                    const int32_t* x_gather_idx, const int32_t* s_scatter_idx, int64_t T, int64_t TK, int H,
                                    int I, int E, int activation, GemmScratch& ws, void* stream) {
-  int rc = check_sizes(TK, H, I, E, "down_projection_backward");
+  int rc = check_gemm_sizes(TK, H, I, E, "down_projection_backward");
   if (rc) return rc;
   SMOE_REQUIRE(activation >= SMOE_ACT_SWIGLU && activation <= SMOE_ACT_SILU, SMOE_ERR_INVALID,
                "down_projection_backward: unknown activation code %d", activation);
@@ -727,7 +711,7 @@ extern "C" int smoe_down_projection_backward(const void* dout, const void* z, co
                                              const int32_t* expert_schedule_order, const int32_t* x_gather_idx,
                                              const int32_t* s_scatter_idx, int64_t T, int64_t TK, int H, int I, int E,
                                              int activation, void* workspace, size_t workspace_bytes, void* stream) {
-  int rc = check_bwd(TK, H, I, E, workspace, workspace_bytes, "down_projection_backward");
+  int rc = check_gemm_call(TK, H, I, E, workspace, workspace_bytes, "down_projection_backward");
   if (rc) return rc;
   GemmScratch ws(workspace, workspace_bytes);
   return smoe::down_projection_backward(dout, z, w2, w2_stride_e, w2_stride_row, b2, dw2, dw2_stride_e, dw2_stride_row, db2,
@@ -740,7 +724,7 @@ int smoe::up_projection_backward(const void* x, const void* w1, int64_t w1_strid
                                  const int32_t* off, const int32_t* expert_schedule_order, const int32_t* x_gather_idx,
                                  int64_t T, int64_t TK, int H, int I, int E, int activation, GemmScratch& ws,
                                  void* stream) {
-  int rc = check_sizes(TK, H, I, E, "up_projection_backward");
+  int rc = check_gemm_sizes(TK, H, I, E, "up_projection_backward");
   if (rc) return rc;
   SMOE_REQUIRE(activation >= SMOE_ACT_SWIGLU && activation <= SMOE_ACT_SILU, SMOE_ERR_INVALID,
                "up_projection_backward: unknown activation code %d", activation);
@@ -794,7 +778,7 @@ extern "C" int smoe_up_projection_backward(const void* x, const void* w1, int64_
                                            const int32_t* expert_schedule_order, const int32_t* x_gather_idx,
                                            int64_t T, int64_t TK, int H, int I, int E, int activation, void* workspace,
                                            size_t workspace_bytes, void* stream) {
-  int rc = check_bwd(TK, H, I, E, workspace, workspace_bytes, "up_projection_backward");
+  int rc = check_gemm_call(TK, H, I, E, workspace, workspace_bytes, "up_projection_backward");
   if (rc) return rc;
   GemmScratch ws(workspace, workspace_bytes);
   return smoe::up_projection_backward(x, w1, w1_stride_e, w1_stride_row, dz, dw1, dw1_stride_e, dw1_stride_row, db1,

@@ -892,22 +892,6 @@ int dz_tile_cols() { return TileCfg<true>::BN; }
 
 using namespace smoe;
 
-static int check_sizes(int64_t TK, int H, int I, int E, const char* who) {
-  SMOE_REQUIRE(TK >= 0 && TK < (1ll << 31), SMOE_ERR_INVALID, "%s: TK out of range", who);
-  SMOE_REQUIRE(E >= 1, SMOE_ERR_INVALID, "%s: E must be >= 1", who);
-  SMOE_REQUIRE(H >= 64 && H % 64 == 0, SMOE_ERR_UNSUPPORTED, "%s: H=%d must be a multiple of 64", who, H);
-  SMOE_REQUIRE(I >= 64 && I % 64 == 0, SMOE_ERR_UNSUPPORTED, "%s: I=%d must be a multiple of 64", who, I);
-  return SMOE_OK;
-}
-
-static int check_common(int64_t TK, int H, int I, int E, const void* ws, size_t ws_bytes, const char* who) {
-  const int rc = check_sizes(TK, H, I, E, who);
-  if (rc) return rc;
-  SMOE_REQUIRE(ws != nullptr && ws_bytes >= smoe_gemm_workspace_bytes(TK, E), SMOE_ERR_WORKSPACE,
-               "%s: workspace too small", who);
-  return SMOE_OK;
-}
-
 extern "C" size_t smoe_gemm_workspace_bytes(int64_t TK, int E) {
   if (TK < 0 || E < 1) return 0;
   return tile_map_bytes(TK, E);
@@ -919,7 +903,7 @@ int smoe::up_projection_forward(const void* x, const void* w1, int64_t w1_stride
                                 void* z, void* y1, const int32_t* off, const int32_t* expert_schedule_order,
                                 const int32_t* x_gather_idx, int64_t T, int64_t TK, int H, int I, int E, int activation,
                                 GemmScratch& ws, void* stream) {
-  const int rc = check_sizes(TK, H, I, E, "up_projection_forward");
+  const int rc = check_gemm_sizes(TK, H, I, E, "up_projection_forward");
   if (rc) return rc;
   SMOE_REQUIRE(activation >= SMOE_ACT_SWIGLU && activation <= SMOE_ACT_SILU, SMOE_ERR_INVALID,
                "up_projection_forward: unknown activation code %d", activation);
@@ -955,7 +939,7 @@ extern "C" int smoe_up_projection_forward(const void* x, const void* w1, int64_t
                                           const int32_t* expert_schedule_order, const int32_t* x_gather_idx, int64_t T,
                                           int64_t TK, int H, int I, int E, int activation, void* workspace,
                                           size_t workspace_bytes, void* stream) {
-  int rc = check_common(TK, H, I, E, workspace, workspace_bytes, "up_projection_forward");
+  int rc = check_gemm_call(TK, H, I, E, workspace, workspace_bytes, "up_projection_forward");
   if (rc) return rc;
   GemmScratch ws(workspace, workspace_bytes);
   return smoe::up_projection_forward(x, w1, w1_stride_e, w1_stride_row, b1, z, y1, off, expert_schedule_order, x_gather_idx,
@@ -965,7 +949,7 @@ extern "C" int smoe_up_projection_forward(const void* x, const void* w1, int64_t
 int smoe::down_projection_forward(const void* y1, const void* w2, int64_t w2_stride_e, int64_t w2_stride_row,
                                   const void* b2, void* y2, const int32_t* off, const int32_t* expert_schedule_order,
                                   int64_t TK, int H, int I, int E, GemmScratch& ws, void* stream) {
-  const int rc = check_sizes(TK, H, I, E, "down_projection_forward");
+  const int rc = check_gemm_sizes(TK, H, I, E, "down_projection_forward");
   if (rc) return rc;
   if (TK == 0) return SMOE_OK;
   SMOE_REQUIRE(y1 && w2 && y2 && off, SMOE_ERR_INVALID, "down_projection_forward: null pointer");
@@ -993,7 +977,7 @@ extern "C" int smoe_down_projection_forward(const void* y1, const void* w2, int6
                                             const void* b2, void* y2, const int32_t* off,
                                             const int32_t* expert_schedule_order, int64_t TK, int H, int I, int E,
                                             void* workspace, size_t workspace_bytes, void* stream) {
-  int rc = check_common(TK, H, I, E, workspace, workspace_bytes, "down_projection_forward");
+  int rc = check_gemm_call(TK, H, I, E, workspace, workspace_bytes, "down_projection_forward");
   if (rc) return rc;
   GemmScratch ws(workspace, workspace_bytes);
   return smoe::down_projection_forward(y1, w2, w2_stride_e, w2_stride_row, b2, y2, off, expert_schedule_order, TK, H, I, E,
@@ -1007,7 +991,7 @@ extern "C" int smoe_down_projection_forward_combine(const void* y1, const void* 
                                                     const int32_t* x_gather_idx, const int32_t* s_scatter_idx,
                                                     int64_t T, int64_t TK, int H, int I, int E, void* workspace,
                                                     size_t workspace_bytes, void* stream) {
-  int rc = check_common(TK, H, I, E, workspace, workspace_bytes, "down_projection_forward_combine");
+  int rc = check_gemm_call(TK, H, I, E, workspace, workspace_bytes, "down_projection_forward_combine");
   if (rc) return rc;
   if (TK == 0) return SMOE_OK;
   SMOE_REQUIRE(y1 && w2 && o && scores && off && x_gather_idx && s_scatter_idx && T > 0, SMOE_ERR_INVALID,

@@ -164,33 +164,7 @@ __global__ __launch_bounds__(64 * RF_WAVES) void route_few_kernel(
   const int id = j < TK ? picks[j] : -1;
   if (id >= 0 && id < E) atomicAdd(&cursor[id], 1);
   __syncthreads();
-  // thread e: the wavefronts' counts of expert e become their starts inside the expert, the total the expert's count
-  int32_t total = 0;
-  if (tid < E) {
-#pragma unroll
-    for (int w = 0; w < RF_WAVES; w++) {
-      const int32_t n = cursors[w * E + tid];
-      cursors[w * E + tid] = total;
-      total += n;
-    }
-  }
-  int32_t upto = total;
-  for (int d = 1; d < 64; d <<= 1) {
-    const int32_t o = __shfl_up(upto, d, 64);
-    if (lane >= d) upto += o;
-  }
-  if (lane == 63) wave_total[wave] = upto;
-  __syncthreads();
-  int32_t begin = upto - total;
-  for (int w = 0; w < wave; w++) begin += wave_total[w];
-  if (tid < E) {
-    freq[tid] = total;
-    off[tid] = begin;
-    if (tid == E - 1) off[E] = begin + total;
-#pragma unroll
-    for (int w = 0; w < RF_WAVES; w++) cursors[w * E + tid] += begin;
-  }
-  __syncthreads();
+  const int32_t total = counts_to_cursors<RF_WAVES>(cursors, E, wave_total, freq, off);
   if (wave * 64 < TK)
     place_slots(id, j, j < TK, lane, nullptr, TK, Trows, E, K, ebits, cursor, gidx, sidx, ridx, tok_off);
   if (loss == nullptr) return;
@@ -202,7 +176,7 @@ __global__ __launch_bounds__(64 * RF_WAVES) void route_few_kernel(
   const float fc = tid < E ? (float)total : 0.f;
   float f = fabsf(fc), d = sum * fc;
   block_sum3(sum, f, d, scratch);
-  if (tid == 0) loss[0] = (float)E * d / (fmaxf(sum, 1e-12f) * fmaxf(f, 1e-12f));
+  if (tid == 0) loss[0] = switch_loss_value(E, sum, f, d);
 }
 
 bool route_few_takes(int64_t T, int H, int E, int K) {

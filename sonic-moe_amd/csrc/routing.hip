@@ -454,33 +454,7 @@ __global__ __launch_bounds__(64 * M1_WAVES) void meta_one_kernel(
   for (int i = 0; i < M1_STEPS; i++)
     if (ids[i] >= 0 && ids[i] < E) atomicAdd(&cursor[ids[i]], 1);
   __syncthreads();
-  // thread e: the wavefronts' counts of expert e become their starts inside the expert, the total the expert's count
-  int32_t total = 0;
-  if (tid < E) {
-#pragma unroll
-    for (int w = 0; w < M1_WAVES; w++) {
-      const int32_t n = lds[w * E + tid];
-      lds[w * E + tid] = total;
-      total += n;
-    }
-  }
-  int32_t upto = total;
-  for (int d = 1; d < 64; d <<= 1) {
-    const int32_t o = __shfl_up(upto, d, 64);
-    if (lane >= d) upto += o;
-  }
-  if (lane == 63) wave_total[wave] = upto;
-  __syncthreads();
-  int32_t begin = upto - total;
-  for (int w = 0; w < wave; w++) begin += wave_total[w];
-  if (tid < E) {
-    freq[tid] = total;
-    off[tid] = begin;
-    if (tid == E - 1) off[E] = begin + total;
-#pragma unroll
-    for (int w = 0; w < M1_WAVES; w++) lds[w * E + tid] += begin;
-  }
-  __syncthreads();
+  counts_to_cursors<M1_WAVES>(lds, E, wave_total, freq, off);
 #pragma unroll
   for (int i = 0; i < M1_STEPS; i++) {
     const int j = first + i * 64;

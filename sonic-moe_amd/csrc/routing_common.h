@@ -205,6 +205,43 @@ SMOE_DEV void place_slots(int e, int j, bool valid, int lane, const int32_t* __r
   }
 }
 
+// The step between the counts and the ranking, of one workgroup whose thread e has expert e (E <= 64 * WAVES).  cursors: WAVES x
+// E words of LDS, the wavefronts' counts, all written before; they become the positions at which each wavefront's slots of an
+// expert begin.  Counts and offsets go to freq and off; returned is the expert's count (0 past the end).  total_of: WAVES words
+// of LDS.  Begins without a barrier and ends with one.
+template <int WAVES>
+SMOE_DEV int32_t counts_to_cursors(int32_t* cursors, int E, int32_t* total_of, int32_t* __restrict__ freq,
+                                   int32_t* __restrict__ off) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int32_t total = 0;
+  if (tid < E) {
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) {
+      const int32_t n = cursors[w * E + tid];
+      cursors[w * E + tid] = total;
+      total += n;
+    }
+  }
+  int32_t upto = total;
+  for (int d = 1; d < 64; d <<= 1) {
+    const int32_t o = __shfl_up(upto, d, 64);
+    if (lane >= d) upto += o;
+  }
+  if (lane == 63) total_of[wave] = upto;
+  __syncthreads();
+  int32_t begin = upto - total;
+  for (int w = 0; w < wave; w++) begin += total_of[w];
+  if (tid < E) {
+    freq[tid] = total;
+    off[tid] = begin;
+    if (tid == E - 1) off[E] = begin + total;
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) cursors[w * E + tid] += begin;
+  }
+  __syncthreads();
+  return total;
+}
+
 // ---- softmax of a row, sums --------------------------------------------------------------------------------------------------
 template <typename T>
 SMOE_DEV float sl_load(const T* p);
@@ -277,6 +314,11 @@ SMOE_DEV void block_sum3(float& a, float& b, float& c, float* scratch /* 3 * 16 
     c += scratch[32 + w];
   }
   __syncthreads();
+}
+
+// The load-balancing loss of the sums of the softmax columns (s), of the counts (f) and of their products (d)
+SMOE_DEV float switch_loss_value(int E, float s, float f, float d) {
+  return (float)E * d / (fmaxf(s, 1e-12f) * fmaxf(f, 1e-12f));
 }
 
 // router_logits, top-K, metadata and loss of few tokens: route_few.hip

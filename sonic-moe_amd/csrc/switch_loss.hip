@@ -125,7 +125,7 @@ __global__ __launch_bounds__(VPL <= 16 ? 1024 : 256) void softmax_colsum_kernel(
   float f = fabsf(fc), d = sum * fc;
   __syncthreads();  // the columns have been read
   block_sum3(sum, f, d, sl_lds);
-  if (threadIdx.x == 0) aux[0] = (float)E * d / (fmaxf(sum, 1e-12f) * fmaxf(f, 1e-12f));
+  if (threadIdx.x == 0) aux[0] = switch_loss_value(E, sum, f, d);
 }
 
 // one workgroup of 1024 threads: acc = sum of the partials, then the scalar.  The threads form 1024 / CW slices of CW
@@ -166,7 +166,7 @@ __global__ __launch_bounds__(1024) void switch_loss_finalize_kernel(const float*
     __syncthreads();
   }
   block_sum3(s, f, d, scratch);
-  if (threadIdx.x == 0) aux[0] = (float)E * d / (fmaxf(s, 1e-12f) * fmaxf(f, 1e-12f));
+  if (threadIdx.x == 0) aux[0] = switch_loss_value(E, s, f, d);
 }
 
 template <typename T, int VPL>

@@ -1,5 +1,5 @@
-"""Routing metadata at the borders of its one-workgroup form (steps of 64 slots, 16 wavefronts, 8192 slots, 512 experts)
-and of the three passes behind it: bit for bit the stable sort of the oracle."""
+"""Routing metadata at the borders of its one-workgroup form (four steps of 64 slots to a wavefront, 16 wavefronts: 4096
+slots; 512 experts) and of the three passes behind it: bit for bit the stable sort of the oracle."""
 
 import numpy as np
 import pytest
@@ -13,7 +13,7 @@ KEYS = ("expert_frequency", "expert_frequency_offset", "x_gather_idx", "s_scatte
 
 
 @pytest.mark.parametrize("E", [1, 8, 100, 512, 513])
-@pytest.mark.parametrize("TK", [1, 63, 64, 65, 1023, 1024, 1025, 2047, 8191, 8192, 8193])
+@pytest.mark.parametrize("TK", [1, 63, 64, 65, 1023, 1024, 1025, 2047, 3072, 3073, 4095, 4096, 4097, 8191, 8192, 8193])
 def test_metadata_borders(dev, TK, E):
     from sonicmoe.functional import _build_metadata
 
