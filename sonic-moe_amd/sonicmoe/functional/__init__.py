@@ -18,9 +18,10 @@ import torch.nn.functional as F
 
 from .. import _lib
 from ..count_cumsum import count_cumsum
-from .._operator import operator, run
+from .._operator import operator, run, stands_in
 from ..enums import ActivationType, is_glu
 from .backward import (
+    ROUTER_DX,
     _down_projection_backward,
     _down_projection_weight_grad,
     _router_logit_grad,
@@ -527,8 +528,8 @@ _REDUCTION = _token_broadcast_backward
 
 def _dx_with_router(ctx, x, router_w, logits_dtype, K) -> bool:
     # (a plain function put in the reduction's place is called as it is)
-    return (ctx.needs_input_grad[0] and _token_broadcast_backward is _REDUCTION
-            and router_dx_takes(x, router_w, logits_dtype, K))
+    return (ctx.needs_input_grad[0] and _token_broadcast_backward is _REDUCTION and stands_in(ROUTER_DX, x, router_w)
+            and router_dx_takes(x, router_w, logits_dtype, K) and router_w.data_ptr() % 16 == 0)
 
 
 def _tc_layer_backward(ctx, dout, dlogits_outside, x, router_w, w1, w2, b2, z, scores, indices, off, gidx, sidx, ridx, tok_off,
@@ -588,7 +589,7 @@ class _OneCallLayerFunction(torch.autograd.Function):
         fast_router = ctx.needs_input_grad[1] and _router_wgrad_takes(x.dtype, E, x)  # (the logits have x's type)
         chunks = router_weight_grad_chunks(T, E, H) if fast_router else 0
         done = None
-        with_router = _dx_with_router(ctx, x, router_w, x.dtype, K)
+        with_router = ctx.needs_input_grad[0] and router_dx_takes(x, router_w, x.dtype, K)
         if (_down_projection_backward, _up_projection_backward, _token_broadcast_backward, _token_broadcast_backward_router,
                 _switch_loss_bwd, _router_logit_grad, _router_weight_grad, _sum_chunks) == layer_call._BACKWARD_OPERATORS:
             done = layer_call.backward(x, dout, z, w1, w2, b2, has_b1, ints, freq, logits, K, activation_type, stream_id, daux,

@@ -7,7 +7,7 @@ from typing import Optional
 import torch
 
 from .. import _lib
-from .._operator import elsewhere, operator, stands_in, torch_elsewhere
+from .._operator import elsewhere, operator, torch_elsewhere
 from ..enums import ACTIVATION_CODE, ActivationType
 from ..utils import expert_major_strides
 from .forward import _check_schedule_order, _elem_dtype, _gather_sum, _gemm_workspace
@@ -222,7 +222,8 @@ def _token_broadcast_backward_router(
     _lib.check(rc, "_token_broadcast_backward_router")
 
 
-_DX = elsewhere(_token_broadcast_backward) | torch_elsewhere("addmm_", "addmm", "addmm.out")
+# what `_token_broadcast_backward_router` stands in for
+ROUTER_DX = elsewhere(_token_broadcast_backward) | torch_elsewhere("addmm_", "addmm", "addmm.out")
 
 # Where dx is formed by `_token_broadcast_backward_router` and not by the reduction and addmm_ (20 us of host time).  Its
 # workgroups read all of the router's weights and add a token's K rows in batches of eight, so the line is by E and E K.
@@ -235,13 +236,14 @@ ROUTER_DX_MAX_E, ROUTER_DX_MAX_EK = 512, 2048
 
 
 def router_dx_takes(x: torch.Tensor, router_w: torch.Tensor, logits_dtype: torch.dtype, K: int) -> bool:
-    """Whether `_token_broadcast_backward_router` forms dx, in the place of a reduction and an addmm_"""
+    """Whether `_token_broadcast_backward_router` forms dx, in the place of a reduction and an addmm_.  For tensors
+    that it may be given (`stands_in` for ROUTER_DX, router_w 16-byte aligned)."""
     E = router_w.size(0)
-    return (stands_in(_DX, x, router_w) and x.dtype in (torch.bfloat16, torch.float16)
+    return (x.dtype in (torch.bfloat16, torch.float16)
             and router_w.dtype == x.dtype and logits_dtype == x.dtype and 1 <= K <= 16
             and E <= ROUTER_DX_MAX_E and E * K <= ROUTER_DX_MAX_EK
             and 0 < x.size(0) < 65536 * 64 - 63  # (64 tokens to a workgroup, 65535 of them)
-            and E % 8 == 0 and x.size(1) % 8 == 0 and router_w.is_contiguous() and router_w.data_ptr() % 16 == 0)
+            and E % 8 == 0 and x.size(1) % 8 == 0 and router_w.is_contiguous())
 
 
 @operator("_softmax_topk_bwd", mutates_args={"dlogits_full"})

@@ -9,7 +9,7 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
-from .._operator import operator, registered, run, stands_in, torch_elsewhere
+from .._operator import operator, run, stands_in, torch_elsewhere
 from ..enums import ACTIVATION_CODE, ActivationType
 from ..utils import expert_major_strides
 
@@ -356,21 +356,22 @@ def _router_logits_pays(T: int, H: int, E: int) -> bool:
     return few and H <= ROUTER_LOGITS_MAX_HIDDEN
 
 
-_LINEAR = torch_elsewhere("linear", "matmul", "mm")
+# what `_router_logits` stands in for
+ROUTER_LINEAR = torch_elsewhere("linear", "matmul", "mm")
 
 
 def router_logits_takes(x: torch.Tensor, router_w: torch.Tensor) -> bool:
-    """Whether `_router_logits` takes these tensors, and is the better one; for tensors that it may be given (`stands_in`)."""
+    """Whether `_router_logits` takes these tensors, and is the better one.  For tensors that it may be given (`stands_in` for
+    ROUTER_LINEAR), and outside autocast."""
     return (x.dtype == router_w.dtype and x.dtype in (torch.bfloat16, torch.float16) and x.dim() == 2
             and x.size(0) > 0 and _router_logits_pays(x.size(0), x.size(1), router_w.size(0))
-            and not registered(_LINEAR) and x.size(1) % 32 == 0 and x.size(1) == router_w.size(1)
-            and x.is_contiguous() and router_w.is_contiguous()
-            and x.data_ptr() % 16 == 0 and router_w.data_ptr() % 16 == 0 and not torch.is_autocast_enabled("cuda"))
+            and x.size(1) % 32 == 0 and x.size(1) == router_w.size(1) and x.is_contiguous() and router_w.is_contiguous()
+            and x.data_ptr() % 16 == 0 and router_w.data_ptr() % 16 == 0)
 
 
 def router_linear(x: torch.Tensor, router_w: torch.Tensor) -> torch.Tensor:
     """F.linear(x, router_w) (nothing of it is differentiated through: the layer's own nodes call it)"""
-    if not (stands_in(_LINEAR, x, router_w) and router_logits_takes(x, router_w)):
+    if not (stands_in(ROUTER_LINEAR, x, router_w) and not torch.is_autocast_enabled("cuda") and router_logits_takes(x, router_w)):
         return torch.nn.functional.linear(x, router_w)
     logits = torch.empty(x.size(0), router_w.size(0), dtype=x.dtype, device=x.device)
     run(_router_logits, x, router_w, logits)

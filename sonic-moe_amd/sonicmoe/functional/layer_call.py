@@ -30,7 +30,7 @@ _FORWARD_OPERATORS = (_f._router_logits, _f._softmax_topk_fwd, _f._topk_fwd, _f.
                       _f._router_forward, _f._switch_loss_fwd)
 _BACKWARD_OPERATORS = (_b._down_projection_backward, _b._up_projection_backward, _b._token_broadcast_backward, _b._token_broadcast_backward_router,
                        _b._switch_loss_bwd, _b._router_logit_grad, _b._router_weight_grad, _b._sum_chunks)
-_BACKWARD_NAMES = elsewhere(*_BACKWARD_OPERATORS)
+_BACKWARD_NAMES = elsewhere(*_BACKWARD_OPERATORS) | _b.ROUTER_DX
 _ELEMENTS = (torch.bfloat16, torch.float16)
 
 
@@ -51,7 +51,7 @@ def _taken(rc: int, what: str) -> bool:
 
 
 def forward_names(routing_metadata) -> frozenset:
-    return elsewhere(*_FORWARD_OPERATORS, routing_metadata)
+    return elsewhere(*_FORWARD_OPERATORS, routing_metadata) | _f.ROUTER_LINEAR
 
 
 class Indices:
@@ -179,7 +179,7 @@ def backward(x, dout, z, w1, w2, b2, has_b1: bool, ints, freq, logits, K: int, a
         return None
     if not (x.is_contiguous() and z.is_contiguous() and ints.is_contiguous() and w1.stride(1) == 1 and w2.stride(1) == 1
             and (b2 is None or (b2.is_contiguous() and b2.data_ptr() != 0))
-            and (router_w is None or (router_w.is_contiguous() and router_w.data_ptr() != 0))
+            and (router_w is None or (router_w.is_contiguous() and router_w.data_ptr() != 0 and router_w.data_ptr() % 16 == 0))
             and (not loss or (freq.is_contiguous() and logits.stride(1) == 1))
             and all(t.data_ptr() != 0 for t in (x, dout, z, w1, w2, ints, *loss))
             and (outside is None or outside.data_ptr() != 0)):

@@ -194,19 +194,17 @@ def _on_gpus(monkeypatch, *numbers, current=0):
         return [torch.empty(rows, 128, dtype=torch.bfloat16, device=f"cuda:{n}") for rows, n in zip((8, 16), numbers)]
 
 
-@pytest.mark.filterwarnings("ignore:Accessing the data pointer")
 @pytest.mark.parametrize("gpus, current, taken", [((0, 0), 0, True), ((0, 1), 0, False), ((1, 0), 0, False), ((1, 1), 0, False),
                                                   ((1, 1), 1, True)])
 def test_kernels_in_the_place_of_torch_operations_stay_on_one_gpu(monkeypatch, gpus, current, taken):
     """F.linear refuses tensors of two GPUs and runs on theirs, not on the current one."""
     from sonicmoe._operator import stands_in, unobserved
-    from sonicmoe.functional.backward import _token_broadcast_backward_router, router_dx_takes
+    from sonicmoe.functional.backward import _token_broadcast_backward_router
     from sonicmoe.functional.forward import _router_logits
 
     x, w = _on_gpus(monkeypatch, *gpus, current=current)
     assert unobserved(frozenset(), x, None, w) == taken
     assert stands_in(frozenset(), x, w) == taken
-    assert router_dx_takes(x, w, x.dtype, 2) == taken
     if gpus[0] != gpus[1]:
         with pytest.raises(RuntimeError, match="one GPU"):
             _router_logits.body(x, w, x)
@@ -221,8 +219,9 @@ def test_tracers_keep_the_router_gemm(monkeypatch, tracer):
     from torch._functorch.aot_autograd import aot_function
     from torch.fx.experimental.proxy_tensor import make_fx
 
-    from sonicmoe.functional import moe_TC_softmax_topk_layer
-    from sonicmoe.functional.backward import router_dx_takes
+    from types import SimpleNamespace
+
+    from sonicmoe.functional import _dx_with_router, moe_TC_softmax_topk_layer
 
     def layer(x, wr, w1, w2):
         return moe_TC_softmax_topk_layer(x, wr, w1.permute(1, 2, 0), None, w2.permute(1, 2, 0), None, 2, 0)
@@ -232,7 +231,7 @@ def test_tracers_keep_the_router_gemm(monkeypatch, tracer):
     graphs = []
     with FakeTensorMode(), torch.no_grad():
         args = [torch.empty(s, dtype=torch.bfloat16, device="cuda:0") for s in ((T, H), (E, H), (E, 2 * I, H), (E, H, I))]
-        assert not router_dx_takes(args[0], args[1], torch.bfloat16, 2)
+        assert not _dx_with_router(SimpleNamespace(needs_input_grad=(True,)), args[0], args[1], torch.bfloat16, 2)
         if tracer == "aot_function":
             got = aot_function(layer, fw_compiler=lambda gm, _: (graphs.append(gm), gm)[1])(*args)
         elif tracer == "make_fx":
@@ -246,22 +245,21 @@ def test_tracers_keep_the_router_gemm(monkeypatch, tracer):
         assert "aten.mm.default" in called and not any("_router_logits" in t for t in called)
 
 
-@pytest.mark.filterwarnings("ignore:Accessing the data pointer")
 @pytest.mark.filterwarnings("ignore:Warning only once for all operators")
 @pytest.mark.parametrize("name, linear, dx", [("aten::mm", False, True), ("aten::linear", False, True), ("aten::addmm_", True, False),
                                               ("aten::addmm.out", True, False), ("aten::tanh", True, True),
                                               ("sonicmoe::_token_broadcast_backward", True, False)])
 def test_implementations_registered_for_what_a_kernel_stands_in_for_are_called(monkeypatch, name, linear, dx):
-    from sonicmoe._operator import stands_in
-    from sonicmoe.functional.backward import router_dx_takes
-    from sonicmoe.functional.forward import _LINEAR, router_logits_takes
+    from sonicmoe._operator import stands_in, unobserved
+    from sonicmoe.functional import _ONE_CALL_NAMES, ROUTER_DX, layer_call
+    from sonicmoe.functional.forward import ROUTER_LINEAR
 
     x, w = _on_gpus(monkeypatch, 0, 0)
     with torch.library._scoped_library(name.split("::")[0], "IMPL") as lib:
         lib.impl(name.split("::")[1], lambda *args, **kwargs: pytest.fail("called"), "CUDA")
-        assert router_logits_takes(x, w) == stands_in(_LINEAR, x, w) == linear
-        assert router_dx_takes(x, w, x.dtype, 2) == dx
-    assert router_logits_takes(x, w) and router_dx_takes(x, w, x.dtype, 2)
+        assert stands_in(ROUTER_LINEAR, x, w) == linear and stands_in(ROUTER_DX, x, w) == dx
+        assert unobserved(_ONE_CALL_NAMES, x, w) == linear and unobserved(layer_call._BACKWARD_NAMES, x, w) == dx
+    assert stands_in(ROUTER_LINEAR, x, w) and stands_in(ROUTER_DX, x, w)
 
 
 def test_a_function_in_the_place_of_the_reduction_is_called(monkeypatch):
@@ -270,10 +268,11 @@ def test_a_function_in_the_place_of_the_reduction_is_called(monkeypatch):
     from sonicmoe import functional
 
     ctx = SimpleNamespace(needs_input_grad=(True,))
-    monkeypatch.setattr(functional, "router_dx_takes", lambda *args: True)
-    assert functional._dx_with_router(ctx, None, None, None, 2)
+    monkeypatch.setattr(functional, "stands_in", lambda *args: True)
+    x, w = torch.empty(8, 64, dtype=torch.bfloat16), torch.empty(16, 64, dtype=torch.bfloat16)
+    assert functional._dx_with_router(ctx, x, w, x.dtype, 2)
     monkeypatch.setattr(functional, "_token_broadcast_backward", lambda *args: None)
-    assert not functional._dx_with_router(ctx, None, None, None, 2)
+    assert not functional._dx_with_router(ctx, x, w, x.dtype, 2)
 
 
 @pytest.mark.parametrize("T, H, E, taken", [
@@ -287,15 +286,10 @@ def test_sizes_of_the_router_kernel(T, H, E, taken):
     assert router_logits_takes(x, w) == taken
 
 
-@pytest.mark.filterwarnings("ignore:Accessing the data pointer")
 @pytest.mark.parametrize("E, K, taken", [(8, 1, True), (128, 16, True), (136, 16, False), (256, 8, True), (512, 4, True),
                                          (512, 5, False), (520, 1, False), (8, 17, False), (12, 2, False)])
-def test_sizes_of_the_dx_kernel(monkeypatch, E, K, taken):
-    from sonicmoe import _operator
+def test_sizes_of_the_dx_kernel(E, K, taken):
     from sonicmoe.functional.backward import router_dx_takes
 
-    monkeypatch.setattr(_operator, "_TENSORS", (FakeTensor,))
-    monkeypatch.setattr(_lib, "current_gpu", lambda: 0)
-    with FakeTensorMode():
-        x, w = (torch.empty(n, 128, dtype=torch.bfloat16, device="cuda:0") for n in (8, E))
+    x, w = (torch.empty(n, 128, dtype=torch.bfloat16, device="meta") for n in (8, E))
     assert router_dx_takes(x, w, x.dtype, K) == taken
