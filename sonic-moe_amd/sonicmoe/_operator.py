@@ -9,6 +9,7 @@ An ExecutionTraceObserver without a profiler around it gives no sign of itself: 
 from __future__ import annotations
 
 import torch
+from torch.fx.experimental.proxy_tensor import get_proxy_mode
 
 from . import _lib
 from ._lib import NoMemory
@@ -67,6 +68,16 @@ def untraced() -> bool:
         and torch._C._functorch.peek_interpreter_stack() is None  # vmap, grad, functionalization
         and not torch._C._is_torch_function_mode_enabled()
         and torch._C._get_tracing_state() is None  # torch.jit.trace
+    )
+
+
+def untransformed() -> bool:
+    """Whether torch calls do what they say, whoever looks on: no vmap, grad or functionalization around them and no trace being
+    recorded.  For eager code only."""
+    return (
+        torch._C._functorch.peek_interpreter_stack() is None
+        and torch._C._get_tracing_state() is None
+        and (torch._C._len_torch_dispatch_stack() == 0 or get_proxy_mode() is None)
     )
 
 

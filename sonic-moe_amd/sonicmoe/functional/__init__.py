@@ -18,7 +18,7 @@ import torch.nn.functional as F
 
 from .. import _lib
 from ..count_cumsum import count_cumsum
-from .._operator import operator, run, stands_in
+from .._operator import operator, run, stands_in, unobserved
 from ..enums import ActivationType, is_glu
 from .backward import (
     ROUTER_DX,
@@ -559,16 +559,38 @@ def _tc_layer_backward(ctx, dout, dlogits_outside, x, router_w, w1, w2, b2, z, s
     return dx, dwr, dw1, db1, dw2, db2, None, None, None, None
 
 
+def _forward_by_operators(x, router_w, w1, b1, w2, b2, K, activation_type, stream_id, with_loss):
+    """layer_call.forward operator by operator"""
+    T, E = x.size(0), router_w.size(0)
+    logits = router_linear(x, router_w)
+    where = layer_call.Indices(T, E, K)
+    ints = torch.empty(where.words, dtype=torch.int32, device=x.device)
+    scores, indices, gidx, sidx, ridx, off, tok_off, acc = where.views(ints)
+    freq = torch.empty(E, dtype=torch.int32, device=x.device)
+    run(_softmax_topk_fwd, logits, scores, indices, E, K)
+    run(_routing_metadata, indices.view(-1), None, T, K, freq, off, gidx, sidx, ridx, tok_off)
+    o, z = _experts_forward(x, w1, b1, w2, b2, scores.view(-1), off, gidx, ridx, tok_off, K, False, activation_type, stream_id,
+                            False)
+    loss = None
+    if with_loss:
+        loss = torch.empty((), dtype=torch.float32, device=x.device)
+        run(_switch_loss_fwd, logits, freq, acc, loss.view(1))
+    return o, logits, z, freq, ints, loss
+
+
 class _OneCallLayerFunction(torch.autograd.Function):
     """_TCLayerFunction whose operators behind the router GEMM run as one call of the library per direction
-    (layer_call.py), with the load-balancing loss as a fourth output if `with_loss`."""
+    (layer_call.py) unless somebody looks on, with the load-balancing loss as a fourth output if `with_loss`."""
 
     @staticmethod
     def forward(ctx, x, router_w, w1, b1, w2, b2, K: int, activation_type: ActivationType, stream_id: int, with_loss: bool):
         x = x.contiguous()
-        done = layer_call.forward(x, router_w, w1, b1, w2, b2, K, activation_type, stream_id, True, with_loss)
-        if done is None:
-            raise layer_call.Refused
+        if unobserved(_ONE_CALL_NAMES):
+            done = layer_call.forward(x, router_w, w1, b1, w2, b2, K, activation_type, stream_id, True, with_loss)
+            if done is None:
+                raise layer_call.Refused
+        else:
+            done = _forward_by_operators(x, router_w, w1, b1, w2, b2, K, activation_type, stream_id, with_loss)
         o, logits, z, freq, ints, loss = done
         # the counts and the logits belong to the caller, who may change them in place: they are kept only for the loss, which
         # is formed from them (as switch_loss keeps them)
@@ -705,14 +727,17 @@ def layer_with_loss(x, router_w, w1, b1, w2, b2, K: int, stream_id: int, activat
         and _SCHEDULE_POLICY == "expert_index"
         and (_softmax_topk_fwd, _routing_metadata, _up_projection_forward, _down_projection_forward, _router_forward,
              _switch_loss_fwd) == _ONE_CALL_OPERATORS
-        and layer_call.takes(x, router_w, w1, b1, w2, b2, K, activation_type, stream_id, _ONE_CALL_NAMES)
+        and layer_call.takes(x, router_w, w1, b1, w2, b2, K, activation_type, stream_id)
         and os.environ.get("SMOE_FUSED_TC_LAYER", "1") != "0"
     ):
         needs_grad = torch.is_grad_enabled() and (
             x.requires_grad or router_w.requires_grad or w1.requires_grad or w2.requires_grad
             or (b1 is not None and (b1.requires_grad or b2.requires_grad)))
         if not needs_grad:
-            done = layer_call.forward(x.contiguous(), router_w, w1, b1, w2, b2, K, activation_type, stream_id, False, with_loss)
+            done = None
+            if unobserved(_ONE_CALL_NAMES):
+                done = layer_call.forward(x.contiguous(), router_w, w1, b1, w2, b2, K, activation_type, stream_id, False,
+                                          with_loss)
             if done is not None:
                 return done[0], done[1], done[3], done[5]
         elif not is_inference_mode_enabled:

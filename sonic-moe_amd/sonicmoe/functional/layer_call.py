@@ -1,9 +1,10 @@
 """The token-choice layer behind (of few tokens: with) its router GEMM as one call of the HIP library per direction (smoe_layer_forward /
 smoe_layer_backward: the operators' entry points in the operators' order, so the same kernels and the same results).
 
-For the common case only: plain 16-bit tensors of one type, nobody looking on the operators, no autocast, no tensor of a
-forward-mode derivative, memory as the operators want it.  Whatever is not like that -- and whatever the library refuses --
-takes the operators one by one, which say what is wrong with it.
+For the common case only: plain 16-bit tensors of one type, no autocast, no tensor of a forward-mode derivative, memory as the
+operators want it (`takes`).  Whatever is not like that -- and whatever the library refuses -- takes the operators one by one,
+which say what is wrong with it.  So does a call that somebody looks on (`unobserved`); what it keeps for its backward pass is
+the same, because who looks on may come and go between a forward pass and its recomputation from a checkpoint.
 """
 
 from __future__ import annotations
@@ -14,7 +15,7 @@ import torch
 from torch.autograd import forward_ad
 
 from .. import _lib
-from .._operator import elsewhere, unobserved
+from .._operator import elsewhere, in_memory, unobserved, untransformed
 from ..enums import ACTIVATION_CODE, is_glu
 from . import backward as _b
 from . import forward as _f
@@ -76,11 +77,12 @@ class Indices:
                 acc.view(torch.float32))
 
 
-def takes(x, router_w, w1, b1, w2, b2, K: int, activation, stream_id: int, names: frozenset) -> bool:
-    """Whether `forward` takes this layer.  (Sizes that the kernels refuse are told by the library.)"""
+def takes(x, router_w, w1, b1, w2, b2, K: int, activation, stream_id: int) -> bool:
+    """Whether `forward` takes this layer if it is `unobserved`.  (Sizes that the kernels refuse are told by the library.)"""
     dtype = x.dtype
     if not (
-        unobserved(names, x, router_w, w1, b1, w2, b2)
+        untransformed()
+        and in_memory(x, router_w, w1, b1, w2, b2)
         and dtype in _ELEMENTS
         and router_w.dtype == dtype and w1.dtype == dtype and w2.dtype == dtype
         and x.dim() == 2 and router_w.dim() == 2 and w1.dim() == 3 and w2.dim() == 3

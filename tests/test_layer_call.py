@@ -352,6 +352,52 @@ def test_module_gradient_of_one_output(dev, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("observer", ["nobody", "profiler", "flop counter", "implementation"])
+@pytest.mark.parametrize("act, bias", [("swiglu", False), ("gelu", True)])
+def test_recomputed_while_somebody_looks_on(dev, observer, act, bias):
+    """A checkpoint compares what a forward pass keeps with what its recomputation does; who looks on may have come since."""
+    from contextlib import ExitStack
+
+    from torch.utils.checkpoint import checkpoint
+    from torch.utils.flop_counter import FlopCounterMode
+
+    moe, x, dy = _module(300, 256, 128, 24, 4, act, bias, torch.bfloat16, dev)
+    called = []
+
+    def loss(own):
+        with torch.no_grad():
+            called.append(True)
+            from sonicmoe.functional.forward import _switch_loss_fwd
+
+            _switch_loss_fwd.body(*own)
+
+    def step(observer):
+        xx = x.clone().requires_grad_()
+        out, aux = checkpoint(moe, xx, use_reentrant=False)
+        with ExitStack() as scope:
+            if observer == "profiler":
+                profile = scope.enter_context(torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]))
+            elif observer == "flop counter":
+                scope.enter_context(FlopCounterMode(display=False))
+            elif observer == "implementation":
+                scope.enter_context(torch.library._scoped_library("sonicmoe", "IMPL")).impl(
+                    "_switch_loss_fwd", lambda *own: loss(own), "CUDA")
+            moe.zero_grad()  # (the flop counter's hooks do not run under autograd.grad)
+            torch.autograd.backward([out, aux], [dy, torch.tensor(0.3, device=dev)])
+        if observer == "profiler":
+            rows = {e.key for e in profile.key_averages()}
+            assert {"sonicmoe::_routing_metadata", "sonicmoe::_up_projection_forward", "sonicmoe::_switch_loss_fwd"} <= rows
+        return [out.detach(), aux.detach(), xx.grad, *[p.grad.clone() for p in moe.parameters()]]
+
+    for i, (a, b) in enumerate(zip(step("nobody"), step(observer))):
+        if (i, observer) == (2, "flop counter"):  # dx: a mode sees the addition onto it, a second rounding of half an eps
+            assert (a - b).float().norm() <= 1.5 * torch.finfo(a.dtype).eps * a.float().norm()
+        else:
+            assert torch.equal(a, b)
+    assert bool(called) == (observer == "implementation")
+
+
+@pytest.mark.gpu
 def test_what_is_left_to_the_operators(dev, monkeypatch):
     """Profilers, autocast, another stream, forward-mode derivatives, odd sizes: as operator by operator, errors included."""
     from sonicmoe.functional import layer_call, moe_TC_softmax_topk_layer
