@@ -56,6 +56,11 @@ def torch_elsewhere(*names: str) -> frozenset:
     return _names("aten", *names)
 
 
+def on_gpu(names: frozenset) -> frozenset:
+    """Those of the names that matter for tensors on a GPU (each costs some 25 ns per question)."""
+    return frozenset(name for name in names if not name.endswith("CPU"))
+
+
 def registered(names: frozenset) -> bool:
     """Whether somebody has registered an implementation under one of these names (or nobody can say)."""
     return _REGISTERED is None or not _REGISTERED.isdisjoint(names)

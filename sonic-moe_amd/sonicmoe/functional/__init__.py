@@ -583,9 +583,10 @@ class _OneCallLayerFunction(torch.autograd.Function):
     (layer_call.py) unless somebody looks on, with the load-balancing loss as a fourth output if `with_loss`."""
 
     @staticmethod
-    def forward(ctx, x, router_w, w1, b1, w2, b2, K: int, activation_type: ActivationType, stream_id: int, with_loss: bool):
+    def forward(ctx, x, router_w, w1, b1, w2, b2, K: int, activation_type: ActivationType, stream_id: int, with_loss: bool,
+                quiet: bool):
         x = x.contiguous()
-        if unobserved(_ONE_CALL_NAMES):
+        if quiet:
             done = layer_call.forward(x, router_w, w1, b1, w2, b2, K, activation_type, stream_id, True, with_loss)
             if done is None:
                 raise layer_call.Refused
@@ -624,14 +625,14 @@ class _OneCallLayerFunction(torch.autograd.Function):
                 dx = None
             elif not with_router:
                 dx.addmm_(dlogits, router_w)
-            return dx, dwr, dw1, db1, dw2, db2, None, None, None, None
+            return dx, dwr, dw1, db1, dw2, db2, None, None, None, None, None
         scores, indices, gidx, sidx, ridx, off, tok_off, acc = layer_call.Indices(T, E, K).views(ints)
         if daux is not None:
             dlogits = torch.empty_like(logits, memory_format=torch.contiguous_format)
             run(_switch_loss_bwd, logits, freq, acc, daux.reshape(1).float().contiguous(), dlogits)
             dlogits_outside = dlogits if dlogits_outside is None else dlogits + dlogits_outside  # (which may be sparse)
-        return _tc_layer_backward(ctx, dout, dlogits_outside, x, router_w, w1, w2, b2, z, scores, indices, off, gidx, sidx, ridx,
-                                  tok_off, K, activation_type, stream_id, x.dtype, has_b1, None, False)
+        return *_tc_layer_backward(ctx, dout, dlogits_outside, x, router_w, w1, w2, b2, z, scores, indices, off, gidx, sidx,
+                                   ridx, tok_off, K, activation_type, stream_id, x.dtype, has_b1, None, False), None
 
 
 class _SwitchLossFunction(torch.autograd.Function):
@@ -721,13 +722,15 @@ def layer_with_loss(x, router_w, w1, b1, w2, b2, K: int, stream_id: int, activat
     it is not asked for, and where the layer runs operator by operator: switch_loss computes it from the other two."""
     b1, b2 = _check_bias(b1, b2)
     activation_type = _as_activation(activation_type)
+    compiling = torch.compiler.is_compiling()
+    quiet = not compiling and unobserved(_ONE_CALL_NAMES)
     if (
-        not torch.compiler.is_compiling()
+        not compiling
         and not (_FUSED_ROUTER or _FUSED_COMBINE or is_using_fp8_forward() or is_using_fp8_backward())
         and _SCHEDULE_POLICY == "expert_index"
         and (_softmax_topk_fwd, _routing_metadata, _up_projection_forward, _down_projection_forward, _router_forward,
              _switch_loss_fwd) == _ONE_CALL_OPERATORS
-        and layer_call.takes(x, router_w, w1, b1, w2, b2, K, activation_type, stream_id)
+        and layer_call.takes(x, router_w, w1, b1, w2, b2, K, activation_type, stream_id, quiet)
         and os.environ.get("SMOE_FUSED_TC_LAYER", "1") != "0"
     ):
         needs_grad = torch.is_grad_enabled() and (
@@ -735,14 +738,14 @@ def layer_with_loss(x, router_w, w1, b1, w2, b2, K: int, stream_id: int, activat
             or (b1 is not None and (b1.requires_grad or b2.requires_grad)))
         if not needs_grad:
             done = None
-            if unobserved(_ONE_CALL_NAMES):
+            if quiet:
                 done = layer_call.forward(x.contiguous(), router_w, w1, b1, w2, b2, K, activation_type, stream_id, False,
                                           with_loss)
             if done is not None:
                 return done[0], done[1], done[3], done[5]
         elif not is_inference_mode_enabled:
             try:
-                return _OneCallLayerFunction.apply(x, router_w, w1, b1, w2, b2, K, activation_type, stream_id, with_loss)
+                return _OneCallLayerFunction.apply(x, router_w, w1, b1, w2, b2, K, activation_type, stream_id, with_loss, quiet)
             except layer_call.Refused:
                 pass
     if os.environ.get("SMOE_FUSED_TC_LAYER", "1") == "0":  # the layer as three autograd nodes, as the reference builds it

@@ -7,7 +7,7 @@ from typing import Optional
 import torch
 
 from .. import _lib
-from .._operator import elsewhere, operator, torch_elsewhere
+from .._operator import elsewhere, on_gpu, operator, torch_elsewhere
 from ..enums import ACTIVATION_CODE, ActivationType
 from ..utils import expert_major_strides
 from .forward import _check_schedule_order, _elem_dtype, _gather_sum, _gemm_workspace
@@ -223,7 +223,7 @@ def _token_broadcast_backward_router(
 
 
 # what `_token_broadcast_backward_router` stands in for
-ROUTER_DX = elsewhere(_token_broadcast_backward) | torch_elsewhere("addmm_", "addmm", "addmm.out")
+ROUTER_DX = on_gpu(elsewhere(_token_broadcast_backward) | torch_elsewhere("addmm_", "addmm", "addmm.out"))
 
 # Where dx is formed by `_token_broadcast_backward_router` and not by the reduction and addmm_ (20 us of host time).  Its
 # workgroups read all of the router's weights and add a token's K rows in batches of eight, so the line is by E and E K.

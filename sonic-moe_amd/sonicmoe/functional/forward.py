@@ -9,7 +9,7 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
-from .._operator import operator, run, stands_in, torch_elsewhere
+from .._operator import on_gpu, operator, run, stands_in, torch_elsewhere
 from ..enums import ACTIVATION_CODE, ActivationType
 from ..utils import expert_major_strides
 
@@ -357,7 +357,7 @@ def _router_logits_pays(T: int, H: int, E: int) -> bool:
 
 
 # what `_router_logits` stands in for
-ROUTER_LINEAR = torch_elsewhere("linear", "matmul", "mm")
+ROUTER_LINEAR = on_gpu(torch_elsewhere("linear", "matmul", "mm"))
 
 
 def router_logits_takes(x: torch.Tensor, router_w: torch.Tensor) -> bool:

@@ -15,7 +15,7 @@ import torch
 from torch.autograd import forward_ad
 
 from .. import _lib
-from .._operator import elsewhere, in_memory, unobserved, untransformed
+from .._operator import elsewhere, in_memory, on_gpu, unobserved, untransformed
 from ..enums import ACTIVATION_CODE, is_glu
 from . import backward as _b
 from . import forward as _f
@@ -31,7 +31,7 @@ _FORWARD_OPERATORS = (_f._router_logits, _f._softmax_topk_fwd, _f._topk_fwd, _f.
                       _f._router_forward, _f._switch_loss_fwd)
 _BACKWARD_OPERATORS = (_b._down_projection_backward, _b._up_projection_backward, _b._token_broadcast_backward, _b._token_broadcast_backward_router,
                        _b._switch_loss_bwd, _b._router_logit_grad, _b._router_weight_grad, _b._sum_chunks)
-_BACKWARD_NAMES = elsewhere(*_BACKWARD_OPERATORS) | _b.ROUTER_DX
+_BACKWARD_NAMES = on_gpu(elsewhere(*_BACKWARD_OPERATORS)) | _b.ROUTER_DX
 _ELEMENTS = (torch.bfloat16, torch.float16)
 
 
@@ -52,7 +52,7 @@ def _taken(rc: int, what: str) -> bool:
 
 
 def forward_names(routing_metadata) -> frozenset:
-    return elsewhere(*_FORWARD_OPERATORS, routing_metadata) | _f.ROUTER_LINEAR
+    return on_gpu(elsewhere(*_FORWARD_OPERATORS, routing_metadata)) | _f.ROUTER_LINEAR
 
 
 class Indices:
@@ -77,11 +77,12 @@ class Indices:
                 acc.view(torch.float32))
 
 
-def takes(x, router_w, w1, b1, w2, b2, K: int, activation, stream_id: int) -> bool:
-    """Whether `forward` takes this layer if it is `unobserved`.  (Sizes that the kernels refuse are told by the library.)"""
+def takes(x, router_w, w1, b1, w2, b2, K: int, activation, stream_id: int, quiet: bool) -> bool:
+    """Whether `forward` takes this layer; if not `quiet`, whether it would, were the operators `unobserved`.  (Sizes that the
+    kernels refuse are told by the library.)"""
     dtype = x.dtype
     if not (
-        untransformed()
+        (quiet or untransformed())
         and in_memory(x, router_w, w1, b1, w2, b2)
         and dtype in _ELEMENTS
         and router_w.dtype == dtype and w1.dtype == dtype and w2.dtype == dtype
@@ -179,12 +180,18 @@ def backward(x, dout, z, w1, w2, b2, has_b1: bool, ints, freq, logits, K: int, a
             and (not loss or (freq.dtype == torch.int32 and freq.shape == (E,) and logits.dtype == dtype
                               and logits.shape == (T, E)))):
         return None
-    if not (x.is_contiguous() and z.is_contiguous() and ints.is_contiguous() and w1.stride(1) == 1 and w2.stride(1) == 1
-            and (b2 is None or (b2.is_contiguous() and b2.data_ptr() != 0))
-            and (router_w is None or (router_w.is_contiguous() and router_w.data_ptr() != 0 and router_w.data_ptr() % 16 == 0))
-            and (not loss or (freq.is_contiguous() and logits.stride(1) == 1))
-            and all(t.data_ptr() != 0 for t in (x, dout, z, w1, w2, ints, *loss))
-            and (outside is None or outside.data_ptr() != 0)):
+    s1, s2 = w1.stride(), w2.stride()
+    if not (x.is_contiguous() and z.is_contiguous() and ints.is_contiguous() and s1[1] == 1 and s2[1] == 1
+            and (b2 is None or b2.is_contiguous()) and (router_w is None or router_w.is_contiguous())
+            and (not loss or (freq.is_contiguous() and logits.stride(1) == 1))):
+        return None
+    p_x, p_dout, p_z, p_w1, p_w2, base = given = (x.data_ptr(), dout.data_ptr(), z.data_ptr(), w1.data_ptr(), w2.data_ptr(),
+                                                  ints.data_ptr())
+    p_b2, p_outside, p_router = [0 if t is None else t.data_ptr() for t in (b2, outside, router_w)]
+    p_loss, p_freq, p_logits = (loss_grad.data_ptr(), freq.data_ptr(), logits.data_ptr()) if loss else (0, 0, 0)
+    # (null means "not given", of router_w that the caller adds its share; the dx kernel wants it aligned)
+    if (0 in given or (loss and 0 in (p_loss, p_freq, p_logits)) or (p_b2 == 0) != (b2 is None)
+            or (p_outside == 0) != (outside is None) or (p_router == 0) != (router_w is None) or p_router % 16 != 0):
         return None
     L = _lib.lib(dtype)
     code, dev = ACTIVATION_CODE[activation], x.device
@@ -198,22 +205,18 @@ def backward(x, dout, z, w1, w2, b2, has_b1: bool, ints, freq, logits, K: int, a
     dlogits = torch.empty(T, E, dtype=dtype, device=dev)
     dwr = torch.empty(E, H, dtype=dtype, device=dev) if chunks else None
     scratch = torch.empty(need, dtype=torch.uint8, device=dev)
-    s1, s2, d1, d2 = w1.stride(), w2.stride(), dw1.stride(), dw2.stride()
+    d1, d2, at = dw1.stride(), dw2.stride(), where.at
     if d1[1] != 1 or d2[1] != 1:
         return None
-    base, at = ints.data_ptr(), where.at
     rc = L.smoe_layer_backward(
         _BACKWARD.pack(
-            x.data_ptr(), dout.data_ptr(), z.data_ptr(), w1.data_ptr(), w2.data_ptr(), 0 if b2 is None else b2.data_ptr(),
-            s1[2], s1[0], s2[2], s2[0],
-            base, base + 4 * at[1], freq.data_ptr() if loss else 0, base + 4 * at[5], base + 4 * at[2], base + 4 * at[3],
-            base + 4 * at[4], logits.data_ptr() if loss else 0, _lib.DT_CODE[dtype], logits.stride(0) if loss else 0,
-            base + 4 * at[7], loss_grad.data_ptr() if loss else 0, 0 if outside is None else outside.data_ptr(),
-            0 if outside is None else outside.stride(0), T, H, I, E, K, code,
+            p_x, p_dout, p_z, p_w1, p_w2, p_b2, s1[2], s1[0], s2[2], s2[0],
+            base, base + 4 * at[1], p_freq, base + 4 * at[5], base + 4 * at[2], base + 4 * at[3], base + 4 * at[4],
+            p_logits, _lib.DT_CODE[dtype], logits.stride(0) if loss else 0, base + 4 * at[7], p_loss,
+            p_outside, 0 if outside is None else outside.stride(0), T, H, I, E, K, code,
             dw1.data_ptr(), dw2.data_ptr(), d1[2], d1[0], d2[2], d2[0],
             0 if db1 is None else db1.data_ptr(), 0 if db2 is None else db2.data_ptr(), dx.data_ptr(), dlogits.data_ptr(),
-            0 if router_w is None else router_w.data_ptr(),
-            0 if dwr is None else dwr.data_ptr(), chunks, scratch.data_ptr(), need,
+            p_router, 0 if dwr is None else dwr.data_ptr(), chunks, scratch.data_ptr(), need,
         ),
         stream_id,
     )

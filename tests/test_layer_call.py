@@ -174,7 +174,7 @@ def test_gradients_of_the_loss_and_of_the_logits_add_up(monkeypatch, sparse):
     seen = []
     monkeypatch.setattr(functional, "run", lambda op, *args: args[-1].fill_(3.0))
     monkeypatch.setattr(functional.layer_call, "backward", lambda *a: None)
-    monkeypatch.setattr(functional, "_tc_layer_backward", lambda ctx, dout, dlogits, *a: seen.append(dlogits))
+    monkeypatch.setattr(functional, "_tc_layer_backward", lambda ctx, dout, dlogits, *a: seen.append(dlogits) or ())
     ints = torch.zeros(functional.layer_call.Indices(T, E, K).words, dtype=torch.int32)
     ctx = SimpleNamespace(cfg=(K, ActivationType.SWIGLU, 0, False), needs_input_grad=(True,) * 6, saved_tensors=(
         torch.zeros(T, H), torch.zeros(E, H), None, torch.zeros(H, I, E), None, None, ints, torch.zeros(E, dtype=torch.int32),
