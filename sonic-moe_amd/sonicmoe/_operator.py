@@ -77,8 +77,8 @@ def untraced() -> bool:
 
 
 def untransformed() -> bool:
-    """Whether torch calls do what they say, whoever looks on: no vmap, grad or functionalization around them and no trace being
-    recorded.  For eager code only."""
+    """Whether torch calls do what they say, whoever looks on: no vmap, grad or functionalization around them and no trace
+    being recorded.  For eager code only."""
     return (
         torch._C._functorch.peek_interpreter_stack() is None
         and torch._C._get_tracing_state() is None
@@ -109,8 +109,8 @@ def unobserved(names: frozenset, *tensors) -> bool:
 
 
 def stands_in(replaced: frozenset, *tensors) -> bool:
-    """Whether an operator may stand in for the operations behind `replaced` (`elsewhere`, `torch_elsewhere`) on these tensors:
-    whoever traces or transforms torch calls keeps them, and can see through them, as does who has registered an
+    """Whether an operator may stand in for the operations behind `replaced` (`elsewhere`, `torch_elsewhere`) on these
+    tensors: whoever traces or transforms torch calls keeps them, and can see through them, as does who has registered an
     implementation of one; and so do tensors without an address to ask for.  (Profilers see the operator.)"""
     return not torch.compiler.is_compiling() and untraced() and not registered(replaced) and in_memory(*tensors)
 

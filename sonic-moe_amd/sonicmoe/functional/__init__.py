@@ -18,7 +18,7 @@ import torch.nn.functional as F
 
 from .. import _lib
 from ..count_cumsum import count_cumsum
-from .._operator import operator, run, stands_in, unobserved
+from .._operator import in_memory, operator, run, stands_in, unobserved
 from ..enums import ActivationType, is_glu
 from .backward import (
     ROUTER_DX,
@@ -612,7 +612,8 @@ class _OneCallLayerFunction(torch.autograd.Function):
         fast_router = ctx.needs_input_grad[1] and _router_wgrad_takes(x.dtype, E, x)  # (the logits have x's type)
         chunks = router_weight_grad_chunks(T, E, H) if fast_router else 0
         done = None
-        with_router = ctx.needs_input_grad[0] and router_dx_takes(x, router_w, x.dtype, K)
+        with_router = (ctx.needs_input_grad[0] and router_dx_takes(x, router_w, x.dtype, K) and in_memory(router_w)
+                       and router_w.data_ptr() % 16 == 0)
         if (_down_projection_backward, _up_projection_backward, _token_broadcast_backward, _token_broadcast_backward_router,
                 _switch_loss_bwd, _router_logit_grad, _router_weight_grad, _sum_chunks) == layer_call._BACKWARD_OPERATORS:
             done = layer_call.backward(x, dout, z, w1, w2, b2, has_b1, ints, freq, logits, K, activation_type, stream_id, daux,
@@ -719,7 +720,7 @@ _ONE_CALL_OPERATORS = (_softmax_topk_fwd, _routing_metadata, _up_projection_forw
 def layer_with_loss(x, router_w, w1, b1, w2, b2, K: int, stream_id: int, activation_type, is_inference_mode_enabled: bool,
                     with_loss: bool):
     """moe_TC_softmax_topk_layer, and its load-balancing loss: (o, router_logits, expert_frequency, loss).  loss is None where
-    it is not asked for, and where the layer runs operator by operator: switch_loss computes it from the other two."""
+    it is not asked for, and where `layer_call.takes` does not take the layer: switch_loss computes it from the other two."""
     b1, b2 = _check_bias(b1, b2)
     activation_type = _as_activation(activation_type)
     compiling = torch.compiler.is_compiling()
